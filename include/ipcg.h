@@ -474,7 +474,9 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
 /* work counts of the last calls, by name: "ccd.candidates" (swept
  * candidates of the last CCD), "ccd.searched" (those whose root box
  * includes the origin), "ccd.spilled" (searches that outgrew the LDS
- * lists), "ccd.wavefront" (searches that outgrew a lane's HBM slab),
+ * lists), "ccd.wavefront" (searches that outgrew a workgroup's lists),
+ * "ccd.unmet" (1 when an expected minimum did not stand and the searches
+ * ran again without it),
  * "hessian.ee_other" (edge-edge collisions of the last Hessian whose type
  * is not the interior one; their projection takes the 9 x 9 path),
  * "hessian.pattern_sorted" (1 when a row of the last Hessian pattern had

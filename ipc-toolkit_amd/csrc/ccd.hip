@@ -3,14 +3,18 @@
 // (tight_inclusion_ccd.cpp:33-336) and the step-size minimum
 // (candidates.cpp:252-292).
 //
-// Three tiers share one device restatement of the algorithm (ti.hpp):
+// Tiers, all with one restatement of the algorithm (ti.hpp):
 //  * LDS tier: one lane per candidate that survived the root pass, its level
 //    lists in LDS (LDS_CAP packed boxes per list).  Almost every candidate
 //    resolves here within a few levels.
-//  * slab tier, for searches that outgrew the LDS lists: persistent lanes
-//    pull candidates from an atomic counter and run the whole breadth-first
-//    search in a private 3 x LANE_CAP box slab in HBM.
-//  * wavefront path, for candidates whose levels outgrow the slab: all of
+//  * sub-wave tier, for searches that outgrew the LDS lists: SUB_W lanes per
+//    search, lists of SUB_CAP boxes.
+//  * group tiers, for searches that outgrew those: a wave per search
+//    with lists of WAVE_CAP, then WIDE_CAP boxes, then a workgroup per
+//    search with lists of BLOCK_CAP boxes in LDS, then SLAB_CAP boxes in
+//    HBM.  Persistent groups pull searches from an atomic counter.
+//    Short lists skip the tiers that need many searches to pay off.
+//  * wavefront path, for candidates whose levels outgrow those too: all of
 //    them advance one level per round of short kernels.  Every box of the
 //    level is evaluated by its own lane (the inclusion test is the work),
 //    the sequential per-level rules are resolved from each candidate's first
@@ -18,6 +22,17 @@
 //    level), children are emitted through a scan and each candidate's next
 //    level is ordered (a merge of the lower / upper t halves, a lane per
 //    box).
+// Expected minimum: a search that outgrows a group's lists goes on with the
+// earliest boxes only (ti_bfs_group's beam); a hit found so bounds its
+// outcome from above.  The smallest such bound of a scene hides boxes at or
+// after it like the running minimum does, so the searches that follow stay
+// small: nearly parallel edges reach hundreds of thousands of boxes a level
+// in an unbounded search and a few thousand below this one.  When no
+// outcome below it turns up, the bound is the minimum itself: the search it
+// came from ends at or before it, and not before it.  That holds for
+// first-stage outcomes; where a first stage ended below SMALL_TOI (the
+// search restarts and may end anywhere) and nothing below the expected
+// minimum was reported, everything is searched again without it.
 // The running minimum lives in device memory as the bit pattern of a
 // non-negative double (unsigned atomic min); every search hides outcomes at
 // or above it, which leaves the final minimum independent of scheduling.
@@ -27,7 +42,8 @@
 #include "ti.hpp"
 
 #include <algorithm>
-#include <mutex>
+#include <cmath>
+#include <cstring>
 
 namespace ipcg {
 
@@ -35,8 +51,32 @@ namespace {
 
 constexpr int CB = 64;
 constexpr int LDS_CAP = 6;
-constexpr int LANE_CAP = 256;
-constexpr int LANES = 131072; // 8 waves per CU at this kernel's register use
+// Tiers above the LDS lists.  Their searches are chains of ~40 dependent
+// levels of a few boxes (median 5 a level on nearly parallel sheets, 18,000
+// at most below the expected minimum), so each tier gives a search the lanes
+// its levels fill.  Two 64 x 64 sheets (120 K searches, 30 K of them past
+// the LDS lists): 24 ms with one lane per search over HBM lists and the
+// wavefront for the rest, 1.6 ms with these tiers; two 8 x 8 sheets 17.3 ->
+// 0.54 ms; the 8 x 512 x 512 stack (13 M searches, 89 K past the LDS lists)
+// 9.2 -> 1.0 ms.
+constexpr int SUB_W = 16;       // lanes of a sub-wave search (8 and 32 measured: within 12 %)
+constexpr int SUB_CAP = 64;     // 1 KB of LDS per search
+constexpr int WAVE_CAP = 128;   // 2 KB of LDS per wave
+constexpr int WIDE_CAP = 1024;  // 16 KB
+constexpr int BLOCK_CAP = 8192; // 128 KB
+constexpr int BLOCK_NW = 8;    // waves of a workgroup search
+constexpr int WAVE_GROUPS = 4096; // persistent groups launched at most
+constexpr int WIDE_GROUPS = 2304;
+constexpr int BLOCK_GROUPS = 256;
+constexpr int SLAB_CAP = 1 << 16;
+constexpr int SLABS = 32; // 1 MB each
+// Where a tier's searches all fit the chip at once in the next tier, the
+// tier only adds its own longest search to the chain of launches:
+constexpr int64_t DIRECT_MAX = 4096; // searches: no LDS tier (1,021: 0.87 -> 0.14 ms)
+constexpr unsigned SUB_MIN = 3072;   // past the LDS lists: no sub-wave tier (884: 0.38 ms saved)
+constexpr unsigned WIDE_MIN = 256;   // past the wave lists: no wide tier
+constexpr int64_t BLOCK_MAX = 4096;   // (unbounded searches only) likewise
+constexpr int64_t EXPECT_MIN_ITER = 1000000; // iteration limit from which a minimum is expected
 // Wavefront batches: searches advanced together (one round of launches and
 // one host check per level for the whole batch), from WF_BATCH, doubled
 // after every batch that fits the box budget up to WF_BATCH_MAX.  Workloads
@@ -66,6 +106,8 @@ struct CCDArgs {
     long max_iter;
     bool bounded;          // hide outcomes >= running minimum
     double* bound;         // running minimum (double bits), one per scene
+    double* expect;        // expected minimum, one per scene (null: none)
+    int* restarted;        // set when a search of the group tiers ends below SMALL_TOI
     const int32_t* vscene; // batched contexts: scene per vertex (null: one scene)
     double* toi_out;       // per-candidate toi (null: not recorded)
     int* any_hit;          // early exit flag (null: no early exit)
@@ -216,10 +258,12 @@ __global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo,
         report(A, ci, pre == 1, 0.0, sc);
         return;
     }
-    TIBound B1 { A.bounded ? A.bound + sc : nullptr, 1.0, SMALL_TOI };
+    const double* const run = A.bounded ? A.bound + sc : nullptr;
+    const double* const expect = A.bounded && A.expect ? A.expect + sc : nullptr;
+    const TIBound B1 { run, expect, 1.0, SMALL_TOI };
     int r = ti_query_lds(q, eff, adj, A.max_iter, false, B1, L, toi);
     if (r == TI_HIT && toi < SMALL_TOI) {
-        TIBound B2 { A.bounded ? A.bound + sc : nullptr, (1.0 / A.rescale) * (1 + 1e-12), 0.0 };
+        const TIBound B2 { run, expect, (1.0 / A.rescale) * (1 + 1e-12), 0.0 };
         r = ti_query_lds(q, A.min_distance, adj, -1, true, B2, L, toi);
         if (r == TI_HIT) toi *= A.rescale;
     }
@@ -235,45 +279,204 @@ __global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo,
     report(A, ci, r == TI_HIT, toi, sc);
 }
 
+// The searches of a tier: `list`, or the list of the tier before (`before`)
+// when that is short enough (at most `skip`) for the tier between to have
+// left it alone.
+struct Searches {
+    const uint32_t* list;
+    const unsigned long long* n;
+    const uint32_t* before;
+    const unsigned long long* n_before;
+    unsigned skip;
+    unsigned long long* work; // next search to take
+};
+
+struct Lists {
+    uint32_t* over; // searches that outgrow this tier
+    unsigned long long* n_over;
+    uint32_t* deep; // searches too deep for packed boxes
+    unsigned long long* n_deep;
+};
+
 // ---------------------------------------------------------------------------
-// slab tier
+// sub-wave tier: SUB_W lanes per search, 64 / SUB_W searches per wave
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(CB) void k_ccd_lanes(CCDArgs A, const uint32_t* todo, int64_t n_todo,
-                                                  TIBox* slab, unsigned long long* work,
-                                                  uint32_t* heavy, unsigned long long* n_heavy)
+// The strategy (tight_inclusion_ccd.cpp:33-75) around one search of a tier:
+// stage 1 with the effective distance; an outcome below SMALL_TOI is searched
+// again from the minimum distance without an iteration limit (stage 2),
+// with the distance or the tolerance halved while the outcome stays 0.
+// `next` tells whether another search follows and sets its parameters.
+struct TIStrategy {
+    TIBound B;
+    double ms, delta, rescale;
+    long max_iter;
+    int tries = 0; // searches of stage 2
+    __device__ TIStrategy(const CCDArgs& A, int sc, double eff, double adj)
+        : B { A.bounded ? A.bound + sc : nullptr, A.bounded && A.expect ? A.expect + sc : nullptr,
+              1.0, SMALL_TOI }
+        , ms(eff)
+        , delta(adj)
+        , rescale(A.rescale)
+        , max_iter(A.max_iter)
+    {
+    }
+    __device__ bool next(const CCDArgs& A, int r, double toi)
+    {
+        if (r != TI_HIT) return false;
+        if (tries == 0) {
+            if (toi >= SMALL_TOI) return false;
+            B.scale = (1.0 / A.rescale) * (1 + 1e-12);
+            B.floor = 0.0;
+            ms = A.min_distance;
+            max_iter = -1;
+        } else {
+            if (toi != 0 || tries >= TI_MAX_NO_ZERO_TOI_ITER) return false;
+            if (10 * delta < ms) ms *= 0.5;
+            else delta *= 0.5;
+        }
+        tries++;
+        return true;
+    }
+    __device__ double outcome(int r, double toi) const
+    {
+        return tries && r == TI_HIT ? toi * rescale : toi;
+    }
+};
+
+template <int W, int CAP>
+__global__ __launch_bounds__(WAVE) void k_ccd_sub(CCDArgs A, Searches Q_in, Lists out)
 {
-    const int64_t lane = (int64_t)blockIdx.x * CB + threadIdx.x;
-    TISlab S;
-    S.cap = LANE_CAP;
-    S.cur = slab + lane * 3 * (int64_t)LANE_CAP;
-    S.lo = S.cur + LANE_CAP;
-    S.hi = S.lo + LANE_CAP;
+    constexpr int PER_WAVE = WAVE / W;
+    __shared__ unsigned long long lists[PER_WAVE][2 * CAP];
+    __shared__ TIQuery Q[PER_WAVE];
+    const int grp = (int)threadIdx.x / W;
+    const bool first = threadIdx.x % W == 0;
+    unsigned long long* const cur = lists[grp];
+    unsigned long long* const nxt = cur + CAP;
+    const unsigned long long n = *Q_in.n;
+    if (n <= Q_in.skip) return; // too few: the wave tier takes them
+    const uint32_t* const todo = Q_in.list;
     for (;;) {
-        if (A.any_hit && __hip_atomic_load(A.any_hit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            break;
-        const int64_t k = (int64_t)atomicAdd(work, 1ull);
-        if (k >= n_todo) break;
-        const int64_t ci = todo[k];
+        unsigned long long k0 = 0;
+        if (threadIdx.x == 0) {
+            const bool quit = A.any_hit
+                && __hip_atomic_load(A.any_hit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            k0 = quit ? ~0ull : atomicAdd(Q_in.work, (unsigned long long)PER_WAVE);
+        }
+        k0 = __shfl(k0, 0, WAVE);
+        if (k0 >= n) return;
+        const unsigned long long k = k0 + (unsigned)grp;
+        if (k < n) {
+            const int64_t ci = todo[k];
+            double eff = 0, adj = 0, toi = INFINITY;
+            int sc = 0, pre;
+            {
+                TIQuery q;
+                pre = candidate_setup(A, ci, q, eff, adj, sc);
+                if (pre < 0) {
+                    ti_param_tol(q, adj);
+                    ti_filter(q, eff > 0);
+                    if (first) Q[grp] = q;
+                }
+            }
+            if (pre >= 0) { // settled by the prologue (not for searches of other tiers)
+                if (first) report(A, ci, pre == 1, 0.0, sc);
+            } else {
+                TIStrategy T(A, sc, eff, adj);
+                int r;
+                for (;;) {
+                    ti_wave_sync();
+                    r = ti_bfs_sub<W>(Q[grp], T.delta, T.ms, T.max_iter, T.B, cur, nxt, CAP, toi);
+                    if (!T.next(A, r, toi)) break;
+                    ti_wave_sync();
+                    if (first) {
+                        ti_param_tol(Q[grp], T.delta);
+                        if (T.tries == 1) ti_filter(Q[grp], T.ms > 0);
+                    }
+                }
+                if (first) {
+                    if (r == TI_OVERFLOW) out.over[atomicAdd(out.n_over, 1ull)] = (uint32_t)ci;
+                    else if (r == TI_DEEP) out.deep[atomicAdd(out.n_deep, 1ull)] = (uint32_t)ci;
+                    else report(A, ci, r == TI_HIT, T.outcome(r, toi), sc);
+                }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// group tiers: NW waves per search, lists of CAP boxes in LDS (NW > 1: then
+// in `slabs`)
+// ---------------------------------------------------------------------------
+template <int NW, int CAP>
+__global__ __launch_bounds__(NW * WAVE) void k_ccd_group(CCDArgs A, Searches Q_in, Lists out,
+                                                         TISlabs slabs)
+{
+    __shared__ unsigned long long lists[2 * CAP];
+    __shared__ TIGroup<NW> G;
+    __shared__ struct {
         TIQuery q;
-        double eff = 0, adj = 0, toi = INFINITY;
-        int sc = 0;
-        const int pre = candidate_setup(A, ci, q, eff, adj, sc);
-        if (pre >= 0) {
-            report(A, ci, pre == 1, 0.0, sc);
+        double eff, adj;
+        unsigned long long k;
+        int sc, pre;
+    } W; // the search in hand, set by the first lane
+    const bool first = threadIdx.x == 0;
+    const bool early = Q_in.before && *Q_in.n_before <= Q_in.skip;
+    const uint32_t* const todo = early ? Q_in.before : Q_in.list;
+    const unsigned long long n = early ? *Q_in.n_before : *Q_in.n;
+    if (!Q_in.before && n <= Q_in.skip) return; // too few: the next tier takes them
+    for (;;) {
+        __syncthreads(); // W has been read
+        if (first) {
+            const bool quit = A.any_hit
+                && __hip_atomic_load(A.any_hit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            W.k = quit ? ~0ull : atomicAdd(Q_in.work, 1ull);
+            if (W.k < n) {
+                TIQuery q;
+                double eff = 0, adj = 0;
+                int sc = 0;
+                W.pre = candidate_setup(A, todo[W.k], q, eff, adj, sc);
+                ti_param_tol(q, adj);
+                ti_filter(q, eff > 0);
+                W.q = q;
+                W.eff = eff;
+                W.adj = adj;
+                W.sc = sc;
+            }
+        }
+        __syncthreads();
+        if (W.k >= n) return;
+        const int64_t ci = todo[W.k];
+        const int sc = W.sc;
+        if (W.pre >= 0) { // settled by the prologue (not for searches of other tiers)
+            if (first) report(A, ci, W.pre == 1, 0.0, sc);
             continue;
         }
-        TIBound B1 { A.bounded ? A.bound + sc : nullptr, 1.0, SMALL_TOI };
-        int r = ti_query(q, eff, adj, A.max_iter, false, B1, S, toi);
-        if (r == TI_HIT && toi < SMALL_TOI) {
-            TIBound B2 { A.bounded ? A.bound + sc : nullptr, (1.0 / A.rescale) * (1 + 1e-12), 0.0 };
-            r = ti_query(q, A.min_distance, adj, -1, true, B2, S, toi);
-            if (r == TI_HIT) toi *= A.rescale;
+        double* const expect = A.bounded && A.expect ? A.expect + sc : nullptr;
+        TIStrategy T(A, sc, W.eff, W.adj);
+        double toi = INFINITY;
+        bool cut = false;
+        int r;
+        for (;;) {
+            const bool beam = expect && T.tries == 0;
+            r = ti_bfs_group<NW>(W.q, T.delta, T.ms, T.max_iter, T.B, lists, lists + CAP, CAP,
+                                 NW > 1 ? &slabs : nullptr, beam, G, toi, cut);
+            if (cut || !T.next(A, r, toi)) break;
+            __syncthreads(); // the query has been read
+            if (first) {
+                ti_param_tol(W.q, T.delta);
+                if (T.tries == 1) ti_filter(W.q, T.ms > 0);
+            }
         }
-        if (r >= TI_OVERFLOW) {
-            heavy[atomicAdd(n_heavy, 1ull)] = (uint32_t)ci;
-            continue;
+        if (!first) continue;
+        if (T.tries) atomicOr(A.restarted, 1);
+        if (cut) {
+            if (r == TI_HIT && toi >= SMALL_TOI) atomic_min_nonneg(expect, toi);
+            if (r != TI_DEEP) r = TI_OVERFLOW;
         }
-        report(A, ci, r == TI_HIT, toi, sc);
+        if (r == TI_OVERFLOW) out.over[atomicAdd(out.n_over, 1ull)] = (uint32_t)ci;
+        else if (r == TI_DEEP) out.deep[atomicAdd(out.n_deep, 1ull)] = (uint32_t)ci;
+        else report(A, ci, r == TI_HIT, T.outcome(r, toi), sc);
     }
 }
 
@@ -348,7 +551,7 @@ __global__ void k_wf_init(CCDArgs A, const uint32_t* heavy, int64_t first, int64
     S.seg_count = 1;
     S.cut = i;
     S.next_start = S.next_count = 0;
-    if (pre >= 0) { // resolved by the prologue (cannot happen for lane overflows)
+    if (pre >= 0) { // resolved by the prologue (cannot happen for searches of other tiers)
         S.done = 1;
         S.hit = pre == 1;
         S.result = 0.0;
@@ -364,8 +567,8 @@ __global__ void k_wf_init(CCDArgs A, const uint32_t* heavy, int64_t first, int64
 __device__ __forceinline__ double wf_bound(const CCDArgs& A, const WFState& S)
 {
     if (!A.bounded) return INFINITY;
-    const double g = __hip_atomic_load(A.bound + S.scene, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
+    const TIBound B { A.bound + S.scene, A.expect ? A.expect + S.scene : nullptr, 1.0, 0.0 };
+    const double g = B.get();
     if (S.stage == 1) return g > SMALL_TOI ? g : SMALL_TOI;
     return g * ((1.0 / A.rescale) * (1 + 1e-12));
 }
@@ -422,7 +625,7 @@ __device__ __forceinline__ void wf_first(bool hit, int owner, int64_t j, unsigne
     if (hit && (!below || prev_owner != owner)) atomicMin(e, (unsigned long long)j);
 }
 
-// The sequential per-level rules of ti_bfs, in parallel: the scan of a
+// The sequential per-level rules of ti_bfs_lds, in parallel: the scan of a
 // level in order ends at the first zero box that is within tolerance or
 // inside the ε box (or any zero box once the level's widths are within
 // tolerance: c1); it finishes the search there if no zero box before it was
@@ -459,6 +662,7 @@ __device__ void wf_search_done(const CCDArgs& A, WFState& S, bool hit, double to
 {
     if (S.stage == 1) {
         if (hit && toi < SMALL_TOI) {
+            atomicOr(A.restarted, 1);
             S.stage = 2;
             S.nz_iter = 0;
             wf_begin_query(S, A.min_distance, S.adj, -1);
@@ -483,7 +687,7 @@ __device__ void wf_search_done(const CCDArgs& A, WFState& S, bool hit, double to
 }
 
 // one lane per candidate: the outcome of the level from its first events
-// (ti_bfs's rules); children may come only from boxes before S.cut
+// (ti_bfs_lds's rules); children may come only from boxes before S.cut
 __global__ void k_wf_decide(CCDArgs A, WFState* st, int64_t nb, const WFBox* boxes,
                             const uint32_t* lpre, unsigned long long* ev, int* error)
 {
@@ -776,26 +980,15 @@ bool wf_batch(Ctx& c, const CCDArgs& A, const uint32_t* heavy, int64_t first, in
     return true;
 }
 
-// The slab tier's box lists (3 x LANE_CAP boxes per lane, up to LANES
-// lanes: 2.4 GB) are one buffer per device shared by every context on it:
-// a context holds the lock while it enqueues its slab launch behind the
-// previous user's (stream event), so the memory does not grow with the
-// number of contexts.
-struct SharedSlab {
-    std::mutex mu;
-    DevBuf buf;
-    hipEvent_t last = nullptr;
-};
-constexpr int SLAB_DEVICES = 64;
-SharedSlab g_slab[SLAB_DEVICES];
-
-SharedSlab& shared_slab(int device)
-{
-    if (device < 0 || device >= SLAB_DEVICES) throw Error(IPCG_ERR_ARG, "device index out of range");
-    return g_slab[device];
-}
-
 } // namespace
+
+// counters of one search over all tiers
+__global__ void k_ccd_begin(unsigned long long* cnt, int n, int at_todo, unsigned long long n_todo,
+                            int* restarted)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) cnt[i] = i == at_todo ? n_todo : 0ull;
+    if (threadIdx.x == 0) *restarted = 0;
+}
 
 __global__ void k_fill_f64(double* p, int n, double v)
 {
@@ -821,29 +1014,32 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         return 1.0;
     }
     if (n >= (1ll << 32)) throw Error(IPCG_ERR_ARG, "too many CCD candidates");
-    // device scalars: bound, work counter, heavy count, hit flag, error, roots
-    c.ccd_status.reserve(512);
+    // device scalars, read back in one copy: running minimum, expected
+    // minimum, list and work counters, hit flag, error, wavefront counts
+    constexpr size_t ST_BYTES = 1024;
+    c.ccd_status.reserve(ST_BYTES);
     char* st = c.ccd_status.as<char>();
     double* bound = reinterpret_cast<double*>(st);
-    unsigned long long* work = reinterpret_cast<unsigned long long*>(st + 64);
-    unsigned long long* n_heavy = reinterpret_cast<unsigned long long*>(st + 128);
+    double* expect = reinterpret_cast<double*>(st + 64);
     int* any_hit = reinterpret_cast<int*>(st + 192);
+    int* restarted = reinterpret_cast<int*>(st + 224);
     int* error = reinterpret_cast<int*>(st + 256);
     unsigned long long* nroot = reinterpret_cast<unsigned long long*>(st + 320);
     unsigned long long* npend = reinterpret_cast<unsigned long long*>(st + 384); // [3]
-    unsigned long long* n_spill = reinterpret_cast<unsigned long long*>(st + 448); // [2]
-    const double one = 1.0;
-    IPCG_HIP(hipMemsetAsync(st, 0, 512, s));
-    if (c.batched()) { // one running minimum per scene
-        c.ccd_sbound.reserve(sizeof(double) * (size_t)nsc);
+    unsigned long long* cnt = reinterpret_cast<unsigned long long*>(st + 512);
+    enum { N_SPILL_A, N_SPILL_A_DEEP, N_SPILL_B, N_SPILL_B_DEEP, N_SUB_A, N_SUB_B, N_OVER, N_WIDE, N_HEAVY,
+           WORK_SUB_A, WORK_SUB_B, WORK_A, WORK_B, WORK_WIDE, WORK_BLOCK, N_SLAB, N_TODO, N_CNT };
+    static_assert(512 + 8 * N_CNT <= ST_BYTES, "status block");
+    IPCG_HIP(hipMemsetAsync(st, 0, ST_BYTES, s));
+    if (c.batched()) { // one running minimum (then one expected minimum) per scene
+        c.ccd_sbound.reserve(sizeof(double) * 2 * (size_t)nsc);
         bound = c.ccd_sbound.as<double>();
-        hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(nsc, 256)), dim3(256), 0, s, bound, nsc, 1.0);
-        IPCG_CHECK_LAUNCH();
-    } else {
-        IPCG_HIP(hipMemcpyAsync(bound, &one, sizeof(double), hipMemcpyHostToDevice, s));
+        expect = bound + nsc;
     }
-    c.ccd_overflow.reserve(sizeof(uint32_t) * (size_t)n);
-    uint32_t* heavy = c.ccd_overflow.as<uint32_t>();
+    hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(nsc, 256)), dim3(256), 0, s, bound, nsc, 1.0);
+    hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(nsc, 256)), dim3(256), 0, s, expect, nsc,
+                       (double)INFINITY);
+    IPCG_CHECK_LAUNCH();
     if (per_cand) c.ccd_toi.reserve(sizeof(double) * (size_t)n);
 
     CCDArgs A;
@@ -866,6 +1062,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     A.max_iter = (long)max_iter;
     A.bounded = !per_cand;
     A.bound = bound;
+    A.expect = nullptr;
+    A.restarted = restarted;
     A.vscene = c.batched() ? c.vscene.as<int32_t>() : nullptr;
     A.toi_out = per_cand ? c.ccd_toi.as<double>() : nullptr;
     A.any_hit = early_exit ? any_hit : nullptr;
@@ -894,93 +1092,212 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     c.stat["ccd.candidates"] = n;
     c.stat["ccd.searched"] = n_todo;
 
-    // One search of every surviving candidate of an index range: the LDS
-    // tier, the slab tier for its overflow, then the wavefront for searches
-    // that outgrew a slab.  The root pass's staging array is free again and
-    // holds the spill list.
-    auto search = [&](int64_t ci_lo, int64_t ci_hi) {
-        uint32_t* spill = c.ccd_stage.as<uint32_t>();
-        IPCG_HIP(hipMemsetAsync(n_spill, 0, 2 * sizeof(unsigned long long), s));
-        IPCG_HIP(hipMemsetAsync(work, 0, sizeof(unsigned long long), s));
-        IPCG_HIP(hipMemsetAsync(n_heavy, 0, sizeof(unsigned long long), s));
-        c.stage_begin("ccd_lds");
-        if (n_todo > 0) {
-            hipLaunchKernelGGL(k_ccd_lds, dim3((unsigned)((n_todo + CB - 1) / CB)), dim3(CB), 0, s,
-                               A, c.ccd_todo.as<uint32_t>(), n_todo, spill, n_spill, ci_lo,
-                               ci_hi);
-            IPCG_CHECK_LAUNCH();
-        }
-        c.stage_end();
-        IPCG_HIP(hipMemcpyAsync(h, n_spill, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                s));
+    // lists of searches, at most n_todo each; the root pass's staging array
+    // is free again and holds one more
+    c.ccd_overflow.reserve(sizeof(uint32_t) * 5 * (size_t)std::max<int64_t>(n_todo, 1));
+    uint32_t* const spill_a = c.ccd_stage.as<uint32_t>();
+    uint32_t* const spill_b = c.ccd_overflow.as<uint32_t>();
+    uint32_t* const over = spill_b + n_todo;
+    uint32_t* const wide = over + n_todo;
+    uint32_t* const heavy = wide + n_todo;
+    uint32_t* const sub = heavy + n_todo;
+    std::vector<double> scene_bound((size_t)(2 * nsc), 0.0); // running, then expected minimums
+    auto read_back = [&]() { // the scalars in h, the scenes' minimums in scene_bound
+        IPCG_HIP(hipMemcpyAsync(h, st, ST_BYTES, hipMemcpyDeviceToHost, s));
+        double* hb = reinterpret_cast<double*>(h) + ST_BYTES / sizeof(double);
+        const size_t nb = sizeof(double) * 2 * (size_t)nsc;
+        const bool pin = ST_BYTES + nb <= PINNED_BYTES;
+        if (c.batched())
+            IPCG_HIP(hipMemcpyAsync(pin ? hb : scene_bound.data(), bound, nb,
+                                    hipMemcpyDeviceToHost, s));
         IPCG_HIP(hipStreamSynchronize(s));
-        const int64_t n2 = (int64_t)h[0];
-        c.stat["ccd.spilled"] += n2;
-        c.stat["ccd.spilled_deep"] += (int64_t)h[1];
-        c.stage_begin("ccd_lanes");
-        if (n2 > 0) {
-            const int64_t ln = std::min<int64_t>(LANES, ((n2 + CB - 1) / CB) * CB);
-            SharedSlab& P = shared_slab(c.device);
-            std::lock_guard<std::mutex> lock(P.mu);
-            // slabs for the lanes launched only; growing frees the old
-            // buffer, which waits for the device to finish with it
-            P.buf.reserve(sizeof(TIBox) * 3 * (size_t)LANE_CAP * (size_t)ln);
-            if (!P.last) IPCG_HIP(hipEventCreateWithFlags(&P.last, hipEventDisableTiming));
-            else IPCG_HIP(hipStreamWaitEvent(s, P.last, 0)); // the previous user's launch
-            hipLaunchKernelGGL(k_ccd_lanes, dim3((unsigned)(ln / CB)), dim3(CB), 0, s, A, spill,
-                               n2, P.buf.as<TIBox>(), work, heavy, n_heavy);
-            IPCG_CHECK_LAUNCH();
-            IPCG_HIP(hipEventRecord(P.last, s));
-        }
-        c.stage_end();
-        IPCG_HIP(hipMemcpyAsync(h, n_heavy, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-        IPCG_HIP(hipStreamSynchronize(s));
-        const int64_t nh = (int64_t)h[0];
-        c.stat["ccd.wavefront"] += nh;
-        if (nh > 0) {
-            c.stage_begin("ccd_wavefront");
-            DevBuf& wst = c.ccd_bound; // per-candidate wavefront state
-            wst.reserve(sizeof(WFState) * (size_t)std::min<int64_t>(nh, WF_BATCH_MAX));
-            WFState* states = wst.as<WFState>();
-            // Batches of heavy candidates advance together.  A batch whose
-            // level outgrows the box budget is abandoned (results are only
-            // reported at the end of a batch, so this has no side effect)
-            // and retried with a quarter of the candidates.
-            int64_t batch = std::min<int64_t>(WF_BATCH, nh);
-            for (int64_t first = 0; first < nh;) {
-                const int64_t nb = std::min<int64_t>(batch, nh - first);
-                const bool ok = wf_batch(c, A, heavy, first, nb, states, early_exit, any_hit,
-                                         error, nroot, npend, h);
-                if (!ok) {
-                    if (nb == 1)
-                        throw Error(IPCG_ERR_NUMERIC, "CCD wavefront level exceeds its box budget");
-                    batch = std::max<int64_t>(1, nb / 4);
-                    continue;
-                }
-                first += nb;
-                batch = std::min<int64_t>(WF_BATCH_MAX, 2 * batch);
-            }
-            c.stage_end();
-            IPCG_HIP(hipMemcpyAsync(h, error, sizeof(int), hipMemcpyDeviceToHost, s));
-            IPCG_HIP(hipStreamSynchronize(s));
-            const int err = *reinterpret_cast<int*>(h);
-            if (err & 2) throw Error(IPCG_ERR_NUMERIC, "CCD wavefront level out of t order");
-            if (err) throw Error(IPCG_ERR_NUMERIC, "CCD root search exceeded the level limit");
+        if (!c.batched()) {
+            scene_bound[0] = *reinterpret_cast<const double*>(h);
+            scene_bound[1] = *reinterpret_cast<const double*>(reinterpret_cast<char*>(h) + 64);
+        } else if (pin) {
+            std::copy(hb, hb + 2 * nsc, scene_bound.begin());
         }
     };
+    auto count = [&](int k) { return (int64_t)h[512 / 8 + k]; };
+    auto lds_tier = [&](int64_t ci_lo, int64_t ci_hi, uint32_t* spill, int n_spill) {
+        c.stage_begin("ccd_lds");
+        hipLaunchKernelGGL(k_ccd_lds, dim3((unsigned)((n_todo + CB - 1) / CB)), dim3(CB), 0, s, A,
+                           c.ccd_todo.as<uint32_t>(), n_todo, spill, cnt + n_spill, ci_lo, ci_hi);
+        IPCG_CHECK_LAUNCH();
+        c.stage_end();
+    };
+    auto out = [&](uint32_t* list, int n_list) {
+        return Lists { list, cnt + n_list, heavy, cnt + N_HEAVY };
+    };
+    auto sub_tier = [&](const uint32_t* list, int n_list, int work, int n_sub) {
+        c.stage_begin("ccd_sub");
+        constexpr int PER_WAVE = WAVE / SUB_W;
+        hipLaunchKernelGGL((k_ccd_sub<SUB_W, SUB_CAP>),
+                           dim3((unsigned)std::min<int64_t>((n_todo + PER_WAVE - 1) / PER_WAVE,
+                                                            WAVE_GROUPS)),
+                           dim3(WAVE), 0, s, A,
+                           Searches { list, cnt + n_list, nullptr, nullptr, SUB_MIN, cnt + work },
+                           out(sub, n_sub));
+        IPCG_CHECK_LAUNCH();
+        c.stage_end();
+    };
+    const TISlabs none { nullptr, nullptr, 0, 0 };
+    auto wave_tier = [&](const Searches& q) {
+        c.stage_begin("ccd_wave");
+        hipLaunchKernelGGL((k_ccd_group<1, WAVE_CAP>),
+                           dim3((unsigned)std::min<int64_t>(n_todo, WAVE_GROUPS)), dim3(WAVE), 0,
+                           s, A, q, out(over, N_OVER), none);
+        IPCG_CHECK_LAUNCH();
+        c.stage_end();
+    };
+    auto wide_tier = [&]() {
+        c.stage_begin("ccd_wide");
+        hipLaunchKernelGGL((k_ccd_group<1, WIDE_CAP>),
+                           dim3((unsigned)std::min<int64_t>(n_todo, WIDE_GROUPS)), dim3(WAVE), 0,
+                           s, A,
+                           Searches { over, cnt + N_OVER, nullptr, nullptr, WIDE_MIN,
+                                      cnt + WORK_WIDE },
+                           out(wide, N_WIDE), none);
+        IPCG_CHECK_LAUNCH();
+        c.stage_end();
+    };
+    auto block_tier = [&]() {
+        c.stage_begin("ccd_block");
+        c.ccd_slab.reserve(sizeof(unsigned long long) * 2 * SLAB_CAP * (size_t)SLABS);
+        hipLaunchKernelGGL((k_ccd_group<BLOCK_NW, BLOCK_CAP>),
+                           dim3((unsigned)std::min<int64_t>(n_todo, BLOCK_GROUPS)),
+                           dim3(BLOCK_NW * WAVE), 0, s, A,
+                           Searches { wide, cnt + N_WIDE, over, cnt + N_OVER, WIDE_MIN,
+                                      cnt + WORK_BLOCK },
+                           out(heavy, N_HEAVY),
+                           TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB, SLABS,
+                                     SLAB_CAP });
+        IPCG_CHECK_LAUNCH();
+        c.stage_end();
+    };
+    // moves a tier's list to the wavefront's (counts as read back)
+    auto to_heavy = [&](const uint32_t* list, int n_list) {
+        const int64_t m = count(n_list);
+        IPCG_HIP(hipMemcpyAsync(heavy + count(N_HEAVY), list, sizeof(uint32_t) * (size_t)m,
+                                hipMemcpyDeviceToDevice, s));
+        h[512 / 8 + N_HEAVY] += (unsigned long long)m;
+    };
+    auto wavefront = [&](int64_t nh) {
+        c.stat["ccd.wavefront"] += nh;
+        c.stage_begin("ccd_wavefront");
+        DevBuf& wst = c.ccd_bound; // per-candidate wavefront state
+        wst.reserve(sizeof(WFState) * (size_t)std::min<int64_t>(nh, WF_BATCH_MAX));
+        WFState* states = wst.as<WFState>();
+        // Batches of heavy candidates advance together.  A batch whose
+        // level outgrows the box budget is abandoned (results are only
+        // reported at the end of a batch, so this has no side effect)
+        // and retried with a quarter of the candidates.
+        int64_t batch = std::min<int64_t>(WF_BATCH, nh);
+        for (int64_t first = 0; first < nh;) {
+            const int64_t nb = std::min<int64_t>(batch, nh - first);
+            const bool ok = wf_batch(c, A, heavy, first, nb, states, early_exit, any_hit, error,
+                                     nroot, npend, h);
+            if (!ok) {
+                if (nb == 1)
+                    throw Error(IPCG_ERR_NUMERIC, "CCD wavefront level exceeds its box budget");
+                batch = std::max<int64_t>(1, nb / 4);
+                continue;
+            }
+            first += nb;
+            batch = std::min<int64_t>(WF_BATCH_MAX, 2 * batch);
+        }
+        c.stage_end();
+        read_back();
+        const int err = *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + 256);
+        if (err & 2) throw Error(IPCG_ERR_NUMERIC, "CCD wavefront level out of t order");
+        if (err) throw Error(IPCG_ERR_NUMERIC, "CCD root search exceeded the level limit");
+    };
+    // Every surviving candidate through the tiers.
+    auto search = [&]() {
+        hipLaunchKernelGGL(k_ccd_begin, dim3(1), dim3(WAVE), 0, s, cnt, (int)N_CNT, (int)N_TODO,
+                           (unsigned long long)n_todo, restarted);
+        IPCG_CHECK_LAUNCH();
+        if (A.bounded) {
+            // Face-vertex and codim candidates first: their roots are isolated
+            // points, so they resolve fast and lower every scene's running and
+            // expected minimum before the edge-edge searches start, which
+            // parallel overlapping edges can make long.  Outcomes below the
+            // minimum do not depend on the order, so neither does the result.
+            if (A.expect && n_todo <= DIRECT_MAX) {
+                // few searches: every one has a wave of its own at once
+                wave_tier({ c.ccd_todo.as<uint32_t>(), cnt + N_TODO, nullptr, nullptr, 0,
+                            cnt + WORK_A });
+            } else {
+                if (c.n_ee < n) {
+                    lds_tier(c.n_ee, n, spill_a, N_SPILL_A);
+                    sub_tier(spill_a, N_SPILL_A, WORK_SUB_A, N_SUB_A);
+                    wave_tier({ sub, cnt + N_SUB_A, spill_a, cnt + N_SPILL_A, SUB_MIN,
+                                cnt + WORK_A });
+                }
+                if (c.n_ee > 0) {
+                    lds_tier(0, c.n_ee, spill_b, N_SPILL_B);
+                    sub_tier(spill_b, N_SPILL_B, WORK_SUB_B, N_SUB_B);
+                    wave_tier({ sub, cnt + N_SUB_B, spill_b, cnt + N_SPILL_B, SUB_MIN,
+                                cnt + WORK_B });
+                }
+            }
+            wide_tier();
+            block_tier();
+            read_back();
+        } else {
+            lds_tier(0, n, spill_a, N_SPILL_A);
+            sub_tier(spill_a, N_SPILL_A, WORK_SUB_A, N_SUB_A);
+            wave_tier({ sub, cnt + N_SUB_A, spill_a, cnt + N_SPILL_A, SUB_MIN, cnt + WORK_A });
+            wide_tier();
+            read_back();
+            // without a bound most of what is left grows past a workgroup's
+            // lists too; many such searches advance faster together
+            const bool from_over = count(N_OVER) <= (int64_t)WIDE_MIN;
+            const int64_t left = from_over ? count(N_OVER) : count(N_WIDE);
+            if (left > BLOCK_MAX) {
+                to_heavy(wide, N_WIDE);
+            } else if (left > 0) {
+                block_tier();
+                read_back();
+            }
+        }
+        c.stat["ccd.spilled"] += count(N_SPILL_A) + count(N_SPILL_B);
+        c.stat["ccd.spilled_deep"] += count(N_SPILL_A_DEEP) + count(N_SPILL_B_DEEP);
+        const int64_t nh = count(N_HEAVY);
+        if (nh > 0) wavefront(nh);
+    };
+    c.stat["ccd.unmet"] = 0;
     c.stat["ccd.wavefront"] = 0;
     c.stat["ccd.spilled"] = 0;
     c.stat["ccd.spilled_deep"] = 0;
-    if (A.bounded) {
-        // Face-vertex and codim candidates first: their roots are isolated
-        // points, so they resolve fast and lower every scene's running
-        // minimum before the edge-edge searches start, which parallel
-        // overlapping edges can make long.  Outcomes below the minimum do not
-        // depend on the order, so neither does the result.
-        search(c.n_ee, n);
-        search(0, c.n_ee);
+    bool hit = false; // an expected minimum stood
+    if (n_todo == 0) {
+        read_back(); // the root pass may have reported hits
     } else {
-        search(0, n);
+        // With a low iteration limit the outcome of a search depends on how
+        // many boxes its bound hides: those keep to the running minimum.
+        const bool expecting = A.bounded && (max_iter <= 0 || max_iter >= EXPECT_MIN_ITER);
+        A.expect = expecting ? expect : nullptr;
+        search();
+        auto flag = [&](size_t at) {
+            return *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + at) != 0;
+        };
+        if (expecting) {
+            bool met = true;
+            for (int k = 0; k < nsc; k++) {
+                if (scene_bound[k] < scene_bound[nsc + k]) continue;
+                if (std::isinf(scene_bound[nsc + k])) continue;
+                if (flag(224)) met = false; // restarted
+                scene_bound[k] = scene_bound[nsc + k];
+                hit = true;
+            }
+            if (!met && !(early_exit && flag(192))) {
+                A.expect = nullptr;
+                hit = false;
+                c.stat["ccd.unmet"]++;
+                search();
+            }
+        }
     }
     if (per_cand) { // toi_out: ee, fv, vv, ev (any null)
         const int64_t cnt[4] = { c.n_ee, c.n_fv, c.n_vv, c.n_ev };
@@ -994,15 +1311,12 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         IPCG_HIP(hipStreamSynchronize(s));
         return 1.0;
     }
-    double* hd = static_cast<double*>(c.pinned);
-    IPCG_HIP(hipMemcpyAsync(hd, any_hit, sizeof(int), hipMemcpyDeviceToHost, s));
-    std::vector<double> per_scene((size_t)nsc);
-    IPCG_HIP(hipMemcpyAsync(per_scene.data(), bound, sizeof(double) * (size_t)nsc,
-                            hipMemcpyDeviceToHost, s));
-    IPCG_HIP(hipStreamSynchronize(s));
-    if (early_exit) return reinterpret_cast<int*>(hd)[0] ? 0.0 : 1.0;
-    if (scene_steps) std::copy(per_scene.begin(), per_scene.end(), scene_steps);
-    return *std::min_element(per_scene.begin(), per_scene.end());
+    if (early_exit) {
+        hit = hit || *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + 192) != 0;
+        return hit ? 0.0 : 1.0;
+    }
+    if (scene_steps) std::copy(scene_bound.begin(), scene_bound.begin() + nsc, scene_steps);
+    return *std::min_element(scene_bound.begin(), scene_bound.begin() + nsc);
 }
 
 } // namespace ipcg
