@@ -474,7 +474,8 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
 /* work counts of the last calls, by name: "ccd.candidates" (swept
  * candidates of the last CCD), "ccd.searched" (those whose root box
  * includes the origin), "ccd.spilled" (searches that outgrew the LDS
- * lists), "ccd.wavefront" (searches that outgrew a workgroup's lists),
+ * lists), "ccd.wavefront" (searches that outgrew a wave's lists too: a workgroup
+ * or the level-by-level wavefront takes them),
  * "ccd.unmet" (1 when an expected minimum did not stand and the searches
  * ran again without it),
  * "hessian.ee_other" (edge-edge collisions of the last Hessian whose type

@@ -152,7 +152,7 @@ static std::vector<DevBuf*> all_bufs(Ctx& c)
                        &c.tv.box, &c.tv.keys, &c.tv.keys2, &c.tv.ids, &c.tv.ids2, &c.tv.nodes, &c.tv.info, &c.tv.root,
                        &c.te.box, &c.te.keys, &c.te.keys2, &c.te.ids, &c.te.ids2, &c.te.nodes, &c.te.info, &c.te.root,
                        &c.tf.box, &c.tf.keys, &c.tf.keys2, &c.tf.ids, &c.tf.ids2, &c.tf.nodes, &c.tf.info, &c.tf.root,
-                       &c.aabb_partial, &c.aabb, &c.sort_tmp, &c.cand_ee, &c.cand_fv, &c.counters,
+                       &c.aabb_partial, &c.aabb, &c.sort_space.status, &c.sort_space.ticket, &c.sort_space.hist, &c.cand_ee, &c.cand_fv, &c.counters,
                        &c.c_ids[0], &c.c_ids[1], &c.c_ids[2], &c.c_ids[3], &c.c_w[0], &c.c_w[1], &c.c_w[2], &c.c_w[3],
                        &c.c_eps, &c.c_dtype, &c.np_keys, &c.np_keys2, &c.np_vals, &c.np_vals2, &c.np_ukeys,
                        &c.np_start, &c.np_tmp, &c.np_raw, &c.red_partial, &c.red_out, &c.grad, &c.hq,

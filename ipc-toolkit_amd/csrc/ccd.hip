@@ -935,18 +935,17 @@ bool wf_batch(Ctx& c, const CCDArgs& A, const uint32_t* heavy, int64_t first, in
         uint32_t* off = c.blk_vals2.as<uint32_t>();
         uint32_t* live = c.wf_live.as<uint32_t>();
         uint32_t* lpre = c.wf_lpre.as<uint32_t>();
-        c.blk_tmp.reserve(scan_tmp_bytes(nbox + 1));
         const unsigned gb = grid_for(nbox, 256, INT32_MAX);
         hipLaunchKernelGGL(k_wf_eval, dim3(gb), dim3(256), 0, s, A, states, cur, nbox, flags, live,
                            error, npend, nroot);
-        exclusive_scan_u32(live, lpre, nbox, lpre + nbox, c.blk_tmp.p, s);
+        exclusive_scan_u32(c.sort_space, live, lpre, nbox, lpre + nbox, s);
         hipLaunchKernelGGL(k_wf_mark, dim3(gb), dim3(256), 0, s, states, cur, nbox, flags, lpre,
                            ev);
         hipLaunchKernelGGL(k_wf_decide, dim3(grid_for(nb, 256)), dim3(256), 0, s, A, states, nb,
                            cur, lpre, ev, error);
         hipLaunchKernelGGL(k_wf_counts, dim3(gb), dim3(256), 0, s, states, cur, flags, nbox, cmask,
                            cnt);
-        exclusive_scan_u32(cnt, off, nbox, off + nbox, c.blk_tmp.p, s);
+        exclusive_scan_u32(c.sort_space, cnt, off, nbox, off + nbox, s);
         hipLaunchKernelGGL(k_wf_nochild, dim3(grid_for(nb, 256)), dim3(256), 0, s, A, states, nb,
                            off, nbox, npend);
         IPCG_CHECK_LAUNCH();
@@ -1082,10 +1081,11 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                        c.ccd_stage.as<uint32_t>());
     IPCG_CHECK_LAUNCH();
     c.shard_sum.reserve(256);
-    const ShardCounts rc = shard_counts(RS.cnt, c.shard_sum.as<unsigned long long>(), c.pinned, s);
+    const ShardCounts rc = shard_counts(RS.cnt, c.shard_sum.as<unsigned long long>(),
+                                        c.shard_off.as<int64_t>(), c.pinned, s);
     if (rc.max > scap) throw Error(IPCG_ERR_NUMERIC, "CCD root pass outgrew its shard");
     c.ccd_todo.reserve(sizeof(uint32_t) * (size_t)std::max<int64_t>(rc.total, 1));
-    shard_compact(c.ccd_stage.as<uint32_t>(), scap, RS.cnt, rc.max, c.ccd_todo.as<uint32_t>(),
+    shard_compact(c.ccd_stage.as<uint32_t>(), scap, rc.max, c.ccd_todo.as<uint32_t>(),
                   c.shard_off.as<int64_t>(), s);
     c.stage_end();
     const int64_t n_todo = rc.total;
@@ -1183,7 +1183,6 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         h[512 / 8 + N_HEAVY] += (unsigned long long)m;
     };
     auto wavefront = [&](int64_t nh) {
-        c.stat["ccd.wavefront"] += nh;
         c.stage_begin("ccd_wavefront");
         DevBuf& wst = c.ccd_bound; // per-candidate wavefront state
         wst.reserve(sizeof(WFState) * (size_t)std::min<int64_t>(nh, WF_BATCH_MAX));
@@ -1263,6 +1262,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         }
         c.stat["ccd.spilled"] += count(N_SPILL_A) + count(N_SPILL_B);
         c.stat["ccd.spilled_deep"] += count(N_SPILL_A_DEEP) + count(N_SPILL_B_DEEP);
+        c.stat["ccd.wavefront"] += count(N_OVER);
         const int64_t nh = count(N_HEAVY);
         if (nh > 0) wavefront(nh);
     };

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "sort.hpp"
 
 #include <map>
 #include <string>
@@ -99,7 +100,7 @@ struct Ctx {
     // broad phase
     Tree tv, te, tf, tcv, tce;
     DevBuf aabb_partial, aabb; // mesh bounds
-    DevBuf sort_tmp;
+    SortSpace sort_space; // scans, sorts and run lengths
     bool cand_valid = false, cand_swept = false;
     DevBuf cand_ee, cand_fv;   // int2 pairs
     DevBuf counters;           // uint64 counters (device)

@@ -299,34 +299,103 @@ __global__ __launch_bounds__(NP_BLOCK) void k_classify(
     }
 }
 
-__global__ void k_iota(uint32_t* v, int64_t n)
+// ---- merge -------------------------------------------------------------------
+// The four streams share every launch of the merge: kind k's contributions
+// are items [off[k], off[k + 1]) of the key arrays.
+struct Merge {
+    int64_t off[5];
+    uint64_t* keys;
+    EERec* ee;   // packed edge-edge records
+    double* cw;  // packed vertex-vertex / edge-vertex weights (real-valued weights only)
+    bool typed;  // edge-edge keys with the distance type
+};
+
+// (min edge, max edge, distance type); edge ids < 2^30
+__device__ __forceinline__ uint64_t ee_typed_key(const EERec& r)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) v[i] = (uint32_t)i;
+    const uint32_t a = (uint32_t)r.ea, b = (uint32_t)r.eb;
+    const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
+    return (lo << 34) | (hi << 4) | (uint64_t)r.dtype;
 }
 
-__global__ void k_ee_keys(const EERec* r, int64_t n, uint64_t* keys, uint32_t* vals)
+// Packs the shard regions of the streams (blockIdx.z: kind, y: shard) and
+// forms the edge-edge keys.  shard_off: SHARDS + 1 offsets per kind.
+__global__ __launch_bounds__(256) void k_merge_gather(Streams S, const int64_t* shard_off, Merge M)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        keys[i] = vv_key(r[i].ea, r[i].eb);
-        vals[i] = (uint32_t)i;
+    const int kind = blockIdx.z, sh = blockIdx.y;
+    const int64_t* const so = shard_off + kind * (SHARDS + 1);
+    const int64_t first = so[sh], m = so[sh + 1] - first;
+    const int64_t in = (int64_t)sh * S.scap, out = M.off[kind] + first;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const int64_t j = (int64_t)blockIdx.x * 1024 + 256 * c + threadIdx.x;
+        if (j >= m) continue;
+        if (kind == 2) {
+            const EERec r = S.ee[in + j];
+            M.ee[first + j] = r;
+            M.keys[out + j] = M.typed ? ee_typed_key(r) : vv_key(r.ea, r.eb);
+        } else {
+            M.keys[out + j] = (kind == 0 ? S.vv : kind == 1 ? S.ev : S.fv)[in + j];
+            if (M.cw && kind < 2) M.cw[out + j] = (kind == 0 ? S.vvw : S.evw)[in + j];
+        }
     }
 }
 
-__global__ void k_ee_gather(const EERec* r, const uint32_t* perm, int64_t n, int2* ids, double* w,
-                            double* eps, int32_t* dtype)
+// keys of edge-edge records appended after the streams'
+__global__ void k_ee_typed_keys(const EERec* r, int64_t n, uint64_t* keys)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        const EERec e = r[perm[i]];
-        ids[i] = make_int2(e.ea, e.eb);
-        w[i] = e.w;
-        eps[i] = e.eps_x;
-        dtype[i] = e.dtype;
+    if (i < n) keys[i] = ee_typed_key(r[i]);
+}
+
+// The merged set with plain counts as weights: runs of equal vertex-vertex
+// and edge-vertex keys; edge-edge and face-vertex contributions are unique.
+struct Merged {
+    const uint64_t* keys[4]; // sorted (0, 1: unique)
+    const uint32_t* perm;    // edge-edge: record per sorted item
+    const uint32_t *start[2], *nu[2];
+    int64_t n[4];
+    const EERec* ee;
+    Areas A;
+    int2* ids[4];
+    double* w[4];
+    double* eps;
+    int32_t* dtype;
+    unsigned group[5]; // workgroups of each kind
+};
+
+__global__ __launch_bounds__(256) void k_merge_out(Merged M)
+{
+    const int kind = blockIdx.x < M.group[1] ? 0
+        : blockIdx.x < M.group[2]            ? 1
+        : blockIdx.x < M.group[3]            ? 2
+                                             : 3;
+    const unsigned g0 = kind == 0 ? 0 : kind == 1 ? M.group[1] : kind == 2 ? M.group[2] : M.group[3];
+    const int64_t i = (int64_t)(blockIdx.x - g0) * 256 + threadIdx.x;
+    if (kind == 2) {
+        if (i >= M.n[2]) return;
+        const EERec e = M.ee[M.perm[i]];
+        M.ids[2][i] = make_int2(e.ea, e.eb);
+        M.w[2][i] = e.w;
+        M.eps[i] = e.eps_x;
+        M.dtype[i] = e.dtype;
+    } else if (kind == 3) {
+        if (i >= M.n[3]) return;
+        const uint64_t k = M.keys[3][i];
+        const int vi = (int)(k & 0xFFFFFFFFu);
+        M.ids[3][i] = make_int2((int)(k >> 32), vi);
+        M.w[3][i] = M.A.va ? 0.25 * M.A.va[vi] : 1.0;
+    } else {
+        const bool ev = kind == 1;
+        if (i >= (ev ? M.n[1] : M.n[0]) || i >= (int64_t)*(ev ? M.nu[1] : M.nu[0])) return;
+        const uint64_t k = (ev ? M.keys[1] : M.keys[0])[i];
+        const uint32_t* const st = ev ? M.start[1] : M.start[0];
+        (ev ? M.ids[1] : M.ids[0])[i] = make_int2((int)(k >> 32), (int)(k & 0xFFFFFFFFu));
+        (ev ? M.w[1] : M.w[0])[i] = (double)(st[i + 1] - st[i]);
     }
 }
 
+// face-vertex output of a real-valued merge
 __global__ void k_keys_to_pairs(const uint64_t* keys, int64_t n, Areas A, int2* ids, double* w)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -334,16 +403,6 @@ __global__ void k_keys_to_pairs(const uint64_t* keys, int64_t n, Areas A, int2* 
         const int vi = (int)(keys[i] & 0xFFFFFFFFu);
         ids[i] = make_int2((int)(keys[i] >> 32), vi);
         w[i] = A.va ? 0.25 * A.va[vi] : 1.0;
-    }
-}
-
-__global__ void k_runs_to_weights(const uint64_t* ukeys, const uint32_t* start, const uint32_t* nu,
-                                  int2* ids, double* w)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < (int64_t)*nu) {
-        ids[i] = make_int2((int)(ukeys[i] >> 32), (int)(ukeys[i] & 0xFFFFFFFFu));
-        w[i] = (double)(start[i + 1] - start[i]);
     }
 }
 
@@ -397,18 +456,6 @@ __global__ void k_run_scatter(const uint64_t* ukeys, int64_t nu, const double* r
     if (i < nu && keep[i]) {
         ids[pos[i]] = make_int2((int)(ukeys[i] >> 32), (int)(ukeys[i] & 0xFFFFFFFFu));
         w[pos[i]] = rw[i];
-    }
-}
-
-// edge-edge merge key: (min edge, max edge, distance type); edge ids < 2^30
-__global__ void k_ee_typed_keys(const EERec* r, int64_t n, uint64_t* keys, uint32_t* vals)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        const uint32_t a = (uint32_t)r[i].ea, b = (uint32_t)r[i].eb;
-        const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
-        keys[i] = (lo << 34) | (hi << 4) | (uint64_t)r[i].dtype;
-        vals[i] = (uint32_t)i;
     }
 }
 
@@ -504,12 +551,6 @@ __global__ __launch_bounds__(NP_BLOCK) void k_conv_slots(
     }
     const unsigned long long at = wave_append(count, nk);
     for (unsigned j = 0; j < nk; j++) out[at + j] = k[j];
-}
-
-__global__ void k_iota_u32(uint32_t* v, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) v[i] = (uint32_t)i;
 }
 
 struct ImOut {
@@ -667,6 +708,9 @@ static void improved_records(Ctx& c, double active2, Areas A, int64_t x[3])
     uint32_t* nu_dev = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 8);
     uint32_t* tot_dev = nu_dev + 2; // three totals
     uint64_t* slot = c.im_slot.as<uint64_t>();
+    // two tag bits above (id << 32 | id)
+    const int ibits = key_bits_for(std::max<int64_t>(c.nV, c.nE)) - 32;
+    const unsigned long long slot_mask = (3ull << 62) | (low_bits(ibits) << 32) | low_bits(ibits);
     IPCG_HIP(hipMemsetAsync(n_act_dev, 0, sizeof(unsigned long long), s));
     hipLaunchKernelGGL(k_conv_slots, dim3(grid_for(nc, NP_BLOCK, INT32_MAX)), dim3(NP_BLOCK), 0, s,
                        c.X[0].as<double>(), c.nV, c.E.as<int32_t>(), c.F.as<int32_t>(),
@@ -684,14 +728,11 @@ static void improved_records(Ctx& c, double active2, Areas A, int64_t x[3])
     c.im_vals2.reserve(sizeof(uint32_t) * (size_t)nact);
     c.im_ukeys.reserve(sizeof(uint64_t) * (size_t)nact);
     c.im_start.reserve(sizeof(uint32_t) * ((size_t)nact + 1));
-    c.np_tmp.reserve(std::max({ radix_tmp_bytes(nact), rle_tmp_bytes(nact), scan_tmp_bytes(nact) }));
-    hipLaunchKernelGGL(k_iota_u32, dim3(grid_for(nact, 256, INT32_MAX)), dim3(256), 0, s,
-                       c.im_vals.as<uint32_t>(), nact);
-    IPCG_CHECK_LAUNCH();
-    radix_sort_pairs(slot, c.im_vals.as<uint32_t>(), c.im_slot2.as<uint64_t>(),
-                     c.im_vals2.as<uint32_t>(), nact, 64, c.np_tmp.p, s);
-    run_length_encode(slot, nact, c.im_ukeys.as<uint64_t>(), c.im_start.as<uint32_t>(), nu_dev,
-                      c.np_tmp.p, s);
+    if (radix_sort_pairs(c.sort_space, slot, c.im_vals.as<uint32_t>(), c.im_slot2.as<uint64_t>(),
+                         c.im_vals2.as<uint32_t>(), nact, slot_mask, true, s))
+        slot = c.im_slot2.as<uint64_t>();
+    run_length_encode(c.sort_space, slot, nact, c.im_ukeys.as<uint64_t>(),
+                      c.im_start.as<uint32_t>(), nu_dev, s);
     const int64_t nu = read_u32(c, nu_dev);
     c.im_cnt.reserve(sizeof(uint32_t) * 3 * (size_t)nu);
     c.im_off.reserve(sizeof(uint32_t) * 3 * (size_t)nu);
@@ -704,8 +745,8 @@ static void improved_records(Ctx& c, double active2, Areas A, int64_t x[3])
                        cnt, nu, O);
     IPCG_CHECK_LAUNCH();
     for (int k = 0; k < 3; k++)
-        exclusive_scan_u32(cnt + k * nu, c.im_off.as<uint32_t>() + k * nu, nu, tot_dev + k,
-                           c.np_tmp.p, s);
+        exclusive_scan_u32(c.sort_space, cnt + k * nu, c.im_off.as<uint32_t>() + k * nu, nu,
+                           tot_dev + k, s);
     uint32_t* h = static_cast<uint32_t*>(c.pinned);
     IPCG_HIP(hipMemcpyAsync(h, tot_dev, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     IPCG_HIP(hipStreamSynchronize(s));
@@ -773,7 +814,8 @@ void np_build(Ctx& c, double dhat, double dmin)
     ShardCounts kc[4];
     int64_t nraw[4];
     c.shard_sum.reserve(256);
-    shard_counts_n(S.cnt, 4, c.shard_sum.as<unsigned long long>(), c.pinned, s, kc);
+    shard_counts_n(S.cnt, 4, c.shard_sum.as<unsigned long long>(), c.shard_off.as<int64_t>(),
+                   c.pinned, s, kc);
     for (int k = 0; k < 4; k++) {
         if (kc[k].max > scap) throw Error(IPCG_ERR_NUMERIC, "collision stream outgrew its shard");
         nraw[k] = kc[k].total;
@@ -786,140 +828,154 @@ void np_build(Ctx& c, double dhat, double dmin)
     }
 
     c.stage_begin("np_merge");
-    int64_t mtot[4];
-    int64_t mx = 1;
+    int64_t m[4];
+    Merge M {};
+    int64_t longest = 0; // largest shard of any stream
     for (int k = 0; k < 4; k++) {
-        mtot[k] = nraw[k] + (k < 3 ? x[k] : 0);
-        mx = std::max(mx, mtot[k]);
+        m[k] = nraw[k] + (k < 3 ? x[k] : 0);
+        M.off[k + 1] = M.off[k] + m[k];
+        longest = std::max(longest, kc[k].max);
     }
-    c.np_keys.reserve(sizeof(uint64_t) * mx);
-    c.np_keys2.reserve(sizeof(uint64_t) * mx);
-    c.np_vals.reserve(sizeof(uint32_t) * mx);
-    c.np_vals2.reserve(sizeof(uint32_t) * mx);
-    c.np_ukeys.reserve(sizeof(uint64_t) * mx);
-    c.np_start.reserve(sizeof(uint32_t) * (mx + 1));
-    c.np_tmp.reserve(std::max({ radix_tmp_bytes(mx), rle_tmp_bytes(mx), scan_tmp_bytes(mx) }));
+    const int64_t mt = std::max<int64_t>(M.off[4], 1);
+    c.np_keys.reserve(sizeof(uint64_t) * mt);
+    c.np_keys2.reserve(sizeof(uint64_t) * mt);
+    c.np_vals.reserve(sizeof(uint32_t) * mt);
+    c.np_vals2.reserve(sizeof(uint32_t) * mt);
+    c.np_ukeys.reserve(sizeof(uint64_t) * mt);
+    c.np_start.reserve(sizeof(uint32_t) * (mt + 4));
+    c.np_eec.reserve(sizeof(EERec) * (size_t)std::max<int64_t>(m[2], 1));
     if (real_w) {
-        c.np_rw.reserve(sizeof(double) * mx);
-        c.np_flag.reserve(sizeof(uint32_t) * mx);
-        c.np_pos.reserve(sizeof(uint32_t) * (mx + 1));
-        c.np_rep.reserve(sizeof(uint32_t) * mx);
+        c.np_cw.reserve(sizeof(double) * mt);
+        c.np_rw.reserve(sizeof(double) * mt);
+        c.np_flag.reserve(sizeof(uint32_t) * mt);
+        c.np_pos.reserve(sizeof(uint32_t) * mt);
+        c.np_rep.reserve(sizeof(uint32_t) * mt);
     }
-    uint64_t* keys = c.np_keys.as<uint64_t>();
-    uint32_t* vals = c.np_vals.as<uint32_t>();
-    uint32_t* nu_dev = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 3);
-    uint32_t* kept_dev = nu_dev + 1;
-    // (id << 32 | id) keys: only the digits that hold id bits can vary, so
-    // the sorts below run those passes without reading the keys back
-    const int ibits = key_bits_for(std::max<int64_t>(std::max<int64_t>(c.nV, c.nE), c.nF)) - 32;
-    const unsigned long long id_mask = (1ull << ibits) - 1ull;
-    const unsigned long long pair_mask = id_mask | (id_mask << 32);
-    auto sort_pairs = [&](int64_t m) {
-        if (radix_sort_pairs_masked(keys, vals, c.np_keys2.as<uint64_t>(),
-                                    c.np_vals2.as<uint32_t>(), m, pair_mask, c.np_tmp.p, s)) {
-            std::swap(c.np_keys, c.np_keys2); // sorted pairs in the second buffers
-            std::swap(c.np_vals, c.np_vals2);
-            keys = c.np_keys.as<uint64_t>();
-            vals = c.np_vals.as<uint32_t>();
-        }
-    };
     for (int k = 0; k < 4; k++) {
-        const int64_t m0 = nraw[k], m = mtot[k];
-        c.c_ids[k].reserve(sizeof(int2) * (size_t)std::max<int64_t>(m, 1));
-        c.c_w[k].reserve(sizeof(double) * (size_t)std::max<int64_t>(m, 1));
-        if (k == 2) {
-            c.c_eps.reserve(sizeof(double) * (size_t)std::max<int64_t>(m, 1));
-            c.c_dtype.reserve(sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1));
-        }
-        c.ncoll[k] = 0;
-        if (m == 0) continue;
-        const unsigned g = grid_for(m, 256, INT32_MAX);
-        const unsigned long long* kcnt = S.cnt + (int64_t)k * SHARDS * SHARD_PAD;
-        int64_t* koff = c.shard_off.as<int64_t>() + k * (SHARDS + 1);
-        if (k == 2) {
-            c.np_eec.reserve(sizeof(EERec) * (size_t)m);
-            EERec* ee = c.np_eec.as<EERec>();
-            if (m0) shard_compact(S.ee, scap, kcnt, kc[k].max, ee, koff, s);
-            if (!real_w) { // one collision per edge-edge candidate: no duplicates
-                hipLaunchKernelGGL(k_ee_keys, dim3(g), dim3(256), 0, s, ee, m, keys, vals);
-                sort_pairs(m);
-                hipLaunchKernelGGL(k_ee_gather, dim3(g), dim3(256), 0, s, ee, vals, m,
-                                   c.c_ids[2].as<int2>(), c.c_w[2].as<double>(),
-                                   c.c_eps.as<double>(), c.c_dtype.as<int32_t>());
-                c.ncoll[2] = m;
-            } else {
-                if (x[2])
-                    IPCG_HIP(hipMemcpyAsync(ee + m0, c.im_ee.p, sizeof(EERec) * (size_t)x[2],
-                                            hipMemcpyDeviceToDevice, s));
-                hipLaunchKernelGGL(k_ee_typed_keys, dim3(g), dim3(256), 0, s, ee, m, keys, vals);
-                radix_sort_pairs(keys, vals, c.np_keys2.as<uint64_t>(), c.np_vals2.as<uint32_t>(),
-                                 m, 64, c.np_tmp.p, s);
-                run_length_encode(keys, m, c.np_ukeys.as<uint64_t>(), c.np_start.as<uint32_t>(),
-                                  nu_dev, c.np_tmp.p, s);
-                const int64_t nu = read_u32(c, nu_dev);
-                const unsigned gu = grid_for(nu, 256, INT32_MAX);
-                hipLaunchKernelGGL(k_ee_runs, dim3(gu), dim3(256), 0, s, c.np_start.as<uint32_t>(),
-                                   nu, vals, ee, c.np_rw.as<double>(), c.np_rep.as<uint32_t>(),
-                                   c.np_flag.as<uint32_t>());
-                exclusive_scan_u32(c.np_flag.as<uint32_t>(), c.np_pos.as<uint32_t>(), nu, kept_dev,
-                                   c.np_tmp.p, s);
-                hipLaunchKernelGGL(k_ee_scatter, dim3(gu), dim3(256), 0, s, ee, nu,
-                                   c.np_rw.as<double>(), c.np_rep.as<uint32_t>(),
-                                   c.np_flag.as<uint32_t>(), c.np_pos.as<uint32_t>(),
-                                   c.c_ids[2].as<int2>(), c.c_w[2].as<double>(),
-                                   c.c_eps.as<double>(), c.c_dtype.as<int32_t>());
-                IPCG_CHECK_LAUNCH();
-                c.ncoll[2] = read_u32(c, kept_dev);
-            }
-        } else {
-            const uint64_t* src = k == 0 ? S.vv : (k == 1 ? S.ev : S.fv);
-            if (m0) shard_compact(src, scap, kcnt, kc[k].max, keys, koff, s);
-            double* cw = nullptr; // compacted contribution weights
-            if (real_w && k < 2) {
-                c.np_cw.reserve(sizeof(double) * (size_t)m);
-                cw = c.np_cw.as<double>();
-                if (m0) shard_compact(k == 0 ? S.vvw : S.evw, scap, kcnt, kc[k].max, cw, koff, s);
-                if (x[k]) {
-                    IPCG_HIP(hipMemcpyAsync(keys + m0, k == 0 ? c.im_vv.p : c.im_ev.p,
-                                            sizeof(uint64_t) * (size_t)x[k], hipMemcpyDeviceToDevice, s));
-                    IPCG_HIP(hipMemcpyAsync(cw + m0, k == 0 ? c.im_vvw.p : c.im_evw.p,
-                                            sizeof(double) * (size_t)x[k], hipMemcpyDeviceToDevice, s));
-                }
-            }
-            hipLaunchKernelGGL(k_iota, dim3(g), dim3(256), 0, s, vals, m);
-            sort_pairs(m);
-            if (k == 3) { // each (face, vertex) candidate is unique
-                hipLaunchKernelGGL(k_keys_to_pairs, dim3(g), dim3(256), 0, s, keys, m, A,
-                                   c.c_ids[3].as<int2>(), c.c_w[3].as<double>());
-                c.ncoll[3] = m;
-            } else {
-                run_length_encode(keys, m, c.np_ukeys.as<uint64_t>(), c.np_start.as<uint32_t>(),
-                                  nu_dev, c.np_tmp.p, s);
-                if (cw) {
-                    const int64_t nu = read_u32(c, nu_dev);
-                    const unsigned gu = grid_for(nu, 256, INT32_MAX);
-                    hipLaunchKernelGGL(k_run_sums, dim3(gu), dim3(256), 0, s,
-                                       c.np_start.as<uint32_t>(), nu, vals, cw,
-                                       c.np_rw.as<double>(), c.np_flag.as<uint32_t>());
-                    exclusive_scan_u32(c.np_flag.as<uint32_t>(), c.np_pos.as<uint32_t>(), nu,
-                                       kept_dev, c.np_tmp.p, s);
-                    hipLaunchKernelGGL(k_run_scatter, dim3(gu), dim3(256), 0, s,
-                                       c.np_ukeys.as<uint64_t>(), nu, c.np_rw.as<double>(),
-                                       c.np_flag.as<uint32_t>(), c.np_pos.as<uint32_t>(),
-                                       c.c_ids[k].as<int2>(), c.c_w[k].as<double>());
-                    IPCG_CHECK_LAUNCH();
-                    c.ncoll[k] = read_u32(c, kept_dev);
-                } else {
-                    hipLaunchKernelGGL(k_runs_to_weights, dim3(g), dim3(256), 0, s,
-                                       c.np_ukeys.as<uint64_t>(), c.np_start.as<uint32_t>(), nu_dev,
-                                       c.c_ids[k].as<int2>(), c.c_w[k].as<double>());
-                    IPCG_CHECK_LAUNCH();
-                    c.ncoll[k] = read_u32(c, nu_dev);
-                }
-            }
-        }
+        c.c_ids[k].reserve(sizeof(int2) * (size_t)std::max<int64_t>(m[k], 1));
+        c.c_w[k].reserve(sizeof(double) * (size_t)std::max<int64_t>(m[k], 1));
+    }
+    c.c_eps.reserve(sizeof(double) * (size_t)std::max<int64_t>(m[2], 1));
+    c.c_dtype.reserve(sizeof(int32_t) * (size_t)std::max<int64_t>(m[2], 1));
+    M.keys = c.np_keys.as<uint64_t>();
+    M.ee = c.np_eec.as<EERec>();
+    M.cw = real_w ? c.np_cw.as<double>() : nullptr;
+    M.typed = real_w;
+    if (longest > 0) {
+        hipLaunchKernelGGL(k_merge_gather, dim3((unsigned)((longest + 1023) / 1024), SHARDS, 4),
+                           dim3(256), 0, s, S, c.shard_off.as<int64_t>(), M);
         IPCG_CHECK_LAUNCH();
     }
+    if (improved) { // the improved contributions follow each stream's
+        for (int k = 0; k < 2; k++) {
+            if (!x[k]) continue;
+            const int64_t at = M.off[k] + nraw[k];
+            IPCG_HIP(hipMemcpyAsync(M.keys + at, k == 0 ? c.im_vv.p : c.im_ev.p,
+                                    sizeof(uint64_t) * (size_t)x[k], hipMemcpyDeviceToDevice, s));
+            IPCG_HIP(hipMemcpyAsync(M.cw + at, k == 0 ? c.im_vvw.p : c.im_evw.p,
+                                    sizeof(double) * (size_t)x[k], hipMemcpyDeviceToDevice, s));
+        }
+        if (x[2]) {
+            IPCG_HIP(hipMemcpyAsync(M.ee + nraw[2], c.im_ee.p, sizeof(EERec) * (size_t)x[2],
+                                    hipMemcpyDeviceToDevice, s));
+            hipLaunchKernelGGL(k_ee_typed_keys, dim3(grid_for(x[2], 256, INT32_MAX)), dim3(256), 0,
+                               s, M.ee + nraw[2], x[2], M.keys + M.off[2] + nraw[2]);
+            IPCG_CHECK_LAUNCH();
+        }
+    }
+    // (id << 32 | id) keys: only the digits that hold id bits can vary
+    const int ibits = key_bits_for(std::max<int64_t>(std::max<int64_t>(c.nV, c.nE), c.nF)) - 32;
+    const unsigned long long pair_mask = low_bits(ibits) | (low_bits(ibits) << 32);
+    const unsigned long long typed_mask = 15ull | (low_bits(ibits) << 4) | (low_bits(ibits) << 34);
+    SortJob jobs[4];
+    for (int k = 0; k < 4; k++)
+        jobs[k] = { M.keys + M.off[k], c.np_keys2.as<uint64_t>() + M.off[k],
+                    c.np_vals.as<uint32_t>() + M.off[k], c.np_vals2.as<uint32_t>() + M.off[k],
+                    m[k], k == 2 && real_w ? typed_mask : pair_mask, true, false };
+    radix_sort_jobs(c.sort_space, jobs, 4, s);
+    const uint64_t* keys[4];
+    const uint32_t* perm[4];
+    for (int k = 0; k < 4; k++) {
+        keys[k] = static_cast<const uint64_t*>(jobs[k].in_alt ? jobs[k].keys_alt : jobs[k].keys);
+        perm[k] = jobs[k].in_alt ? jobs[k].vals_alt : jobs[k].vals;
+    }
+    uint32_t* nu_dev = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 3);
+    uint64_t* ukeys[3];
+    uint32_t* start[3];
+    for (int k = 0; k < 3; k++) {
+        ukeys[k] = c.np_ukeys.as<uint64_t>() + M.off[k];
+        start[k] = c.np_start.as<uint32_t>() + M.off[k] + k;
+        c.ncoll[k] = 0;
+        if (k < 2 || real_w)
+            run_length_encode(c.sort_space, keys[k], m[k], ukeys[k], start[k], nu_dev + k, s);
+    }
+    auto read_three = [&](const uint32_t* dev, int64_t* out) {
+        uint32_t* h = static_cast<uint32_t*>(c.pinned);
+        IPCG_HIP(hipMemcpyAsync(h, dev, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        IPCG_HIP(hipStreamSynchronize(s));
+        for (int k = 0; k < 3; k++) out[k] = h[k];
+    };
+    if (!real_w) {
+        Merged O {};
+        for (int k = 0; k < 4; k++) {
+            O.keys[k] = k < 2 ? ukeys[k] : keys[k];
+            O.n[k] = m[k];
+            O.ids[k] = c.c_ids[k].as<int2>();
+            O.w[k] = c.c_w[k].as<double>();
+            O.group[k + 1] = O.group[k] + (unsigned)((m[k] + 255) / 256);
+            if (k < 2) {
+                O.start[k] = start[k];
+                O.nu[k] = nu_dev + k;
+            }
+        }
+        O.perm = perm[2];
+        O.ee = M.ee;
+        O.A = A;
+        O.eps = c.c_eps.as<double>();
+        O.dtype = c.c_dtype.as<int32_t>();
+        if (O.group[4] > 0) {
+            hipLaunchKernelGGL(k_merge_out, dim3(O.group[4]), dim3(256), 0, s, O);
+            IPCG_CHECK_LAUNCH();
+        }
+        int64_t nu[3];
+        read_three(nu_dev, nu);
+        c.ncoll[0] = m[0] ? nu[0] : 0;
+        c.ncoll[1] = m[1] ? nu[1] : 0;
+        c.ncoll[2] = m[2]; // one collision per edge-edge candidate: no duplicates
+    } else {
+        int64_t nu[3];
+        read_three(nu_dev, nu);
+        uint32_t* const kept_dev = nu_dev + 3;
+        for (int k = 0; k < 3; k++) {
+            if (m[k] == 0) nu[k] = 0;
+            const unsigned gu = grid_for(nu[k], 256, INT32_MAX);
+            double* const rw = c.np_rw.as<double>() + M.off[k];
+            uint32_t* const flag = c.np_flag.as<uint32_t>() + M.off[k];
+            uint32_t* const pos = c.np_pos.as<uint32_t>() + M.off[k];
+            uint32_t* const rep = c.np_rep.as<uint32_t>() + M.off[k];
+            if (nu[k] && k == 2)
+                hipLaunchKernelGGL(k_ee_runs, dim3(gu), dim3(256), 0, s, start[k], nu[k], perm[k],
+                                   M.ee, rw, rep, flag);
+            else if (nu[k])
+                hipLaunchKernelGGL(k_run_sums, dim3(gu), dim3(256), 0, s, start[k], nu[k], perm[k],
+                                   M.cw + M.off[k], rw, flag);
+            exclusive_scan_u32(c.sort_space, flag, pos, nu[k], kept_dev + k, s);
+            if (nu[k] && k == 2)
+                hipLaunchKernelGGL(k_ee_scatter, dim3(gu), dim3(256), 0, s, M.ee, nu[k], rw, rep,
+                                   flag, pos, c.c_ids[2].as<int2>(), c.c_w[2].as<double>(),
+                                   c.c_eps.as<double>(), c.c_dtype.as<int32_t>());
+            else if (nu[k])
+                hipLaunchKernelGGL(k_run_scatter, dim3(gu), dim3(256), 0, s, ukeys[k], nu[k], rw,
+                                   flag, pos, c.c_ids[k].as<int2>(), c.c_w[k].as<double>());
+            IPCG_CHECK_LAUNCH();
+        }
+        if (m[3])
+            hipLaunchKernelGGL(k_keys_to_pairs, dim3(grid_for(m[3], 256, INT32_MAX)), dim3(256), 0,
+                               s, keys[3], m[3], A, c.c_ids[3].as<int2>(), c.c_w[3].as<double>());
+        IPCG_CHECK_LAUNCH();
+        read_three(kept_dev, c.ncoll);
+    }
+    c.ncoll[3] = m[3]; // each (face, vertex) candidate is unique
     c.stage_end();
     c.coll_dmin = dmin;
     c.coll_valid = true;

@@ -1185,8 +1185,7 @@ __device__ __forceinline__ uint64_t spread3(uint64_t v)
 }
 
 __global__ __launch_bounds__(256) void k_row_keys(const double* X, int nV, const int32_t* vscene,
-                                                  const double* aabb, uint64_t* keys,
-                                                  uint32_t* ids)
+                                                  const double* aabb, uint64_t* keys)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nV) return;
@@ -1206,7 +1205,6 @@ __global__ __launch_bounds__(256) void k_row_keys(const double* X, int nV, const
         code |= spread3((uint64_t)t) << (2 - k);
     }
     keys[i] = ((uint64_t)sc << 39) | code;
-    ids[i] = (uint32_t)i;
 }
 
 static void build_row_order(Ctx& c)
@@ -1219,16 +1217,17 @@ static void build_row_order(Ctx& c)
     c.ro_keys2.reserve(sizeof(uint64_t) * (size_t)n);
     c.ro_ids.reserve(sizeof(uint32_t) * (size_t)n);
     c.ro_ids2.reserve(sizeof(uint32_t) * (size_t)n);
-    c.blk_tmp.reserve(radix_tmp_bytes(n));
     hipLaunchKernelGGL(k_row_keys, dim3(grid_for(n, 256)), dim3(256), 0, s, c.X[0].as<double>(),
                        c.nV, c.batched() ? c.vscene.as<int32_t>() : nullptr, c.aabb.as<double>(),
-                       c.ro_keys.as<uint64_t>(), c.ro_ids.as<uint32_t>());
+                       c.ro_keys.as<uint64_t>());
     IPCG_CHECK_LAUNCH();
     int bits = 39;
     if (c.batched())
         while ((1ll << (bits - 39)) < c.n_scenes) bits++;
-    radix_sort_pairs(c.ro_keys.as<uint64_t>(), c.ro_ids.as<uint32_t>(), c.ro_keys2.as<uint64_t>(),
-                     c.ro_ids2.as<uint32_t>(), n, bits, c.blk_tmp.p, s);
+    if (radix_sort_pairs(c.sort_space, c.ro_keys.as<uint64_t>(), c.ro_ids.as<uint32_t>(),
+                         c.ro_keys2.as<uint64_t>(), c.ro_ids2.as<uint32_t>(), n, low_bits(bits),
+                         true, s))
+        std::swap(c.ro_ids, c.ro_ids2);
     c.ro_ready = true;
 }
 
@@ -1253,7 +1252,6 @@ void require_incidences(Ctx& c, const CollView& C, const CollRanges& G, int64_t 
     c.inc_vals.reserve(sizeof(uint32_t) * mk);
     c.inc_vals2.reserve(sizeof(uint32_t) * mk);
     c.inc_ptr.reserve(sizeof(uint32_t) * ((size_t)c.nV + 1));
-    c.blk_tmp.reserve(radix_tmp_bytes(mk));
     uint32_t* keys = c.inc_keys.as<uint32_t>();
     uint32_t* vals = c.inc_vals.as<uint32_t>();
     int64_t io = 0;
@@ -1267,8 +1265,8 @@ void require_incidences(Ctx& c, const CollView& C, const CollRanges& G, int64_t 
     IPCG_CHECK_LAUNCH();
     int vb = 1;
     while ((1ll << vb) <= c.nV) vb++;
-    if (radix_sort_pairs_all(keys, vals, c.inc_keys2.as<uint32_t>(), c.inc_vals2.as<uint32_t>(),
-                             M, vb, c.blk_tmp.p, s)) { // sorted pairs in the second buffers
+    if (radix_sort_pairs(c.sort_space, keys, vals, c.inc_keys2.as<uint32_t>(),
+                         c.inc_vals2.as<uint32_t>(), M, low_bits(vb), false, s)) { // sorted pairs in the second buffers
         std::swap(c.inc_keys, c.inc_keys2);
         std::swap(c.inc_vals, c.inc_vals2);
         keys = c.inc_keys.as<uint32_t>();
@@ -1341,8 +1339,6 @@ void hess_pattern(Ctx& c)
     c.blk_vals2.reserve(sizeof(uint32_t) * nk);
     c.blk_ukeys.reserve(sizeof(uint64_t) * nk);
     c.blk_start.reserve(sizeof(uint32_t) * (nk + 1));
-    c.blk_tmp.reserve(std::max(std::max(radix_tmp_bytes(nk), rle_tmp_bytes(nk)),
-                               scan_tmp_bytes(3 * (int64_t)c.nV + 1)));
     const size_t nv1 = (size_t)c.nV + 1;
     c.hp_mark.reserve(sizeof(uint32_t) * nv1 * 3);
     uint32_t* mark = c.hp_mark.as<uint32_t>();
@@ -1362,17 +1358,19 @@ void hess_pattern(Ctx& c)
     IPCG_CHECK_LAUNCH();
     int vb = 1;
     while ((1ll << vb) <= c.nV) vb++;
-    radix_sort_pairs(keys, vals, c.blk_keys2.as<uint64_t>(), c.blk_vals2.as<uint32_t>(), npair,
-                     32 + vb, c.blk_tmp.p, s);
+    if (radix_sort_pairs(c.sort_space, keys, vals, c.blk_keys2.as<uint64_t>(),
+                         c.blk_vals2.as<uint32_t>(), npair,
+                         low_bits(vb) | (low_bits(vb) << 32), false, s))
+        keys = c.blk_keys2.as<uint64_t>();
     uint32_t* nu_dev = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 9);
-    run_length_encode(keys, npair, c.blk_ukeys.as<uint64_t>(), c.blk_start.as<uint32_t>(), nu_dev,
-                      c.blk_tmp.p, s);
+    run_length_encode(c.sort_space, keys, npair, c.blk_ukeys.as<uint64_t>(),
+                      c.blk_start.as<uint32_t>(), nu_dev, s);
     hipLaunchKernelGGL(k_pair_degree, dim3(grid_for(nk, 256, INT32_MAX)), dim3(256), 0, s,
                        c.blk_ukeys.as<uint64_t>(), nu_dev, deg);
     hipLaunchKernelGGL(k_add_mark, dim3(grid_for(c.nV, 256)), dim3(256), 0, s, mark, c.nV, deg);
     c.hp_bptr.reserve(sizeof(uint32_t) * nv1);
     uint32_t* bptr = c.hp_bptr.as<uint32_t>();
-    exclusive_scan_u32(deg, bptr, c.nV, bptr + c.nV, c.blk_tmp.p, s);
+    exclusive_scan_u32(c.sort_space, deg, bptr, c.nV, bptr + c.nV, s);
     IPCG_CHECK_LAUNCH();
     uint32_t* h = static_cast<uint32_t*>(c.pinned);
     IPCG_HIP(hipMemcpyAsync(h, bptr + c.nV, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -1399,7 +1397,6 @@ bool hess_pattern_incidences(Ctx& c, int64_t M)
     c.blk_keys.reserve(sizeof(int32_t) * 4 * (size_t)std::max<int64_t>(M, 1));
     c.hp_mark.reserve(sizeof(uint32_t) * nv1 * 3);
     c.hp_bptr.reserve(sizeof(uint32_t) * nv1);
-    c.blk_tmp.reserve(scan_tmp_bytes(std::max<int64_t>(c.nV, 1)));
     uint32_t* cnt = c.hp_mark.as<uint32_t>();
     uint32_t* bptr = c.hp_bptr.as<uint32_t>();
     int32_t* stage = c.blk_keys.as<int32_t>();
@@ -1408,7 +1405,7 @@ bool hess_pattern_incidences(Ctx& c, int64_t M)
     const unsigned gw = grid_for((int64_t)c.nV * WAVE, 256, INT32_MAX); // a wave per vertex
     hipLaunchKernelGGL(k_pattern_rows, dim3(gw), dim3(256), 0, s, c.inc_ptr.as<uint32_t>(),
                        c.inc_vtx.as<int4>(), c.nV, stage, cnt, ovf);
-    exclusive_scan_u32(cnt, bptr, c.nV, bptr + c.nV, c.blk_tmp.p, s);
+    exclusive_scan_u32(c.sort_space, cnt, bptr, c.nV, bptr + c.nV, s);
     IPCG_CHECK_LAUNCH();
     uint32_t* h = static_cast<uint32_t*>(c.pinned);
     IPCG_HIP(hipMemcpyAsync(h, bptr + c.nV, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -1477,10 +1474,9 @@ void pot_hessian(Ctx& c, double dhat, double kappa, int psd)
         uint32_t* flag = c.ee_other.as<uint32_t>();
         uint32_t* pos = flag + ne;
         uint32_t* list = pos + ne;
-        c.blk_tmp.reserve(scan_tmp_bytes(ne));
         hipLaunchKernelGGL(k_ee_other_flags, dim3(grid_for(ne, 256, INT32_MAX)), dim3(256), 0, s, C.dtype, ne, flag);
         uint32_t* n_other = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 11);
-        exclusive_scan_u32(flag, pos, ne, n_other, c.blk_tmp.p, s);
+        exclusive_scan_u32(c.sort_space, flag, pos, ne, n_other, s);
         hipLaunchKernelGGL(k_ee_other_list, dim3(grid_for(ne, 256, INT32_MAX)), dim3(256), 0, s, flag, pos, ne, list);
         IPCG_CHECK_LAUNCH();
         uint32_t* h = static_cast<uint32_t*>(c.pinned);

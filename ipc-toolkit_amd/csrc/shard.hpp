@@ -48,47 +48,40 @@ struct ShardCounts {
 };
 
 // Counts of the last producer launch over nsets consecutive counter sets
-// (set k at cnt_dev + k * SHARDS * SHARD_PAD): each set's total and largest
-// shard are reduced on the device into sum_dev (2 * nsets u64) and read
-// back in one small copy with one synchronisation of the stream, together
-// with *extra_dev when it is given.
+// (set k at cnt_dev + k * SHARDS * SHARD_PAD): one launch leaves the
+// exclusive offsets of each set's shards in off_dev (SHARDS + 1 int64 per
+// set) and reduces each set's total and largest shard into sum_dev (2 * nsets
+// u64, then *extra_dev), read back in one small copy with one synchronisation
+// of the stream.
 ShardCounts shard_counts(const unsigned long long* cnt_dev, unsigned long long* sum_dev,
-                         void* pinned, hipStream_t s);
+                         int64_t* off_dev, void* pinned, hipStream_t s);
 void shard_counts_n(const unsigned long long* cnt_dev, int nsets, unsigned long long* sum_dev,
-                    void* pinned, hipStream_t s, ShardCounts* out, const int* extra_dev = nullptr,
-                    int* extra = nullptr);
-
-// exclusive offsets of the shard counts, each clipped to scap (SHARDS + 1
-// int64 on the device)
-void shard_offsets(const unsigned long long* cnt_dev, int64_t scap, int64_t* off_dev,
-                   hipStream_t s);
+                    int64_t* off_dev, void* pinned, hipStream_t s, ShardCounts* out,
+                    const int* extra_dev = nullptr, int* extra = nullptr);
 
 template <class T>
-__global__ __launch_bounds__(256) void k_shard_copy(const T* in, int64_t scap,
-                                                    const unsigned long long* cnt,
-                                                    const int64_t* off, T* out)
+__global__ __launch_bounds__(256) void k_shard_copy(const T* in, int64_t scap, const int64_t* off,
+                                                    T* out)
 {
     const int sh = blockIdx.y;
-    const int64_t n = (int64_t)cnt[(int64_t)sh * SHARD_PAD];
-    const int64_t lim = n < scap ? n : scap;
+    const int64_t first = off[sh], n = off[sh + 1] - first;
     const int64_t base = (int64_t)blockIdx.x * 1024 + threadIdx.x;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int64_t j = base + 256 * k;
-        if (j < lim) out[off[sh] + j] = in[(int64_t)sh * scap + j];
+        if (j < n) out[first + j] = in[(int64_t)sh * scap + j];
     }
 }
 
-// Packs the shard regions of `in` into `out` (off_dev: SHARDS + 1 int64).
+// Packs the shard regions of `in` into `out` (off_dev: SHARDS + 1 offsets,
+// no shard larger than scap; max_count: the largest shard).
 template <class T>
-void shard_compact(const T* in, int64_t scap, const unsigned long long* cnt_dev, int64_t max_count,
-                   T* out, int64_t* off_dev, hipStream_t s)
+void shard_compact(const T* in, int64_t scap, int64_t max_count, T* out, const int64_t* off_dev,
+                   hipStream_t s)
 {
     if (max_count <= 0) return;
-    shard_offsets(cnt_dev, scap, off_dev, s);
-    const int64_t m = std::min<int64_t>(max_count, scap);
-    hipLaunchKernelGGL(k_shard_copy<T>, dim3((unsigned)((m + 1023) / 1024), SHARDS), dim3(256), 0,
-                       s, in, scap, cnt_dev, off_dev, out);
+    hipLaunchKernelGGL(k_shard_copy<T>, dim3((unsigned)((max_count + 1023) / 1024), SHARDS),
+                       dim3(256), 0, s, in, scap, off_dev, out);
     IPCG_CHECK_LAUNCH();
 }
 

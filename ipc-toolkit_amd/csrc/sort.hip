@@ -1,18 +1,33 @@
 // Device-wide scan, stable LSD radix sort and run-length encoding.
 //
-// Radix sort pass (8-bit digit, 256-thread blocks, 2048-key tiles):
-//   1. per-tile digit histogram (LDS atomics) -> counts[digit][tile]
-//   2. exclusive scan of counts in digit-major order -> tile base offsets
-//   3. per-tile stable ranking: each wave owns 512 consecutive keys, ranks
-//      a 64-key chunk at a time by matching digits with 8 ballots, keeps a
-//      running per-digit count in LDS; wave counts are prefix-summed across
-//      the block, then every key is written to base + wave prefix + rank.
-// 64-bit or 32-bit keys.  Passes whose digit is constant over all keys are
-// skipped where the caller asks for it (a read-back of the varying bits).
+// Scans, run lengths and sort passes read their input once and run in one
+// launch each: a tile publishes its own sum, then adds up the sums of the
+// tiles before it until it meets one that already knows its prefix
+// (decoupled look-back, Merrill & Garland 2016).  Tiles take their index
+// from an atomic ticket, so a tile only ever waits for tiles that are already
+// running and publish without waiting for anything.  A published word holds
+// the launch's epoch, its state and the value together: one relaxed 64-bit
+// atomic, no fences (on gfx950 a device-scope fence writes back and
+// invalidates an L2), and no clearing between launches.
+//
+// Radix sort (8-bit digits): jobs (independent arrays) share every launch.
+// Arrays of up to SB_MAX keys are sorted by one workgroup in LDS, all
+// digits in one launch.  Larger ones take one histogram launch for all
+// digits and one launch per digit over tiles of keys: each wave owns
+// consecutive keys, ranks a 64-key chunk at a time by matching digits with 8
+// ballots and keeps a running per-digit count in LDS; wave counts are
+// prefix-summed across the workgroup, the look-back (a thread per digit) gives
+// the tile's first slot of every digit, and the keys leave in digit order
+// through LDS.  Tiles hold 2048 keys (short arrays: more workgroups) or,
+// past BIG_TILES of those, 4096 64-bit or 8192 32-bit keys: a ticket takes
+// about 12 ns whatever the width of the launch (75 M 32-bit keys: 0.49 ms
+// a pass, 0.82 ms with 2048-key tiles, 0.76 ms in the three launches before).
+//
+// The form before took three to five launches per digit and array.  Three
+// Morton arrays (8 K, 24 K and 16 K keys): 0.42 ms in 88 launches before,
+// 0.15 ms in 10 now; 6.3 M, 4.2 M and 2.1 M keys: 1.30 ms before, 1.17 ms now.
 #include "shard.hpp"
 #include "sort.hpp"
-
-#include <utility>
 
 namespace ipcg {
 
@@ -136,9 +151,11 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_one(const T* in, T* out, in
     if (threadIdx.x == 0 && total) *total = tot;
 }
 
-template <class T>
-void exclusive_scan(const T* in, T* out, int64_t n, T* total, void* tmp, hipStream_t s)
+// u64 sums (two packed counts) do not fit a look-back word: three launches
+void scan_three(const uint64_t* in, uint64_t* out, int64_t n, uint64_t* total, void* tmp,
+                hipStream_t s)
 {
+    using T = uint64_t;
     const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
     T* partial = static_cast<T*>(tmp);
     if (n <= 0) {
@@ -158,156 +175,446 @@ void exclusive_scan(const T* in, T* out, int64_t n, T* total, void* tmp, hipStre
     IPCG_CHECK_LAUNCH();
 }
 
+// ---- look-back ---------------------------------------------------------------
+// word: epoch (30 bits) | state (2 bits) | value (32 bits)
+constexpr unsigned LB_SUM = 1, LB_PREFIX = 2;
+
+__device__ __forceinline__ void lb_publish(unsigned long long* w, unsigned epoch, unsigned state,
+                                           uint32_t value)
+{
+    __hip_atomic_store(w, ((unsigned long long)(epoch << 2 | state) << 32) | value,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sum of the values of tiles 0 .. tile - 1, word k at w[k * stride].  All
+// tiles in flight publish their sums at about the same time, so a tile walks
+// back over many of them: LB_WINDOW words are read at once (one memory round
+// trip) and used as far as they are there.
+constexpr int LB_WINDOW = 8;
+
+__device__ __forceinline__ uint32_t lb_before(const unsigned long long* w, int64_t stride,
+                                              int64_t tile, unsigned epoch)
+{
+    uint32_t sum = 0;
+    bool done = tile == 0;
+    for (int64_t k = tile - 1; !done;) {
+        unsigned long long x[LB_WINDOW];
+#pragma unroll
+        for (int j = 0; j < LB_WINDOW; j++) {
+            const int64_t at = k - j > 0 ? k - j : 0;
+            x[j] = __hip_atomic_load(w + at * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        bool there = true;
+        int used = 0;
+#pragma unroll
+        for (int j = 0; j < LB_WINDOW; j++) {
+            const unsigned tag = (unsigned)(x[j] >> 32);
+            there = there && !done && tag >> 2 == epoch;
+            if (there) {
+                sum += (uint32_t)x[j];
+                used++;
+                done = (tag & 3u) == LB_PREFIX; // tile 0 publishes its prefix
+            }
+        }
+        if (used == 0) __builtin_amdgcn_s_sleep(1); // the next word is not there yet
+        k -= used;
+    }
+    return sum;
+}
+
+// The same for one value per tile, read by a whole wave: 64 words at once.
+__device__ __forceinline__ uint32_t lb_before_wave(const unsigned long long* w, int64_t tile,
+                                                   unsigned epoch)
+{
+    uint32_t sum = 0;
+    for (int64_t k = tile - 1; k >= 0;) {
+        const int64_t at = k - lane_id();
+        const unsigned long long x = at >= 0
+            ? __hip_atomic_load(w + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+            : 0ull;
+        const unsigned tag = (unsigned)(x >> 32);
+        const unsigned long long there = __ballot(at >= 0 && tag >> 2 == epoch);
+        const unsigned long long prefix =
+            __ballot(at >= 0 && tag >> 2 == epoch && (tag & 3u) == LB_PREFIX);
+        // words up to the first one missing, or up to the first prefix
+        int m = __builtin_ctzll(~there | (1ull << 63));
+        if (there == ~0ull) m = WAVE;
+        const int p = prefix ? __ffsll((long long)prefix) - 1 : WAVE;
+        const bool done = p < m;
+        const int use = done ? p + 1 : m;
+        uint32_t v = lane_id() < use ? (uint32_t)x : 0u;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+        sum += v;
+        if (done) break;
+        if (use == 0) __builtin_amdgcn_s_sleep(1);
+        k -= use;
+    }
+    return sum;
+}
+
+// This workgroup's tile; the last ticket of a launch winds the counter back
+// for the next.  Every thread must call it.
+__device__ __forceinline__ int64_t lb_ticket(unsigned* ticket, unsigned tiles)
+{
+    __shared__ unsigned t;
+    if (threadIdx.x == 0) {
+        t = atomicAdd(ticket, 1u);
+        if (t == tiles - 1)
+            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return t;
+}
+
+// exclusive prefix of this tile's total over the tiles before it, the same in
+// every thread
+__device__ __forceinline__ uint32_t lb_scan(unsigned long long* w, int64_t tile, uint32_t total,
+                                            unsigned epoch)
+{
+    __shared__ uint32_t before;
+    if (threadIdx.x < WAVE) {
+        if (threadIdx.x == 0) lb_publish(w + tile, epoch, tile ? LB_SUM : LB_PREFIX, total);
+        const uint32_t b = lb_before_wave(w, tile, epoch);
+        if (threadIdx.x == 0) {
+            if (tile) lb_publish(w + tile, epoch, LB_PREFIX, b + total);
+            before = b;
+        }
+    }
+    __syncthreads();
+    return before;
+}
+
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan(const uint32_t* in, uint32_t* out, int64_t n,
+                                                     uint32_t* total, unsigned long long* w,
+                                                     unsigned* ticket, unsigned epoch)
+{
+    const int64_t tile = lb_ticket(ticket, gridDim.x);
+    const int64_t base = tile * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    uint32_t v[SCAN_ITEMS];
+    uint32_t s = 0;
+#pragma unroll
+    for (int j = 0; j < SCAN_ITEMS; j++) {
+        v[j] = base + j < n ? in[base + j] : 0;
+        s += v[j];
+    }
+    uint32_t tot;
+    uint32_t off = block_exclusive_scan<uint32_t>(s, tot);
+    const uint32_t before = lb_scan(w, tile, tot, epoch);
+    off += before;
+#pragma unroll
+    for (int j = 0; j < SCAN_ITEMS; j++) {
+        if (base + j < n) out[base + j] = off;
+        off += v[j];
+    }
+    if (threadIdx.x == 0 && total && tile == (int64_t)gridDim.x - 1) *total = before + tot;
+}
+
+// Sorted keys -> unique keys, first position of each run (start[number of
+// runs] = n) and the number of runs.
+__global__ __launch_bounds__(SCAN_BLOCK) void k_rle(const uint64_t* keys, int64_t n,
+                                                    uint64_t* ukeys, uint32_t* start, uint32_t* nu,
+                                                    unsigned long long* w, unsigned* ticket,
+                                                    unsigned epoch)
+{
+    const int64_t tile = lb_ticket(ticket, gridDim.x);
+    const int64_t base = tile * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    uint64_t k[SCAN_ITEMS];
+    bool head[SCAN_ITEMS];
+    uint32_t s = 0;
+    uint64_t prev = base > 0 && base < n ? keys[base - 1] : 0;
+#pragma unroll
+    for (int j = 0; j < SCAN_ITEMS; j++) {
+        const int64_t i = base + j;
+        k[j] = i < n ? keys[i] : 0;
+        head[j] = i < n && (i == 0 || k[j] != prev);
+        prev = k[j];
+        s += head[j];
+    }
+    uint32_t tot;
+    uint32_t off = block_exclusive_scan<uint32_t>(s, tot);
+    const uint32_t before = lb_scan(w, tile, tot, epoch);
+    off += before;
+#pragma unroll
+    for (int j = 0; j < SCAN_ITEMS; j++)
+        if (head[j]) {
+            ukeys[off] = k[j];
+            start[off] = (uint32_t)(base + j);
+            off++;
+        }
+    if (threadIdx.x == 0 && tile == (int64_t)gridDim.x - 1) {
+        *nu = before + tot;
+        start[before + tot] = (uint32_t)n;
+    }
+}
+
 // ---------------------------------------------------------------------------
 constexpr int RS_BLOCK = 256;
 constexpr int RS_WAVES = RS_BLOCK / WAVE;
 constexpr int RS_CHUNKS = 8; // 64-key chunks per wave
 constexpr int RS_TILE = RS_BLOCK * RS_CHUNKS;
+constexpr int BIG_BLOCK = 512;
+constexpr int64_t BIG_TILES = 2048;
+template <class K> constexpr int big_chunks() { return sizeof(K) == 8 ? 8 : 16; }
 
-template <class K>
-__global__ __launch_bounds__(RS_BLOCK) void k_radix_hist(const K* keys, int64_t n, int shift,
-                                                         uint32_t* counts, int64_t ntiles)
+constexpr int MAX_DIGITS = 8;
+
+// one array of a sort as the kernels see it
+struct KeyJob {
+    const void* keys;
+    const uint32_t* vals; // null: the positions
+    void* okeys;
+    uint32_t* ovals;
+    int64_t n;
+    unsigned long long mask;       // bits that may vary
+    int64_t tile0, ntiles;         // its tiles of the launch
+    int shift;                     // this launch's digit, -1: none
+    const uint32_t* hist;          // counts of that digit
+    unsigned long long* status;    // look-back words, 256 per tile
+};
+struct KeyJobs {
+    KeyJob j[SORT_JOBS];
+    int n;
+};
+
+// Ranks 64 keys by digit among the wave's keys so far: lanes of one digit
+// count up from wcnt[d] (the wave's running counts).
+__device__ __forceinline__ uint32_t wave_rank(uint32_t d, bool valid, uint32_t* wcnt,
+                                              unsigned long long lt)
 {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+    unsigned long long peers = __ballot(valid);
 #pragma unroll
-    for (int j = 0; j < RS_CHUNKS; j++) {
-        const int64_t i = base + (int64_t)j * RS_BLOCK + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xFF], 1u);
+    for (int b = 0; b < 8; b++) {
+        const unsigned long long m = __ballot((d >> b) & 1);
+        peers &= ((d >> b) & 1) ? m : ~m;
     }
-    __syncthreads();
-    counts[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    const uint32_t r = (uint32_t)__popcll(peers & lt);
+    const uint32_t before = valid ? wcnt[d] : 0;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && r == 0) wcnt[d] = before + (uint32_t)__popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+    return before + r;
 }
 
-// Stable scatter of one 8-bit digit.  Each wave ranks its keys per digit
-// with ballots; the block turns the per-wave counts into offsets, places
-// the tile's keys in LDS in digit order, and writes each digit's run to its
-// global range so that neighbouring lanes write neighbouring addresses.
-template <class K>
-__global__ __launch_bounds__(RS_BLOCK) void k_radix_scatter(
-    const K* keys, const uint32_t* vals, K* okeys, uint32_t* ovals, int64_t n, int shift,
-    const uint32_t* offsets, int64_t ntiles)
+// Per digit d (threads 0 .. 255): wave counts -> offsets within the digit;
+// dstart[d] = first slot of the digit in the tile.  Returns the digit's
+// total.  Every thread of the workgroup must call it.
+template <int WAVES>
+__device__ __forceinline__ uint32_t digit_starts(uint32_t (*wcnt)[256], uint32_t* dstart,
+                                                 uint32_t* wtot)
 {
-    __shared__ uint32_t wcnt[RS_WAVES][256];
+    const int d = threadIdx.x, lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    uint32_t total = 0, x = 0;
+    if (d < 256) {
+        uint32_t c[WAVES]; // every read before the writes
+#pragma unroll
+        for (int ww = 0; ww < WAVES; ww++) c[ww] = wcnt[ww][d];
+#pragma unroll
+        for (int ww = 0; ww < WAVES; ww++) {
+            wcnt[ww][d] = total;
+            total += c[ww];
+        }
+        x = total;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, WAVE);
+            if (lane >= o) x += y;
+        }
+        if (lane == WAVE - 1) wtot[w] = x;
+    }
+    __syncthreads();
+    if (d < 256) {
+        uint32_t wpre = 0;
+#pragma unroll
+        for (int ww = 0; ww < 256 / WAVE; ww++)
+            if (ww < w) wpre += wtot[ww];
+        dstart[d] = wpre + x - total;
+    }
+    __syncthreads();
+    return total;
+}
+
+// All digits of an array of at most SB_MAX keys in one workgroup: keys and
+// values stay in registers and cross LDS once per digit (112 KB).
+constexpr int SB_BLOCK = 1024;
+constexpr int SB_WAVES = SB_BLOCK / WAVE;
+constexpr int SB_CHUNKS = 8;
+constexpr int64_t SB_MAX = (int64_t)SB_BLOCK * SB_CHUNKS;
+
+template <class K> __global__ __launch_bounds__(SB_BLOCK) void k_sort_block(KeyJobs J)
+{
+    __shared__ K sk[SB_MAX];
+    __shared__ uint32_t sv[SB_MAX];
+    __shared__ uint32_t wcnt[SB_WAVES][256];
+    __shared__ uint32_t dstart[256], wtot[256 / WAVE];
+    const KeyJob j = J.j[blockIdx.x];
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    // waves share the keys evenly, in chunks of 64
+    const int n = (int)j.n, chunks = (n + SB_BLOCK - 1) / SB_BLOCK;
+    const int base = w * chunks * WAVE + lane;
+    K k[SB_CHUNKS];
+    uint32_t v[SB_CHUNKS], rank[SB_CHUNKS];
+#pragma unroll
+    for (int c = 0; c < SB_CHUNKS; c++) {
+        const int i = base + c * WAVE;
+        const bool in = c < chunks && i < n;
+        k[c] = in ? static_cast<const K*>(j.keys)[i] : 0;
+        v[c] = in ? (j.vals ? j.vals[i] : (uint32_t)i) : 0;
+    }
+    for (int shift = 0; shift < 8 * (int)sizeof(K); shift += 8) {
+        if (((j.mask >> shift) & 0xFFull) == 0) continue;
+        for (int i = threadIdx.x; i < SB_WAVES * 256; i += SB_BLOCK) (&wcnt[0][0])[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < SB_CHUNKS; c++)
+            if (c < chunks)
+                rank[c] = wave_rank((uint32_t)(k[c] >> shift) & 0xFF, base + c * WAVE < n,
+                                    wcnt[w], lt);
+        __syncthreads();
+        digit_starts<SB_WAVES>(wcnt, dstart, wtot);
+#pragma unroll
+        for (int c = 0; c < SB_CHUNKS; c++)
+            if (c < chunks && base + c * WAVE < n) {
+                const uint32_t d = (uint32_t)(k[c] >> shift) & 0xFF;
+                const uint32_t at = dstart[d] + wcnt[w][d] + rank[c];
+                sk[at] = k[c];
+                sv[at] = v[c];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < SB_CHUNKS; c++)
+            if (c < chunks && base + c * WAVE < n) {
+                k[c] = sk[base + c * WAVE];
+                v[c] = sv[base + c * WAVE];
+            }
+    }
+#pragma unroll
+    for (int c = 0; c < SB_CHUNKS; c++) {
+        const int i = base + c * WAVE;
+        if (c < chunks && i < n) {
+            static_cast<K*>(j.okeys)[i] = k[c];
+            j.ovals[i] = v[c];
+        }
+    }
+}
+
+// Digit counts of every job and digit (hist: SORT_JOBS x MAX_DIGITS x 256,
+// zero on entry).
+template <class K>
+__global__ __launch_bounds__(RS_BLOCK) void k_sort_hist(KeyJobs J, uint32_t* hist)
+{
+    __shared__ uint32_t h[MAX_DIGITS][256];
+    int q = 0;
+    while (q + 1 < J.n && (int64_t)blockIdx.x >= J.j[q + 1].tile0) q++;
+    const K* const keys = static_cast<const K*>(J.j[q].keys);
+    const int64_t n = J.j[q].n, stride = J.j[q].ntiles * RS_TILE;
+    const unsigned long long mask = J.j[q].mask;
+#pragma unroll
+    for (int p = 0; p < MAX_DIGITS; p++) h[p][threadIdx.x] = 0;
+    __syncthreads();
+    for (int64_t base = ((int64_t)blockIdx.x - J.j[q].tile0) * RS_TILE; base < n; base += stride)
+#pragma unroll
+        for (int c = 0; c < RS_CHUNKS; c++) {
+            const int64_t i = base + c * RS_BLOCK + threadIdx.x;
+            if (i < n) {
+                const K k = keys[i];
+#pragma unroll
+                for (int p = 0; p < (int)sizeof(K); p++)
+                    if ((mask >> (8 * p)) & 0xFFull) atomicAdd(&h[p][(k >> (8 * p)) & 0xFF], 1u);
+            }
+        }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < MAX_DIGITS; p++) {
+        const uint32_t c = h[p][threadIdx.x];
+        if (c) atomicAdd(hist + (q * MAX_DIGITS + p) * 256 + threadIdx.x, c);
+    }
+}
+
+// One stable digit pass of every job that has this digit.  `clear`: the
+// other histogram buffer, zeroed for the next sort.
+template <class K, int BLOCK, int CHUNKS>
+__global__ __launch_bounds__(BLOCK, 4) void k_sort_pass(KeyJobs J, unsigned tiles,
+                                                        unsigned* ticket, unsigned epoch,
+                                                        uint32_t* clear)
+{
+    constexpr int WAVES = BLOCK / WAVE, TILE = BLOCK * CHUNKS;
+    __shared__ uint32_t wcnt[WAVES][256];
     __shared__ uint32_t tile_off[256];
     __shared__ uint32_t dstart[256]; // first slot of each digit in the tile
-    __shared__ uint32_t wtot[RS_WAVES];
-    __shared__ K sk[RS_TILE];
-    __shared__ uint32_t sv[RS_TILE];
+    __shared__ uint32_t wtot[256 / WAVE], gtot[256 / WAVE];
+    __shared__ K sk[TILE];
+    __shared__ uint32_t sv[TILE];
     const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
-    for (int i = threadIdx.x; i < RS_WAVES * 256; i += RS_BLOCK) (&wcnt[0][0])[i] = 0;
-    tile_off[threadIdx.x] = offsets[(int64_t)threadIdx.x * ntiles + blockIdx.x];
-    __syncthreads();
-    const int64_t tile0 = (int64_t)blockIdx.x * RS_TILE;
-    const int64_t base = tile0 + (int64_t)w * (RS_CHUNKS * WAVE);
-    const unsigned long long lt = (1ull << lane) - 1ull;
-    K k[RS_CHUNKS];
-    uint32_t v[RS_CHUNKS];
-    uint32_t rank[RS_CHUNKS];
-#pragma unroll
-    for (int c = 0; c < RS_CHUNKS; c++) {
-        const int64_t i = base + c * WAVE + lane;
-        const bool valid = i < n;
-        k[c] = valid ? keys[i] : 0;
-        v[c] = valid ? vals[i] : 0;
-        const uint32_t d = (uint32_t)(k[c] >> shift) & 0xFF;
-        unsigned long long peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const unsigned long long m = __ballot((d >> b) & 1);
-            peers &= ((d >> b) & 1) ? m : ~m;
-        }
-        const uint32_t r = (uint32_t)__popcll(peers & lt);
-        const uint32_t before = valid ? wcnt[w][d] : 0;
-        __builtin_amdgcn_wave_barrier();
-        if (valid && r == 0) wcnt[w][d] = before + (uint32_t)__popcll(peers);
-        __builtin_amdgcn_wave_barrier();
-        rank[c] = before + r;
-    }
-    __syncthreads();
-    // per digit: wave counts -> offsets within the digit, digit total
-    uint32_t total;
-    {
-        const int d = threadIdx.x; // RS_BLOCK == 256 digits
-        uint32_t run = 0;
-#pragma unroll
-        for (int ww = 0; ww < RS_WAVES; ww++) {
-            const uint32_t c = wcnt[ww][d];
-            wcnt[ww][d] = run;
-            run += c;
-        }
-        total = run;
-    }
-    // exclusive scan of the digit totals: within each wave, then across
-    uint32_t x = total;
+    const int64_t t = lb_ticket(ticket, tiles);
+    if (clear && t == 0)
+        for (int i = threadIdx.x; i < SORT_JOBS * MAX_DIGITS * 256; i += BLOCK) clear[i] = 0;
+    int q = 0;
+    while (q + 1 < J.n && t >= J.j[q + 1].tile0) q++;
+    const KeyJob& j = J.j[q];
+    const K* const keys = static_cast<const K*>(j.keys);
+    const int64_t n = j.n, tile = t - j.tile0;
+    const int shift = j.shift;
+    for (int i = threadIdx.x; i < WAVES * 256; i += BLOCK) (&wcnt[0][0])[i] = 0;
+    // first slot of every digit in the output
+    const bool digit = threadIdx.x < 256; // a thread per digit
+    const uint32_t gh = digit ? j.hist[threadIdx.x] : 0;
+    uint32_t gx = gh;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, WAVE);
-        if (lane >= o) x += y;
+        const uint32_t y = __shfl_up(gx, o, WAVE);
+        if (lane >= o) gx += y;
     }
-    if (lane == WAVE - 1) wtot[w] = x;
+    if (digit && lane == WAVE - 1) gtot[w] = gx;
     __syncthreads();
-    uint32_t wpre = 0;
+    uint32_t first = gx - gh;
 #pragma unroll
-    for (int ww = 0; ww < RS_WAVES; ww++)
-        if (ww < w) wpre += wtot[ww];
-    dstart[threadIdx.x] = wpre + x - total;
+    for (int ww = 0; ww < 256 / WAVE; ww++)
+        if (ww < w) first += gtot[ww];
+    const int64_t at0 = tile * TILE;
+    const int64_t base = at0 + (int64_t)w * (CHUNKS * WAVE) + lane;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    K k[CHUNKS];
+    uint32_t v[CHUNKS];
+    uint32_t rank[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++) {
+        const int64_t i = base + c * WAVE;
+        k[c] = i < n ? keys[i] : 0;
+        v[c] = i < n ? (j.vals ? j.vals[i] : (uint32_t)i) : 0;
+    }
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++)
+        rank[c] = wave_rank((uint32_t)(k[c] >> shift) & 0xFF, base + c * WAVE < n, wcnt[w], lt);
     __syncthreads();
-    // keys in digit order in LDS
+    const uint32_t total = digit_starts<WAVES>(wcnt, dstart, wtot);
+    if (digit) {
+        unsigned long long* const word = j.status + threadIdx.x;
+        lb_publish(word + 256 * tile, epoch, tile ? LB_SUM : LB_PREFIX, total);
+        const uint32_t before = lb_before(word, 256, tile, epoch);
+        if (tile) lb_publish(word + 256 * tile, epoch, LB_PREFIX, before + total);
+        tile_off[threadIdx.x] = first + before;
+    }
+    // keys in digit order in LDS, then each digit's run to its place, so
+    // that neighbouring lanes write neighbouring addresses
 #pragma unroll
-    for (int c = 0; c < RS_CHUNKS; c++) {
-        const int64_t i = base + c * WAVE + lane;
-        if (i < n) {
+    for (int c = 0; c < CHUNKS; c++)
+        if (base + c * WAVE < n) {
             const uint32_t d = (uint32_t)(k[c] >> shift) & 0xFF;
             const uint32_t lp = dstart[d] + wcnt[w][d] + rank[c];
             sk[lp] = k[c];
             sv[lp] = v[c];
         }
-    }
     __syncthreads();
-    const int tn = (int)(n - tile0 < RS_TILE ? n - tile0 : RS_TILE);
-    for (int j = threadIdx.x; j < tn; j += RS_BLOCK) {
-        const K key = sk[j];
+    const int tn = (int)(n - at0 < TILE ? n - at0 : TILE);
+    for (int i = threadIdx.x; i < tn; i += BLOCK) {
+        const K key = sk[i];
         const uint32_t d = (uint32_t)(key >> shift) & 0xFF;
-        const int64_t pos = (int64_t)tile_off[d] + (j - (int)dstart[d]);
-        okeys[pos] = key;
-        ovals[pos] = sv[j];
+        const int64_t pos = (int64_t)tile_off[d] + (i - (int)dstart[d]);
+        static_cast<K*>(j.okeys)[pos] = key;
+        j.ovals[pos] = sv[i];
     }
-}
-
-// xor-fold of all keys against the first one: bits that vary
-template <class K>
-__global__ __launch_bounds__(256) void k_vary_bits(const K* keys, int64_t n,
-                                                   unsigned long long* out)
-{
-    const uint64_t k0 = keys[0];
-    uint64_t acc = 0;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * 256)
-        acc |= keys[i] ^ k0;
-    // wave reduce
-    for (int o = 32; o > 0; o >>= 1) acc |= __shfl_xor(acc, o, WAVE);
-    if (threadIdx.x % WAVE == 0 && acc) atomicOr(out, (unsigned long long)acc);
-}
-
-__global__ void k_rle_flags(const uint64_t* keys, int64_t n, uint32_t* flags)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flags[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u;
-}
-
-__global__ void k_rle_scatter(const uint64_t* keys, int64_t n, const uint32_t* flags,
-                              const uint32_t* pos, uint64_t* ukeys, uint32_t* start,
-                              const uint32_t* nu)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && flags[i]) {
-        ukeys[pos[i]] = keys[i];
-        start[pos[i]] = (uint32_t)i;
-    }
-    if (i == 0) start[*nu] = (uint32_t)n;
 }
 
 } // namespace
@@ -317,203 +624,241 @@ size_t scan_tmp_bytes(int64_t n)
     return sizeof(uint64_t) * (size_t)((n + SCAN_TILE - 1) / SCAN_TILE + 1) + 256;
 }
 
-void exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_dev,
-                        void* tmp, hipStream_t s)
+// Makes room for `words` look-back words and returns the launch's epoch.
+// Old words never match a new epoch; new memory is cleared once.
+static unsigned lb_begin(SortSpace& ws, int64_t words, hipStream_t s)
 {
-    exclusive_scan<uint32_t>(in, out, n, total_dev, tmp, s);
+    constexpr unsigned EPOCHS = 1u << 30;
+    const size_t bytes = sizeof(unsigned long long) * (size_t)words;
+    bool clear = bytes > ws.status.bytes;
+    ws.status.reserve(bytes);
+    if (++ws.epoch == EPOCHS) {
+        ws.epoch = 1;
+        clear = true;
+    }
+    if (clear) IPCG_HIP(hipMemsetAsync(ws.status.p, 0, ws.status.bytes, s));
+    if (!ws.ticket.p) {
+        ws.ticket.reserve(256);
+        IPCG_HIP(hipMemsetAsync(ws.ticket.p, 0, ws.ticket.bytes, s));
+    }
+    return ws.epoch;
+}
+
+void exclusive_scan_u32(SortSpace& ws, const uint32_t* in, uint32_t* out, int64_t n,
+                        uint32_t* total_dev, hipStream_t s)
+{
+    if (n <= 0) {
+        if (total_dev) IPCG_HIP(hipMemsetAsync(total_dev, 0, sizeof(uint32_t), s));
+        return;
+    }
+    const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
+    if (nb == 1) {
+        hipLaunchKernelGGL(k_scan_one<uint32_t>, dim3(1), dim3(SCAN_BLOCK), 0, s, in, out, n,
+                           total_dev);
+        IPCG_CHECK_LAUNCH();
+        return;
+    }
+    const unsigned epoch = lb_begin(ws, nb, s);
+    hipLaunchKernelGGL(k_scan, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, out, n, total_dev,
+                       ws.status.as<unsigned long long>(), ws.ticket.as<unsigned>(), epoch);
+    IPCG_CHECK_LAUNCH();
 }
 
 void exclusive_scan_u64(const uint64_t* in, uint64_t* out, int64_t n, uint64_t* total_dev,
                         void* tmp, hipStream_t s)
 {
-    exclusive_scan<uint64_t>(in, out, n, total_dev, tmp, s);
+    scan_three(in, out, n, total_dev, tmp, s);
 }
 
-size_t radix_tmp_bytes(int64_t n)
-{
-    const int64_t ntiles = (n + RS_TILE - 1) / RS_TILE;
-    const int64_t nc = 256 * ntiles;
-    return 2 * sizeof(uint32_t) * (size_t)nc + scan_tmp_bytes(nc) + 1024;
-}
-
-// LSD passes over the low key_bits bits.  skip_constant: one pass over the
-// keys and a read-back find the digits that vary, and only those passes run;
-// otherwise every pass runs without any host round trip (a constant digit
-// costs a stable identity pass).  Returns true when the sorted pairs ended
-// in keys_alt / vals_alt (copy_back false and an odd number of passes).
-template <class K>
-static bool radix_sort(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, int64_t n,
-                       int key_bits, void* tmp, hipStream_t s, bool skip_constant,
-                       bool copy_back, unsigned long long bit_mask = ~0ull)
-{
-    if (n <= 1) return false;
-    const int64_t ntiles = (n + RS_TILE - 1) / RS_TILE;
-    const int64_t nc = 256 * ntiles;
-    char* t = static_cast<char*>(tmp);
-    unsigned long long* vary = reinterpret_cast<unsigned long long*>(t);
-    uint32_t* counts = reinterpret_cast<uint32_t*>(t + 256);
-    uint32_t* offsets = counts + nc;
-    void* stmp = offsets + nc;
-    unsigned long long hv = bit_mask; // digits without a bit here are constant
-    if (skip_constant) { // which bits vary at all (one small D2H read per sort)
-        IPCG_HIP(hipMemsetAsync(vary, 0, sizeof(unsigned long long), s));
-        hipLaunchKernelGGL(k_vary_bits<K>, dim3(grid_for(n, 256, 1024)), dim3(256), 0, s, keys,
-                           n, vary);
-        IPCG_CHECK_LAUNCH();
-        IPCG_HIP(hipMemcpyAsync(&hv, vary, sizeof(hv), hipMemcpyDeviceToHost, s));
-        IPCG_HIP(hipStreamSynchronize(s));
-    }
-    K* ki = keys;
-    uint32_t* vi = vals;
-    K* ko = keys_alt;
-    uint32_t* vo = vals_alt;
-    for (int shift = 0; shift < key_bits; shift += 8) {
-        if (((hv >> shift) & 0xFFull) == 0) continue;
-        hipLaunchKernelGGL(k_radix_hist<K>, dim3((unsigned)ntiles), dim3(RS_BLOCK), 0, s, ki, n,
-                           shift, counts, ntiles);
-        exclusive_scan_u32(counts, offsets, nc, nullptr, stmp, s);
-        hipLaunchKernelGGL(k_radix_scatter<K>, dim3((unsigned)ntiles), dim3(RS_BLOCK), 0, s, ki,
-                           vi, ko, vo, n, shift, offsets, ntiles);
-        IPCG_CHECK_LAUNCH();
-        std::swap(ki, ko);
-        std::swap(vi, vo);
-    }
-    if (ki == keys) return false;
-    if (!copy_back) return true;
-    IPCG_HIP(hipMemcpyAsync(keys, ki, sizeof(K) * n, hipMemcpyDeviceToDevice, s));
-    IPCG_HIP(hipMemcpyAsync(vals, vi, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-    return false;
-}
-
-void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
-                      int64_t n, int key_bits, void* tmp, hipStream_t s)
-{
-    radix_sort(keys, vals, keys_alt, vals_alt, n, key_bits, tmp, s, true, true);
-}
-
-bool radix_sort_pairs_all(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
-                          uint32_t* vals_alt, int64_t n, int key_bits, void* tmp, hipStream_t s)
-{
-    return radix_sort(keys, vals, keys_alt, vals_alt, n, key_bits, tmp, s, false, false);
-}
-
-bool radix_sort_pairs_masked(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
-                             uint32_t* vals_alt, int64_t n, unsigned long long bit_mask,
-                             void* tmp, hipStream_t s)
-{
-    return radix_sort(keys, vals, keys_alt, vals_alt, n, 64, tmp, s, false, false, bit_mask);
-}
-
-bool radix_sort_pairs_all(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
-                          uint32_t* vals_alt, int64_t n, int key_bits, void* tmp, hipStream_t s)
-{
-    if (key_bits > 32) throw Error(IPCG_ERR_ARG, "32-bit keys hold at most 32 key bits");
-    return radix_sort(keys, vals, keys_alt, vals_alt, n, key_bits, tmp, s, false, false);
-}
-
-size_t rle_tmp_bytes(int64_t n)
-{
-    return 2 * sizeof(uint32_t) * (size_t)(n + 1) + scan_tmp_bytes(n) + 256;
-}
-
-void run_length_encode(const uint64_t* keys, int64_t n, uint64_t* unique_keys,
-                       uint32_t* run_start, uint32_t* n_unique_dev, void* tmp, hipStream_t s)
+void run_length_encode(SortSpace& ws, const uint64_t* keys, int64_t n, uint64_t* unique_keys,
+                       uint32_t* run_start, uint32_t* n_unique_dev, hipStream_t s)
 {
     if (n <= 0) {
         IPCG_HIP(hipMemsetAsync(n_unique_dev, 0, sizeof(uint32_t), s));
         IPCG_HIP(hipMemsetAsync(run_start, 0, sizeof(uint32_t), s));
         return;
     }
-    uint32_t* flags = static_cast<uint32_t*>(tmp);
-    uint32_t* pos = flags + (n + 1);
-    void* stmp = pos + (n + 1);
-    // one thread per key: the grid must cover all n keys
-    hipLaunchKernelGGL(k_rle_flags, dim3(grid_for(n, 256, INT32_MAX)), dim3(256), 0, s, keys, n,
-                       flags);
-    exclusive_scan_u32(flags, pos, n, n_unique_dev, stmp, s);
-    hipLaunchKernelGGL(k_rle_scatter, dim3(grid_for(n, 256, INT32_MAX)), dim3(256), 0, s, keys, n, flags,
-                       pos, unique_keys, run_start, n_unique_dev);
+    const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
+    const unsigned epoch = lb_begin(ws, nb, s);
+    hipLaunchKernelGGL(k_rle, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, keys, n, unique_keys,
+                       run_start, n_unique_dev, ws.status.as<unsigned long long>(),
+                       ws.ticket.as<unsigned>(), epoch);
     IPCG_CHECK_LAUNCH();
 }
 
-__global__ void k_shard_offsets(const unsigned long long* cnt, int64_t scap, int64_t* off)
+template <class K> static void sort_jobs(SortSpace& ws, SortJob* jobs, int njobs, hipStream_t s)
 {
-    __shared__ int64_t v[SHARDS];
-    const int t = threadIdx.x;
-    const int64_t c = (int64_t)cnt[(int64_t)t * SHARD_PAD];
-    v[t] = c < scap ? c : scap;
-    __syncthreads();
-    if (t == 0) {
-        int64_t acc = 0;
-        for (int i = 0; i < SHARDS; i++) {
-            off[i] = acc;
-            acc += v[i];
+    if (njobs > SORT_JOBS) throw Error(IPCG_ERR_ARG, "too many arrays in one sort");
+    KeyJobs small {}, large {};
+    SortJob* of_large[SORT_JOBS];
+    int64_t tiles = 0;
+    for (int q = 0; q < njobs; q++) {
+        SortJob& j = jobs[q];
+        if (sizeof(K) < 8) j.mask &= (1ull << (8 * sizeof(K) % 64)) - 1ull;
+        j.in_alt = false;
+        if (j.n >= (1ll << 32)) throw Error(IPCG_ERR_ARG, "too many keys for one sort");
+        if (j.n <= 0) continue;
+        KeyJob k {};
+        k.keys = j.keys;
+        k.vals = j.iota ? nullptr : j.vals;
+        k.okeys = j.keys;
+        k.ovals = j.vals;
+        k.n = j.n;
+        k.mask = j.mask;
+        if (j.n <= SB_MAX) {
+            small.j[small.n++] = k;
+            continue;
         }
-        off[SHARDS] = acc;
+        if (j.mask == 0) throw Error(IPCG_ERR_ARG, "a sort needs key bits");
+        k.ntiles = (j.n + RS_TILE - 1) / RS_TILE; // (short tiles)
+        tiles += k.ntiles;
+        of_large[large.n] = &j;
+        large.j[large.n++] = k;
     }
+    if (small.n) {
+        hipLaunchKernelGGL(k_sort_block<K>, dim3(small.n), dim3(SB_BLOCK), 0, s, small);
+        IPCG_CHECK_LAUNCH();
+    }
+    if (!large.n) return;
+    constexpr size_t HIST = SORT_JOBS * MAX_DIGITS * 256; // one buffer
+    const bool fresh = !ws.hist.p || ws.torn;
+    ws.hist.reserve(sizeof(uint32_t) * 2 * HIST);
+    if (fresh) IPCG_HIP(hipMemsetAsync(ws.hist.p, 0, sizeof(uint32_t) * 2 * HIST, s));
+    ws.torn = true; // until every launch below is in the stream
+    uint32_t* const hist = ws.hist.as<uint32_t>() + (ws.flip ? HIST : 0);
+    uint32_t* const other = ws.hist.as<uint32_t>() + (ws.flip ? 0 : HIST);
+    ws.flip = !ws.flip;
+    { // at most HIST_GROUPS workgroups per array (each adds up to 2048 counts)
+        constexpr int64_t HIST_GROUPS = 512;
+        KeyJobs h = large;
+        int64_t at = 0;
+        for (int q = 0; q < h.n; q++) {
+            h.j[q].tile0 = at;
+            h.j[q].ntiles = h.j[q].ntiles < HIST_GROUPS ? h.j[q].ntiles : HIST_GROUPS;
+            at += h.j[q].ntiles;
+        }
+        hipLaunchKernelGGL(k_sort_hist<K>, dim3((unsigned)at), dim3(RS_BLOCK), 0, s, h, hist);
+        IPCG_CHECK_LAUNCH();
+    }
+    const bool big = tiles > BIG_TILES;
+    const int tile = big ? BIG_BLOCK * big_chunks<K>() : RS_TILE;
+    for (int q = 0; q < large.n; q++) large.j[q].ntiles = (large.j[q].n + tile - 1) / tile;
+    bool first = true;
+    for (int p = 0; p < (int)sizeof(K); p++) {
+        KeyJobs pass {};
+        int64_t at = 0;
+        for (int q = 0; q < large.n; q++) {
+            KeyJob& k = large.j[q];
+            SortJob& j = *of_large[q];
+            if (((k.mask >> (8 * p)) & 0xFFull) == 0) continue;
+            K* const a = static_cast<K*>(j.keys);
+            K* const b = static_cast<K*>(j.keys_alt);
+            k.keys = j.in_alt ? b : a;
+            k.vals = j.iota ? nullptr : (j.in_alt ? j.vals_alt : j.vals);
+            k.okeys = j.in_alt ? a : b;
+            k.ovals = j.in_alt ? j.vals : j.vals_alt;
+            k.shift = 8 * p;
+            k.hist = hist + (q * MAX_DIGITS + p) * 256;
+            KeyJob out = k;
+            out.tile0 = at;
+            at += k.ntiles;
+            pass.j[pass.n++] = out;
+            j.in_alt = !j.in_alt;
+            j.iota = false; // the values exist from here on
+        }
+        if (!pass.n) continue;
+        const unsigned epoch = lb_begin(ws, 256 * at, s);
+        for (int q = 0; q < pass.n; q++)
+            pass.j[q].status = ws.status.as<unsigned long long>() + 256 * pass.j[q].tile0;
+        if (big)
+            hipLaunchKernelGGL((k_sort_pass<K, BIG_BLOCK, big_chunks<K>()>), dim3((unsigned)at),
+                               dim3(BIG_BLOCK), 0, s, pass, (unsigned)at,
+                               ws.ticket.as<unsigned>(), epoch, first ? other : nullptr);
+        else
+            hipLaunchKernelGGL((k_sort_pass<K, RS_BLOCK, RS_CHUNKS>), dim3((unsigned)at),
+                               dim3(RS_BLOCK), 0, s, pass, (unsigned)at,
+                               ws.ticket.as<unsigned>(), epoch, first ? other : nullptr);
+        IPCG_CHECK_LAUNCH();
+        first = false;
+    }
+    ws.torn = false;
 }
 
-// one workgroup per counter set: its total and its largest shard count
+void radix_sort_jobs(SortSpace& ws, SortJob* jobs, int njobs, hipStream_t s)
+{
+    sort_jobs<uint64_t>(ws, jobs, njobs, s);
+}
+
+bool radix_sort_pairs(SortSpace& ws, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
+                      uint32_t* vals_alt, int64_t n, unsigned long long bit_mask, bool iota,
+                      hipStream_t s)
+{
+    SortJob j { keys, keys_alt, vals, vals_alt, n, bit_mask, iota, false };
+    sort_jobs<uint64_t>(ws, &j, 1, s);
+    return j.in_alt;
+}
+
+bool radix_sort_pairs(SortSpace& ws, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
+                      uint32_t* vals_alt, int64_t n, unsigned long long bit_mask, bool iota,
+                      hipStream_t s)
+{
+    SortJob j { keys, keys_alt, vals, vals_alt, n, bit_mask, iota, false };
+    sort_jobs<uint32_t>(ws, &j, 1, s);
+    return j.in_alt;
+}
+
+// one workgroup per counter set: the offsets of its shards, its total and its
+// largest shard count
 __global__ __launch_bounds__(SHARDS) void k_shard_summary(const unsigned long long* cnt,
+                                                          const int* extra, int64_t* off,
                                                           unsigned long long* out)
 {
-    __shared__ unsigned long long wsum[SHARDS / WAVE], wmax[SHARDS / WAVE];
+    static_assert(SHARDS == SCAN_BLOCK, "block_exclusive_scan");
+    __shared__ unsigned long long wmax[SHARDS / WAVE];
     const unsigned long long v =
         cnt[(int64_t)blockIdx.x * SHARDS * SHARD_PAD + (int64_t)threadIdx.x * SHARD_PAD];
-    unsigned long long sm = v, mx = v;
+    unsigned long long mx = v, total;
     for (int o = WAVE / 2; o > 0; o >>= 1) {
-        sm += __shfl_xor(sm, o, WAVE);
         const unsigned long long y = __shfl_xor(mx, o, WAVE);
         mx = y > mx ? y : mx;
     }
-    if (threadIdx.x % WAVE == 0) {
-        wsum[threadIdx.x / WAVE] = sm;
-        wmax[threadIdx.x / WAVE] = mx;
-    }
-    __syncthreads();
+    if (threadIdx.x % WAVE == 0) wmax[threadIdx.x / WAVE] = mx;
+    int64_t* const so = off + (int64_t)blockIdx.x * (SHARDS + 1);
+    so[threadIdx.x] = (int64_t)block_exclusive_scan<unsigned long long>(v, total);
     if (threadIdx.x == 0) {
-        unsigned long long t = 0, m = 0;
-        for (int w = 0; w < SHARDS / WAVE; w++) {
-            t += wsum[w];
-            m = wmax[w] > m ? wmax[w] : m;
-        }
-        out[2 * blockIdx.x] = t;
+        so[SHARDS] = (int64_t)total;
+        unsigned long long m = 0;
+        for (int w = 0; w < SHARDS / WAVE; w++) m = wmax[w] > m ? wmax[w] : m;
+        out[2 * blockIdx.x] = total;
         out[2 * blockIdx.x + 1] = m;
+        if (blockIdx.x == 0) out[2 * gridDim.x] = extra ? (unsigned long long)(unsigned)*extra : 0ull;
     }
 }
 
 void shard_counts_n(const unsigned long long* cnt_dev, int nsets, unsigned long long* sum_dev,
-                    void* pinned, hipStream_t s, ShardCounts* out, const int* extra_dev,
-                    int* extra)
+                    int64_t* off_dev, void* pinned, hipStream_t s, ShardCounts* out,
+                    const int* extra_dev, int* extra)
 {
-    hipLaunchKernelGGL(k_shard_summary, dim3(nsets), dim3(SHARDS), 0, s, cnt_dev, sum_dev);
+    hipLaunchKernelGGL(k_shard_summary, dim3(nsets), dim3(SHARDS), 0, s, cnt_dev, extra_dev,
+                       off_dev, sum_dev);
     IPCG_CHECK_LAUNCH();
     unsigned long long* h = static_cast<unsigned long long*>(pinned);
-    IPCG_HIP(hipMemcpyAsync(h, sum_dev, sizeof(unsigned long long) * 2 * nsets,
+    IPCG_HIP(hipMemcpyAsync(h, sum_dev, sizeof(unsigned long long) * (2 * nsets + 1),
                             hipMemcpyDeviceToHost, s));
-    if (extra_dev)
-        IPCG_HIP(hipMemcpyAsync(h + 2 * nsets, extra_dev, sizeof(int), hipMemcpyDeviceToHost, s));
     IPCG_HIP(hipStreamSynchronize(s));
     for (int k = 0; k < nsets; k++) {
         out[k].total = (int64_t)h[2 * k];
         out[k].max = (int64_t)h[2 * k + 1];
     }
-    if (extra_dev && extra) *extra = *reinterpret_cast<const int*>(h + 2 * nsets);
+    if (extra) *extra = (int)h[2 * nsets];
 }
 
 ShardCounts shard_counts(const unsigned long long* cnt_dev, unsigned long long* sum_dev,
-                         void* pinned, hipStream_t s)
+                         int64_t* off_dev, void* pinned, hipStream_t s)
 {
     ShardCounts r;
-    shard_counts_n(cnt_dev, 1, sum_dev, pinned, s, &r);
+    shard_counts_n(cnt_dev, 1, sum_dev, off_dev, pinned, s, &r);
     return r;
-}
-
-void shard_offsets(const unsigned long long* cnt_dev, int64_t scap, int64_t* off_dev,
-                   hipStream_t s)
-{
-    hipLaunchKernelGGL(k_shard_offsets, dim3(1), dim3(SHARDS), 0, s, cnt_dev, scap, off_dev);
-    IPCG_CHECK_LAUNCH();
 }
 
 } // namespace ipcg
