@@ -51,6 +51,10 @@ namespace {
 
 constexpr int CB = 64;
 constexpr int LDS_CAP = 6;
+// boxes a lane's search may visit (8 x 512 x 512 sheets, LDS and sub-wave tier:
+// 4.9 ms without, 4.7 at 32, 4.5 at 24, 4.5 at 16; two 193 x 193 sheets 2.9,
+// 2.9, 2.9 and 3.3)
+constexpr long LDS_BUDGET = 24;
 // Tiers above the LDS lists.  Their searches are chains of ~40 dependent
 // levels of a few boxes (median 5 a level on nearly parallel sheets, 18,000
 // at most below the expected minimum), so each tier gives a search the lanes
@@ -130,9 +134,9 @@ __device__ __forceinline__ void report(const CCDArgs& A, int64_t ci, bool hit, d
 
 // Strategy prologue (ccd_strategy + *_ccd of tight_inclusion_ccd.cpp):
 // gathers the stencil, returns 1 (hit at toi = 0), 0 (miss) or -1 (search
-// needed, q / eff / adj set); `scene` receives the candidate's scene.
-__device__ int candidate_setup(const CCDArgs& A, int64_t ci, TIQuery& q, double& eff, double& adj,
-                               int& scene)
+// needed, q's positions, its scale, eff and adj set); `scene` receives the candidate's scene.
+__device__ int candidate_setup(const CCDArgs& A, int64_t ci, TIQuery& q, TIScale& sc, double& eff,
+                               double& adj, int& scene)
 {
     // candidates [0, n_ee) edge-edge, then face-vertex, codim vertex-vertex
     // and codim edge-vertex; point-point and point-edge run as degenerate
@@ -169,6 +173,7 @@ __device__ int candidate_setup(const CCDArgs& A, int64_t ci, TIQuery& q, double&
     const bool is_ee = kind != 1;
     scene = A.vscene ? A.vscene[ids[0]] : 0;
     d3 p0[4];
+    double e[12];
     bool moving = false;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -177,9 +182,9 @@ __device__ int candidate_setup(const CCDArgs& A, int64_t ci, TIQuery& q, double&
         q.s[3 * j] = p0[j].x;
         q.s[3 * j + 1] = p0[j].y;
         q.s[3 * j + 2] = p0[j].z;
-        q.e[3 * j] = p1.x;
-        q.e[3 * j + 1] = p1.y;
-        q.e[3 * j + 2] = p1.z;
+        e[3 * j] = p1.x;
+        e[3 * j + 1] = p1.y;
+        e[3 * j + 2] = p1.z;
         moving |= p1.x != p0[j].x || p1.y != p0[j].y || p1.z != p0[j].z;
     }
     q.vf = !is_ee;
@@ -200,6 +205,9 @@ __device__ int candidate_setup(const CCDArgs& A, int64_t ci, TIQuery& q, double&
     eff = (1.0 - A.rescale) * (d0 - dmin);
     eff = eff < 1e-4 ? eff : 1e-4;
     eff += dmin;
+#pragma unroll
+    for (int k = 0; k < 12; k++) q.d[k] = e[k] - q.s[k];
+    ti_scale(q.s, e, q.vf, sc);
     return -1;
 }
 
@@ -216,11 +224,12 @@ __global__ __launch_bounds__(256) void k_ccd_root(CCDArgs A, Shards S, uint32_t*
         TIQuery q;
         double eff = 0, adj = 0;
         int sc = 0;
-        const int pre = candidate_setup(A, ci, q, eff, adj, sc);
+        TIScale scale;
+        const int pre = candidate_setup(A, ci, q, scale, eff, adj, sc);
         if (pre >= 0) {
             report(A, ci, pre == 1, 0.0, sc);
         } else {
-            ti_filter(q, eff > 0);
+            ti_filter(q, scale, eff > 0);
             bool box_in;
             double w[3];
             search = ti_inclusion(q, TIBox { 0.0, 0.0, 0.0 }, 1.0, 1.0, 1.0, eff, box_in, w);
@@ -233,74 +242,6 @@ __global__ __launch_bounds__(256) void k_ccd_root(CCDArgs A, Shards S, uint32_t*
     if (search && slot < S.scap) stage[sh * S.scap + slot] = (uint32_t)ci;
 }
 
-// ---------------------------------------------------------------------------
-// LDS tier
-// ---------------------------------------------------------------------------
-// ci_lo, ci_hi: only the candidates of this index range are searched (a
-// phase of the search; the others return at once)
-__global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo, int64_t n_todo,
-                                                uint32_t* spill, unsigned long long* n_spill,
-                                                int64_t ci_lo, int64_t ci_hi)
-{
-    __shared__ unsigned long long lists[3 * LDS_CAP * CB];
-    const int64_t k = (int64_t)xcd_block() * CB + threadIdx.x;
-    if (k >= n_todo) return;
-    if (A.any_hit && __hip_atomic_load(A.any_hit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        return;
-    const TILdsLists L { lists + threadIdx.x, CB, LDS_CAP };
-    const int64_t ci = todo[k];
-    if (ci < ci_lo || ci >= ci_hi) return;
-    TIQuery q;
-    double eff = 0, adj = 0, toi = INFINITY;
-    int sc = 0;
-    const int pre = candidate_setup(A, ci, q, eff, adj, sc);
-    if (pre >= 0) {
-        report(A, ci, pre == 1, 0.0, sc);
-        return;
-    }
-    const double* const run = A.bounded ? A.bound + sc : nullptr;
-    const double* const expect = A.bounded && A.expect ? A.expect + sc : nullptr;
-    const TIBound B1 { run, expect, 1.0, SMALL_TOI };
-    int r = ti_query_lds(q, eff, adj, A.max_iter, false, B1, L, toi);
-    if (r == TI_HIT && toi < SMALL_TOI) {
-        const TIBound B2 { run, expect, (1.0 / A.rescale) * (1 + 1e-12), 0.0 };
-        r = ti_query_lds(q, A.min_distance, adj, -1, true, B2, L, toi);
-        if (r == TI_HIT) toi *= A.rescale;
-    }
-    if (r >= TI_OVERFLOW) {
-        spill[atomicAdd(n_spill, 1ull)] = (uint32_t)ci;
-        // searches spilled for depth (the rest: for list length), counted
-        // per wave
-        const unsigned long long deep = __ballot(r == TI_DEEP);
-        if (deep && (unsigned)lane_id() == (unsigned)(__ffsll((long long)deep) - 1))
-            atomicAdd(n_spill + 1, (unsigned long long)__popcll(deep));
-        return;
-    }
-    report(A, ci, r == TI_HIT, toi, sc);
-}
-
-// The searches of a tier: `list`, or the list of the tier before (`before`)
-// when that is short enough (at most `skip`) for the tier between to have
-// left it alone.
-struct Searches {
-    const uint32_t* list;
-    const unsigned long long* n;
-    const uint32_t* before;
-    const unsigned long long* n_before;
-    unsigned skip;
-    unsigned long long* work; // next search to take
-};
-
-struct Lists {
-    uint32_t* over; // searches that outgrow this tier
-    unsigned long long* n_over;
-    uint32_t* deep; // searches too deep for packed boxes
-    unsigned long long* n_deep;
-};
-
-// ---------------------------------------------------------------------------
-// sub-wave tier: SUB_W lanes per search, 64 / SUB_W searches per wave
-// ---------------------------------------------------------------------------
 // The strategy (tight_inclusion_ccd.cpp:33-75) around one search of a tier:
 // stage 1 with the effective distance; an outcome below SMALL_TOI is searched
 // again from the minimum distance without an iteration limit (stage 2),
@@ -343,12 +284,90 @@ struct TIStrategy {
     }
 };
 
+// ---------------------------------------------------------------------------
+// LDS tier
+// ---------------------------------------------------------------------------
+// ci_lo, ci_hi: only the candidates of this index range are searched (a
+// phase of the search; the others return at once)
+__global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo, int64_t n_todo,
+                                                uint32_t* spill, unsigned long long* n_spill,
+                                                int64_t ci_lo, int64_t ci_hi)
+{
+    __shared__ unsigned long long lists[3 * LDS_CAP * CB];
+    const int64_t k = (int64_t)xcd_block() * CB + threadIdx.x;
+    if (k >= n_todo) return;
+    if (A.any_hit && __hip_atomic_load(A.any_hit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        return;
+    const TILdsLists L { lists + threadIdx.x, CB, LDS_CAP };
+    const int64_t ci = todo[k];
+    if (ci < ci_lo || ci >= ci_hi) return;
+    TIQuery q;
+    double eff = 0, adj = 0, toi = INFINITY;
+    int sc = 0;
+    {
+        TIScale scale;
+        const int pre = candidate_setup(A, ci, q, scale, eff, adj, sc);
+        if (pre >= 0) {
+            report(A, ci, pre == 1, 0.0, sc);
+            return;
+        }
+        ti_param_tol(q, scale, adj);
+        ti_filter(q, scale, eff > 0);
+    }
+    TIStrategy T(A, sc, eff, adj);
+    int r;
+    for (;;) {
+        r = ti_bfs_lds(q, T.delta, T.ms, T.max_iter, T.B, L, LDS_BUDGET, toi);
+        if (!T.next(A, r, toi)) break;
+        TIScale scale; // gathered again: too rare to keep
+        (void)candidate_setup(A, ci, q, scale, eff, adj, sc);
+        ti_param_tol(q, scale, T.delta);
+        ti_filter(q, scale, T.ms > 0);
+    }
+    if (r >= TI_OVERFLOW) {
+        spill[atomicAdd(n_spill, 1ull)] = (uint32_t)ci;
+        // searches spilled for depth (the rest: for list length), counted
+        // per wave
+        const unsigned long long deep = __ballot(r == TI_DEEP);
+        if (deep && (unsigned)lane_id() == (unsigned)(__ffsll((long long)deep) - 1))
+            atomicAdd(n_spill + 1, (unsigned long long)__popcll(deep));
+        return;
+    }
+    report(A, ci, r == TI_HIT, T.outcome(r, toi), sc);
+}
+
+// The searches of a tier: `list`, or the list of the tier before (`before`)
+// when that is short enough (at most `skip`) for the tier between to have
+// left it alone.
+struct Searches {
+    const uint32_t* list;
+    const unsigned long long* n;
+    const uint32_t* before;
+    const unsigned long long* n_before;
+    unsigned skip;
+    unsigned long long* work; // next search to take
+};
+
+struct Lists {
+    uint32_t* over; // searches that outgrow this tier
+    unsigned long long* n_over;
+    uint32_t* deep; // searches too deep for packed boxes
+    unsigned long long* n_deep;
+};
+
+// ---------------------------------------------------------------------------
+// sub-wave tier: SUB_W lanes per search, 64 / SUB_W searches per wave
+// ---------------------------------------------------------------------------
+// (WAVE, 4): 128 registers a lane and four waves a SIMD; what spills (184
+// bytes a lane) is the setup's.  16 scenes of nearly parallel sheets: 4.3 ms
+// at two waves a SIMD, 3.3 at four, 4.3 at five.
 template <int W, int CAP>
-__global__ __launch_bounds__(WAVE) void k_ccd_sub(CCDArgs A, Searches Q_in, Lists out)
+__global__ __launch_bounds__(WAVE, 4) void k_ccd_sub(CCDArgs A, Searches Q_in, Lists out)
 {
     constexpr int PER_WAVE = WAVE / W;
     __shared__ unsigned long long lists[PER_WAVE][2 * CAP];
     __shared__ TIQuery Q[PER_WAVE];
+    __shared__ TIScale C[PER_WAVE];
     const int grp = (int)threadIdx.x / W;
     const bool first = threadIdx.x % W == 0;
     unsigned long long* const cur = lists[grp];
@@ -372,11 +391,15 @@ __global__ __launch_bounds__(WAVE) void k_ccd_sub(CCDArgs A, Searches Q_in, List
             int sc = 0, pre;
             {
                 TIQuery q;
-                pre = candidate_setup(A, ci, q, eff, adj, sc);
+                TIScale scale;
+                pre = candidate_setup(A, ci, q, scale, eff, adj, sc);
                 if (pre < 0) {
-                    ti_param_tol(q, adj);
-                    ti_filter(q, eff > 0);
-                    if (first) Q[grp] = q;
+                    ti_param_tol(q, scale, adj);
+                    ti_filter(q, scale, eff > 0);
+                    if (first) {
+                        Q[grp] = q;
+                        C[grp] = scale;
+                    }
                 }
             }
             if (pre >= 0) { // settled by the prologue (not for searches of other tiers)
@@ -390,8 +413,8 @@ __global__ __launch_bounds__(WAVE) void k_ccd_sub(CCDArgs A, Searches Q_in, List
                     if (!T.next(A, r, toi)) break;
                     ti_wave_sync();
                     if (first) {
-                        ti_param_tol(Q[grp], T.delta);
-                        if (T.tries == 1) ti_filter(Q[grp], T.ms > 0);
+                        ti_param_tol(Q[grp], C[grp], T.delta);
+                        if (T.tries == 1) ti_filter(Q[grp], C[grp], T.ms > 0);
                     }
                 }
                 if (first) {
@@ -416,6 +439,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_ccd_group(CCDArgs A, Searches Q_i
     __shared__ TIGroup<NW> G;
     __shared__ struct {
         TIQuery q;
+        TIScale scale;
         double eff, adj;
         unsigned long long k;
         int sc, pre;
@@ -433,12 +457,16 @@ __global__ __launch_bounds__(NW * WAVE) void k_ccd_group(CCDArgs A, Searches Q_i
             W.k = quit ? ~0ull : atomicAdd(Q_in.work, 1ull);
             if (W.k < n) {
                 TIQuery q;
+                TIScale scale;
                 double eff = 0, adj = 0;
                 int sc = 0;
-                W.pre = candidate_setup(A, todo[W.k], q, eff, adj, sc);
-                ti_param_tol(q, adj);
-                ti_filter(q, eff > 0);
-                W.q = q;
+                W.pre = candidate_setup(A, todo[W.k], q, scale, eff, adj, sc);
+                if (W.pre < 0) {
+                    ti_param_tol(q, scale, adj);
+                    ti_filter(q, scale, eff > 0);
+                    W.q = q;
+                    W.scale = scale;
+                }
                 W.eff = eff;
                 W.adj = adj;
                 W.sc = sc;
@@ -464,8 +492,8 @@ __global__ __launch_bounds__(NW * WAVE) void k_ccd_group(CCDArgs A, Searches Q_i
             if (cut || !T.next(A, r, toi)) break;
             __syncthreads(); // the query has been read
             if (first) {
-                ti_param_tol(W.q, T.delta);
-                if (T.tries == 1) ti_filter(W.q, T.ms > 0);
+                ti_param_tol(W.q, W.scale, T.delta);
+                if (T.tries == 1) ti_filter(W.q, W.scale, T.ms > 0);
             }
         }
         if (!first) continue;
@@ -490,6 +518,7 @@ struct WFBox {
 
 struct WFState {
     TIQuery q;
+    TIScale scale;
     int64_t ci;
     double ms, delta, adj, eff;
     double wt, wu, wv;
@@ -511,8 +540,8 @@ __device__ void wf_begin_query(WFState& S, double ms, double delta, long max_itr
     S.ms = ms;
     S.delta = delta;
     S.max_itr = max_itr;
-    ti_param_tol(S.q, delta);
-    ti_filter(S.q, ms > 0);
+    ti_param_tol(S.q, S.scale, delta);
+    ti_filter(S.q, S.scale, ms > 0);
     S.wt = S.wu = S.wv = 1.0;
     S.toi_skip = 4;
     S.temp_toi = INFINITY;
@@ -538,7 +567,7 @@ __global__ void k_wf_init(CCDArgs A, const uint32_t* heavy, int64_t first, int64
     WFState S;
     S.ci = heavy[first + i];
     double eff = 0, adj = 0;
-    const int pre = candidate_setup(A, S.ci, S.q, eff, adj, S.scene);
+    const int pre = candidate_setup(A, S.ci, S.q, S.scale, eff, adj, S.scene);
     S.done = 0;
     S.hit = 0;
     S.result = INFINITY;

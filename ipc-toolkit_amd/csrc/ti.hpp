@@ -41,113 +41,162 @@ enum TIResult : int { TI_MISS = 0, TI_HIT = 1, TI_OVERFLOW = 2, TI_DEEP = 3 };
 constexpr int TI_MAX_LEVELS = 1024;
 constexpr int TI_MAX_NO_ZERO_TOI_ITER = 64;
 
-// F(t,u,v) along one axis.  x0/x1: 12 doubles at t=0 / t=1 in the order
-// (ea0, ea1, eb0, eb1) or (p, t0, t1, t2).
-IPCG_HD double ti_f_ee(const double* s, const double* e, int d, double t, double u, double v)
-{
-    const double a0 = (e[0 + d] - s[0 + d]) * t + s[0 + d];
-    const double a1 = (e[3 + d] - s[3 + d]) * t + s[3 + d];
-    const double b0 = (e[6 + d] - s[6 + d]) * t + s[6 + d];
-    const double b1 = (e[9 + d] - s[9 + d]) * t + s[9 + d];
-    const double va = (a1 - a0) * u + a0;
-    const double vb = (b1 - b0) * v + b0;
-    return va - vb;
-}
-
-IPCG_HD double ti_f_vf(const double* s, const double* e, int d, double t, double u, double v)
-{
-    const double p = (e[0 + d] - s[0 + d]) * t + s[0 + d];
-    const double t0 = (e[3 + d] - s[3 + d]) * t + s[3 + d];
-    const double t1 = (e[6 + d] - s[6 + d]) * t + s[6 + d];
-    const double t2 = (e[9 + d] - s[9 + d]) * t + s[9 + d];
-    const double pt = (t1 - t0) * u + (t2 - t0) * v + t0;
-    return p - pt;
-}
-
 struct TIQuery {
-    double s[12], e[12];
+    double s[12], d[12]; // positions at t=0, differences to t=1
     bool vf;
     double err[3];
     double tol[3];
     double itol[3]; // 1 / tol: widths are powers of two, so 2^-k / tol is itol scaled
 };
 
-IPCG_HD double linf3(const double* a, const double* b)
+// What the tolerances and the filter of a query need of its positions.
+struct TIScale {
+    double len3[3]; // 3 max |dF| along t, u, v over the cube's corners
+    double mag[3];  // per axis, max(|x|, 1)
+};
+
+// F(t,u,v) along one axis, points in the order (ea0, ea1, eb0, eb1) or
+// (p, t0, t1, t2):
+//   edge-edge    (a1 - a0) u + a0 - ((b1 - b0) v + b0)
+//   vertex-face  p - ((t1 - t0) u + (t2 - t0) v + t0)
+// with every point x = d t + s.
+template <bool VF>
+IPCG_HD double ti_corner(const TIQuery& q, int k, double t, double u, double v)
 {
-    double m = 0;
-    for (int k = 0; k < 3; k++) {
-        const double x = fabs(b[k] - a[k]);
-        m = x > m ? x : m;
+    const double x0 = q.d[0 + k] * t + q.s[0 + k];
+    const double x1 = q.d[3 + k] * t + q.s[3 + k];
+    const double x2 = q.d[6 + k] * t + q.s[6 + k];
+    const double x3 = q.d[9 + k] * t + q.s[9 + k];
+    if (VF) {
+        const double pt = (x2 - x1) * u + (x3 - x1) * v + x1;
+        return x0 - pt;
     }
-    return m;
+    const double va = (x1 - x0) * u + x0;
+    const double vb = (x3 - x2) * v + x2;
+    return va - vb;
 }
 
-// Parameter tolerances delta / (3 max |dF| along t, u, v over cube corners)
-IPCG_HD void ti_param_tol(TIQuery& q, double delta)
+// Smallest and largest F over the eight corners [t0,t1] x [u0,u1] x [v0,v1].
+// u enters one product and v another, and every rounded operation is
+// monotone in each operand, so the extremes over the corners of one t are
+// the same chain of operations over the extremes of the products: the same
+// doubles as the eight corners give, in about 55 operations an axis instead
+// of 75.  Where overflow, infinities or NaN occur (the range is not finite)
+// the corners are compared one by one.
+template <bool VF>
+IPCG_HD void ti_range(const TIQuery& q, int k, double t0, double t1, double u0, double u1,
+                      double v0, double v1, double& mn, double& mx)
 {
-    double p[8][3];
-    for (int k = 0; k < 3; k++) {
-        const double* s = q.s;
-        const double* e = q.e;
-        if (q.vf) {
-            p[0][k] = s[k] - s[3 + k];
-            p[1][k] = s[k] - s[9 + k];
-            p[3][k] = s[k] - (s[6 + k] + s[9 + k] - s[3 + k]);
-            p[2][k] = s[k] - s[6 + k];
-            p[4][k] = e[k] - e[3 + k];
-            p[5][k] = e[k] - e[9 + k];
-            p[7][k] = e[k] - (e[6 + k] + e[9 + k] - e[3 + k]);
-            p[6][k] = e[k] - e[6 + k];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const double t = j ? t1 : t0;
+        const double x0 = q.d[0 + k] * t + q.s[0 + k];
+        const double x1 = q.d[3 + k] * t + q.s[3 + k];
+        const double x2 = q.d[6 + k] * t + q.s[6 + k];
+        const double x3 = q.d[9 + k] * t + q.s[9 + k];
+        double lo, hi;
+        if (VF) {
+            const double eu = x2 - x1, ev = x3 - x1;
+            const double a = eu * u0, b = eu * u1, c = ev * v0, e = ev * v1;
+            lo = x0 - (fmax(a, b) + fmax(c, e) + x1);
+            hi = x0 - (fmin(a, b) + fmin(c, e) + x1);
         } else {
-            p[0][k] = s[k] - s[6 + k];
-            p[1][k] = s[k] - s[9 + k];
-            p[3][k] = s[3 + k] - s[9 + k];
-            p[2][k] = s[3 + k] - s[6 + k];
-            p[4][k] = e[k] - e[6 + k];
-            p[5][k] = e[k] - e[9 + k];
-            p[7][k] = e[3 + k] - e[9 + k];
-            p[6][k] = e[3 + k] - e[6 + k];
+            const double ea = x1 - x0, eb = x3 - x2;
+            const double a = ea * u0 + x0, b = ea * u1 + x0;
+            const double c = eb * v0 + x2, e = eb * v1 + x2;
+            lo = fmin(a, b) - fmax(c, e);
+            hi = fmax(a, b) - fmin(c, e);
+        }
+        mn = j == 0 ? lo : fmin(mn, lo);
+        mx = j == 0 ? hi : fmax(mx, hi);
+    }
+    if (!(mx - mn < INFINITY)) {
+        for (int c = 0; c < 8; c++) {
+            const double f =
+                ti_corner<VF>(q, k, (c & 4) ? t1 : t0, (c & 2) ? u1 : u0, (c & 1) ? v1 : v0);
+            mn = (c == 0 || f < mn) ? f : mn;
+            mx = (c == 0 || f > mx) ? f : mx;
         }
     }
-    double dl = linf3(p[0], p[4]), x;
-    if ((x = linf3(p[1], p[5])) > dl) dl = x;
-    if ((x = linf3(p[3], p[7])) > dl) dl = x;
-    if ((x = linf3(p[2], p[6])) > dl) dl = x;
-    double lu = linf3(p[0], p[2]);
-    if ((x = linf3(p[4], p[6])) > lu) lu = x;
-    if ((x = linf3(p[5], p[7])) > lu) lu = x;
-    if ((x = linf3(p[1], p[3])) > lu) lu = x;
-    double lv = linf3(p[0], p[1]);
-    if ((x = linf3(p[4], p[5])) > lv) lv = x;
-    if ((x = linf3(p[6], p[7])) > lv) lv = x;
-    if ((x = linf3(p[2], p[3])) > lv) lv = x;
-    q.tol[0] = delta / (3 * dl);
-    q.tol[1] = delta / (3 * lu);
-    q.tol[2] = delta / (3 * lv);
-    for (int k = 0; k < 3; k++) q.itol[k] = 1.0 / q.tol[k];
 }
 
-// Published floating-point filter: max(|x|, 1)^3 * c per axis.
-IPCG_HD void ti_filter(TIQuery& q, bool use_ms)
+// s, e: 12 positions at t=0 / t=1.  One axis at a time: few values live at
+// once.
+IPCG_HD void ti_scale(const double* s, const double* e, bool vf, TIScale& c)
 {
-    const double c = q.vf ? (use_ms ? 7.549516567451064e-15 : 6.661338147750939e-15)
-                          : (use_ms ? 7.105427357601002e-15 : 6.217248937900877e-15);
+    double dl = 0, lu = 0, lv = 0;
+    auto grow = [](double& m, double a, double b) {
+        const double x = fabs(b - a);
+        m = x > m ? x : m;
+    };
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-        double m = fabs(q.s[k]);
+        double p[8];
+        if (vf) {
+            p[0] = s[k] - s[3 + k];
+            p[1] = s[k] - s[9 + k];
+            p[3] = s[k] - (s[6 + k] + s[9 + k] - s[3 + k]);
+            p[2] = s[k] - s[6 + k];
+            p[4] = e[k] - e[3 + k];
+            p[5] = e[k] - e[9 + k];
+            p[7] = e[k] - (e[6 + k] + e[9 + k] - e[3 + k]);
+            p[6] = e[k] - e[6 + k];
+        } else {
+            p[0] = s[k] - s[6 + k];
+            p[1] = s[k] - s[9 + k];
+            p[3] = s[3 + k] - s[9 + k];
+            p[2] = s[3 + k] - s[6 + k];
+            p[4] = e[k] - e[6 + k];
+            p[5] = e[k] - e[9 + k];
+            p[7] = e[3 + k] - e[9 + k];
+            p[6] = e[3 + k] - e[6 + k];
+        }
+        grow(dl, p[0], p[4]);
+        grow(dl, p[1], p[5]);
+        grow(dl, p[3], p[7]);
+        grow(dl, p[2], p[6]);
+        grow(lu, p[0], p[2]);
+        grow(lu, p[4], p[6]);
+        grow(lu, p[5], p[7]);
+        grow(lu, p[1], p[3]);
+        grow(lv, p[0], p[1]);
+        grow(lv, p[4], p[5]);
+        grow(lv, p[6], p[7]);
+        grow(lv, p[2], p[3]);
+        double m = fabs(s[k]);
+#pragma unroll
         for (int i = 0; i < 4; i++) {
-            const double a = fabs(q.s[3 * i + k]), b = fabs(q.e[3 * i + k]);
+            const double a = fabs(s[3 * i + k]), b = fabs(e[3 * i + k]);
             m = a > m ? a : m;
             m = b > m ? b : m;
         }
-        const double dl = m > 1 ? m : 1;
-        q.err[k] = dl * dl * dl * c;
+        c.mag[k] = m > 1 ? m : 1;
     }
+    c.len3[0] = 3 * dl;
+    c.len3[1] = 3 * lu;
+    c.len3[2] = 3 * lv;
+}
+
+// Parameter tolerances delta / (3 max |dF| along t, u, v over cube corners)
+IPCG_HD void ti_param_tol(TIQuery& q, const TIScale& c, double delta)
+{
+    for (int k = 0; k < 3; k++) {
+        q.tol[k] = delta / c.len3[k];
+        q.itol[k] = 1.0 / q.tol[k];
+    }
+}
+
+// Published floating-point filter: max(|x|, 1)^3 * c per axis.
+IPCG_HD void ti_filter(TIQuery& q, const TIScale& c, bool use_ms)
+{
+    const double f = q.vf ? (use_ms ? 7.549516567451064e-15 : 6.661338147750939e-15)
+                          : (use_ms ? 7.105427357601002e-15 : 6.217248937900877e-15);
+    for (int k = 0; k < 3; k++) q.err[k] = c.mag[k] * c.mag[k] * c.mag[k] * f;
 }
 
 // Inclusion of the origin in the corner box of F over [t,t+wt]x[u,u+wu]x
 // [v,v+wv], inflated by err and ms.  The kind is a template argument so the
-// eight corner evaluations of an axis are one straight block (shared
-// subexpressions computed once), not eight branches on q.vf.
+// evaluation of an axis is one straight block, not branches on q.vf.
 template <bool VF>
 IPCG_HD bool ti_inclusion_k(const TIQuery& q, const TIBox& b, double wt, double wu, double wv,
                             double ms, bool& box_in, double* width)
@@ -155,18 +204,8 @@ IPCG_HD bool ti_inclusion_k(const TIQuery& q, const TIBox& b, double wt, double 
     box_in = true;
     const double t1 = b.t + wt, u1 = b.u + wu, v1 = b.v + wv;
     for (int d = 0; d < 3; d++) {
-        double mn = 0, mx = 0, f0 = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const double t = (c & 4) ? t1 : b.t;
-            const double u = (c & 2) ? u1 : b.u;
-            const double v = (c & 1) ? v1 : b.v;
-            const double f = VF ? ti_f_vf(q.s, q.e, d, t, u, v) : ti_f_ee(q.s, q.e, d, t, u, v);
-            f0 = c == 0 ? f : f0;
-            mn = c == 0 ? f : fmin(mn, f);
-            mx = c == 0 ? f : fmax(mx, f);
-        }
-        if (f0 != f0) mn = mx = f0; // fmin and fmax drop a NaN, comparisons keep the first
+        double mn, mx;
+        ti_range<VF>(q, d, b.t, t1, b.u, u1, b.v, v1, mn, mx);
         width[d] = mx - mn;
         const double eps = q.err[d];
         if (mn - ms > eps || mx + ms < -eps) return false;
@@ -182,10 +221,10 @@ IPCG_HD bool ti_inclusion(const TIQuery& q, const TIBox& b, double wt, double wu
                 : ti_inclusion_k<false>(q, b, wt, wu, wv, ms, box_in, width);
 }
 
-// The same test for a query in LDS, the three axes together; `tol` tells
-// whether every width of the corner box is within co_tol (meaningful when the
+// The same test for a query in LDS, AXES axes at a time (3: shortest chain, 1:
+// fewer registers); `tol` tells whether every width of the corner box is within co_tol (meaningful when the
 // origin is included).
-template <bool VF>
+template <bool VF, int AXES>
 __device__ __forceinline__ bool ti_inclusion_tol_k(const TIQuery& q, const TIBox& b, double wt,
                                                    double wu, double wv, double ms, double co_tol,
                                                    bool& box_in, bool& tol)
@@ -193,20 +232,10 @@ __device__ __forceinline__ bool ti_inclusion_tol_k(const TIQuery& q, const TIBox
     box_in = tol = true;
     const double t1 = b.t + wt, u1 = b.u + wu, v1 = b.v + wv;
     bool zero = true;
-#pragma unroll
+#pragma unroll AXES
     for (int d = 0; d < 3; d++) {
-        double mn = 0, mx = 0, f0 = 0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const double t = (c & 4) ? t1 : b.t;
-            const double u = (c & 2) ? u1 : b.u;
-            const double v = (c & 1) ? v1 : b.v;
-            const double f = VF ? ti_f_vf(q.s, q.e, d, t, u, v) : ti_f_ee(q.s, q.e, d, t, u, v);
-            f0 = c == 0 ? f : f0;
-            mn = c == 0 ? f : fmin(mn, f);
-            mx = c == 0 ? f : fmax(mx, f);
-        }
-        if (f0 != f0) mn = mx = f0; // fmin and fmax drop a NaN, comparisons keep the first
+        double mn, mx;
+        ti_range<VF>(q, d, b.t, t1, b.u, u1, b.v, v1, mn, mx);
         const double eps = q.err[d];
         if (!(mx - mn <= co_tol)) tol = false;
         if (mn - ms > eps || mx + ms < -eps) zero = false;
@@ -215,12 +244,13 @@ __device__ __forceinline__ bool ti_inclusion_tol_k(const TIQuery& q, const TIBox
     return zero;
 }
 
+template <int AXES>
 __device__ __forceinline__ bool ti_inclusion_tol(const TIQuery& q, const TIBox& b, double wt,
                                                  double wu, double wv, double ms, double co_tol,
                                                  bool& box_in, bool& tol)
 {
-    return q.vf ? ti_inclusion_tol_k<true>(q, b, wt, wu, wv, ms, co_tol, box_in, tol)
-                : ti_inclusion_tol_k<false>(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
+    return q.vf ? ti_inclusion_tol_k<true, AXES>(q, b, wt, wu, wv, ms, co_tol, box_in, tol)
+                : ti_inclusion_tol_k<false, AXES>(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
 }
 
 // The axis a level is split along: the first with the largest width over
@@ -286,12 +316,12 @@ __device__ __forceinline__ unsigned long long ti_pack(unsigned it, unsigned iu, 
            ((unsigned long long)iu << TI_LDS_BITS) | iv;
 }
 
+// Searches of more than `budget` boxes overflow too: the wave waits for its
+// longest search, and the tiers above search long ones faster.
 __device__ inline int ti_bfs_lds(const TIQuery& q, double co_tol, double ms, long max_itr,
-                                 const TIBound& B, const TILdsLists& L, double& toi,
-                                 double& out_tol)
+                                 const TIBound& B, const TILdsLists& L, long budget, double& toi)
 {
-    out_tol = co_tol;
-    double temp_out_tol = co_tol, temp_toi = INFINITY;
+    double temp_toi = INFINITY;
     double toi_skip = 4;
     bool use_skip = false;
     long refine = 0;
@@ -307,18 +337,7 @@ __device__ inline int ti_bfs_lds(const TIQuery& q, double co_tol, double ms, lon
         const double wt = ldexp(1.0, -kt), wu = ldexp(1.0, -ku), wv = ldexp(1.0, -kv);
         bool level_less_tol = true, level_root = false;
         const bool c1 = wt <= q.tol[0] && wu <= q.tol[1] && wv <= q.tol[2];
-        int axis = 0;
-        {
-            double best = -INFINITY;
-            const double w3[3] = { wt, wu, wv };
-            for (int i = 0; i < 3; i++) {
-                const double r = w3[i] > q.tol[i] ? w3[i] / q.tol[i] : -INFINITY;
-                if (r > best) {
-                    best = r;
-                    axis = i;
-                }
-            }
-        }
+        const int axis = ti_axis(q, wt, wu, wv);
         const int nk = (axis == 0 ? kt : axis == 1 ? ku : kv) + 1;
         int nlo = 0, nhi = 0;
         for (int i = 0; i < ncur; i++) {
@@ -330,6 +349,7 @@ __device__ inline int ti_bfs_lds(const TIQuery& q, double co_tol, double ms, lon
                             ldexp((double)iv, -kv) };
             if (b.t >= toi_skip || b.t >= bound) continue;
             refine++;
+            if (refine > budget) return TI_OVERFLOW;
             bool box_in;
             double tw[3];
             if (!ti_inclusion(q, b, wt, wu, wv, ms, box_in, tw)) continue;
@@ -343,14 +363,10 @@ __device__ inline int ti_bfs_lds(const TIQuery& q, double co_tol, double ms, lon
             if (max_itr > 0) {
                 if (!level_root) {
                     temp_toi = b.t;
-                    double m = co_tol;
-                    for (int k = 0; k < 3; k++) m = tw[k] > m ? tw[k] : m;
-                    temp_out_tol = m;
                     level_root = true;
                 }
                 if (refine > max_itr) {
                     toi = temp_toi;
-                    out_tol = temp_out_tol;
                     return TI_HIT;
                 }
             }
@@ -616,7 +632,7 @@ __device__ inline int ti_bfs_group(const TIQuery& q, double co_tol, double ms, l
             const unsigned iv = (unsigned)pb & TI_LDS_MASK;
             const TIBox b { ldexp((double)it, -kt), ldexp((double)iu, -ku), ldexp((double)iv, -kv) };
             live = i < ncur && !(b.t >= toi_skip || b.t >= bound);
-            if (live) zero = ti_inclusion_tol(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
+            if (live) zero = ti_inclusion_tol<3>(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
             const bool stop = zero && (c1 || tol || box_in);
             const bool past = zero && max_itr > 0 && refine + i + 1 > max_itr;
             // children: both halves of t; the halves of u or v that can hold
@@ -801,7 +817,7 @@ __device__ inline int ti_bfs_sub(const TIQuery& q, double co_tol, double ms, lon
             const TIBox b { ldexp((double)it, -kt), ldexp((double)iu, -ku), ldexp((double)iv, -kv) };
             const bool live = i < ncur && !(b.t >= toi_skip || b.t >= bound);
             bool zero = false, tol = false, box_in = false;
-            if (live) zero = ti_inclusion_tol(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
+            if (live) zero = ti_inclusion_tol<1>(q, b, wt, wu, wv, ms, co_tol, box_in, tol);
             const bool past = zero && max_itr > 0 && refine + i + 1 > max_itr;
             const unsigned hu = axis == 1 ? 2 * iu + 1 : iu, hv = axis == 1 ? iv : 2 * iv + 1;
             const unsigned lu = axis == 1 ? 2 * iu : iu, lv = axis == 1 ? iv : 2 * iv;
@@ -911,44 +927,6 @@ __device__ inline int ti_bfs_sub(const TIQuery& q, double co_tol, double ms, lon
         return TI_HIT;
     }
     return TI_MISS;
-}
-
-// ticcd::{edgeEdge,vertexFace}CCD with the automatic error filter and the
-// no_zero_toi loop around a one-lane search.
-template <class Search>
-__device__ inline int ti_query_with(TIQuery& q, double ms, double tolerance, long max_itr,
-                                    bool no_zero_toi, const Search& bfs, double& toi)
-{
-    ti_param_tol(q, tolerance);
-    ti_filter(q, ms > 0);
-    int r;
-    double out_tol;
-    for (int it = 0;; it++) {
-        r = bfs(q, tolerance, ms, max_itr, toi, out_tol);
-        if (it + 1 >= TI_MAX_NO_ZERO_TOI_ITER) break;
-        if (!(no_zero_toi && r == TI_HIT && toi == 0)) break;
-        if (out_tol > tolerance) {
-            break; // unreachable with unlimited iterations (out_tol == tolerance)
-        } else if (10 * tolerance < ms) {
-            ms *= 0.5;
-        } else {
-            tolerance *= 0.5;
-            ti_param_tol(q, tolerance);
-        }
-    }
-    return r;
-}
-
-__device__ inline int ti_query_lds(TIQuery& q, double ms, double tolerance, long max_itr,
-                                   bool no_zero_toi, const TIBound& B, const TILdsLists& L,
-                                   double& toi)
-{
-    return ti_query_with(
-        q, ms, tolerance, max_itr, no_zero_toi,
-        [&](const TIQuery& qq, double co_tol, double m, long mi, double& t, double& ot) {
-            return ti_bfs_lds(qq, co_tol, m, mi, B, L, t, ot);
-        },
-        toi);
 }
 
 } // namespace ipcg
