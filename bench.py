@@ -34,22 +34,20 @@ FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 (vector and matrix), TFLOP/s
 # and FP64 flops it must execute, counted from the algorithm).
 # Hessian record of one collision: ids, weight (+ eps, dtype for EE), the
 # stencil's points, and the packed projected Hessian written out.
-REC_BYTES = {"ee": 8 + 8 + 8 + 4 + 4 * 24 + 45 * 8,
-             "fv": 8 + 8 + 4 * 24 + 45 * 8,
-             "ev": 8 + 8 + 3 * 24 + 21 * 8}
+REC_BYTES = {"ee": 8 + 8 + 8 + 4 + 4 * 24 + 28 * 8,
+             "fv": 8 + 8 + 4 * 24 + 28 * 8,
+             "ev": 8 + 8 + 3 * 24 + 28 * 8,
+             "vv": 8 + 8 + 2 * 24 + 28 * 8}
 # Jacobi PSD projection of an n x n matrix: SWEEPS[n] sweeps of n(n-1)/2
 # rotations (12n + 7 flops each), a convergence sum per sweep (n(n+1)
 # flops) and the reconstruction V diag(lambda) V^T (3n flops per packed
 # entry); SWEEPS is the mean sweep count measured on contact stencils.
-SWEEPS = {3: 4, 6: 6, 9: 7}
+SWEEPS = {5: 5, 9: 7}
 PSD_FLOPS = {n: SWEEPS[n] * (n * (n - 1) // 2 * (12 * n + 7) + n * (n + 1))
-             + 3 * n * n * (n + 1) // 2 for n in (3, 6, 9)}
-# Rank-5 path for a 9 x 9 matrix: 5 Lanczos steps (matrix-vector product,
-# two reorthogonalization passes), T = Q^T A Q (6 products + 21 dots), the
-# residual A - Q T Q^T (45 entries x 36 terms), a 6 x 6 Jacobi (5 sweeps),
-# the Ritz vectors and the reconstruction.
-KRYLOV9_FLOPS = (5 * (162 + 2 * 3 * 36 + 20) + (6 * 162 + 21 * 18) + 45 * 36 * 3
-                 + 5 * (15 * (12 * 6 + 7) + 42) + 9 * 6 * 6 * 2 + 45 * 6 * 3)
+             + 3 * n * n * (n + 1) // 2 for n in (5, 9)}
+# Unmollified collision: the frame of the closest points (about 200 flops),
+# the 5 x 5 matrix and its projection, and the record from it (about 150).
+FRAME_FLOPS = 350 + PSD_FLOPS[5]
 # Tight-Inclusion: one box = the 8 corners of F along 3 axes (about 70 flops
 # per axis); a candidate that survives the root pass visits 5.0 boxes on
 # average on the sheet-stack workload (counted in-kernel).
@@ -459,7 +457,7 @@ def main():
 
     ccd_work = {k: ctx.counter(k) for k in ("ccd.candidates", "ccd.searched", "ccd.spilled",
                                               "ccd.spilled_deep", "ccd.wavefront")}
-    ee_other = ctx.counter("hessian.ee_other")
+    ee_moll = ctx.counter("hessian.ee_other")
     counts = ctx.collision_counts()
     ctx.broad_phase(False, 0.5 * sc.dhat)
     ne_s, nf_s = [len(x) for x in ctx.candidates()]
@@ -485,11 +483,11 @@ def main():
         "bp_traverse_fv.swept": (24 * nV + 8 * nf_d, 0),
         "np_classify": (8 * (ne_s + nf_s) + 16 * pairs, 0),
         "energy": (16 * pairs + 8, 0),
-        "hessian_records.ee": (REC_BYTES["ee"] * (n_ee - ee_other),
-                               KRYLOV9_FLOPS * (n_ee - ee_other)),
-        "hessian_records.ee_other": (REC_BYTES["ee"] * ee_other, PSD_FLOPS[9] * ee_other),
-        "hessian_records.fv": (REC_BYTES["fv"] * n_fv, KRYLOV9_FLOPS * n_fv),
-        "hessian_records.ev": (REC_BYTES["ev"] * n_ev, PSD_FLOPS[6] * n_ev),
+        "hessian_records": (REC_BYTES["ee"] * (n_ee - ee_moll) + REC_BYTES["fv"] * n_fv
+                            + REC_BYTES["ev"] * n_ev + REC_BYTES["vv"] * n_vv,
+                            FRAME_FLOPS * (pairs - ee_moll)),
+        "hessian_records.mollified": ((REC_BYTES["ee"] + 18 * 8) * ee_moll,
+                                      PSD_FLOPS[9] * ee_moll),
         "hessian_assemble": (12 * nnz + 8 * (3 * nV + 1), 0),
         "ccd_root": (200 * (ne_d + nf_d), 0),
         "ccd_lds": (204 * searched, TI_BOX_FLOPS * TI_BOXES_PER_SEARCH * searched),

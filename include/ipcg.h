@@ -478,8 +478,8 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
  * or the level-by-level wavefront takes them),
  * "ccd.unmet" (1 when an expected minimum did not stand and the searches
  * ran again without it),
- * "hessian.ee_other" (edge-edge collisions of the last Hessian whose type
- * is not the interior one; their projection takes the 9 x 9 path),
+ * "hessian.ee_other" (edge-edge collisions of the last Hessian under their
+ * mollifier; their projection takes the 9 x 9 path),
  * "hessian.pattern_sorted" (1 when a row of the last Hessian pattern had
  * more than 256 distinct block columns and the pattern was built by a
  * sort of all stencil pairs instead of the per-row hash),

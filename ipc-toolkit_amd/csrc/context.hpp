@@ -135,9 +135,10 @@ struct Ctx {
     DevBuf blk_mask, row_cnt, rowptr, col, val;
     DevBuf hp_mark, hp_bptr, hp_bcol; // block pattern of the collision set
     DevBuf inc_keys, inc_keys2, inc_vals, inc_vals2, inc_ptr; // vertex -> (collision, point)
-    DevBuf ee_other;                  // edge-edge collisions of non-interior types (list)
+    DevBuf ee_mollified;              // mollified edge-edge collisions (list)
     DevBuf inc_vtx;                   // stencil vertices per sorted incidence (int4)
-    DevBuf hrec;                      // projected Hessian per collision (Q basis)
+    DevBuf hrec;                      // projected Hessian record per collision
+    DevBuf hrec_ext;                  // rest of the full records (mollified edge-edge)
     DevBuf gn_out, gn_p;              // Gauss-Newton diagonal (3 nV) and direction (3 nV)
     DevBuf fric;                      // friction record per collision (global order)
     bool fric_valid = false;

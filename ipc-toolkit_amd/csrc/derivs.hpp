@@ -285,9 +285,9 @@ IPCG_HD void add_sym_outer(double* Hq, double alpha, const d3* a, const d3* b)
 }
 
 // ---------------------------------------------------------------------------
-// 1/sqrt(x) for x in [1, 2]: the hardware estimate refined by two Newton
-// steps (each squares the relative error), a few ulp from 1.0 / sqrt(x) at
-// a fraction of the instructions of a correctly rounded sqrt and divide.
+// 1/sqrt(x) and 1/x for normal x: the hardware estimate refined by two Newton
+// steps (each squares the relative error), a few ulp from the correctly
+// rounded ones at a fraction of their instructions.
 // ---------------------------------------------------------------------------
 IPCG_HD double rsqrt_nr(double x)
 {
@@ -301,8 +301,24 @@ IPCG_HD double rsqrt_nr(double x)
 #endif
 }
 
+IPCG_HD double rcp_nr(double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+#else
+    return 1.0 / x;
+#endif
+}
+
 // ---------------------------------------------------------------------------
-// PSD projection (cyclic Jacobi, eigenvectors accumulated in registers)
+// PSD projection (cyclic Jacobi, eigenvectors accumulated in registers).
+// The tangent of a rotation, h / (|d| + sqrt(d^2 + h^2)) for h = 2 a_pq and
+// d = a_qq - a_pp, may be a few ulp off: c and s are normalized to the
+// tangent that was computed, and the entry set to 0 is off by as many ulp.
+// (Rounded division and square root were two thirds of a rotation's
+// instructions on a 5 x 5 matrix.)
 // method: 0 none, 1 clamp, 2 abs (PSDProjectionMethod, eigen_ext.hpp:202-206)
 // ---------------------------------------------------------------------------
 template <int N>
@@ -331,9 +347,10 @@ IPCG_HD void project_psd(double* A /* packed N */, int method)
             for (int q = p + 1; q < N; q++) {
                 const double apq = A[sp(p, q)];
                 const double app = A[sp(p, p)], aqq = A[sp(q, q)];
-                const double theta = (aqq - app) / (2 * apq);
-                double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1));
-                t = apq == 0.0 ? 0.0 : t;
+                const double dd = aqq - app, h = 2 * apq, x = dd * dd + h * h;
+                double t = h * rcp_nr(fabs(dd) + x * rsqrt_nr(x));
+                t = dd < 0 ? -t : t;
+                t = x >= 1e-290 ? t : 0.0; // (both entries vanish)
                 const double c = rsqrt_nr(t * t + 1), s = t * c; // |t| <= 1
 #pragma unroll
                 for (int k = 0; k < N; k++) {
@@ -371,196 +388,187 @@ IPCG_HD void project_psd(double* A /* packed N */, int method)
 }
 
 // ---------------------------------------------------------------------------
-// PSD projection of a 9 x 9 matrix of rank at most KR (contact stencils of
-// the point-triangle and edge-edge interior types have rank 5 in the
-// translation-free basis: 3 positive and 2 negative eigenvalues).
+// Hessian of b(d) of an unmollified stencil in five coordinates.
 //
-// Lanczos from b = A w (w fixed, b in the range of A) with full
-// reorthogonalization builds an orthonormal basis Q of the Krylov space
-// until the next vector vanishes; the eigen-pairs of T = Q^T A Q (at most
-// KR x KR, cyclic Jacobi) give A = (Q V) diag(lambda) (Q V)^T.  The result
-// is accepted only if the residual |A - Q T Q^T|_F is at most 1e-12 |A|_F
-// (the Krylov space holds the whole range of A); otherwise A is left
-// untouched and false is returned (the caller runs project_psd<9>).
+// Let q be the vector between the closest points (points weighted by c, sum
+// 0), n its direction and e1, e2 the other axes of an orthonormal frame:
+//   plane (point-triangle, interior edge-edge): n normal to the plane,
+//   line  (point-line): e1 along the line,
+//   point (point-point): any e1, e2.
+// With sigma = n . q, d = sigma^2 and rho_k the rotation of the frame about
+// the closest points (linear in n . dx: the point weights r_k), the second
+// derivative of d / 2 along dx is
+//   (n . dq)^2 - 2 sum_k rho_k (e_k . dq) - sum_k rho_k^2 + sum_k y_k (e_k . dq)^2
+// with y_k = 1 along the axes in which the nearest feature does not extend
+// (rho_k = 0 there).  So the energy Hessian acts on n (x) R^3 and e_k (x) c
+// only: five orthonormal coordinates z0..z2 = n (x) (c^, f1, f2) and
+// e_k (x) c^, where it is
+//   4 d b'' + 2 b' on the n . dq term, 2 b' on the others,
+// and its projection is that of a 5 x 5 matrix.
 // ---------------------------------------------------------------------------
-template <int KR>
-IPCG_HD bool project_psd_krylov9(double* A /* packed 9 */, int method)
+struct ContactFrame {
+    d3 n, e1, e2;
+    double c[4], r1[4], r2[4]; // point weights
+    double y1, y2;
+};
+
+IPCG_HD d3 unit(const d3& v) { return scale(v, 1.0 / sqrt(sqn(v))); }
+
+// two axes completing the unit vector a (Duff et al., "Building an
+// Orthonormal Basis, Revisited", JCGT 2017)
+IPCG_HD void complement(const d3& a, d3& b, d3& c)
+{
+    const double sg = a.z < 0 ? -1.0 : 1.0;
+    const double h = -1.0 / (sg + a.z), xy = a.x * a.y * h;
+    b = { 1.0 + sg * a.x * a.x * h, sg * xy, -sg * a.x };
+    c = { xy, sg + a.y * a.y * h, -a.y };
+}
+
+// 4-point weights to the Q basis
+IPCG_HD d3 weights_q(const double* w)
+{
+    return { 0.5 * ((w[0] - w[1]) + (w[2] - w[3])), 0.5 * ((w[0] + w[1]) - (w[2] + w[3])),
+             0.5 * ((w[0] - w[1]) - (w[2] - w[3])) };
+}
+
+// plane through the origin along u, v (weights U, V), w (weights W) to it
+IPCG_HD void frame_plane(const d3& w, const d3& u, const d3& v, const double* W, const double* U,
+                         const double* V, ContactFrame& f)
 {
 #pragma clang fp contract(fast)
-    constexpr int N = 9;
-    if (method == 0) return true;
-    double nA2 = 0;
+    const double lu = sqrt(sqn(u)), iu = 1.0 / lu;
+    f.e1 = scale(u, iu);
+    const d3 m = cross(u, v);
+    const double in = 1.0 / sqrt(sqn(m));
+    f.n = scale(m, in);
+    f.e2 = cross(f.n, f.e1);
+    const double v1 = dot(v, f.e1), w2 = dot(w, f.e2);
+    const double k2 = lu * in;
+    const double b = w2 * k2, a = dot(w, f.e1) * iu - v1 * in * w2;
+    const double sig = dot(w, f.n);
+    const double su = sig * iu, s2u = -sig * v1 * in, s2v = sig * k2;
+    f.y1 = f.y2 = 0;
 #pragma unroll
-    for (int i = 0; i < N; i++)
-#pragma unroll
-        for (int j = 0; j <= i; j++) nA2 += (i == j ? 1.0 : 2.0) * A[sp(i, j)] * A[sp(i, j)];
-    if (!(nA2 > 0)) return true; // the zero matrix is its own projection
-    if (!(nA2 < 1e300)) return false;
-    auto matvec = [&](const double* x, double* y) {
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            double acc = 0;
-#pragma unroll
-            for (int j = 0; j < N; j++) acc += A[sp(i, j)] * x[j];
-            y[i] = acc;
-        }
-    };
-    constexpr double w[N] = { 0.3719, -0.6541, 0.2333, 0.8123, -0.1427,
-                              0.5021, -0.7433, 0.0679, 0.4517 };
-    double Q[KR][N], al[KR], be[KR];
-#pragma unroll
-    for (int k = 0; k < KR; k++) {
-        al[k] = be[k] = 0;
-#pragma unroll
-        for (int i = 0; i < N; i++) Q[k][i] = 0;
+    for (int x = 0; x < 4; x++) {
+        f.c[x] = (W[x] - a * U[x]) - b * V[x];
+        f.r1[x] = su * U[x];
+        f.r2[x] = s2u * U[x] + s2v * V[x];
     }
-    double u[N];
-    matvec(w, u);
-    const double tiny = 1e-13 * sqrt(nA2);
-    double nb = 0;
+}
+
+// Line l0 l1, w0 and w1 from its ends to the point (weights W from l0, L
+// along the line).  The direction off the line comes from w0 x w1, the
+// vectors of the squared distance: a rounded unit vector along the line would
+// turn it by |w| / |r| roundings.
+IPCG_HD void frame_line(const d3& w, const d3& w1, const d3& e, const double* W, const double* L,
+                        ContactFrame& f)
+{
+#pragma clang fp contract(fast)
+    const double e2 = sqn(e), ie = 1.0 / sqrt(e2), ie2 = 1.0 / e2;
+    f.e1 = scale(e, ie);
+    const d3 m = cross(w1, w);
+    const double m2 = sqn(m);
+    d3 b, c;
+    complement(f.e1, b, c);
+    f.e2 = m2 > 0 ? scale(m, 1.0 / sqrt(m2)) : b;
+    f.n = cross(f.e1, f.e2);
+    const double a = dot(w, e) * ie2, s = sqrt(m2) * ie2;
+    f.y1 = 0;
+    f.y2 = 1;
 #pragma unroll
-    for (int i = 0; i < N; i++) nb += u[i] * u[i];
-    nb = sqrt(nb);
-    if (!(nb > tiny)) return false;
+    for (int x = 0; x < 4; x++) {
+        f.c[x] = W[x] - a * L[x];
+        f.r1[x] = s * L[x];
+        f.r2[x] = 0;
+    }
+}
+
+IPCG_HD void frame_point(const d3& w, const double* W, ContactFrame& f)
+{
+    const double w2 = sqn(w);
+    f.n = w2 > 0 ? scale(w, 1.0 / sqrt(w2)) : d3 { 1, 0, 0 };
+    complement(f.n, f.e1, f.e2);
+    f.y1 = f.y2 = 1;
 #pragma unroll
-    for (int i = 0; i < N; i++) Q[0][i] = u[i] / nb;
-    int m = 0; // Krylov dimension
-    bool closed = false;
+    for (int x = 0; x < 4; x++) {
+        f.c[x] = W[x];
+        f.r1[x] = f.r2[x] = 0;
+    }
+}
+
+// Projected Hessian from the frame and the derivatives f1, f2 of the energy
+// by d, as a record of FRAME_LEN values: n, c, M (packed 3 x 3), R (3 rows),
+// T (packed 3 x 3), with the 3 x 3 block of the 4-point Q basis rows k, l
+//   M_kl n n^T + c_k R_l n^T + c_l n R_k^T + c_k c_l T.
+// The 5 x 5 matrix is scaled to entries of at most 1 for the projection.
+constexpr int FRAME_LEN = 27;
+
+IPCG_HD void frame_hessian(const ContactFrame& f, double d, double f1, double f2, int method,
+                           double* o)
+{
+#pragma clang fp contract(fast)
+    const d3 cq = weights_q(f.c), q1 = weights_q(f.r1), q2 = weights_q(f.r2);
+    const double cl2 = sqn(cq), cl = sqrt(cl2);
+    const d3 ch = scale(cq, 1.0 / cl);
+    d3 g1, g2;
+    complement(ch, g1, g2);
+    const double a[3] = { dot(q1, ch), dot(q1, g1), dot(q1, g2) };
+    const double b[3] = { dot(q2, ch), dot(q2, g1), dot(q2, g2) };
+    const double k = 2 * f1, kc = -k * cl;
+    double B[15];
 #pragma unroll
-    for (int k = 0; k < KR; k++) {
-        if (!closed) {
-            matvec(Q[k], u);
-            double a = 0;
+    for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int i = 0; i < N; i++) a += Q[k][i] * u[i];
-            al[k] = a;
-            // full reorthogonalization, twice
+        for (int j = 0; j <= i; j++) B[sp(i, j)] = -k * (a[i] * a[j] + b[i] * b[j]);
+    B[0] += (4 * d * f2 + k) * cl2;
 #pragma unroll
-            for (int pass = 0; pass < 2; pass++)
+    for (int j = 0; j < 3; j++) {
+        B[sp(3, j)] = kc * a[j];
+        B[sp(4, j)] = kc * b[j];
+    }
+    B[sp(3, 3)] = k * cl2 * f.y1;
+    B[sp(4, 4)] = k * cl2 * f.y2;
+    B[sp(4, 3)] = 0;
+    if (method != 0) {
+        double mx = 0;
 #pragma unroll
-                for (int j = 0; j <= k; j++) {
-                    double d = 0;
+        for (int e = 0; e < 15; e++) mx = fmax(mx, fabs(B[e]));
+        if (mx > 0) { // (a NaN stays in its entry)
+            const double im = 1.0 / mx;
 #pragma unroll
-                    for (int i = 0; i < N; i++) d += Q[j][i] * u[i];
+            for (int e = 0; e < 15; e++) B[e] *= im;
+            project_psd<5>(B, method);
 #pragma unroll
-                    for (int i = 0; i < N; i++) u[i] -= d * Q[j][i];
-                }
-            double b = 0;
-#pragma unroll
-            for (int i = 0; i < N; i++) b += u[i] * u[i];
-            b = sqrt(b);
-            m = k + 1;
-            if (b <= tiny) {
-                closed = true;
-            } else if (k + 1 < KR) {
-                be[k] = b;
-#pragma unroll
-                for (int i = 0; i < N; i++) Q[k + 1][i] = u[i] / b;
-            }
+            for (int e = 0; e < 15; e++) B[e] *= mx;
         }
     }
-    if (!closed) return false;
-    // T = Q^T A Q in the basis (tridiagonal up to rounding: use the exact
-    // projection so the residual test sees the same matrix)
-    double T[KR * (KR + 1) / 2];
+    // M = F B_zz F^T over F = (c^, g1, g2), R = F B_zy (e1, e2)^T, and the
+    // in-frame part T = sum B_yy e e^T
+    const double F[3][3] = { { ch.x, g1.x, g2.x }, { ch.y, g1.y, g2.y }, { ch.z, g1.z, g2.z } };
+    o[0] = f.n.x; o[1] = f.n.y; o[2] = f.n.z;
+    o[3] = ch.x; o[4] = ch.y; o[5] = ch.z;
 #pragma unroll
-    for (int k = 0; k < KR; k++) {
-        matvec(Q[k], u);
+    for (int i = 0; i < 3; i++) {
+        double t[3];
 #pragma unroll
-        for (int l = 0; l <= k; l++) {
-            double d = 0;
+        for (int j = 0; j < 3; j++)
+            t[j] = F[i][0] * B[sp(0, j)] + F[i][1] * B[sp(1, j)] + F[i][2] * B[sp(2, j)];
 #pragma unroll
-            for (int i = 0; i < N; i++) d += Q[l][i] * u[i];
-            T[sp(k, l)] = d;
-        }
+        for (int j = 0; j <= i; j++)
+            o[6 + sp(i, j)] = t[0] * F[j][0] + t[1] * F[j][1] + t[2] * F[j][2];
+        const double p = F[i][0] * B[sp(3, 0)] + F[i][1] * B[sp(3, 1)] + F[i][2] * B[sp(3, 2)];
+        const double q = F[i][0] * B[sp(4, 0)] + F[i][1] * B[sp(4, 1)] + F[i][2] * B[sp(4, 2)];
+        o[12 + 3 * i] = p * f.e1.x + q * f.e2.x;
+        o[13 + 3 * i] = p * f.e1.y + q * f.e2.y;
+        o[14 + 3 * i] = p * f.e1.z + q * f.e2.z;
     }
-    (void)m;
-    // residual |A - Q T Q^T|_F
-    double r2 = 0;
+    const double u[3] = { f.e1.x, f.e1.y, f.e1.z }, v[3] = { f.e2.x, f.e2.y, f.e2.z };
 #pragma unroll
-    for (int i = 0; i < N; i++)
+    for (int r = 0; r < 3; r++)
 #pragma unroll
-        for (int j = 0; j <= i; j++) {
-            double x = A[sp(i, j)];
-#pragma unroll
-            for (int k = 0; k < KR; k++)
-#pragma unroll
-                for (int l = 0; l < KR; l++) x -= Q[k][i] * T[sp(k, l)] * Q[l][j];
-            r2 += (i == j ? 1.0 : 2.0) * x * x;
-        }
-    if (!(r2 <= 1e-24 * nA2)) return false;
-    // eigen-pairs of T (unused dimensions are zero rows: zero eigenvalues)
-    double V[KR][KR];
-#pragma unroll
-    for (int i = 0; i < KR; i++)
-#pragma unroll
-        for (int j = 0; j < KR; j++) V[i][j] = i == j ? 1.0 : 0.0;
-#pragma clang loop unroll(disable)
-    for (int sweep = 0; sweep < 16; sweep++) {
-        double off = 0, tot = 0;
-#pragma unroll
-        for (int i = 0; i < KR; i++) {
-            tot += T[sp(i, i)] * T[sp(i, i)];
-#pragma unroll
-            for (int j = 0; j < i; j++) off += T[sp(i, j)] * T[sp(i, j)];
-        }
-        tot += 2 * off;
-        if (!(off > 1e-30 * tot)) break;
-#pragma unroll
-        for (int p = 0; p < KR; p++)
-#pragma unroll
-            for (int q = p + 1; q < KR; q++) {
-                const double apq = T[sp(p, q)];
-                const double app = T[sp(p, p)], aqq = T[sp(q, q)];
-                const double theta = (aqq - app) / (2 * apq);
-                double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1));
-                t = apq == 0.0 ? 0.0 : t;
-                const double c = rsqrt_nr(t * t + 1), s = t * c;
-#pragma unroll
-                for (int k = 0; k < KR; k++) {
-                    if (k == p || k == q) continue;
-                    const double akp = T[sp(k, p)], akq = T[sp(k, q)];
-                    T[sp(k, p)] = c * akp - s * akq;
-                    T[sp(k, q)] = s * akp + c * akq;
-                }
-                T[sp(p, p)] = app - t * apq;
-                T[sp(q, q)] = aqq + t * apq;
-                T[sp(p, q)] = 0.0;
-#pragma unroll
-                for (int k = 0; k < KR; k++) {
-                    const double vkp = V[k][p], vkq = V[k][q];
-                    V[k][p] = c * vkp - s * vkq;
-                    V[k][q] = s * vkp + c * vkq;
-                }
-            }
-    }
-    // W = Q^T V (N x KR columns), A = W diag(lambda+) W^T
-    double lam[KR];
-#pragma unroll
-    for (int c = 0; c < KR; c++) {
-        const double l = T[sp(c, c)];
-        lam[c] = l >= 0 ? l : (method == 1 ? 0.0 : -l);
-    }
-    double W[N][KR];
-#pragma unroll
-    for (int i = 0; i < N; i++)
-#pragma unroll
-        for (int c = 0; c < KR; c++) {
-            double x = 0;
-#pragma unroll
-            for (int k = 0; k < KR; k++) x += Q[k][i] * V[k][c];
-            W[i][c] = x;
-        }
-#pragma unroll
-    for (int i = 0; i < N; i++)
-#pragma unroll
-        for (int j = 0; j <= i; j++) {
-            double acc = 0;
-#pragma unroll
-            for (int c = 0; c < KR; c++) acc += W[i][c] * lam[c] * W[j][c];
-            A[sp(i, j)] = acc;
-        }
-    return true;
+        for (int t = 0; t <= r; t++)
+            o[21 + sp(r, t)] = B[sp(3, 3)] * u[r] * u[t] + B[sp(4, 4)] * v[r] * v[t]
+                + B[sp(4, 3)] * (u[r] * v[t] + v[r] * u[t]);
 }
 
 } // namespace ipcg

@@ -367,10 +367,8 @@ __global__ __launch_bounds__(PB) void k_gn_quadratic_form(CollView C, const doub
     }
 }
 
-template <int KIND> struct HqTraits {
-    static constexpr int NP = StencilTraits<KIND>::NP;
-    static constexpr int N = 3 * (NP - 1);
-    static constexpr int LEN = N * (N + 1) / 2;
+struct CollRanges {
+    int64_t goff[5]; // global collision index ranges per kind
 };
 
 // ---- symbolic phase: block pattern of the collision set ---------------------
@@ -462,10 +460,6 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-struct CollRanges {
-    int64_t goff[5]; // global collision index ranges per kind
-};
 
 constexpr int PH_BITS = 9;
 constexpr int PH = 1 << PH_BITS; // hash slots per wave (LDS: 8 waves per SIMD fit)
@@ -594,88 +588,111 @@ __global__ __launch_bounds__(256) void k_gradient_rows(CollRanges G, GradRecs R,
 }
 
 // ---- numeric phase without global atomics ------------------------------------
-// (1) every collision writes its PSD-projected Hessian in the Q basis
-//     (packed 3K x 3K) to a record;
+// (1) every collision writes its PSD-projected Hessian in the 4-point Q basis
+//     to a record, so one code path expands all kinds (unused points have
+//     weight 0 and get zero blocks);
 // (2) the (vertex, collision, point) incidences are sorted by vertex;
 // (3) one wave per vertex owns its block row: the lanes walk the vertex's
 //     incidences, expand each record to the row's 3x3 blocks and add them
 //     into the row's accumulators in LDS, then the wave writes the row.
-// Every record holds the projected Hessian in the 4-point Q basis (packed
-// 9 x 9, REC_LEN values), so one code path expands all kinds.  A stencil of
-// NP < 4 points is projected in its own NP-point basis and mapped exactly:
-// with T[k][m] = sum_{x<NP} q4(x,k) qNP(x,m), the 4-point matrix
-// T B T^T expands to the same point blocks (Q4 Q4^T = I - 11^T/4 and the
-// columns of Q_NP sum to zero) and to zero blocks for the unused points.
-constexpr int REC_LEN = 45;
+// A record is the FRAME_LEN values of frame_hessian and a last value 0.  A
+// mollified edge-edge collision has a full packed 9 x 9 matrix: its first
+// FRAME_LEN entries in the record, the last value 1, and the other REC_EXT
+// entries in a second array indexed by the edge-edge collision.  224 bytes
+// instead of 360 for the full matrix: the row kernel is bound by the lines
+// that its gathers touch.
+constexpr int REC_LEN = FRAME_LEN + 1;
+constexpr int REC_EXT = 45 - FRAME_LEN;
 
-// PATH (4-point stencils): REC_ALL projects every collision with the 9 x 9
-// Jacobi; REC_LOW projects by the rank-5 Krylov path (falling back to the
-// Jacobi for a matrix it does not capture) and, for edge-edge, takes only
-// the interior (EA_EB) type, whose Hessians have rank 5; REC_LIST takes the
-// collisions listed in `only` (the other edge-edge types) with the Jacobi.
-enum { REC_ALL = 0, REC_LOW = 1, REC_LIST = 2 };
-
-template <int KIND, int PATH = REC_ALL>
-__global__ __launch_bounds__(64) void k_hessian_records(CollView C, const double* X, int nV,
-                                                        BarrierParams bp, double* rec,
-                                                        const uint32_t* only = nullptr,
-                                                        int64_t n_only = 0)
+template <int KIND>
+__device__ __forceinline__ void record_inputs(const CollView& C, int64_t i, const double* X, int nV,
+                                              d3* P)
 {
-    constexpr int NP = StencilTraits<KIND>::NP;
-    constexpr int K = NP - 1;
-    constexpr int LEN = HqTraits<KIND>::LEN;
-    const int64_t t = (int64_t)xcd_block() * 64 + threadIdx.x;
-    int64_t i = t;
-    if constexpr (PATH == REC_LIST) {
-        if (t >= n_only) return;
-        i = only[t];
-    } else {
-        if (i >= C.n[KIND]) return;
-    }
-    if constexpr (PATH == REC_LOW && KIND == K_EE)
-        if (C.dtype[i] != EE_EA_EB) return;
     int v[4];
     stencil_ids<KIND>(C, i, v);
-    d3 P[4];
 #pragma unroll
-    for (int j = 0; j < NP; j++) P[j] = ldx(X, nV, v[j]);
-    double H[LEN];
-    if constexpr (PATH == REC_LOW && NP == 4) {
-        const bool psd = stencil_hessian_q<KIND>(KIND == K_EE ? C.dtype[i] : 0, P, C.w[KIND][i],
-                                                 KIND == K_EE ? C.eps[i] : 0.0, bp, H, true);
-        if (psd && !project_psd_krylov9<6>(H, bp.psd)) project_psd<9>(H, bp.psd);
-    } else {
-        stencil_hessian_q<KIND>(KIND == K_EE ? C.dtype[i] : 0, P, C.w[KIND][i],
-                                KIND == K_EE ? C.eps[i] : 0.0, bp, H);
+    for (int j = 0; j < StencilTraits<KIND>::NP; j++) P[j] = ldx(X, nV, v[j]);
+}
+
+// A lane per collision of any kind: the kinds differ in the frame only, the
+// 5 x 5 projection and the expansion are one code.  Mollified edge-edge
+// collisions (rank up to 9) go to `list` for k_hessian_mollified.  Bound by
+// the FP64 rotations of the projection (registers: three waves a SIMD) and by
+// the 224 bytes written per collision.
+__global__ __launch_bounds__(256, 2) void k_hessian_records(CollView C, CollRanges G, const double* X,
+                                                         int nV, BarrierParams bp, double* rec,
+                                                         uint32_t* list, unsigned long long* n_list)
+{
+    const int64_t g = (int64_t)xcd_block() * 256 + threadIdx.x;
+    bool mollified = false;
+    uint32_t ee = 0;
+    if (g < G.goff[4]) {
+        d3 P[4];
+        ContactFrame f;
+        double d2, w;
+        if (g < G.goff[1]) {
+            record_inputs<K_VV>(C, g, X, nV, P);
+            w = C.w[K_VV][g];
+            d2 = stencil_dist2(K_VV, 0, P);
+            stencil_frame<K_VV>(0, P, f);
+        } else if (g < G.goff[2]) {
+            const int64_t i = g - G.goff[1];
+            record_inputs<K_EV>(C, i, X, nV, P);
+            w = C.w[K_EV][i];
+            d2 = stencil_dist2(K_EV, 0, P);
+            stencil_frame<K_EV>(0, P, f);
+        } else if (g < G.goff[3]) {
+            const int64_t i = g - G.goff[2];
+            ee = (uint32_t)i;
+            record_inputs<K_EE>(C, i, X, nV, P);
+            w = C.w[K_EE][i];
+            const int t = C.dtype[i];
+            mollified = mollifier(P, C.eps[i]).active;
+            d2 = stencil_dist2(K_EE, t, P);
+            stencil_frame<K_EE>(t, P, f);
+        } else {
+            const int64_t i = g - G.goff[3];
+            record_inputs<K_FV>(C, i, X, nV, P);
+            w = C.w[K_FV][i];
+            d2 = stencil_dist2(K_FV, 0, P);
+            stencil_frame<K_FV>(0, P, f);
+        }
+        if (!mollified) {
+            double H[REC_LEN];
+            frame_hessian(f, d2, w * bar_f1(d2, bp), w * bar_f2(d2, bp), bp.psd, H);
+            H[FRAME_LEN] = 0;
+            double2* o = reinterpret_cast<double2*>(rec + (int64_t)REC_LEN * g);
+#pragma unroll
+            for (int e = 0; e < REC_LEN / 2; e++) o[e] = make_double2(H[2 * e], H[2 * e + 1]);
+        }
     }
-    double* o = rec + (int64_t)REC_LEN * i;
-    if constexpr (NP == 4) {
+    unsigned pre;
+    const unsigned long long at = wave_append_bits(n_list, mollified, false, pre);
+    if (mollified) list[at + pre] = ee;
+}
+
+// The mollified edge-edge collisions listed by k_hessian_records, with the
+// 9 x 9 Jacobi (a wave a SIMD: matrix and eigenvectors fill the registers).
+// rec, ext: the edge-edge records.
+__global__ __launch_bounds__(64) void k_hessian_mollified(CollView C, const double* X, int nV,
+                                                          BarrierParams bp, double* rec,
+                                                          double* ext, const uint32_t* list,
+                                                          const unsigned long long* n_list)
+{
+    const int64_t n = (int64_t)*n_list;
+    for (int64_t t = (int64_t)blockIdx.x * 64 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 64) {
+        const int64_t i = list[t];
+        d3 P[4];
+        record_inputs<K_EE>(C, i, X, nV, P);
+        double H[45];
+        stencil_hessian_mollified(C.dtype[i], P, C.w[K_EE][i], C.eps[i], bp, H);
+        double* o = rec + (int64_t)REC_LEN * i;
 #pragma unroll
-        for (int e = 0; e < LEN; e++) o[e] = H[e];
-    } else {
-        double T[3][K];
+        for (int e = 0; e < FRAME_LEN; e++) o[e] = H[e];
+        o[FRAME_LEN] = 1;
+        double* x = ext + (int64_t)REC_EXT * i;
 #pragma unroll
-        for (int k = 0; k < 3; k++)
-#pragma unroll
-            for (int m = 0; m < K; m++) {
-                double t = 0;
-#pragma unroll
-                for (int x = 0; x < NP; x++) t += QBasis<4>::q(x, k) * QBasis<NP>::q(x, m);
-                T[k][m] = t;
-            }
-#pragma unroll
-        for (int p = 0; p < 9; p++)
-#pragma unroll
-            for (int q = 0; q <= p; q++) {
-                const int k = p / 3, r = p % 3, l = q / 3, t = q % 3;
-                double acc = 0;
-#pragma unroll
-                for (int m = 0; m < K; m++)
-#pragma unroll
-                    for (int n = 0; n < K; n++)
-                        acc += T[k][m] * T[l][n] * H[sp(3 * m + r, 3 * n + t)];
-                o[sp(p, q)] = acc;
-            }
+        for (int e = 0; e < REC_EXT; e++) x[e] = H[FRAME_LEN + e];
     }
 }
 
@@ -728,22 +745,6 @@ __global__ __launch_bounds__(256) void k_gap_ptr(const uint32_t* keys, int64_t M
     vptr[v] = (uint32_t)lo;
 }
 
-// edge-edge collisions of the other (non-interior) types, whose Hessians
-// have higher rank: flags, then the list at the scanned positions
-__global__ __launch_bounds__(256) void k_ee_other_flags(const int32_t* dtype, int64_t n,
-                                                        uint32_t* flag)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) flag[i] = dtype[i] != EE_EA_EB ? 1u : 0u;
-}
-
-__global__ __launch_bounds__(256) void k_ee_other_list(const uint32_t* flag, const uint32_t* pos,
-                                                       int64_t n, uint32_t* list)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n && flag[i]) list[pos[i]] = (uint32_t)i;
-}
-
 // stencil vertices of every sorted incidence (-1 for unused points)
 __global__ __launch_bounds__(256) void k_inc_vertices(CollView C, CollRanges G,
                                                       const uint32_t* inc, int64_t M, int4* out)
@@ -761,75 +762,52 @@ __global__ __launch_bounds__(256) void k_inc_vertices(CollView C, CollRanges G,
 
 constexpr int RW = 64; // block columns per accumulation window (one per lane)
 
-// Adds the contributions of one collision (record h in the 4-point basis,
-// stencil vertices vs, the row vertex is point a) to the window of the row's
-// blocks whose columns are cols[0, RW) (sorted, padded with INT32_MAX).  The
-// record stays in memory (read through the cache) and is expanded one block
-// row r at a time, so few values are live at once.
-__device__ __forceinline__ void row_accumulate(const double* h, int a, int4 vs,
-                                               const int32_t* cols, double (*acc)[9],
-                                               uint32_t* msk)
+constexpr int RD = 8; // copies of the diagonal block's accumulator
+
+// Window slot of a column (-1: none or outside this window)
+__device__ __forceinline__ int row_slot(const int32_t* cols, int col)
 {
-    constexpr int K = 3;
-    // window slot of each stencil point's column (-1: unused point or outside
-    // this window)
-    int slot[4];
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const int col = b == 0 ? vs.x : b == 1 ? vs.y : b == 2 ? vs.z : vs.w;
-        slot[b] = -1;
-        if (col < 0 || col < cols[0] || col > cols[RW - 1]) continue;
-        int lo = 0, hi = RW;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (cols[mid] < col) lo = mid + 1;
-            else hi = mid;
-        }
-        if (lo < RW && cols[lo] == col) slot[b] = lo;
+    if (col < 0 || col < cols[0] || col > cols[RW - 1]) return -1;
+    int lo = 0, hi = RW;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (cols[mid] < col) lo = mid + 1;
+        else hi = mid;
     }
-    uint32_t mask[4] = { 0, 0, 0, 0 };
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        // G[l][t] = sum_k q(a,k) H[3k+r][3l+t]
-        double G[K][3];
-#pragma unroll
-        for (int l = 0; l < K; l++)
-#pragma unroll
-            for (int t = 0; t < 3; t++) {
-                double x = 0;
-#pragma unroll
-                for (int k = 0; k < K; k++) x += QBasis<4>::q(a, k) * h[sp(3 * k + r, 3 * l + t)];
-                G[l][t] = x;
-            }
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            if (slot[b] < 0) continue;
-#pragma unroll
-            for (int t = 0; t < 3; t++) {
-                double x = 0;
-#pragma unroll
-                for (int l = 0; l < K; l++) x += QBasis<4>::q(b, l) * G[l][t];
-                if (x != 0) { // exact zeros are not triplets (local_to_global.hpp:291)
-                    atomicAdd(&acc[slot[b]][3 * r + t], x);
-                    mask[b] |= 1u << (3 * r + t);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-        if (mask[b]) atomicOr(&msk[slot[b]], mask[b]);
+    return lo < RW && cols[lo] == col ? lo : -1;
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_hessian_rows(const double* rec, const uint32_t* vptr,
-                                                      const uint32_t* inc, const int4* inc_vtx,
-                                                      const uint32_t* bptr,
-                                                      const int32_t* bcol, int nV, double* bval,
-                                                      uint32_t* bmask, const uint32_t* order)
+// Adds block row r.. of one point pair to its accumulator; exact zeros are
+// not triplets (local_to_global.hpp:291)
+__device__ __forceinline__ void row_add(double* acc, uint32_t* msk, const double* x)
+{
+    uint32_t mask = 0;
+#pragma unroll
+    for (int e = 0; e < 9; e++)
+        if (x[e] != 0) {
+            atomicAdd(&acc[e], x[e]);
+            mask |= 1u << e;
+        }
+    if (mask) atomicOr(msk, mask);
+}
+
+// A wave per vertex.  Every lane of a gather touches lines of its own, so a
+// load costs a cycle per lane whatever its width: records are read once, 16
+// bytes at a time (14 loads; the full matrix read by blocks took 81).  All
+// incidences of a row add to its diagonal block: RD copies of it keep the
+// LDS adds of a wave off one address.  The few full matrices are expanded by
+// the whole wave, a lane per entry of the four blocks: as a branch of each
+// lane they doubled the kernel's time (spills, and most waves hold one).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_hessian_rows(
+    const double* rec, const double* ext, int64_t ee0, const uint32_t* vptr, const uint32_t* inc,
+    const int4* inc_vtx, const uint32_t* bptr, const int32_t* bcol, int nV, double* bval,
+    uint32_t* bmask, const uint32_t* order)
 {
     __shared__ double acc[256 / WAVE][RW][9];
     __shared__ uint32_t msk[256 / WAVE][RW];
     __shared__ int32_t cols[256 / WAVE][RW];
+    __shared__ double dacc[256 / WAVE][RD][9];
+    __shared__ uint32_t dmsk[256 / WAVE][RD];
     const int wv = threadIdx.x / WAVE, l = lane_id();
     const int64_t w = ((int64_t)xcd_block() * 256 + threadIdx.x) / WAVE; // uniform per wave
     if (w >= nV) return;
@@ -841,26 +819,141 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         for (int e = 0; e < 9; e++) acc[wv][l][e] = 0;
         msk[wv][l] = 0;
         cols[wv][l] = w0 + l < m ? bcol[row_s + w0 + l] : INT32_MAX;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        (&dacc[wv][0][0])[l] = 0;
+        if (l < RD * 9 - WAVE) (&dacc[wv][0][0])[WAVE + l] = 0;
+        if (l < RD) dmsk[wv][l] = 0;
+        wave_sync();
+        const int self = row_slot(cols[wv], (int)v); // uniform
+        bool some_full = false;
         for (uint32_t j = i0 + l; j < i1; j += WAVE) {
-            const uint32_t x = inc[j];
-            row_accumulate(rec + (int64_t)REC_LEN * (x >> 2), (int)(x & 3u), inc_vtx[j], cols[wv],
-                           acc[wv], msk[wv]);
+            const uint32_t id = inc[j];
+            const int4 vs = inc_vtx[j];
+            double h[REC_LEN];
+            const double2* src = reinterpret_cast<const double2*>(rec + (int64_t)REC_LEN * (id >> 2));
+#pragma unroll
+            for (int e = 0; e < REC_LEN / 2; e++) {
+                const double2 t = src[e];
+                h[2 * e] = t.x;
+                h[2 * e + 1] = t.y;
+            }
+            if (h[FRAME_LEN] != 0) {
+                some_full = true;
+            } else {
+#pragma clang fp contract(fast)
+                const int a = (int)(id & 3u);
+                const double qa[3] = { QBasis<4>::q(a, 0), QBasis<4>::q(a, 1),
+                                       QBasis<4>::q(a, 2) };
+                const double* n = h;
+                const double* c = h + 3;
+                const double* M = h + 6;
+                const double* R = h + 12;
+                const double* T = h + 21;
+                const double ca = qa[0] * c[0] + qa[1] * c[1] + qa[2] * c[2];
+                double ma[3], Y[9];
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    ma[k] = qa[0] * M[sp(0, k)] + qa[1] * M[sp(1, k)] + qa[2] * M[sp(2, k)];
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    const double ra = qa[0] * R[t] + qa[1] * R[3 + t] + qa[2] * R[6 + t];
+#pragma unroll
+                    for (int r = 0; r < 3; r++) Y[3 * r + t] = n[r] * ra + ca * T[sp(r, t)];
+                }
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const int col = b == 0 ? vs.x : b == 1 ? vs.y : b == 2 ? vs.z : vs.w;
+                    const int slot = b == a ? self : row_slot(cols[wv], col);
+                    if (slot < 0) continue;
+                    double mb = 0, cb = 0, x[9];
+#pragma unroll
+                    for (int k = 0; k < 3; k++) {
+                        mb += QBasis<4>::q(b, k) * ma[k];
+                        cb += QBasis<4>::q(b, k) * c[k];
+                    }
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        double rb = 0;
+#pragma unroll
+                        for (int k = 0; k < 3; k++) rb += QBasis<4>::q(b, k) * R[3 * k + r];
+                        const double xr = mb * n[r] + ca * rb;
+#pragma unroll
+                        for (int t = 0; t < 3; t++) x[3 * r + t] = xr * n[t] + cb * Y[3 * r + t];
+                    }
+                    row_add(b == a ? dacc[wv][l % RD] : acc[wv][slot],
+                            b == a ? &dmsk[wv][l % RD] : &msk[wv][slot], x);
+                }
+            }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // (a loop of its own: inside the first one its address arithmetic
+        // stays live across the closed form, which then spills)
+        for (uint32_t j0 = __any(some_full) ? i0 : i1; j0 < i1; j0 += WAVE) {
+            const bool on = j0 + l < i1;
+            const uint32_t id = on ? inc[j0 + l] : 0u;
+            const int4 vs = on ? inc_vtx[j0 + l] : make_int4(-1, -1, -1, -1);
+            const bool is_full = on && rec[(int64_t)REC_LEN * (id >> 2) + FRAME_LEN] != 0;
+            unsigned long long full = __ballot(is_full);
+            uint32_t slots = 0; // of the four points, 255: none
+            if (is_full) {
+                slots = (uint32_t)(row_slot(cols[wv], vs.x) & 255)
+                    | (uint32_t)(row_slot(cols[wv], vs.y) & 255) << 8
+                    | (uint32_t)(row_slot(cols[wv], vs.z) & 255) << 16
+                    | (uint32_t)(row_slot(cols[wv], vs.w) & 255) << 24;
+            }
+            while (full) { // two at a time: both matrices' loads in flight
+                int e9 = l; // (opaque: not hoisted out of the loops, which would spill)
+                asm volatile("" : "+v"(e9));
+                const int b = e9 / 9, r = e9 % 9 / 3, t = e9 % 3;
+                const bool two = (full & (full - 1)) != 0;
+                const int s0 = __ffsll(full) - 1;
+                full &= full - 1;
+                const int s1 = two ? __ffsll(full) - 1 : s0;
+                full &= full - 1;
+                if (l >= 36) continue;
+                double x[2] = { 0, 0 };
+#pragma unroll
+                for (int y = 0; y < 2; y++) {
+#pragma clang fp contract(fast)
+                    const uint32_t fid = __builtin_amdgcn_readlane(id, y ? s1 : s0);
+                    const int64_t g = fid >> 2;
+                    const int a = (int)(fid & 3u);
+                    const double* hr = rec + (int64_t)REC_LEN * g;
+                    const double* he = ext + (int64_t)REC_EXT * (g - ee0) - FRAME_LEN;
+#pragma unroll
+                    for (int k = 0; k < 3; k++)
+#pragma unroll
+                        for (int i = 0; i < 3; i++) {
+                            const int e = sp(3 * k + r, 3 * i + t);
+                            x[y] += QBasis<4>::q(a, k) * QBasis<4>::q(b, i)
+                                * (e < FRAME_LEN ? hr : he)[e];
+                        }
+                }
+#pragma unroll
+                for (int y = 0; y < 2; y++) {
+                    const uint32_t sl = __builtin_amdgcn_readlane(slots, y ? s1 : s0);
+                    const uint32_t slot = (sl >> (8 * b)) & 255u;
+                    if (slot < (uint32_t)RW && x[y] != 0 && (y == 0 || two)) {
+                        atomicAdd(&acc[wv][slot][3 * r + t], x[y]);
+                        atomicOr(&msk[wv][slot], 1u << (3 * r + t));
+                    }
+                }
+            }
+        }
+        wave_sync();
+        if (self >= 0 && l < 9) { // (alone: no lane reads or adds here now)
+            double t = 0;
+#pragma unroll
+            for (int k = 0; k < RD; k++) t += dacc[wv][k][l];
+            acc[wv][self][l] += t;
+        }
+        if (self >= 0 && l < RD && dmsk[wv][l]) atomicOr(&msk[wv][self], dmsk[wv][l]);
+        wave_sync();
         if (w0 + l < m) {
             const int64_t u = (int64_t)row_s + w0 + l;
 #pragma unroll
             for (int e = 0; e < 9; e++) bval[9 * u + e] = acc[wv][l][e];
             bmask[u] = msk[wv][l];
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
     }
 }
 
@@ -1441,7 +1534,7 @@ static CollRanges hess_prepare(Ctx& c, const CollView& C)
     return G;
 }
 
-static void hess_assemble(Ctx& c);
+static void hess_assemble(Ctx& c, const double* ext, int64_t ee0);
 
 void pot_hessian(Ctx& c, double dhat, double kappa, int psd)
 {
@@ -1455,55 +1548,31 @@ void pot_hessian(Ctx& c, double dhat, double kappa, int psd)
     // projected Hessian records, REC_LEN values per collision in global
     // collision order
     double* rec = c.hrec.as<double>();
-    // one launch per stencil kind, each its own timed stage
-    if (C.n[0]) {
-        c.stage_begin("hessian_records.vv");
-        hipLaunchKernelGGL(k_hessian_records<K_VV>, dim3(grid_for(C.n[0], 64, INT32_MAX)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[0]);
+    if (G.goff[4] > 0) {
+        unsigned long long* n_list = c.counters.as<unsigned long long>() + 11;
+        c.ee_mollified.reserve(sizeof(uint32_t) * (size_t)std::max<int64_t>(C.n[2], 1));
+        uint32_t* list = c.ee_mollified.as<uint32_t>();
+        c.hrec_ext.reserve(sizeof(double) * REC_EXT * (size_t)std::max<int64_t>(C.n[2], 1));
+        double* ext = c.hrec_ext.as<double>();
+        c.stage_begin("hessian_records");
+        IPCG_HIP(hipMemsetAsync(n_list, 0, sizeof(*n_list), s));
+        hipLaunchKernelGGL(k_hessian_records, dim3(grid_for(G.goff[4], 256, INT32_MAX)), dim3(256), 0, s, C, G, X, c.nV, bp, rec, list, n_list);
         c.stage_end();
-    }
-    if (C.n[1]) {
-        c.stage_begin("hessian_records.ev");
-        hipLaunchKernelGGL(k_hessian_records<K_EV>, dim3(grid_for(C.n[1], 64, INT32_MAX)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[1]);
-        c.stage_end();
-    }
-    if (C.n[2]) {
-        // interior edge-edge Hessians by the rank-5 path, the other types
-        // (listed by a scan of their flags) by the 9 x 9 Jacobi
-        const int64_t ne = C.n[2];
-        c.ee_other.reserve(sizeof(uint32_t) * 3 * (size_t)ne);
-        uint32_t* flag = c.ee_other.as<uint32_t>();
-        uint32_t* pos = flag + ne;
-        uint32_t* list = pos + ne;
-        hipLaunchKernelGGL(k_ee_other_flags, dim3(grid_for(ne, 256, INT32_MAX)), dim3(256), 0, s, C.dtype, ne, flag);
-        uint32_t* n_other = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 11);
-        exclusive_scan_u32(c.sort_space, flag, pos, ne, n_other, s);
-        hipLaunchKernelGGL(k_ee_other_list, dim3(grid_for(ne, 256, INT32_MAX)), dim3(256), 0, s, flag, pos, ne, list);
-        IPCG_CHECK_LAUNCH();
-        uint32_t* h = static_cast<uint32_t*>(c.pinned);
-        IPCG_HIP(hipMemcpyAsync(h, n_other, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        IPCG_HIP(hipStreamSynchronize(s));
-        const int64_t no = h[0];
-        c.stat["hessian.ee_other"] = no;
-        c.stage_begin("hessian_records.ee");
-        hipLaunchKernelGGL((k_hessian_records<K_EE, REC_LOW>), dim3(grid_for(ne, 64, INT32_MAX)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[2], nullptr, (int64_t)0);
-        c.stage_end();
-        if (no > 0) {
-            c.stage_begin("hessian_records.ee_other");
-            hipLaunchKernelGGL((k_hessian_records<K_EE, REC_LIST>), dim3(grid_for(no, 64, INT32_MAX)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[2], list, no);
+        if (C.n[2]) {
+            c.stage_begin("hessian_records.mollified");
+            hipLaunchKernelGGL(k_hessian_mollified, dim3(grid_for(C.n[2], 64, 2048)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[2], ext, list, n_list);
             c.stage_end();
         }
-    }
-    if (C.n[3]) {
-        c.stage_begin("hessian_records.fv");
-        hipLaunchKernelGGL((k_hessian_records<K_FV, REC_LOW>), dim3(grid_for(C.n[3], 64, INT32_MAX)), dim3(64), 0, s, C, X, c.nV, bp, rec + REC_LEN * G.goff[3], nullptr, (int64_t)0);
-        c.stage_end();
+        IPCG_HIP(hipMemcpyAsync(static_cast<int64_t*>(c.pinned) + 1, n_list, sizeof(*n_list), hipMemcpyDeviceToHost, s));
     }
     IPCG_CHECK_LAUNCH();
-    hess_assemble(c);
+    hess_assemble(c, c.hrec_ext.as<double>(), G.goff[2]); // waits for the stream
+    c.stat["hessian.ee_other"] = G.goff[4] > 0 ? static_cast<int64_t*>(c.pinned)[1] : 0;
 }
 
-// block rows from the records in c.hrec, then the CSR
-static void hess_assemble(Ctx& c)
+// block rows from the records in c.hrec (ext: REC_EXT further values of the
+// full ones, by collision - ee0), then the CSR
+static void hess_assemble(Ctx& c, const double* ext, int64_t ee0)
 {
     hipStream_t s = c.stream;
     const double* rec = c.hrec.as<double>();
@@ -1516,7 +1585,7 @@ static void hess_assemble(Ctx& c)
     const int32_t* bcol = c.hp_bcol.as<int32_t>();
     c.stage_begin("hessian_rows");
     const unsigned gwr = grid_for((int64_t)c.nV * WAVE, 256, INT32_MAX); // a wave per vertex
-    hipLaunchKernelGGL(k_hessian_rows, dim3(gwr), dim3(256), 0, s, rec, c.inc_ptr.as<uint32_t>(),
+    hipLaunchKernelGGL(k_hessian_rows, dim3(gwr), dim3(256), 0, s, rec, ext, ee0, c.inc_ptr.as<uint32_t>(),
                        c.inc_vals.as<uint32_t>(), c.inc_vtx.as<int4>(), bptr, bcol, c.nV, bval,
                        bmask, row_order(c));
     IPCG_CHECK_LAUNCH();
@@ -2026,24 +2095,31 @@ __device__ void psd2(double& a, double& b, double& d, int method)
     d = m1 * y * y + m0 * x * x;
 }
 
-// Hessian records in the 4-point Q basis (REC_LEN packed values)
-template <int KIND>
-__global__ __launch_bounds__(PB) void k_fric_hessian_records(CollView C, const FricRec* R,
-                                                             const double* Vel, int nV,
-                                                             FricParams fp, double* rec)
+// Hessian records (the form of frame_hessian with only the c_k c_l T term:
+// c the friction weights, T the tangential matrix), a lane per collision of
+// any kind.
+__global__ __launch_bounds__(PB) void k_fric_hessian_records(CollView C, CollRanges G,
+                                                             const FricRec* R, const double* Vel,
+                                                             int nV, FricParams fp, double* rec)
 {
     const int64_t i = (int64_t)xcd_block() * PB + threadIdx.x;
-    if (i >= C.n[KIND]) return;
-    double* o = rec + (int64_t)REC_LEN * i;
+    if (i >= G.goff[4]) return;
     const FricRec r = R[i];
     double m00 = 0, m01 = 0, m11 = 0;
     double sq[3] = { 0, 0, 0 };
     if (r.keep != 0) {
-        int v[4];
-        stencil_ids<KIND>(C, i, v);
         double u[2], norm, g[4];
-        fric_local<KIND>(r, Vel, nV, v, fp.eps_v, r.ms_eff, r.mk_eff, u, norm);
-        fric_coef<KIND>(r.beta, g);
+        auto local = [&](auto kind, int64_t k) {
+            constexpr int KIND = decltype(kind)::value;
+            int v[4];
+            stencil_ids<KIND>(C, k, v);
+            fric_local<KIND>(r, Vel, nV, v, fp.eps_v, r.ms_eff, r.mk_eff, u, norm);
+            fric_coef<KIND>(r.beta, g);
+        };
+        if (i < G.goff[1]) local(std::integral_constant<int, K_VV>(), i);
+        else if (i < G.goff[2]) local(std::integral_constant<int, K_EV>(), i - G.goff[1]);
+        else if (i < G.goff[3]) local(std::integral_constant<int, K_EE>(), i - G.goff[2]);
+        else local(std::integral_constant<int, K_FV>(), i - G.goff[3]);
         const double f1x = smooth_mu_f1_over_x(norm, r.ms_eff, r.mk_eff, fp.eps_v);
         const double scale = r.s;
         if (norm > fp.eps_v) { // sliding: f2 = 0, rank one along u_perp
@@ -2080,10 +2156,18 @@ __global__ __launch_bounds__(PB) void k_fric_hessian_records(CollView C, const F
             const double pb0 = r.P[b] * r.an[0], pb1 = r.P[3 + b] * r.an[1];
             A[a][b] = pa0 * (m00 * pb0 + m01 * pb1) + pa1 * (m01 * pb0 + m11 * pb1);
         }
+    double o[REC_LEN];
 #pragma unroll
-    for (int I = 0; I < 9; I++)
+    for (int e = 0; e < REC_LEN; e++) o[e] = 0;
 #pragma unroll
-        for (int J = 0; J <= I; J++) o[sp(I, J)] = sq[I / 3] * sq[J / 3] * A[I % 3][J % 3];
+    for (int a = 0; a < 3; a++) {
+        o[3 + a] = sq[a];
+#pragma unroll
+        for (int b = 0; b <= a; b++) o[21 + sp(a, b)] = A[a][b];
+    }
+    double2* out = reinterpret_cast<double2*>(rec + (int64_t)REC_LEN * i);
+#pragma unroll
+    for (int e = 0; e < REC_LEN / 2; e++) out[e] = make_double2(o[2 * e], o[2 * e + 1]);
 }
 
 } // namespace
@@ -2245,13 +2329,10 @@ void fric_hessian(Ctx& c, double eps_v, int psd)
     double* rec = c.hrec.as<double>();
     const double* Vel = c.vel.as<double>();
     c.stage_begin("friction_hessian_records");
-    if (C.n[0]) hipLaunchKernelGGL(k_fric_hessian_records<K_VV>, dim3(grid_for(C.n[0], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[0], Vel, c.nV, fp, rec + REC_LEN * G.goff[0]);
-    if (C.n[1]) hipLaunchKernelGGL(k_fric_hessian_records<K_EV>, dim3(grid_for(C.n[1], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[1], Vel, c.nV, fp, rec + REC_LEN * G.goff[1]);
-    if (C.n[2]) hipLaunchKernelGGL(k_fric_hessian_records<K_EE>, dim3(grid_for(C.n[2], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[2], Vel, c.nV, fp, rec + REC_LEN * G.goff[2]);
-    if (C.n[3]) hipLaunchKernelGGL(k_fric_hessian_records<K_FV>, dim3(grid_for(C.n[3], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[3], Vel, c.nV, fp, rec + REC_LEN * G.goff[3]);
+    if (G.goff[4] > 0) hipLaunchKernelGGL(k_fric_hessian_records, dim3(grid_for(G.goff[4], PB, INT32_MAX)), dim3(PB), 0, s, C, G, R, Vel, c.nV, fp, rec);
     IPCG_CHECK_LAUNCH();
     c.stage_end();
-    hess_assemble(c);
+    hess_assemble(c, nullptr, 0); // no full records
 }
 
 

@@ -175,50 +175,72 @@ IPCG_HD void stencil_gradient(int dtype, const d3* P, double w, double eps_x,
     }
 }
 
-// PSD-projected energy Hessian in the Q basis (packed 3(NP-1) square).
-// defer_psd: leave the projection to the caller; the return value says
-// whether the reference projects this stencil's Hessian at all.
-template <int KIND, int NP = StencilTraits<KIND>::NP>
-IPCG_HD bool stencil_hessian_q(int dtype, const d3* P, double w, double eps_x,
-                               const BarrierParams& bp, double* Hq, bool defer_psd = false)
+// (a select of the values: one of the addresses would put P into scratch)
+IPCG_HD d3 pick(bool c, const d3& a, const d3& b)
 {
-    constexpr int kind = KIND;
-    constexpr int K = NP - 1, N = 3 * K;
+    return { c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z };
+}
+
+// Frame of an unmollified stencil's distance.
+template <int KIND> IPCG_HD void stencil_frame(int dtype, const d3* P, ContactFrame& f)
+{
+    if constexpr (KIND == K_VV) {
+        const double W[4] = { 1, -1, 0, 0 };
+        frame_point(sub(P[0], P[1]), W, f);
+    } else if constexpr (KIND == K_EV) {
+        const double W[4] = { 1, -1, 0, 0 }, L[4] = { 0, -1, 1, 0 };
+        frame_line(sub(P[0], P[1]), sub(P[0], P[2]), sub(P[2], P[1]), W, L, f);
+    } else if constexpr (KIND == K_FV) {
+        const double W[4] = { 1, -1, 0, 0 }, U[4] = { 0, -1, 1, 0 }, V[4] = { 0, -1, 0, 1 };
+        frame_plane(sub(P[0], P[1]), sub(P[2], P[1]), sub(P[3], P[1]), W, U, V, f);
+    } else if (dtype < EE_EA_EB0) { // corner against corner
+        const int a = (dtype >> 1) & 1, b = dtype & 1;
+        const double W[4] = { a ? 0. : 1., a ? 1. : 0., b ? 0. : -1., b ? -1. : 0. };
+        frame_point(sub(pick(a, P[1], P[0]), pick(b, P[3], P[2])), W, f);
+    } else if (dtype < EE_EA_EB) { // corner p against the other edge's line
+        const bool ea = dtype == EE_EA_EB0 || dtype == EE_EA_EB1; // the line is ea
+        const bool second = dtype == EE_EA_EB1 || dtype == EE_EA1_EB;
+        const d3 l0 = pick(ea, P[0], P[2]), l1 = pick(ea, P[1], P[3]);
+        const d3 p = pick(ea, pick(second, P[3], P[2]), pick(second, P[1], P[0]));
+        const double p0 = second ? 0. : 1., p1 = second ? 1. : 0.;
+        const double W[4] = { ea ? -1. : p0, ea ? 0. : p1, ea ? p0 : -1., ea ? p1 : 0. };
+        const double L[4] = { ea ? -1. : 0., ea ? 1. : 0., ea ? 0. : -1., ea ? 0. : 1. };
+        frame_line(sub(p, l0), sub(p, l1), sub(l1, l0), W, L, f);
+    } else {
+        const double W[4] = { -1, 0, 1, 0 }, U[4] = { -1, 1, 0, 0 }, V[4] = { 0, 0, -1, 1 };
+        frame_plane(sub(P[2], P[0]), sub(P[1], P[0]), sub(P[3], P[2]), W, U, V, f);
+    }
+}
+
+// Projected Hessian (packed 9 x 9, Q basis) of w m f(d) for an edge-edge
+// stencil under its mollifier.
+IPCG_HD void stencil_hessian_mollified(int dtype, const d3* P, double w, double eps_x,
+                                       const BarrierParams& bp, double* Hq)
+{
 #pragma unroll
-    for (int i = 0; i < N * (N + 1) / 2; i++) Hq[i] = 0;
-    const double d2 = stencil_dist2(kind, dtype, P);
-    const Moll M = kind == K_EE ? mollifier(P, eps_x) : Moll { 1.0, 0.0, 0.0, false };
+    for (int i = 0; i < 45; i++) Hq[i] = 0;
+    const double d2 = stencil_dist2(K_EE, dtype, P);
+    const Moll M = mollifier(P, eps_x);
     const int mpl[2] = { 1, 3 }, mmi[2] = { 0, 2 };
-    if (kind == K_EE && M.m <= 0) { // normal_potential.cpp:188-192: no projection
-        if constexpr (KIND == K_EE) {
-            const double f = bar_f(d2, bp);
-            Red<2> X;
-            cross2_derivs(sub(P[1], P[0]), sub(P[3], P[2]), X);
-            d3 gx[K];
-            to_qspace<NP>(X, mpl, mmi, w * f * M.m1, gx, Hq);
-            add_sym_outer<K>(Hq, 0.5 * w * f * M.m2, gx, gx);
-        }
-        return false;
+    const double f = bar_f(d2, bp);
+    Red<2> X;
+    cross2_derivs(sub(P[1], P[0]), sub(P[3], P[2]), X);
+    d3 gx[3];
+    if (M.m <= 0) { // normal_potential.cpp:188-192: no projection
+        to_qspace<4>(X, mpl, mmi, w * f * M.m1, gx, Hq);
+        add_sym_outer<3>(Hq, 0.5 * w * f * M.m2, gx, gx);
+        return;
     }
     const double f1 = bar_f1(d2, bp), f2 = bar_f2(d2, bp);
-    d3 gq[K];
-    with_distance_derivs<KIND>(dtype, P, [&](auto& red, const int* pl, const int* mi) {
-        to_qspace<NP>(red, pl, mi, w * M.m * f1, gq, Hq);
+    d3 gq[3];
+    with_distance_derivs<K_EE>(dtype, P, [&](auto& red, const int* pl, const int* mi) {
+        to_qspace<4>(red, pl, mi, w * M.m * f1, gq, Hq);
     });
-    add_sym_outer<K>(Hq, 0.5 * w * M.m * f2, gq, gq);
-    if constexpr (KIND == K_EE) {
-        if (M.active) {
-            const double f = bar_f(d2, bp);
-            Red<2> X;
-            cross2_derivs(sub(P[1], P[0]), sub(P[3], P[2]), X);
-            d3 gx[K];
-            to_qspace<NP>(X, mpl, mmi, w * f * M.m1, gx, Hq);
-            add_sym_outer<K>(Hq, 0.5 * w * f * M.m2, gx, gx);
-            add_sym_outer<K>(Hq, w * f1 * M.m1, gq, gx);
-        }
-    }
-    if (!defer_psd) project_psd<N>(Hq, bp.psd);
-    return true;
+    add_sym_outer<3>(Hq, 0.5 * w * M.m * f2, gq, gq);
+    to_qspace<4>(X, mpl, mmi, w * f * M.m1, gx, Hq);
+    add_sym_outer<3>(Hq, 0.5 * w * f * M.m2, gx, gx);
+    add_sym_outer<3>(Hq, w * f1 * M.m1, gq, gx);
+    project_psd<9>(Hq, bp.psd);
 }
 
 } // namespace ipcg
