@@ -477,10 +477,8 @@ def main():
     n_vv, n_ev, n_ee, n_fv = [int(x) for x in counts]
     searched = int(ccd_work["ccd.searched"])
     model = {  # stage: (bytes, flops) per launch
-        "bp_traverse_ee.static": (24 * nE + 8 * ne_s, 0),
-        "bp_traverse_fv.static": (24 * nV + 8 * nf_s, 0),
-        "bp_traverse_ee.swept": (24 * nE + 8 * ne_d, 0),
-        "bp_traverse_fv.swept": (24 * nV + 8 * nf_d, 0),
+        "bp_traverse_both.static": (24 * (nE + nV) + 8 * (ne_s + nf_s), 0),
+        "bp_traverse_both.swept": (24 * (nE + nV) + 8 * (ne_d + nf_d), 0),
         "np_classify": (8 * (ne_s + nf_s) + 16 * pairs, 0),
         "energy": (16 * pairs + 8, 0),
         "hessian_records": (REC_BYTES["ee"] * (n_ee - ee_moll) + REC_BYTES["fv"] * n_fv

@@ -28,7 +28,10 @@ constexpr int BP_BLOCK = 256;
 constexpr int TR_BLOCK = 128;
 constexpr int TR_STACK = 64;  // lbvh.cpp:378 MAX_STACK_SIZE
 constexpr int TR_LSTACK = 16; // entries per lane kept in LDS; the rest in HBM
-constexpr int TR_BUF = 4;     // overlapping leaves a lane holds before the wave settles them
+constexpr int64_t TR_FEW = 1 << 18, TR_FEWER = 1 << 16; // queries: see wave_queries
+constexpr int TR_SHARE = 2;   // steps between two chances of idle lanes to take over subtrees
+constexpr int TR_IDLE = 4;    // idle lanes that make it worth the exchange
+constexpr int TR_QUEUE = 256; // overlapping leaves that a wave holds before it settles them
 
 // AABB::from_point (+ swept union), aabb.cpp:21-55
 __device__ __forceinline__ void vbox(const double* X0, const double* X1, int nV, int i, double r,
@@ -657,22 +660,69 @@ struct ForestArgs {
     const uint32_t* tids;    // target tree: primitive per sorted leaf
 };
 
-// BLOCK: workgroup size (64, 128 or 256), chosen per launch by the
-// context's autotuner or TR_BLOCK.
-template <int MODE, int SWEPT, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_traverse(
-    const float* qbox, const uint32_t* qids, int nq, const Node* nodes, const int32_t* root_p,
-    const int4* leaf, const float* tbox, int nleaves, Filter flt, const int32_t* qmap, int2* out,
-    Shards S, int* deep, int* status, ForestArgs fa)
+struct TraverseArgs {
+    const float* qbox;
+    const uint32_t* qids;
+    int nq;
+    const Node* nodes;
+    const int32_t* root;
+    const int4* leaf;
+    const float* tbox;
+    int nleaves;
+    Filter flt;
+    const int32_t* qmap;
+    int2* out;
+    Shards S;
+    int* deep; // TR_STACK - TR_LSTACK ints per lane of the launch
+    int* status;
+    ForestArgs fa;
+    int qw; // queries a wave starts with (its first lanes; the others share)
+};
+
+template <int BLOCK> struct TrShared {
+    int stack[TR_LSTACK][BLOCK];
+    int leaf[BLOCK / WAVE][TR_QUEUE];
+    unsigned char lane[BLOCK / WAVE][TR_QUEUE];
+    unsigned char donor[BLOCK / WAVE][WAVE];
+};
+
+// LDS written by some lanes of the wave is read by others
+__device__ __forceinline__ void wave_fence()
 {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The walk of one workgroup's queries (block: its index in the query set's
+// launch range).  stack: postponed right children, the first TR_LSTACK
+// entries of each lane in LDS (small enough for full occupancy), deeper ones
+// in the lane's own HBM slots.
+template <int MODE, int BLOCK>
+__device__ __forceinline__ void traverse(const TraverseArgs& A, unsigned block,
+                                         TrShared<BLOCK>& sh_mem)
+{
+    const float* const qbox = A.qbox;
+    const uint32_t* const qids = A.qids;
+    const int nq = A.nq, nleaves = A.nleaves;
+    const Node* const nodes = A.nodes;
+    const int32_t* const root_p = A.root;
+    const int4* const leaf = A.leaf;
+    const float* const tbox = A.tbox;
+    const Filter& flt = A.flt;
+    const int32_t* const qmap = A.qmap;
+    int2* const out = A.out;
+    const Shards& S = A.S;
+    int* const status = A.status;
+    const ForestArgs& fa = A.fa;
+    int(*const stack)[BLOCK] = sh_mem.stack;
     constexpr bool TRI = MODE == TR_EE || MODE == TR_VV;
-    // The traversal stack of postponed right children: the first TR_LSTACK
-    // entries in LDS (small enough for full occupancy), deeper ones in the
-    // query's own HBM slots (deep: TR_STACK - TR_LSTACK ints per query).
-    __shared__ int stack[TR_LSTACK][BLOCK];
     const int t = threadIdx.x;
-    const int qpos = (int)xcd_block() * BLOCK + t;
-    bool active = qpos < nq;
+    const int64_t q0 = ((int64_t)block * (BLOCK / WAVE) + t / WAVE) * A.qw + t % WAVE;
+    const bool has_query = t % WAVE < A.qw && q0 < nq;
+    const int qpos = has_query ? (int)q0 : 0;
+    bool active = has_query;
+    int* const deep = A.deep + ((int64_t)block * BLOCK + t) * (TR_STACK - TR_LSTACK) - TR_LSTACK;
     float q[6] = { 0, 0, 0, 0, 0, 0 };
     Query qr { 0, { -1, -1, -1 } };
     if (active) {
@@ -690,41 +740,73 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
     }
     const int nin = nleaves - 1; // internal nodes
     const int sh = wave_shard();
-    // Overlapping leaves wait in registers (their positions, up to TR_BUF
-    // per lane) and the wave settles them together when a lane could
-    // overflow or the walks end: the leaf records are loaded for all of them
-    // at once (one memory round trip per flush instead of one per iteration
-    // with a hit), the filters drop pairs, and one append per wave writes
-    // the rest.
-    int buf[TR_BUF];
-#pragma unroll
-    for (int k = 0; k < TR_BUF; k++) buf[k] = -1;
-    unsigned nb = 0;
+    // Overlapping leaves (position and lane) wait in the wave's queue in LDS.
+    // Past half of it, or when the walks end, a lane takes every 64th entry:
+    // the leaf records of all of them are loaded at once, the filters drop
+    // pairs, and one append writes the rest.  (The append's round trip is the
+    // dear part: with four entries held per lane the busiest lane forced one
+    // every few steps, for a handful of pairs each; 11.4 against 9.4 ms for
+    // the static walks of 8 sheets of 512^2.)
+    int* const qleaf = sh_mem.leaf[t / WAVE];
+    unsigned char* const qlane = sh_mem.lane[t / WAVE];
+    unsigned nb = 0; // uniform
+    int owner = t % WAVE; // lane whose query this lane walks
+    auto push = [&](int h) {
+        const unsigned long long m = __ballot(h >= 0);
+        if (h >= 0) {
+            const unsigned at = nb + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            qleaf[at] = h;
+            qlane[at] = (unsigned char)owner;
+        }
+        nb += (unsigned)__popcll(m);
+    };
     int2* const reg = out + sh * S.scap;
     auto flush = [&]() {
-        int4 rec[TR_BUF]; // every load first, then the filters
+        constexpr int R = TR_QUEUE / WAVE;
+        wave_fence();
+        int lp[R], ln[R];
 #pragma unroll
-        for (int k = 0; k < TR_BUF; k++) {
-            rec[k] = make_int4(-1, -1, -1, -1);
-            if (nb > (unsigned)k) rec[k] = leaf[buf[k]];
+        for (int k = 0; k < R; k++) {
+            const unsigned i = k * WAVE + t % WAVE;
+            lp[k] = i < nb ? qleaf[i] : -1;
+            ln[k] = i < nb ? qlane[i] : 0;
         }
-        int2 hit[TR_BUF];
+        int4 rec[R]; // every load first, then the filters
 #pragma unroll
-        for (int k = 0; k < TR_BUF; k++)
-            hit[k] = nb > (unsigned)k ? leaf_pair<MODE>(flt, qr, rec[k]) : make_int2(-1, -1);
-        unsigned nv = 0;
+        for (int k = 0; k < R; k++) {
+            rec[k] = make_int4(-1, -1, -1, -1);
+            if (lp[k] >= 0) rec[k] = leaf[lp[k]];
+        }
+        int2 hit[R];
+        unsigned before[R], total = 0;
 #pragma unroll
-        for (int k = 0; k < TR_BUF; k++) nv += hit[k].x >= 0 ? 1u : 0u;
-        const int64_t first = (int64_t)shard_append(S, sh, nv);
-        int64_t at = first;
+        for (int k = 0; k < R; k++) {
+            Query q2;
+            q2.id = __shfl(qr.id, ln[k], WAVE);
 #pragma unroll
-        for (int k = 0; k < TR_BUF; k++)
-            if (hit[k].x >= 0) {
-                if (at < S.scap) reg[at] = hit[k];
-                at++;
-            }
+            for (int v = 0; v < 3; v++) q2.v[v] = __shfl(qr.v[v], ln[k], WAVE);
+            hit[k] = lp[k] >= 0 ? leaf_pair<MODE>(flt, q2, rec[k]) : make_int2(-1, -1);
+            const unsigned long long m = __ballot(hit[k].x >= 0);
+            before[k] = total + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            total += (unsigned)__popcll(m);
+        }
+        if (total) {
+            unsigned long long base = 0;
+            if (t % WAVE == 0)
+                base = atomicAdd(S.cnt + (int64_t)sh * SHARD_PAD, (unsigned long long)total);
+            const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)base);
+            const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(base >> 32));
+            const int64_t first = (int64_t)(((unsigned long long)hi << 32) | lo);
+#pragma unroll
+            for (int k = 0; k < R; k++)
+                if (hit[k].x >= 0 && first + before[k] < S.scap) reg[first + before[k]] = hit[k];
+        }
         nb = 0;
+        wave_fence();
     };
+    int single = -1; // the only leaf of a one-leaf tree
     int node = 0;
     if (active) {
         int root = root_p[0];
@@ -742,19 +824,56 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
             if (!TRI) {
                 const int lp = ~root;
                 const float* b = tbox + (int64_t)6 * (fa.tids ? fa.tids[lp] : 0);
-                if (overlap(q, b, b + 3)) {
-                    buf[0] = lp;
-                    nb = 1;
-                }
+                if (overlap(q, b, b + 3)) single = lp;
             }
             active = false;
         } else {
             node = root;
         }
     }
-    int sp = 0, steps = 0;
+    push(single);
+    // Postponed children of the lane: entries [sb, sp) (those below sb were
+    // given away).  Lanes of a wave finish at different times; every
+    // TR_SHARE steps the idle ones take the oldest postponed child, the
+    // largest subtree left, of a busy lane each and walk it with that lane's
+    // query (9.4 to 8.4 ms there, 0.29 to 0.21 ms on 4 sheets of 97^2).
+    int sb = 0, sp = 0, steps = 0, round = 0;
+    int pos = qpos; // of the query walked
+    unsigned char* const donor = sh_mem.donor[t / WAVE];
     const int max_steps = 2 * nleaves + 64; // each node is visited at most once per query
     while (__any(active)) {
+        if (++round % TR_SHARE == 0) {
+            const bool gives = active && sp > sb && sb < TR_LSTACK;
+            const bool takes = !active;
+            const unsigned long long mg = __ballot(gives), mt = __ballot(takes);
+            const unsigned ng = (unsigned)__popcll(mg), nt = (unsigned)__popcll(mt);
+            if (ng > 0 && nt >= TR_IDLE) {
+                const unsigned long long mine = gives ? mg : mt;
+                const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mine >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0u));
+                if (gives) donor[rank] = (unsigned char)(t % WAVE);
+                wave_fence();
+                const bool got = takes && rank < ng;
+                const int src = got ? donor[rank] : t % WAVE;
+#pragma unroll
+                for (int k = 0; k < 6; k++) {
+                    const float v = __shfl(q[k], src, WAVE);
+                    q[k] = got ? v : q[k];
+                }
+                const int pos2 = __shfl(pos, src, WAVE), own2 = __shfl(owner, src, WAVE),
+                          sb2 = __shfl(sb, src, WAVE);
+                if (got) {
+                    pos = pos2;
+                    owner = own2;
+                    node = stack[sb2][t - t % WAVE + src];
+                    sb = sp = steps = 0;
+                    active = true;
+                } else if (gives && rank < nt) {
+                    sb++;
+                }
+                wave_fence();
+            }
+        }
         int h0 = -1, h1 = -1;
         bool nd_ok = true;
         if (active) {
@@ -771,8 +890,8 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
             // branch-free tests (bitwise, no short-circuit)
             bool o0 = nd_ok & overlap(q, nd.lo0, nd.hi0), o1 = nd_ok & overlap(q, nd.lo1, nd.hi1);
             if (TRI) {
-                o0 = o0 & (nd.r0 > qpos);
-                o1 = o1 & (nd.r1 > qpos);
+                o0 = o0 & (nd.r0 > pos);
+                o1 = o1 & (nd.r1 > pos);
             }
             const bool l0 = nd.c0 < 0, l1 = nd.c1 < 0;
             h0 = (o0 & l0) ? ~nd.c0 : -1;
@@ -780,7 +899,7 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
             const bool t0 = o0 & !l0, t1 = o1 & !l1;
             if (!nd_ok) {
             } else if (!t0 && !t1) {
-                if (sp == 0) active = false;
+                if (sp == sb) active = false;
                 else {
                     --sp;
                     // the LDS entries by an LDS read; the deep ones through a
@@ -790,14 +909,14 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
                         node = stack[sp][t];
                     else
                         node = __builtin_nontemporal_load(
-                            &deep[(int64_t)qpos * (TR_STACK - TR_LSTACK) + sp - TR_LSTACK]);
+                            &deep[sp]);
                 }
             } else {
                 node = t0 ? nd.c0 : nd.c1;
                 if (t0 && t1) {
                     if (sp < TR_LSTACK) stack[sp++][t] = nd.c1;
                     else if (sp < TR_STACK) {
-                        deep[(int64_t)qpos * (TR_STACK - TR_LSTACK) + sp - TR_LSTACK] = nd.c1;
+                        deep[sp] = nd.c1;
                         sp++;
                     } else {
                         atomicOr(status, 1);
@@ -806,46 +925,62 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(
                 }
             }
         }
-        // (nb <= TR_BUF - 2 here) queue h0 then h1 without branches:
-        // constant indices keep the buffer in registers, a missing hit
-        // matches no slot
-        {
-            const unsigned s0 = h0 >= 0 ? nb : (unsigned)TR_BUF;
-            nb += h0 >= 0 ? 1u : 0u;
-            const unsigned s1 = h1 >= 0 ? nb : (unsigned)TR_BUF;
-            nb += h1 >= 0 ? 1u : 0u;
-#pragma unroll
-            for (int k = 0; k < TR_BUF; k++)
-                buf[k] = s0 == (unsigned)k ? h0 : (s1 == (unsigned)k ? h1 : buf[k]);
-        }
-        if (__any(nb > TR_BUF - 2)) flush(); // all lanes together
+        push(h0);
+        push(h1);
+        if (nb > TR_QUEUE - 2 * WAVE) flush(); // room for the next step's
     }
-    if (__any(nb > 0)) flush();
+    if (nb > 0) flush();
 }
-struct TraverseArgs {
-    const float* qbox;
-    const uint32_t* qids;
-    int nq;
-    const Node* nodes;
-    const int32_t* root;
-    const int4* leaf;
-    const float* tbox;
-    int nleaves;
-    Filter flt;
-    const int32_t* qmap;
-    int2* out;
-    Shards S;
-    int* deep;
-    int* status;
-    ForestArgs fa;
-};
+
+// BLOCK: workgroup size (64, 128 or 256), chosen per launch by the
+// context's autotuner or TR_BLOCK.
+template <int MODE, int SWEPT, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_traverse(TraverseArgs a)
+{
+    __shared__ TrShared<BLOCK> m;
+    traverse<MODE, BLOCK>(a, xcd_block(), m);
+}
+
+// Edge-edge and face-vertex walks side by side (workgroups [0, nb_ee) and
+// the rest).  Bound by the chain of dependent node loads of the longest walk
+// (small scenes: two launches in a row take two of them) and by node reads
+// from L2 (large ones).  With the wave's queue and the shared subtrees,
+// static walks of 4 sheets of 97^2 go from 0.395 + 0.292 to 0.138 ms, of
+// 8 sheets of 512^2 from 8.35 + 3.09 to 8.33 ms.
+template <int SWEPT>
+__global__ __launch_bounds__(TR_BLOCK) void k_traverse_both(TraverseArgs ee, TraverseArgs fv,
+                                                            unsigned nb_ee)
+{
+    __shared__ TrShared<TR_BLOCK> m;
+    if (blockIdx.x < nb_ee)
+        traverse<TR_EE, TR_BLOCK>(ee, xcd_block(blockIdx.x, nb_ee), m);
+    else
+        traverse<TR_FV, TR_BLOCK>(fv, xcd_block(blockIdx.x - nb_ee, gridDim.x - nb_ee), m);
+}
+
+unsigned traverse_blocks(int64_t nq, int qw, int block)
+{
+    return grid_for(nq, block / WAVE * qw);
+}
+
+// HBM stack ints of a walk of nq queries (its largest workgroup size)
+int64_t deep_ints(int64_t nq, int qw)
+{
+    return ((nq + qw - 1) / qw + 4) * WAVE * (TR_STACK - TR_LSTACK);
+}
+
+// A walk of few queries leaves most of the chip idle and takes the time of
+// its longest wave: its waves start with part of their lanes busy, and the
+// others take over subtrees.  Static walks with 64, 16, 8 queries a wave: 0.091,
+// 0.039, 0.033 ms for 33K queries (two 64^2 sheets), 0.207, 0.138, 0.141 ms for
+// 149K (4 sheets of 97^2), 0.086, 0.125 ms for the 450K short walks of 11 spheres.
+int wave_queries(int64_t nq) { return nq <= TR_FEWER ? 8 : nq <= TR_FEW ? 16 : WAVE; }
 
 template <int MODE, int SWEPT, int BLOCK>
 void launch_traverse_b(const TraverseArgs& a, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_traverse<MODE, SWEPT, BLOCK>), dim3(grid_for(a.nq, BLOCK)), dim3(BLOCK),
-                       0, s, a.qbox, a.qids, a.nq, a.nodes, a.root, a.leaf, a.tbox, a.nleaves,
-                       a.flt, a.qmap, a.out, a.S, a.deep, a.status, a.fa);
+    hipLaunchKernelGGL((k_traverse<MODE, SWEPT, BLOCK>), dim3(traverse_blocks(a.nq, a.qw, BLOCK)),
+                       dim3(BLOCK), 0, s, a);
 }
 
 template <int MODE, int SWEPT> void launch_traverse(int block, const TraverseArgs& a, hipStream_t s)
@@ -1319,8 +1454,8 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
     c.counters.reserve(sizeof(unsigned long long) * 4);
     Filter flt { c.E.as<int32_t>(), c.F.as<int32_t>(), c.has_patch ? c.patch.as<int32_t>() : nullptr,
                  c.n_dynamic, c.n_codim_filter };
-    int* status = reinterpret_cast<int*>(c.counters.as<unsigned long long>() + 2);
-    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES);
+    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(unsigned long long));
+    int* status = reinterpret_cast<int*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
     c.shard_off.reserve(sizeof(int64_t) * 4 * (SHARDS + 1));
     unsigned long long* cnt[4];
     for (int k = 0; k < 4; k++) cnt[k] = c.shard_cnt.as<unsigned long long>() + k * SHARDS * SHARD_PAD;
@@ -1330,9 +1465,13 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
     DevBuf* final_list[4] = { &c.cand_ee, &c.cand_fv, &c.cand_vv, &c.cand_ev };
     int64_t* final_n[4] = { &c.n_ee, &c.n_fv, &c.n_vv, &c.n_ev };
     const int lists = codim ? 4 : 2;
-    // deep traversal stack entries, per query of the largest query set
-    const int64_t nq_max = std::max<int64_t>(std::max<int64_t>(c.nE, c.nV), 1);
-    c.tr_deep.reserve(sizeof(int) * (size_t)nq_max * (TR_STACK - TR_LSTACK));
+    // one launch for both walks, unless the launch shapes are being tuned
+    const bool both = !c.autotune && c.nE >= 2 && c.nF >= 1;
+    // deep traversal stack entries: per query of the largest query set, or
+    // of both sets when they walk at once
+    const int qw = wave_queries((int64_t)c.nE + c.nV);
+    const int64_t deep_ee = deep_ints(c.nE, qw), deep_fv = deep_ints(c.nV, qw);
+    c.tr_deep.reserve(sizeof(int) * (size_t)(both ? deep_ee + deep_fv : std::max(deep_ee, deep_fv)));
     int* deep = c.tr_deep.as<int>();
     for (int attempt = 0; attempt < 3; attempt++) {
         // per-shard regions; their sum bounds a list until a retry grows it
@@ -1340,8 +1479,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
             if (*scap[k] == 0) *scap[k] = std::max<int64_t>(1024, guess[k] / SHARDS);
             c.cand_stage[k].reserve(sizeof(int2) * (size_t)(SHARDS * *scap[k]));
         }
-        IPCG_HIP(hipMemsetAsync(c.shard_cnt.p, 0, 4 * SHARD_CNT_BYTES, s));
-        IPCG_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+        IPCG_HIP(hipMemsetAsync(c.shard_cnt.p, 0, 4 * SHARD_CNT_BYTES + sizeof(int), s));
         const Shards S0 { cnt[0], c.scap_ee }, S1 { cnt[1], c.scap_fv };
         if (sap) {
             c.stage_begin("bp_sweep");
@@ -1364,31 +1502,45 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
             c.stage_end();
         } else {
             const std::string tag = swept ? ".swept" : ".static";
-            if (c.nE >= 2) {
-                const TraverseArgs a { c.te.box.as<float>(), c.te.ids.as<uint32_t>(), c.nE,
-                                       c.te.nodes.as<Node>(), c.te.root.as<int32_t>(),
-                                       c.te.leaf.as<int4>(), c.te.box.as<float>(), c.nE, flt,
-                                       nullptr, c.cand_stage[0].as<int2>(), S0, deep, status,
-                                       forest_args(c, c.te) };
-                c.stage_begin("bp_traverse_ee");
-                tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], [&](int b) {
-                    if (swept) launch_traverse<TR_EE, 1>(b, a, s);
-                    else launch_traverse<TR_EE, 0>(b, a, s);
-                });
+            const TraverseArgs ee { c.te.box.as<float>(), c.te.ids.as<uint32_t>(), c.nE,
+                                    c.te.nodes.as<Node>(), c.te.root.as<int32_t>(),
+                                    c.te.leaf.as<int4>(), c.te.box.as<float>(), c.nE, flt,
+                                    nullptr, c.cand_stage[0].as<int2>(), S0, deep, status,
+                                    forest_args(c, c.te), qw };
+            const TraverseArgs fv { c.tv.box.as<float>(), c.tv.ids.as<uint32_t>(), c.nV,
+                                    c.tf.nodes.as<Node>(), c.tf.root.as<int32_t>(),
+                                    c.tf.leaf.as<int4>(), c.tf.box.as<float>(), c.nF, flt,
+                                    nullptr, c.cand_stage[1].as<int2>(), S1,
+                                    both ? deep + deep_ee : deep, status,
+                                    forest_args(c, c.tf), qw };
+            if (both) {
+                const unsigned nb_ee = traverse_blocks(c.nE, qw, TR_BLOCK),
+                               nb_fv = traverse_blocks(c.nV, qw, TR_BLOCK);
+                c.stage_begin("bp_traverse_both");
+                if (swept)
+                    hipLaunchKernelGGL(k_traverse_both<1>, dim3(nb_ee + nb_fv), dim3(TR_BLOCK), 0,
+                                       s, ee, fv, nb_ee);
+                else
+                    hipLaunchKernelGGL(k_traverse_both<0>, dim3(nb_ee + nb_fv), dim3(TR_BLOCK), 0,
+                                       s, ee, fv, nb_ee);
                 c.stage_end();
-            }
-            if (c.nF >= 1) {
-                const TraverseArgs a { c.tv.box.as<float>(), c.tv.ids.as<uint32_t>(), c.nV,
-                                       c.tf.nodes.as<Node>(), c.tf.root.as<int32_t>(),
-                                       c.tf.leaf.as<int4>(), c.tf.box.as<float>(), c.nF, flt,
-                                       nullptr, c.cand_stage[1].as<int2>(), S1, deep, status,
-                                       forest_args(c, c.tf) };
-                c.stage_begin("bp_traverse_fv");
-                tuned_traverse(c, "bp_traverse_fv" + tag, cnt[1], [&](int b) {
-                    if (swept) launch_traverse<TR_FV, 1>(b, a, s);
-                    else launch_traverse<TR_FV, 0>(b, a, s);
-                });
-                c.stage_end();
+            } else {
+                if (c.nE >= 2) {
+                    c.stage_begin("bp_traverse_ee");
+                    tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], [&](int b) {
+                        if (swept) launch_traverse<TR_EE, 1>(b, ee, s);
+                        else launch_traverse<TR_EE, 0>(b, ee, s);
+                    });
+                    c.stage_end();
+                }
+                if (c.nF >= 1) {
+                    c.stage_begin("bp_traverse_fv");
+                    tuned_traverse(c, "bp_traverse_fv" + tag, cnt[1], [&](int b) {
+                        if (swept) launch_traverse<TR_FV, 1>(b, fv, s);
+                        else launch_traverse<TR_FV, 0>(b, fv, s);
+                    });
+                    c.stage_end();
+                }
             }
         }
         if (codim) {
@@ -1399,7 +1551,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                                        c.tcv.nodes.as<Node>(), c.tcv.root.as<int32_t>(),
                                        c.tcv.leaf.as<int4>(), c.tcv.box.as<float>(), c.n_cv, flt,
                                        c.cv.as<int32_t>(), c.cand_stage[2].as<int2>(), S2, deep,
-                                       status, forest_args(c, c.tcv) };
+                                       status, forest_args(c, c.tcv), qw };
                 if (swept) launch_traverse<TR_VV, 1>(TR_BLOCK, a, s);
                 else launch_traverse<TR_VV, 0>(TR_BLOCK, a, s);
             }
@@ -1408,7 +1560,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                                        c.tce.nodes.as<Node>(), c.tce.root.as<int32_t>(),
                                        c.tce.leaf.as<int4>(), c.tce.box.as<float>(), c.n_ce, flt,
                                        c.cv.as<int32_t>(), c.cand_stage[3].as<int2>(), S3, deep,
-                                       status, forest_args(c, c.tce) };
+                                       status, forest_args(c, c.tce), qw };
                 if (swept) launch_traverse<TR_EV, 1>(TR_BLOCK, a, s);
                 else launch_traverse<TR_EV, 0>(TR_BLOCK, a, s);
             }
@@ -1476,11 +1628,12 @@ void bp_edge_face(Ctx& c, double inflation)
     Filter flt { c.E.as<int32_t>(), c.F.as<int32_t>(), c.has_patch ? c.patch.as<int32_t>() : nullptr,
                  c.n_dynamic, c.n_codim_filter };
     c.counters.reserve(sizeof(unsigned long long) * 4);
-    int* status = reinterpret_cast<int*>(c.counters.as<unsigned long long>() + 2);
-    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES);
+    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(unsigned long long));
+    int* status = reinterpret_cast<int*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
     c.shard_off.reserve(sizeof(int64_t) * 4 * (SHARDS + 1));
     unsigned long long* cnt = c.shard_cnt.as<unsigned long long>();
-    c.tr_deep.reserve(sizeof(int) * (size_t)c.nE * (TR_STACK - TR_LSTACK));
+    const int qw = wave_queries(c.nE);
+    c.tr_deep.reserve(sizeof(int) * (size_t)deep_ints(c.nE, qw));
     for (int attempt = 0; attempt < 3; attempt++) {
         if (c.scap_ef == 0) c.scap_ef = std::max<int64_t>(1024, 8 * (int64_t)c.nE / SHARDS);
         c.cand_stage[0].reserve(sizeof(int2) * (size_t)(SHARDS * c.scap_ef));
@@ -1491,7 +1644,7 @@ void bp_edge_face(Ctx& c, double inflation)
         const TraverseArgs a { c.te.box.as<float>(), c.te.ids.as<uint32_t>(), c.nE,
                                c.tf.nodes.as<Node>(), c.tf.root.as<int32_t>(), c.tf.leaf.as<int4>(),
                                c.tf.box.as<float>(), c.nF, flt, nullptr, c.cand_stage[0].as<int2>(),
-                               S0, c.tr_deep.as<int>(), status, forest_args(c, c.tf) };
+                               S0, c.tr_deep.as<int>(), status, forest_args(c, c.tf), qw };
         launch_traverse<TR_EF, 0>(TR_BLOCK, a, s);
         IPCG_CHECK_LAUNCH();
         c.stage_end();

@@ -80,12 +80,13 @@ struct DevBuf {
 // workgroups: spatially ordered work (Morton-sorted queries, sorted
 // collisions) then shares one L2.  A bijection of [0, gridDim.x).
 constexpr unsigned NUM_XCD = 8;
-__device__ __forceinline__ unsigned xcd_block()
+// (b, nb: a range of a launch's workgroups, for one that holds several)
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
 {
-    const unsigned b = blockIdx.x, nb = gridDim.x;
     const unsigned q = nb / NUM_XCD, r = nb % NUM_XCD, x = b % NUM_XCD;
     return x * q + (x < r ? x : r) + b / NUM_XCD;
 }
+__device__ __forceinline__ unsigned xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 // ---- wave64 helpers -------------------------------------------------------
 __device__ __forceinline__ int lane_id() { return __lane_id(); }

@@ -1,0 +1,59 @@
+"""Tree walks: waves that start with 8, 16 or 64 queries, subtrees handed
+between lanes, the queue of overlapping leaves and edge-edge beside
+face-vertex walks in one launch, against the oracle's candidates and the
+separate launches of the autotuned path.  Candidate sets are exact."""
+import numpy as np
+import pytest
+
+from conftest import pair_set
+
+pytestmark = pytest.mark.gpu
+
+
+def pile(n):
+    """n triangles through one another: every wave's queue fills at each
+    step, and all the work belongs to few lanes"""
+    rng = np.random.default_rng(5)
+    V = rng.normal(size=(3 * n, 3))
+    F = np.arange(3 * n, dtype=np.int32).reshape(-1, 3)
+    return V, F
+
+
+def edges(F):
+    return np.unique(np.sort(np.concatenate([F[:, [0, 1]], F[:, [1, 2]], F[:, [2, 0]]]), axis=1),
+                     axis=0).astype(np.int32)
+
+
+def check(ctx, O, V, E, F, r):
+    ctx.upload_mesh(V, E, F)
+    ctx.upload_positions(0, V)
+    ctx.broad_phase(False, r)
+    ee, fv = ctx.candidates()
+    ee_o, fv_o = O.candidates(V, E, F, r)
+    assert len(ee) == len(ee_o) and pair_set(ee) == pair_set(ee_o)
+    assert len(fv) == len(fv_o) and pair_set(fv) == pair_set(fv_o)
+    return ee, fv
+
+
+@pytest.mark.parametrize("n", [2, 5, 22, 64, 150])
+def test_pile_of_triangles(ctx, O, n):
+    V, F = pile(n)
+    check(ctx, O, V, edges(F), F, 1e-3)
+
+
+# nE + nV just below and above 2^16 and 2^18 (a sheet of n^2 vertices has
+# 4 n^2 - 4 n + 1 of them)
+@pytest.mark.parametrize("n", [128, 129, 256, 257])
+def test_walks_at_the_limits_of_the_starting_widths(ctx, O, scenes, n):
+    s = scenes.stacked_sheets(n, 1, seed=2, h=1.0 / 511)
+    V = s.V.copy()
+    V[::7] *= 0.98  # some far overlaps
+    print("case", n, len(s.E) + len(V), flush=True)
+    ee, fv = check(ctx, O, V, s.E, s.F, 0.5 * s.dhat)
+    ctx.set_autotune(True)
+    try:
+        ctx.broad_phase(False, 0.5 * s.dhat)
+        ee2, fv2 = ctx.candidates()
+    finally:
+        ctx.set_autotune(False)
+    assert pair_set(ee) == pair_set(ee2) and pair_set(fv) == pair_set(fv2)
