@@ -406,11 +406,47 @@ __global__ void k_keys_to_pairs(const uint64_t* keys, int64_t n, Areas A, int2* 
     }
 }
 
-// Sum of wt(j), j in [s, e), taken in ascending order of value (equal
-// values in any order): the same double whatever order the contributions
-// arrived in.  Runs are a handful of entries, so a repeated minimum scan.
-template <class W>
-__device__ double sorted_sum(uint32_t s, uint32_t e, W wt)
+// LDS written by some lanes of the wave is read by others
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sum of the n <= N values wt(s + j) in ascending order, by a bitonic network
+// in registers (every load in flight at once; the places past n hold the
+// largest value and are not added).
+template <int N, class W> __device__ __forceinline__ double network_sum(uint32_t s, uint32_t n, W wt)
+{
+    double v[N];
+    bool nan = false;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        v[j] = INFINITY;
+        if ((uint32_t)j < n) v[j] = wt(s + j);
+        nan |= v[j] != v[j];
+    }
+#pragma unroll
+    for (int k = 2; k <= N; k *= 2)
+#pragma unroll
+        for (int j = k / 2; j > 0; j /= 2)
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if ((i ^ j) > i) {
+                    const double lo = fmin(v[i], v[i ^ j]), hi = fmax(v[i], v[i ^ j]);
+                    v[i] = (i & k) == 0 ? lo : hi;
+                    v[i ^ j] = (i & k) == 0 ? hi : lo;
+                }
+    double sum = 0.0;
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if ((uint32_t)j < n) sum += v[j];
+    return nan ? NAN : sum; // NaN contributions have no place in the order
+}
+
+// Repeated minimum scan, for runs that outgrow the other ways.
+template <class W> __device__ double scan_sum(uint32_t s, uint32_t e, W wt)
 {
     double sum = 0.0, last = 0.0;
     uint32_t done = 0;
@@ -437,13 +473,72 @@ __device__ double sorted_sum(uint32_t s, uint32_t e, W wt)
     return sum;
 }
 
-// real-valued merge of a vertex-vertex / edge-vertex run
-__global__ void k_run_sums(const uint32_t* start, int64_t nu, const uint32_t* perm,
-                           const double* cw, double* rw, uint32_t* keep)
+// Sum of a run of n <= RUN_WAVE values by the wave: every value's rank by
+// comparison with the others in LDS (buf: 2 RUN_WAVE doubles), then the sum
+// of the ranked values.  All lanes call it, with the same run.
+constexpr uint32_t RUN_WAVE = 512;
+
+template <class W>
+__device__ __forceinline__ double wave_sum(uint32_t s, uint32_t n, W wt, double* buf)
 {
+    const uint32_t l = (uint32_t)lane_id();
+    double* const by_rank = buf + RUN_WAVE;
+    bool nan = false;
+    for (uint32_t j = l; j < n; j += WAVE) {
+        const double x = wt(s + j);
+        buf[j] = x;
+        nan |= x != x;
+    }
+    if (__any(nan)) return NAN; // NaN contributions have no place in the order
+    wave_lds_fence();
+    for (uint32_t j = l; j < n; j += WAVE) {
+        const double x = buf[j];
+        uint32_t rank = 0;
+        for (uint32_t k = 0; k < n; k++) rank += buf[k] < x || (buf[k] == x && k < j) ? 1u : 0u;
+        by_rank[rank] = x;
+    }
+    wave_lds_fence();
+    double sum = 0.0;
+    for (uint32_t k = 0; k < n; k++) sum += by_rank[k];
+    wave_lds_fence();
+    return sum;
+}
+
+// Sum of wt(j), j in [s, e) (none where s == e), taken in ascending order of
+// value (equal values in any order): the same double whatever order the
+// contributions arrived in.  All lanes of the wave call it.  Runs up to 16
+// go through a network in the lane's registers, longer ones are taken by the
+// wave one after the other; a minimum scan by each lane, e - s passes of dependent
+// loads, took 1.10 ms for the two launches of the area-weighted merge of 5 sheets of
+// 127^2, now 0.24.
+template <class W> __device__ __forceinline__ double sorted_sum(uint32_t s, uint32_t e, W wt, double* buf)
+{
+    const uint32_t n = e - s;
+    double sum = n <= 16 ? network_sum<16>(s, n, wt) : 0.0;
+    unsigned long long more = __ballot(n > 16);
+    while (more) {
+        const int src = __ffsll(more) - 1;
+        more &= more - 1;
+        const uint32_t rs = __builtin_amdgcn_readlane(s, src), rn = __builtin_amdgcn_readlane(n, src);
+        double w;
+        if (rn <= RUN_WAVE) w = wave_sum(rs, rn, wt, buf);
+        else w = scan_sum(rs, rs + rn, wt);
+        if (lane_id() == src) sum = w;
+    }
+    return sum;
+}
+
+// real-valued merge of a vertex-vertex / edge-vertex run
+__global__ __launch_bounds__(256) void k_run_sums(const uint32_t* start, int64_t nu,
+                                                  const uint32_t* perm, const double* cw,
+                                                  double* rw, uint32_t* keep)
+{
+    __shared__ double buf[256 / WAVE][2 * RUN_WAVE];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t s = i < nu ? start[i] : 0, e = i < nu ? start[i + 1] : 0;
+    const double w = sorted_sum(s, e, [&](uint32_t j) { return cw[perm[j]]; },
+                                buf[threadIdx.x / WAVE]);
     if (i < nu) {
-        const double w = sorted_sum(start[i], start[i + 1], [&](uint32_t j) { return cw[perm[j]]; });
         rw[i] = w;
         keep[i] = w != 0.0;
     }
@@ -459,16 +554,19 @@ __global__ void k_run_scatter(const uint64_t* ukeys, int64_t nu, const double* r
     }
 }
 
-__global__ void k_ee_runs(const uint32_t* start, int64_t nu, const uint32_t* perm, const EERec* r,
-                          double* rw, uint32_t* rep, uint32_t* keep)
+__global__ __launch_bounds__(256) void k_ee_runs(const uint32_t* start, int64_t nu,
+                                                 const uint32_t* perm, const EERec* r, double* rw,
+                                                 uint32_t* rep, uint32_t* keep)
 {
+    __shared__ double buf[256 / WAVE][2 * RUN_WAVE];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t s = i < nu ? start[i] : 0, e = i < nu ? start[i + 1] : 0;
+    const double w = sorted_sum(s, e, [&](uint32_t j) { return r[perm[j]].w; },
+                                buf[threadIdx.x / WAVE]);
     if (i < nu) {
-        const uint32_t s = start[i], e = start[i + 1];
         uint32_t best = perm[s];
         for (uint32_t j = s + 1; j < e; j++)
             if (r[perm[j]].rank < r[best].rank) best = perm[j];
-        const double w = sorted_sum(s, e, [&](uint32_t j) { return r[perm[j]].w; });
         rw[i] = w;
         rep[i] = best;
         keep[i] = w != 0.0;
@@ -505,52 +603,75 @@ __device__ __forceinline__ uint64_t conv_key(int tag, uint64_t k)
 // vertices, candidates.cpp:583-620), 4 per edge-edge candidate (each edge
 // with the other's vertices, candidates.cpp:665-692), 6 per face-vertex
 // candidate (the face's edges, candidates.cpp:640-663, then its vertices);
-// a pair whose sub-element distance is active is appended to `out` (one
-// atomic per wave), so the sort sees only the active pairs.  Every lane
-// reaches the append (its count may be 0).
+// a pair whose sub-element distance is active is appended to `out`, so the
+// sort sees only the active pairs.  A workgroup takes CONV_CHUNKS candidates a
+// thread and collects the keys in LDS: one device-wide atomic (12 ns each,
+// whoever issues it) per CONV_ROOM keys or workgroup.  With one per wave they
+// were all of the kernel's 1.36 ms on 5 sheets of 127^2; now 0.32.
+constexpr int CONV_CHUNKS = 8;
+constexpr unsigned CONV_ROOM = 1536;                  // keys that leave room for a chunk
+constexpr unsigned CONV_BUF = CONV_ROOM + 6 * NP_BLOCK; // six keys a candidate
+
 __global__ __launch_bounds__(NP_BLOCK) void k_conv_slots(
     const double* X, int nV, const int32_t* E, const int32_t* F, const int32_t* F2E, const int2* ev,
     int64_t n_ev, const int2* ee, int64_t n_ee, const int2* fv, int64_t n_fv, double active2,
     unsigned long long* count, uint64_t* out)
 {
-    const int64_t i = (int64_t)xcd_block() * NP_BLOCK + threadIdx.x;
-    uint64_t k[6];
-    unsigned nk = 0;
-    if (i < n_ev) {
-        const int2 c = ev[i];
-        const d3 p = ldx(X, nV, c.y);
-        for (int j = 0; j < 2; j++) {
-            const int vj = E[2 * (int64_t)c.x + j];
-            if (pp_dist2(p, ldx(X, nV, vj)) < active2) k[nk++] = conv_key(CV_EV_VV, vv_key(c.y, vj));
-        }
-    } else if (i < n_ev + n_ee) {
-        const int2 c = ee[i - n_ev];
-        for (int s = 0; s < 2; s++) {
-            const int ei = s ? c.y : c.x, ej = s ? c.x : c.y;
-            const d3 q0 = ldx(X, nV, E[2 * (int64_t)ei]), q1 = ldx(X, nV, E[2 * (int64_t)ei + 1]);
+    __shared__ uint64_t buf[CONV_BUF];
+    __shared__ unsigned held;
+    __shared__ unsigned long long base;
+    if (threadIdx.x == 0) held = 0;
+    __syncthreads();
+    const int64_t n = n_ev + n_ee + n_fv;
+    const int64_t i0 = (int64_t)xcd_block() * (NP_BLOCK * CONV_CHUNKS);
+    for (int ch = 0; ch < CONV_CHUNKS; ch++) {
+        const int64_t i = i0 + ch * NP_BLOCK + threadIdx.x;
+        auto emit = [&](uint64_t k) { buf[atomicAdd(&held, 1u)] = k; };
+        if (i < n_ev) {
+            const int2 c = ev[i];
+            const d3 p = ldx(X, nV, c.y);
             for (int j = 0; j < 2; j++) {
-                const int vj = E[2 * (int64_t)ej + j];
-                const d3 p = ldx(X, nV, vj);
+                const int vj = E[2 * (int64_t)c.x + j];
+                if (pp_dist2(p, ldx(X, nV, vj)) < active2) emit(conv_key(CV_EV_VV, vv_key(c.y, vj)));
+            }
+        } else if (i < n_ev + n_ee) {
+            const int2 c = ee[i - n_ev];
+            for (int s = 0; s < 2; s++) {
+                const int ei = s ? c.y : c.x, ej = s ? c.x : c.y;
+                const d3 q0 = ldx(X, nV, E[2 * (int64_t)ei]),
+                         q1 = ldx(X, nV, E[2 * (int64_t)ei + 1]);
+                for (int j = 0; j < 2; j++) {
+                    const int vj = E[2 * (int64_t)ej + j];
+                    const d3 p = ldx(X, nV, vj);
+                    if (pe_dist2(p, q0, q1, point_edge_type(p, q0, q1)) < active2)
+                        emit(conv_key(CV_EE_EV, pair_key(ei, vj)));
+                }
+            }
+        } else if (i < n) {
+            const int2 c = fv[i - n_ev - n_ee];
+            const d3 p = ldx(X, nV, c.y);
+            for (int j = 0; j < 3; j++) {
+                const int ei = F2E[3 * (int64_t)c.x + j];
+                const d3 q0 = ldx(X, nV, E[2 * (int64_t)ei]),
+                         q1 = ldx(X, nV, E[2 * (int64_t)ei + 1]);
                 if (pe_dist2(p, q0, q1, point_edge_type(p, q0, q1)) < active2)
-                    k[nk++] = conv_key(CV_EE_EV, pair_key(ei, vj));
+                    emit(conv_key(CV_FV_EV, pair_key(ei, c.y)));
+            }
+            for (int j = 0; j < 3; j++) {
+                const int vj = F[3 * (int64_t)c.x + j];
+                if (pp_dist2(p, ldx(X, nV, vj)) < active2) emit(conv_key(CV_FV_VV, vv_key(c.y, vj)));
             }
         }
-    } else if (i < n_ev + n_ee + n_fv) {
-        const int2 c = fv[i - n_ev - n_ee];
-        const d3 p = ldx(X, nV, c.y);
-        for (int j = 0; j < 3; j++) {
-            const int ei = F2E[3 * (int64_t)c.x + j];
-            const d3 q0 = ldx(X, nV, E[2 * (int64_t)ei]), q1 = ldx(X, nV, E[2 * (int64_t)ei + 1]);
-            if (pe_dist2(p, q0, q1, point_edge_type(p, q0, q1)) < active2)
-                k[nk++] = conv_key(CV_FV_EV, pair_key(ei, c.y));
+        __syncthreads();
+        const unsigned m = held; // uniform
+        if (m > CONV_ROOM || (ch + 1 == CONV_CHUNKS && m > 0)) {
+            if (threadIdx.x == 0) base = atomicAdd(count, (unsigned long long)m);
+            __syncthreads();
+            for (unsigned j = threadIdx.x; j < m; j += NP_BLOCK) out[base + j] = buf[j];
+            if (threadIdx.x == 0) held = 0;
         }
-        for (int j = 0; j < 3; j++) {
-            const int vj = F[3 * (int64_t)c.x + j];
-            if (pp_dist2(p, ldx(X, nV, vj)) < active2) k[nk++] = conv_key(CV_FV_VV, vv_key(c.y, vj));
-        }
+        __syncthreads();
     }
-    const unsigned long long at = wave_append(count, nk);
-    for (unsigned j = 0; j < nk; j++) out[at + j] = k[j];
 }
 
 struct ImOut {
@@ -712,7 +833,7 @@ static void improved_records(Ctx& c, double active2, Areas A, int64_t x[3])
     const int ibits = key_bits_for(std::max<int64_t>(c.nV, c.nE)) - 32;
     const unsigned long long slot_mask = (3ull << 62) | (low_bits(ibits) << 32) | low_bits(ibits);
     IPCG_HIP(hipMemsetAsync(n_act_dev, 0, sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(k_conv_slots, dim3(grid_for(nc, NP_BLOCK, INT32_MAX)), dim3(NP_BLOCK), 0, s,
+    hipLaunchKernelGGL(k_conv_slots, dim3(grid_for(nc, NP_BLOCK * CONV_CHUNKS, INT32_MAX)), dim3(NP_BLOCK), 0, s,
                        c.X[0].as<double>(), c.nV, c.E.as<int32_t>(), c.F.as<int32_t>(),
                        c.F2E.as<int32_t>(), c.cand_ev.as<int2>(), c.n_ev, c.cand_ee.as<int2>(),
                        c.n_ee, c.cand_fv.as<int2>(), c.n_fv, active2, n_act_dev, slot);
