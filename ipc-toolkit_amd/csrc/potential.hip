@@ -64,6 +64,38 @@ __device__ __forceinline__ void stencil_ids(const CollView& C, int64_t i, int* v
     }
 }
 
+// The four kinds in one launch: the workgroups of a kind follow those of the
+// one before it, `block` threads each.  (A launch per kind cost 5 us each: a
+// line-search trial of two 33^2 sheets has 2,000 collisions of three kinds.)
+struct KindBlocks {
+    unsigned first[5];
+};
+
+KindBlocks kind_blocks(const CollView& C, int block)
+{
+    KindBlocks K { { 0, 0, 0, 0, 0 } };
+    int64_t at = 0;
+    for (int k = 0; k < 4; k++) {
+        at += (C.n[k] + block - 1) / block;
+        grid_for(at, 1); // more blocks than a grid holds are an error
+        K.first[k + 1] = (unsigned)at;
+    }
+    grid_for(at * block, block);
+    return K;
+}
+
+// f(kind, b, nb): workgroup b of the kind's nb
+template <class Fn> __device__ __forceinline__ void by_kind(const KindBlocks& K, Fn&& f)
+{
+    const unsigned b = blockIdx.x;
+    if (b < K.first[1]) f(std::integral_constant<int, K_VV>(), b, K.first[1]);
+    else if (b < K.first[2])
+        f(std::integral_constant<int, K_EV>(), b - K.first[1], K.first[2] - K.first[1]);
+    else if (b < K.first[3])
+        f(std::integral_constant<int, K_EE>(), b - K.first[2], K.first[3] - K.first[2]);
+    else f(std::integral_constant<int, K_FV>(), b - K.first[3], K.first[4] - K.first[3]);
+}
+
 template <int KIND>
 __device__ __forceinline__ double collision_energy(const CollView& C, const double* X, int nV,
                                                    const BarrierParams& bp, int64_t i)
@@ -92,13 +124,15 @@ __device__ __forceinline__ void block_partial(double e, double* partial)
     }
 }
 
-template <int KIND>
-__global__ __launch_bounds__(PB) void k_energy(CollView C, const double* X, int nV,
+__global__ __launch_bounds__(PB) void k_energy(CollView C, KindBlocks K, const double* X, int nV,
                                                BarrierParams bp, double* partial)
 {
-    const int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x;
     double e = 0;
-    if (i < C.n[KIND]) e = collision_energy<KIND>(C, X, nV, bp, i);
+    by_kind(K, [&](auto kind, unsigned b, unsigned) {
+        constexpr int KIND = decltype(kind)::value;
+        const int64_t i = (int64_t)b * PB + threadIdx.x;
+        if (i < C.n[KIND]) e = collision_energy<KIND>(C, X, nV, bp, i);
+    });
     block_partial(e, partial);
 }
 
@@ -198,12 +232,15 @@ __global__ __launch_bounds__(256) void k_sum_scenes(const double* partial, const
 // Atomic-free gradient: every collision writes its 3 NP derivatives to a
 // record (point-major), then one wave per vertex sums the records of the
 // vertex's incidences in a fixed order.
+struct KindRecs {
+    double* rec[4];
+};
+
 template <int KIND>
-__global__ __launch_bounds__(PB) void k_gradient_records(CollView C, const double* X, int nV,
-                                                         BarrierParams bp, double* rec)
+__device__ __forceinline__ void gradient_record(const CollView& C, int64_t i, const double* X,
+                                                int nV, const BarrierParams& bp, double* rec)
 {
     constexpr int NP = StencilTraits<KIND>::NP;
-    const int64_t i = (int64_t)xcd_block() * PB + threadIdx.x;
     if (i >= C.n[KIND]) return;
     int v[4];
     stencil_ids<KIND>(C, i, v);
@@ -220,6 +257,16 @@ __global__ __launch_bounds__(PB) void k_gradient_records(CollView C, const doubl
         o[3 * j + 1] = g[j].y;
         o[3 * j + 2] = g[j].z;
     }
+}
+
+__global__ __launch_bounds__(PB) void k_gradient_records(CollView C, KindBlocks K, const double* X,
+                                                         int nV, BarrierParams bp, KindRecs out)
+{
+    by_kind(K, [&](auto kind, unsigned b, unsigned nb) {
+        constexpr int KIND = decltype(kind)::value;
+        gradient_record<KIND>(C, (int64_t)xcd_block(b, nb) * PB + threadIdx.x, X, nV, bp,
+                              out.rec[KIND]);
+    });
 }
 
 // ---- Gauss-Newton helpers (normal_potential.cpp:236-308) -----------------
@@ -332,15 +379,17 @@ __global__ __launch_bounds__(PB) void k_gn_diag_records(CollView C, const double
 }
 
 // normal_potential.cpp:272-308; p: 3 nV RowMajor
-template <int KIND>
-__global__ __launch_bounds__(PB) void k_gn_quadratic_form(CollView C, const double* X, int nV,
+__global__ __launch_bounds__(PB) void k_gn_quadratic_form(CollView C, KindBlocks K,
+                                                          const double* X, int nV,
                                                           BarrierParams bp, const double* p,
                                                           double* partial)
 {
-    constexpr int NP = StencilTraits<KIND>::NP;
-    const int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x;
     double e = 0;
-    if (i < C.n[KIND]) {
+    by_kind(K, [&](auto kind, unsigned b, unsigned) {
+        constexpr int KIND = decltype(kind)::value;
+        constexpr int NP = StencilTraits<KIND>::NP;
+        const int64_t i = (int64_t)b * PB + threadIdx.x;
+        if (i >= C.n[KIND]) return;
         int v[4];
         stencil_ids<KIND>(C, i, v);
         d3 P[4], Q[4];
@@ -355,16 +404,8 @@ __global__ __launch_bounds__(PB) void k_gn_quadratic_form(CollView C, const doub
         const double d2 = dot_seq(t, t);
         const double qt = dot_seq(q, t);
         e = C.w[KIND][i] * (4.0 * bar_f2(d2, bp) * (qt * qt) + 2.0 * bar_f1(d2, bp) * dot_seq(q, q));
-    }
-    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, WAVE);
-    __shared__ double s[PB / WAVE];
-    if (threadIdx.x % WAVE == 0) s[threadIdx.x / WAVE] = e;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0;
-        for (int j = 0; j < PB / WAVE; j++) t += s[j];
-        partial[blockIdx.x] = t;
-    }
+    });
+    block_partial(e, partial);
 }
 
 struct CollRanges {
@@ -697,20 +738,25 @@ __global__ __launch_bounds__(64) void k_hessian_mollified(CollView C, const doub
 }
 
 // (vertex, global collision g, point a): key vertex, value g << 2 | a
-template <int KIND>
-__global__ __launch_bounds__(256) void k_incidence(CollView C, int64_t goff, int64_t ioff,
+__global__ __launch_bounds__(256) void k_incidence(CollView C, KindBlocks K, CollRanges G,
                                                    uint32_t* keys, uint32_t* vals)
 {
-    constexpr int NP = StencilTraits<KIND>::NP;
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= C.n[KIND]) return;
-    int v[4];
-    stencil_ids<KIND>(C, i, v);
+    by_kind(K, [&](auto kind, unsigned b, unsigned) {
+        constexpr int KIND = decltype(kind)::value;
+        constexpr int NP = StencilTraits<KIND>::NP;
+        const int64_t i = (int64_t)b * 256 + threadIdx.x;
+        if (i >= C.n[KIND]) return;
+        // incidences of the kinds before this one
+        const int64_t ioff = (KIND > K_VV ? 2 * C.n[K_VV] : 0) + (KIND > K_EV ? 3 * C.n[K_EV] : 0)
+            + (KIND > K_EE ? 4 * C.n[K_EE] : 0);
+        int v[4];
+        stencil_ids<KIND>(C, i, v);
 #pragma unroll
-    for (int a = 0; a < NP; a++) {
-        keys[ioff + (int64_t)NP * i + a] = (uint32_t)v[a];
-        vals[ioff + (int64_t)NP * i + a] = (uint32_t)(((goff + i) << 2) | a);
-    }
+        for (int a = 0; a < NP; a++) {
+            keys[ioff + (int64_t)NP * i + a] = (uint32_t)v[a];
+            vals[ioff + (int64_t)NP * i + a] = (uint32_t)(((G.goff[KIND] + i) << 2) | a);
+        }
+    });
 }
 
 // First incidence of every vertex in the sorted keys (vptr[nV] = M): lane i
@@ -1093,24 +1139,15 @@ double pot_energy(Ctx& c, double dhat, double kappa)
     hipStream_t s = c.stream;
     CollView C = view(c);
     const BarrierParams bp = barrier_params(c, dhat, kappa, 0);
-    int64_t nb[4], tot = 0;
-    for (int k = 0; k < 4; k++) {
-        nb[k] = (C.n[k] + PB - 1) / PB;
-        tot += nb[k];
-    }
+    const KindBlocks KB = kind_blocks(C, PB);
+    const int64_t tot = KB.first[4];
     c.red_partial.reserve(sizeof(double) * (size_t)std::max<int64_t>(tot, 1));
     c.red_out.reserve(sizeof(double) * 2);
     double* part = c.red_partial.as<double>();
     const double* X = c.X[0].as<double>();
     c.stage_begin("energy");
-    int64_t o = 0;
-    if (nb[0]) hipLaunchKernelGGL(k_energy<K_VV>, dim3(nb[0]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[0];
-    if (nb[1]) hipLaunchKernelGGL(k_energy<K_EV>, dim3(nb[1]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[1];
-    if (nb[2]) hipLaunchKernelGGL(k_energy<K_EE>, dim3(nb[2]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[2];
-    if (nb[3]) hipLaunchKernelGGL(k_energy<K_FV>, dim3(nb[3]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_energy, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, X, c.nV, bp, part);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, s, part, tot, c.red_out.as<double>());
     IPCG_CHECK_LAUNCH();
     c.stage_end();
@@ -1167,25 +1204,16 @@ void pot_energy_noalloc(Ctx& c, double dhat, double kappa, double* d_out)
     hipStream_t s = c.stream;
     CollView C = view(c);
     const BarrierParams bp = barrier_params(c, dhat, kappa, 0);
-    int64_t nb[4], tot = 0;
-    for (int k = 0; k < 4; k++) {
-        nb[k] = (C.n[k] + PB - 1) / PB;
-        tot += nb[k];
-    }
+    const KindBlocks KB = kind_blocks(C, PB);
+    const int64_t tot = KB.first[4];
     if (tot > NOALLOC_PARTIALS)
         throw Error(IPCG_ERR_ARG, "collision set too large for the allocation-free energy: "
                                       + std::to_string(tot) + " blocks of "
                                       + std::to_string(PB) + " collisions, at most "
                                       + std::to_string(NOALLOC_PARTIALS));
     const double* X = c.X[0].as<double>();
-    int64_t o = 0;
-    if (nb[0]) hipLaunchKernelGGL(k_energy<K_VV>, dim3(nb[0]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[0];
-    if (nb[1]) hipLaunchKernelGGL(k_energy<K_EV>, dim3(nb[1]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[1];
-    if (nb[2]) hipLaunchKernelGGL(k_energy<K_EE>, dim3(nb[2]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
-    o += nb[2];
-    if (nb[3]) hipLaunchKernelGGL(k_energy<K_FV>, dim3(nb[3]), dim3(PB), 0, s, C, X, c.nV, bp, part + o);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_energy, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, X, c.nV, bp, part);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, s, part, tot, d_out);
     IPCG_CHECK_LAUNCH();
 }
@@ -1347,14 +1375,9 @@ void require_incidences(Ctx& c, const CollView& C, const CollRanges& G, int64_t 
     c.inc_ptr.reserve(sizeof(uint32_t) * ((size_t)c.nV + 1));
     uint32_t* keys = c.inc_keys.as<uint32_t>();
     uint32_t* vals = c.inc_vals.as<uint32_t>();
-    int64_t io = 0;
-    if (C.n[0]) hipLaunchKernelGGL(k_incidence<K_VV>, dim3(grid_for(C.n[0], 256, INT32_MAX)), dim3(256), 0, s, C, G.goff[0], io, keys, vals);
-    io += 2 * C.n[0];
-    if (C.n[1]) hipLaunchKernelGGL(k_incidence<K_EV>, dim3(grid_for(C.n[1], 256, INT32_MAX)), dim3(256), 0, s, C, G.goff[1], io, keys, vals);
-    io += 3 * C.n[1];
-    if (C.n[2]) hipLaunchKernelGGL(k_incidence<K_EE>, dim3(grid_for(C.n[2], 256, INT32_MAX)), dim3(256), 0, s, C, G.goff[2], io, keys, vals);
-    io += 4 * C.n[2];
-    if (C.n[3]) hipLaunchKernelGGL(k_incidence<K_FV>, dim3(grid_for(C.n[3], 256, INT32_MAX)), dim3(256), 0, s, C, G.goff[3], io, keys, vals);
+    const KindBlocks KB = kind_blocks(C, 256);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_incidence, dim3(KB.first[4]), dim3(256), 0, s, C, KB, G, keys, vals);
     IPCG_CHECK_LAUNCH();
     int vb = 1;
     while ((1ll << vb) <= c.nV) vb++;
@@ -1404,10 +1427,12 @@ void pot_gradient(Ctx& c, double dhat, double kappa)
         ro += 3 * (int64_t)npk[k] * C.n[k];
     }
     c.stage_begin("gradient");
-    if (C.n[0]) hipLaunchKernelGGL(k_gradient_records<K_VV>, dim3(grid_for(C.n[0], PB, INT32_MAX)), dim3(PB), 0, s, C, X, c.nV, bp, const_cast<double*>(R.rec[0]));
-    if (C.n[1]) hipLaunchKernelGGL(k_gradient_records<K_EV>, dim3(grid_for(C.n[1], PB, INT32_MAX)), dim3(PB), 0, s, C, X, c.nV, bp, const_cast<double*>(R.rec[1]));
-    if (C.n[2]) hipLaunchKernelGGL(k_gradient_records<K_EE>, dim3(grid_for(C.n[2], PB, INT32_MAX)), dim3(PB), 0, s, C, X, c.nV, bp, const_cast<double*>(R.rec[2]));
-    if (C.n[3]) hipLaunchKernelGGL(k_gradient_records<K_FV>, dim3(grid_for(C.n[3], PB, INT32_MAX)), dim3(PB), 0, s, C, X, c.nV, bp, const_cast<double*>(R.rec[3]));
+    KindRecs out;
+    for (int k = 0; k < 4; k++) out.rec[k] = const_cast<double*>(R.rec[k]);
+    const KindBlocks KB = kind_blocks(C, PB);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_gradient_records, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, X, c.nV, bp,
+                           out);
     const unsigned gw = grid_for((int64_t)c.nV * WAVE, 256, INT32_MAX); // a wave per vertex
     hipLaunchKernelGGL(k_gradient_rows, dim3(gw), dim3(256), 0, s, G, R, c.inc_ptr.as<uint32_t>(),
                        c.inc_vals.as<uint32_t>(), c.nV, g, row_order(c));
@@ -1664,25 +1689,17 @@ double pot_gn_quadratic_form(Ctx& c, double dhat, double kappa, const double* p_
     if (c.nV)
         IPCG_HIP(hipMemcpyAsync(c.gn_p.p, p_host, sizeof(double) * 3 * (size_t)c.nV,
                                 hipMemcpyHostToDevice, s));
-    int64_t nb[4], tot = 0;
-    for (int k = 0; k < 4; k++) {
-        nb[k] = (C.n[k] + PB - 1) / PB;
-        tot += nb[k];
-    }
+    const KindBlocks KB = kind_blocks(C, PB);
+    const int64_t tot = KB.first[4];
     c.red_partial.reserve(sizeof(double) * (size_t)std::max<int64_t>(tot, 1));
     c.red_out.reserve(sizeof(double) * 2);
     double* part = c.red_partial.as<double>();
     const double* X = c.X[0].as<double>();
     const double* p = c.gn_p.as<double>();
     c.stage_begin("gn_quadratic_form");
-    int64_t o = 0;
-    if (nb[0]) hipLaunchKernelGGL(k_gn_quadratic_form<K_VV>, dim3(nb[0]), dim3(PB), 0, s, C, X, c.nV, bp, p, part + o);
-    o += nb[0];
-    if (nb[1]) hipLaunchKernelGGL(k_gn_quadratic_form<K_EV>, dim3(nb[1]), dim3(PB), 0, s, C, X, c.nV, bp, p, part + o);
-    o += nb[1];
-    if (nb[2]) hipLaunchKernelGGL(k_gn_quadratic_form<K_EE>, dim3(nb[2]), dim3(PB), 0, s, C, X, c.nV, bp, p, part + o);
-    o += nb[2];
-    if (nb[3]) hipLaunchKernelGGL(k_gn_quadratic_form<K_FV>, dim3(nb[3]), dim3(PB), 0, s, C, X, c.nV, bp, p, part + o);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_gn_quadratic_form, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, X, c.nV,
+                           bp, p, part);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, s, part, tot, c.red_out.as<double>());
     IPCG_CHECK_LAUNCH();
     c.stage_end();
@@ -1945,38 +1962,33 @@ __device__ __forceinline__ void fric_local(const FricRec& r, const double* Vel, 
     norm = sqrt(u[0] * u[0] + u[1] * u[1]);
 }
 
-template <int KIND>
-__global__ __launch_bounds__(PB) void k_fric_energy(CollView C, const FricRec* R, const double* Vel,
-                                                    int nV, FricParams fp, double* partial)
+__global__ __launch_bounds__(PB) void k_fric_energy(CollView C, KindBlocks K, CollRanges G,
+                                                    const FricRec* recs, const double* Vel, int nV,
+                                                    FricParams fp, double* partial)
 {
-    const int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x;
     double e = 0;
-    if (i < C.n[KIND] && R[i].keep != 0) {
-        int v[4];
-        stencil_ids<KIND>(C, i, v);
-        double u[2], norm;
-        fric_local<KIND>(R[i], Vel, nV, v, fp.eps_v, R[i].ms_eff, R[i].mk_eff, u, norm);
-        e = R[i].s * smooth_mu_f0(norm, R[i].ms_eff, R[i].mk_eff, fp.eps_v);
-    }
-    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, WAVE);
-    __shared__ double sh[PB / WAVE];
-    if (threadIdx.x % WAVE == 0) sh[threadIdx.x / WAVE] = e;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0;
-        for (int j = 0; j < PB / WAVE; j++) t += sh[j];
-        partial[blockIdx.x] = t;
-    }
+    by_kind(K, [&](auto kind, unsigned b, unsigned) {
+        constexpr int KIND = decltype(kind)::value;
+        const int64_t i = (int64_t)b * PB + threadIdx.x;
+        const FricRec* const R = recs + G.goff[KIND];
+        if (i < C.n[KIND] && R[i].keep != 0) {
+            int v[4];
+            stencil_ids<KIND>(C, i, v);
+            double u[2], norm;
+            fric_local<KIND>(R[i], Vel, nV, v, fp.eps_v, R[i].ms_eff, R[i].mk_eff, u, norm);
+            e = R[i].s * smooth_mu_f0(norm, R[i].ms_eff, R[i].mk_eff, fp.eps_v);
+        }
+    });
+    block_partial(e, partial);
 }
 
 // gradient records: 3 NP values per collision, point major
 template <int KIND>
-__global__ __launch_bounds__(PB) void k_fric_gradient_records(CollView C, const FricRec* R,
-                                                              const double* Vel, int nV,
-                                                              FricParams fp, double* rec)
+__device__ __forceinline__ void fric_gradient_record(const CollView& C, int64_t i, const FricRec* R,
+                                                     const double* Vel, int nV,
+                                                     const FricParams& fp, double* rec)
 {
     constexpr int NP = StencilTraits<KIND>::NP;
-    const int64_t i = (int64_t)xcd_block() * PB + threadIdx.x;
     if (i >= C.n[KIND]) return;
     double* o = rec + (int64_t)3 * NP * i;
     const FricRec r = R[i];
@@ -1997,6 +2009,18 @@ __global__ __launch_bounds__(PB) void k_fric_gradient_records(CollView C, const 
 #pragma unroll
         for (int k = 0; k < 3; k++)
             o[3 * j + k] = (g[j] * r.P[k] * r.an[0]) * g0 + (g[j] * r.P[3 + k] * r.an[1]) * g1;
+}
+
+__global__ __launch_bounds__(PB) void k_fric_gradient_records(CollView C, KindBlocks K,
+                                                              CollRanges G, const FricRec* R,
+                                                              const double* Vel, int nV,
+                                                              FricParams fp, KindRecs out)
+{
+    by_kind(K, [&](auto kind, unsigned b, unsigned nb) {
+        constexpr int KIND = decltype(kind)::value;
+        fric_gradient_record<KIND>(C, (int64_t)xcd_block(b, nb) * PB + threadIdx.x,
+                                   R + G.goff[KIND], Vel, nV, fp, out.rec[KIND]);
+    });
 }
 
 // per-collision anisotropy (n x 2 each, null: keep), effective coefficients
@@ -2256,24 +2280,16 @@ double fric_energy(Ctx& c, double eps_v)
     const CollRanges G = ranges(C, M);
     const FricRec* R = c.fric.as<FricRec>();
     const FricParams fp { eps_v, 0 };
-    int64_t nb[4], tot = 0;
-    for (int k = 0; k < 4; k++) {
-        nb[k] = (C.n[k] + PB - 1) / PB;
-        tot += nb[k];
-    }
+    const KindBlocks KB = kind_blocks(C, PB);
+    const int64_t tot = KB.first[4];
     c.red_partial.reserve(sizeof(double) * (size_t)std::max<int64_t>(tot, 1));
     c.red_out.reserve(sizeof(double) * 2);
     double* part = c.red_partial.as<double>();
     const double* Vel = c.vel.as<double>();
     c.stage_begin("friction_energy");
-    int64_t o = 0;
-    if (nb[0]) hipLaunchKernelGGL(k_fric_energy<K_VV>, dim3(nb[0]), dim3(PB), 0, s, C, R + G.goff[0], Vel, c.nV, fp, part + o);
-    o += nb[0];
-    if (nb[1]) hipLaunchKernelGGL(k_fric_energy<K_EV>, dim3(nb[1]), dim3(PB), 0, s, C, R + G.goff[1], Vel, c.nV, fp, part + o);
-    o += nb[1];
-    if (nb[2]) hipLaunchKernelGGL(k_fric_energy<K_EE>, dim3(nb[2]), dim3(PB), 0, s, C, R + G.goff[2], Vel, c.nV, fp, part + o);
-    o += nb[2];
-    if (nb[3]) hipLaunchKernelGGL(k_fric_energy<K_FV>, dim3(nb[3]), dim3(PB), 0, s, C, R + G.goff[3], Vel, c.nV, fp, part + o);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_fric_energy, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, G, R, Vel, c.nV,
+                           fp, part);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, s, part, tot, c.red_out.as<double>());
     IPCG_CHECK_LAUNCH();
     c.stage_end();
@@ -2306,10 +2322,12 @@ void fric_gradient(Ctx& c, double eps_v)
     }
     const double* Vel = c.vel.as<double>();
     c.stage_begin("friction_gradient");
-    if (C.n[0]) hipLaunchKernelGGL(k_fric_gradient_records<K_VV>, dim3(grid_for(C.n[0], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[0], Vel, c.nV, fp, const_cast<double*>(GR.rec[0]));
-    if (C.n[1]) hipLaunchKernelGGL(k_fric_gradient_records<K_EV>, dim3(grid_for(C.n[1], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[1], Vel, c.nV, fp, const_cast<double*>(GR.rec[1]));
-    if (C.n[2]) hipLaunchKernelGGL(k_fric_gradient_records<K_EE>, dim3(grid_for(C.n[2], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[2], Vel, c.nV, fp, const_cast<double*>(GR.rec[2]));
-    if (C.n[3]) hipLaunchKernelGGL(k_fric_gradient_records<K_FV>, dim3(grid_for(C.n[3], PB, INT32_MAX)), dim3(PB), 0, s, C, R + G.goff[3], Vel, c.nV, fp, const_cast<double*>(GR.rec[3]));
+    KindRecs out;
+    for (int k = 0; k < 4; k++) out.rec[k] = const_cast<double*>(GR.rec[k]);
+    const KindBlocks KB = kind_blocks(C, PB);
+    if (KB.first[4])
+        hipLaunchKernelGGL(k_fric_gradient_records, dim3(KB.first[4]), dim3(PB), 0, s, C, KB, G, R,
+                           Vel, c.nV, fp, out);
     const unsigned gw = grid_for((int64_t)c.nV * WAVE, 256, INT32_MAX); // a wave per vertex
     hipLaunchKernelGGL(k_gradient_rows, dim3(gw), dim3(256), 0, s, G, GR, c.inc_ptr.as<uint32_t>(),
                        c.inc_vals.as<uint32_t>(), c.nV, c.grad.as<double>(), row_order(c));

@@ -84,3 +84,34 @@ def test_hessian_of_every_stencil(ctx, O, shape, dmin):
         assert ctx.counter("hessian.ee_other") > 0
     if shape == "soup":
         assert ctx.counter("hessian.ee_other") < counts[2]  # mostly the closed form
+
+
+ALONE = {  # one collision of one kind: the launch over the kinds has a single workgroup
+    "vv": ([[0, 0, 0], [0, 0, 1], [0, 1, 0.5], [-5e-3, 0, 0], [-1, 0, 0.2], [-1, 1, 0.2]],
+           [[0, 1, 2], [3, 4, 5]]),
+    "fv": ([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0.2, 0.3, 5e-3], [0.3, 0.2, 2.0], [0.1, 0.2, 2.0]],
+           [[0, 1, 2], [3, 4, 5]]),
+    "ee": ([[0, 0, 0], [1, 0, 0], [0.5, 0, -1], [0.4, -0.5, 5e-3], [0.5, 0.6, 5e-3], [0.5, 0, 1]],
+           [[0, 1, 2], [3, 4, 5]]),
+}
+
+
+@pytest.mark.parametrize("kind", sorted(ALONE))
+def test_one_kind_alone(ctx, O, kind):
+    V, F = np.array(ALONE[kind][0], float), np.array(ALONE[kind][1], np.int32)
+    E = np.unique(np.sort(np.concatenate([F[:, [0, 1]], F[:, [1, 2]], F[:, [2, 0]]]), axis=1),
+                  axis=0).astype(np.int32)
+    ctx.upload_mesh(V, E, F)
+    ctx.upload_positions(0, V)
+    ctx.build_collisions(DHAT)
+    ee, fv = O.candidates(V, E, F, 0.5 * DHAT)
+    co = O.build_collisions(V, E, F, ee, fv, DHAT)
+    counts = dict(zip(("vv", "ev", "ee", "fv"), (int(x) for x in ctx.collision_counts())))
+    print("case", kind, counts, flush=True)
+    assert counts == {k: int(k == kind) for k in counts}
+    e = O.barrier_energy(co, V, E, F, DHAT, KAPPA)
+    assert abs(ctx.energy(DHAT, KAPPA) - e) <= 1e-12 * abs(e)
+    g = O.barrier_gradient(co, V, E, F, DHAT, KAPPA)
+    assert np.linalg.norm(ctx.gradient(DHAT, KAPPA).ravel() - g.ravel()) <= 1e-12 * np.linalg.norm(g)
+    assert sparse_rel_err(ctx.hessian(DHAT, KAPPA, "clamp"),
+                          O.barrier_hessian(co, V, E, F, DHAT, KAPPA, "clamp")) <= 1e-10
