@@ -837,6 +837,60 @@ __device__ __forceinline__ void row_add(double* acc, uint32_t* msk, const double
     if (mask) atomicOr(msk, mask);
 }
 
+// full matrices among a wave's 64 incidences from which each lane expands
+// its own: one after the other they take about 1.5 us a pair (two aligned
+// sheets have dozens a row: the rows of 64 such scenes 11.9 -> 9.3 ms)
+constexpr int ROW_FULL = 8;
+
+// A full matrix by one lane, one block row r at a time, so few values are
+// live at once (slots: the four points' columns, 255: none).
+__device__ __forceinline__ void row_add_full(const double* rec, const double* ext, int64_t ee0,
+                                             uint32_t id, uint32_t slots, double (*dacc)[9],
+                                             uint32_t* dmsk, double (*acc)[9], uint32_t* msk)
+{
+#pragma clang fp contract(fast)
+    const int64_t g = id >> 2;
+    const int a = (int)(id & 3u), l = lane_id();
+    const double* hr = rec + (int64_t)REC_LEN * g;
+    const double* he = ext + (int64_t)REC_EXT * (g - ee0);
+    uint32_t mask[4] = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        double G[3][3]; // G[i][t] = sum_k q(a, k) H[3 k + r][3 i + t]
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                double x = 0;
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    const int e = sp(3 * k + r, 3 * i + t);
+                    x += QBasis<4>::q(a, k) * (e < FRAME_LEN ? hr[e] : he[e - FRAME_LEN]);
+                }
+                G[i][t] = x;
+            }
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const uint32_t slot = (slots >> (8 * b)) & 255u;
+            if (slot >= (uint32_t)RW) continue;
+            double* const to = b == a ? dacc[l % RD] : acc[slot];
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                double x = 0;
+#pragma unroll
+                for (int i = 0; i < 3; i++) x += QBasis<4>::q(b, i) * G[i][t];
+                if (x != 0) {
+                    atomicAdd(&to[3 * r + t], x);
+                    mask[b] |= 1u << (3 * r + t);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+        if (mask[b]) atomicOr(b == a ? &dmsk[l % RD] : &msk[(slots >> (8 * b)) & 255u], mask[b]);
+}
+
 // A wave per vertex.  Every lane of a gather touches lines of its own, so a
 // load costs a cycle per lane whatever its width: records are read once, 16
 // bytes at a time (14 loads; the full matrix read by blocks took 81).  All
@@ -944,6 +998,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                     | (uint32_t)(row_slot(cols[wv], vs.y) & 255) << 8
                     | (uint32_t)(row_slot(cols[wv], vs.z) & 255) << 16
                     | (uint32_t)(row_slot(cols[wv], vs.w) & 255) << 24;
+            }
+            if (__popcll(full) >= ROW_FULL) {
+                if (is_full) row_add_full(rec, ext, ee0, id, slots, dacc[wv], dmsk[wv], acc[wv], msk[wv]);
+                full = 0;
             }
             while (full) { // two at a time: both matrices' loads in flight
                 int e9 = l; // (opaque: not hoisted out of the loops, which would spill)
