@@ -6,12 +6,13 @@
 // formed in those variables (quotient rule on d = N / D with N, D low-degree
 // polynomials) and mapped into the n-1 dimensional subspace orthogonal to
 // rigid translations, spanned by an orthonormal basis Q of the stencil's
-// point space (Hadamard rows for 4 points, Helmert rows for 3, (1,-1)/sqrt2
-// for 2).  The energy Hessian H_x of a stencil satisfies H_x = Q B Q^T with
+// point space (Hadamard rows of 4 points).  The energy Hessian H_x of a
+// stencil satisfies H_x = Q B Q^T with
 // B = Q^T H_x Q (3(n-1) x 3(n-1)), and the translation directions are
 // exact null vectors, so PSD(H_x) = Q PSD(B) Q^T: the eigen-problem of the
 // reference's project_to_psd (eigen_ext.tpp:63-108) on 12x12 matrices is
-// solved here on 9x9 ones, in registers, with cyclic Jacobi.
+// solved here on 9x9 ones (mollified edge pairs) or, in the frame of the
+// closest points, on 5x5 ones (all others), in registers, with cyclic Jacobi.
 #pragma once
 
 #include "geometry.hpp"
@@ -176,21 +177,10 @@ IPCG_HD void triple_derivs(const d3& w, const d3& u, const d3& v, Red<3>& out)
 }
 
 // ---------------------------------------------------------------------------
-// Orthonormal translation-free bases Q (n points x K = n-1 columns)
+// Orthonormal translation-free basis Q (4 points x 3 columns; stencils of
+// fewer points give the others weight 0)
 // ---------------------------------------------------------------------------
 template <int NP> struct QBasis;
-template <> struct QBasis<2> {
-    static IPCG_HD double q(int x, int k) { return x == 0 ? M_SQRT1_2 : -M_SQRT1_2; }
-};
-template <> struct QBasis<3> {
-    static IPCG_HD double q(int x, int k)
-    {
-        // (1,-1,0)/sqrt2, (1,1,-2)/sqrt6
-        constexpr double r6 = 0.40824829046386301637; // 1/sqrt(6)
-        if (k == 0) return x == 0 ? M_SQRT1_2 : (x == 1 ? -M_SQRT1_2 : 0.0);
-        return x == 2 ? -2 * r6 : r6;
-    }
-};
 template <> struct QBasis<4> {
     static IPCG_HD double q(int x, int k)
     {

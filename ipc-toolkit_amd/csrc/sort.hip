@@ -350,7 +350,6 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_rle(const uint64_t* keys, int64_
 
 // ---------------------------------------------------------------------------
 constexpr int RS_BLOCK = 256;
-constexpr int RS_WAVES = RS_BLOCK / WAVE;
 constexpr int RS_CHUNKS = 8; // 64-key chunks per wave
 constexpr int RS_TILE = RS_BLOCK * RS_CHUNKS;
 constexpr int BIG_BLOCK = 512;
