@@ -474,8 +474,8 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
  * includes the origin), "ccd.spilled" (searches that outgrew the LDS
  * lists), "ccd.wavefront" (searches that outgrew a wave's lists too: a workgroup
  * or the level-by-level wavefront takes them),
- * "ccd.unmet" (1 when an expected minimum did not stand and the searches
- * ran again without it),
+ * "ccd.unmet" (scenes, at most 1 in a plain context, whose expected minimum
+ * did not stand and whose searches ran again without it),
  * "hessian.ee_other" (edge-edge collisions of the last Hessian under their
  * mollifier; their projection takes the 9 x 9 path),
  * "hessian.pattern_sorted" (1 when a row of the last Hessian pattern had

@@ -30,9 +30,11 @@
 // in an unbounded search and a few thousand below this one.  When no
 // outcome below it turns up, the bound is the minimum itself: the search it
 // came from ends at or before it, and not before it.  That holds for
-// first-stage outcomes; where a first stage ended below SMALL_TOI (the
-// search restarts and may end anywhere) and nothing below the expected
-// minimum was reported, everything is searched again without it.
+// first-stage outcomes: where a search that may have given its scene's bound
+// (one that outgrew a group's lists before) ended its first stage below
+// SMALL_TOI, it restarts and may end anywhere.  A scene with such a restart and
+// nothing below its expected minimum is searched again without it; the
+// other scenes of a batch keep their outcomes.
 // The running minimum lives in device memory as the bit pattern of a
 // non-negative double (unsigned atomic min); every search hides outcomes at
 // or above it, which leaves the final minimum independent of scheduling.
@@ -111,7 +113,8 @@ struct CCDArgs {
     bool bounded;          // hide outcomes >= running minimum
     double* bound;         // running minimum (double bits), one per scene
     double* expect;        // expected minimum, one per scene (null: none)
-    int* restarted;        // set when a search of the group tiers ends below SMALL_TOI
+    int* restarted;        // one per scene: a search handed on by a group tier restarted
+    const uint8_t* redo;   // one per scene (null: all): search these only (LDS tier)
     const int32_t* vscene; // batched contexts: scene per vertex (null: one scene)
     double* toi_out;       // per-candidate toi (null: not recorded)
     int* any_hit;          // early exit flag (null: no early exit)
@@ -130,6 +133,15 @@ __device__ __forceinline__ void report(const CCDArgs& A, int64_t ci, bool hit, d
         if (A.any_hit) atomicOr(A.any_hit, 1);
     }
     if (A.toi_out) A.toi_out[ci] = hit ? toi : INFINITY;
+}
+
+// the scene of a candidate (batched contexts), as candidate_setup reports it
+__device__ __forceinline__ int candidate_scene(const CCDArgs& A, int64_t ci)
+{
+    if (ci < A.n_ee) return A.vscene[A.E[2 * (int64_t)A.ee[ci].x]];
+    if ((ci -= A.n_ee) < A.n_fv) return A.vscene[A.fv[ci].y];
+    if ((ci -= A.n_fv) < A.n_vv) return A.vscene[A.vv[ci].x];
+    return A.vscene[A.ev[ci - A.n_vv].y];
 }
 
 // Strategy prologue (ccd_strategy + *_ccd of tight_inclusion_ccd.cpp):
@@ -301,6 +313,7 @@ __global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo,
     const TILdsLists L { lists + threadIdx.x, CB, LDS_CAP };
     const int64_t ci = todo[k];
     if (ci < ci_lo || ci >= ci_hi) return;
+    if (A.redo && !A.redo[candidate_scene(A, ci)]) return;
     TIQuery q;
     double eff = 0, adj = 0, toi = INFINITY;
     int sc = 0;
@@ -346,6 +359,7 @@ struct Searches {
     const unsigned long long* n_before;
     unsigned skip;
     unsigned long long* work; // next search to take
+    bool cut;                 // searches that outgrew a group's lists before
 };
 
 struct Lists {
@@ -497,7 +511,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_ccd_group(CCDArgs A, Searches Q_i
             }
         }
         if (!first) continue;
-        if (T.tries) atomicOr(A.restarted, 1);
+        if (T.tries && Q_in.cut) atomicOr(A.restarted + sc, 1);
         if (cut) {
             if (r == TI_HIT && toi >= SMALL_TOI) atomic_min_nonneg(expect, toi);
             if (r != TI_DEEP) r = TI_OVERFLOW;
@@ -691,7 +705,7 @@ __device__ void wf_search_done(const CCDArgs& A, WFState& S, bool hit, double to
 {
     if (S.stage == 1) {
         if (hit && toi < SMALL_TOI) {
-            atomicOr(A.restarted, 1);
+            atomicOr(A.restarted + S.scene, 1);
             S.stage = 2;
             S.nz_iter = 0;
             wf_begin_query(S, A.min_distance, S.adj, -1);
@@ -1012,10 +1026,10 @@ bool wf_batch(Ctx& c, const CCDArgs& A, const uint32_t* heavy, int64_t first, in
 
 // counters of one search over all tiers
 __global__ void k_ccd_begin(unsigned long long* cnt, int n, int at_todo, unsigned long long n_todo,
-                            int* restarted)
+                            int* restarted, int n_scenes)
 {
     for (int i = threadIdx.x; i < n; i += blockDim.x) cnt[i] = i == at_todo ? n_todo : 0ull;
-    if (threadIdx.x == 0) *restarted = 0;
+    for (int i = threadIdx.x; i < n_scenes; i += blockDim.x) restarted[i] = 0;
 }
 
 __global__ void k_fill_f64(double* p, int n, double v)
@@ -1059,10 +1073,16 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
            WORK_SUB_A, WORK_SUB_B, WORK_A, WORK_B, WORK_WIDE, WORK_BLOCK, N_SLAB, N_TODO, N_CNT };
     static_assert(512 + 8 * N_CNT <= ST_BYTES, "status block");
     IPCG_HIP(hipMemsetAsync(st, 0, ST_BYTES, s));
-    if (c.batched()) { // one running minimum (then one expected minimum) per scene
-        c.ccd_sbound.reserve(sizeof(double) * 2 * (size_t)nsc);
+    // batched contexts: running minimums, expected minimums, restart flags
+    // and redo marks of all scenes
+    const size_t scene_bytes = (2 * sizeof(double) + sizeof(int)) * (size_t)nsc; // (read back)
+    uint8_t* redo = nullptr;
+    if (c.batched()) {
+        c.ccd_sbound.reserve(scene_bytes + (size_t)nsc);
         bound = c.ccd_sbound.as<double>();
         expect = bound + nsc;
+        restarted = reinterpret_cast<int*>(expect + nsc);
+        redo = reinterpret_cast<uint8_t*>(restarted + nsc);
     }
     hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(nsc, 256)), dim3(256), 0, s, bound, nsc, 1.0);
     hipLaunchKernelGGL(k_fill_f64, dim3(grid_for(nsc, 256)), dim3(256), 0, s, expect, nsc,
@@ -1092,6 +1112,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     A.bound = bound;
     A.expect = nullptr;
     A.restarted = restarted;
+    A.redo = nullptr;
     A.vscene = c.batched() ? c.vscene.as<int32_t>() : nullptr;
     A.toi_out = per_cand ? c.ccd_toi.as<double>() : nullptr;
     A.any_hit = early_exit ? any_hit : nullptr;
@@ -1130,21 +1151,25 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     uint32_t* const wide = over + n_todo;
     uint32_t* const heavy = wide + n_todo;
     uint32_t* const sub = heavy + n_todo;
-    std::vector<double> scene_bound((size_t)(2 * nsc), 0.0); // running, then expected minimums
-    auto read_back = [&]() { // the scalars in h, the scenes' minimums in scene_bound
+    // running minimums, expected minimums, restart flags of the scenes
+    std::vector<char> scene_out(scene_bytes, 0);
+    const double* const run = reinterpret_cast<const double*>(scene_out.data());
+    const double* const expected = run + nsc;
+    const int* const restarts = reinterpret_cast<const int*>(expected + nsc);
+    auto read_back = [&]() { // the scalars in h, the scenes' values in scene_out
         IPCG_HIP(hipMemcpyAsync(h, st, ST_BYTES, hipMemcpyDeviceToHost, s));
-        double* hb = reinterpret_cast<double*>(h) + ST_BYTES / sizeof(double);
-        const size_t nb = sizeof(double) * 2 * (size_t)nsc;
-        const bool pin = ST_BYTES + nb <= PINNED_BYTES;
+        char* const hb = reinterpret_cast<char*>(h);
+        const bool pin = ST_BYTES + scene_bytes <= PINNED_BYTES;
         if (c.batched())
-            IPCG_HIP(hipMemcpyAsync(pin ? hb : scene_bound.data(), bound, nb,
+            IPCG_HIP(hipMemcpyAsync(pin ? hb + ST_BYTES : scene_out.data(), bound, scene_bytes,
                                     hipMemcpyDeviceToHost, s));
         IPCG_HIP(hipStreamSynchronize(s));
         if (!c.batched()) {
-            scene_bound[0] = *reinterpret_cast<const double*>(h);
-            scene_bound[1] = *reinterpret_cast<const double*>(reinterpret_cast<char*>(h) + 64);
+            std::memcpy(scene_out.data(), hb, sizeof(double));
+            std::memcpy(scene_out.data() + sizeof(double), hb + 64, sizeof(double));
+            std::memcpy(scene_out.data() + 2 * sizeof(double), hb + 224, sizeof(int));
         } else if (pin) {
-            std::copy(hb, hb + 2 * nsc, scene_bound.begin());
+            std::memcpy(scene_out.data(), hb + ST_BYTES, scene_bytes);
         }
     };
     auto count = [&](int k) { return (int64_t)h[512 / 8 + k]; };
@@ -1165,7 +1190,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                            dim3((unsigned)std::min<int64_t>((n_todo + PER_WAVE - 1) / PER_WAVE,
                                                             WAVE_GROUPS)),
                            dim3(WAVE), 0, s, A,
-                           Searches { list, cnt + n_list, nullptr, nullptr, SUB_MIN, cnt + work },
+                           Searches { list, cnt + n_list, nullptr, nullptr, SUB_MIN, cnt + work,
+                                      false },
                            out(sub, n_sub));
         IPCG_CHECK_LAUNCH();
         c.stage_end();
@@ -1185,7 +1211,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                            dim3((unsigned)std::min<int64_t>(n_todo, WIDE_GROUPS)), dim3(WAVE), 0,
                            s, A,
                            Searches { over, cnt + N_OVER, nullptr, nullptr, WIDE_MIN,
-                                      cnt + WORK_WIDE },
+                                      cnt + WORK_WIDE, true },
                            out(wide, N_WIDE), none);
         IPCG_CHECK_LAUNCH();
         c.stage_end();
@@ -1197,7 +1223,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                            dim3((unsigned)std::min<int64_t>(n_todo, BLOCK_GROUPS)),
                            dim3(BLOCK_NW * WAVE), 0, s, A,
                            Searches { wide, cnt + N_WIDE, over, cnt + N_OVER, WIDE_MIN,
-                                      cnt + WORK_BLOCK },
+                                     cnt + WORK_BLOCK, true },
                            out(heavy, N_HEAVY),
                            TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB, SLABS,
                                      SLAB_CAP });
@@ -1243,7 +1269,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     // Every surviving candidate through the tiers.
     auto search = [&]() {
         hipLaunchKernelGGL(k_ccd_begin, dim3(1), dim3(WAVE), 0, s, cnt, (int)N_CNT, (int)N_TODO,
-                           (unsigned long long)n_todo, restarted);
+                           (unsigned long long)n_todo, restarted, nsc);
         IPCG_CHECK_LAUNCH();
         if (A.bounded) {
             // Face-vertex and codim candidates first: their roots are isolated
@@ -1254,19 +1280,19 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
             if (A.expect && n_todo <= DIRECT_MAX) {
                 // few searches: every one has a wave of its own at once
                 wave_tier({ c.ccd_todo.as<uint32_t>(), cnt + N_TODO, nullptr, nullptr, 0,
-                            cnt + WORK_A });
+                            cnt + WORK_A, false });
             } else {
                 if (c.n_ee < n) {
                     lds_tier(c.n_ee, n, spill_a, N_SPILL_A);
                     sub_tier(spill_a, N_SPILL_A, WORK_SUB_A, N_SUB_A);
                     wave_tier({ sub, cnt + N_SUB_A, spill_a, cnt + N_SPILL_A, SUB_MIN,
-                                cnt + WORK_A });
+                                cnt + WORK_A, false });
                 }
                 if (c.n_ee > 0) {
                     lds_tier(0, c.n_ee, spill_b, N_SPILL_B);
                     sub_tier(spill_b, N_SPILL_B, WORK_SUB_B, N_SUB_B);
                     wave_tier({ sub, cnt + N_SUB_B, spill_b, cnt + N_SPILL_B, SUB_MIN,
-                                cnt + WORK_B });
+                                cnt + WORK_B, false });
                 }
             }
             wide_tier();
@@ -1275,7 +1301,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         } else {
             lds_tier(0, n, spill_a, N_SPILL_A);
             sub_tier(spill_a, N_SPILL_A, WORK_SUB_A, N_SUB_A);
-            wave_tier({ sub, cnt + N_SUB_A, spill_a, cnt + N_SPILL_A, SUB_MIN, cnt + WORK_A });
+            wave_tier({ sub, cnt + N_SUB_A, spill_a, cnt + N_SPILL_A, SUB_MIN, cnt + WORK_A,
+                        false });
             wide_tier();
             read_back();
             // without a bound most of what is left grows past a workgroup's
@@ -1300,32 +1327,43 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     c.stat["ccd.spilled"] = 0;
     c.stat["ccd.spilled_deep"] = 0;
     bool hit = false; // an expected minimum stood
+    auto any_reported = [&]() {
+        return *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + 192) != 0;
+    };
+    std::vector<double> step((size_t)nsc, 1.0); // per scene
     if (n_todo == 0) {
         read_back(); // the root pass may have reported hits
+        std::copy(run, run + nsc, step.begin());
     } else {
         // With a low iteration limit the outcome of a search depends on how
         // many boxes its bound hides: those keep to the running minimum.
         const bool expecting = A.bounded && (max_iter <= 0 || max_iter >= EXPECT_MIN_ITER);
         A.expect = expecting ? expect : nullptr;
         search();
-        auto flag = [&](size_t at) {
-            return *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + at) != 0;
-        };
+        std::copy(run, run + nsc, step.begin());
+        std::vector<uint8_t> again; // scenes whose expected minimum may not stand
         if (expecting) {
-            bool met = true;
             for (int k = 0; k < nsc; k++) {
-                if (scene_bound[k] < scene_bound[nsc + k]) continue;
-                if (std::isinf(scene_bound[nsc + k])) continue;
-                if (flag(224)) met = false; // restarted
-                scene_bound[k] = scene_bound[nsc + k];
-                hit = true;
+                if (run[k] < expected[k] || std::isinf(expected[k])) continue;
+                if (restarts[k]) {
+                    again.resize((size_t)nsc, 0);
+                    again[k] = 1;
+                } else {
+                    step[k] = expected[k];
+                    hit = true;
+                }
             }
-            if (!met && !(early_exit && flag(192))) {
-                A.expect = nullptr;
-                hit = false;
-                c.stat["ccd.unmet"]++;
-                search();
+        }
+        if (!again.empty() && !(early_exit && (hit || any_reported()))) {
+            c.stat["ccd.unmet"] = std::count(again.begin(), again.end(), (uint8_t)1);
+            A.expect = nullptr;
+            if (c.batched()) {
+                IPCG_HIP(hipMemcpyAsync(redo, again.data(), (size_t)nsc, hipMemcpyHostToDevice, s));
+                A.redo = redo;
             }
+            search();
+            for (int k = 0; k < nsc; k++)
+                if (again[k]) step[k] = run[k];
         }
     }
     if (per_cand) { // toi_out: ee, fv, vv, ev (any null)
@@ -1340,12 +1378,9 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         IPCG_HIP(hipStreamSynchronize(s));
         return 1.0;
     }
-    if (early_exit) {
-        hit = hit || *reinterpret_cast<const int*>(reinterpret_cast<const char*>(h) + 192) != 0;
-        return hit ? 0.0 : 1.0;
-    }
-    if (scene_steps) std::copy(scene_bound.begin(), scene_bound.begin() + nsc, scene_steps);
-    return *std::min_element(scene_bound.begin(), scene_bound.begin() + nsc);
+    if (early_exit) return hit || any_reported() ? 0.0 : 1.0;
+    if (scene_steps) std::copy(step.begin(), step.end(), scene_steps);
+    return *std::min_element(step.begin(), step.end());
 }
 
 } // namespace ipcg
