@@ -474,6 +474,9 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
  * includes the origin), "ccd.spilled" (searches that outgrew the LDS
  * lists), "ccd.wavefront" (searches that outgrew a wave's lists too: a workgroup
  * or the level-by-level wavefront takes them),
+ * "ccd.expected" (scenes, at most 1 in a plain context, for which a search cut
+ * to its earliest boxes gave an expected minimum; iteration limits below the
+ * default search without one),
  * "ccd.unmet" (scenes, at most 1 in a plain context, whose expected minimum
  * did not stand and whose searches ran again without it),
  * "hessian.ee_other" (edge-edge collisions of the last Hessian under their

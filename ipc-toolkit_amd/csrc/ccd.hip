@@ -82,7 +82,13 @@ constexpr int64_t DIRECT_MAX = 4096; // searches: no LDS tier (1,021: 0.87 -> 0.
 constexpr unsigned SUB_MIN = 3072;   // past the LDS lists: no sub-wave tier (884: 0.38 ms saved)
 constexpr unsigned WIDE_MIN = 256;   // past the wave lists: no wide tier
 constexpr int64_t BLOCK_MAX = 4096;   // (unbounded searches only) likewise
-constexpr int64_t EXPECT_MIN_ITER = 1000000; // iteration limit from which a minimum is expected
+// Iteration limit from which a minimum is expected: the library's default.  A
+// search that meets its limit ends early, so the step then lies anywhere
+// between the smallest outcome of the searches alone and the step without a
+// limit, nearer the latter the more boxes a bound hides.  A caller who lowers the
+// limit keeps the bound of finished searches alone (two aligned 10 x 10
+// sheets: a million boxes are met, ten million on none of the scenes tried).
+constexpr int64_t EXPECT_MIN_ITER = 10000000;
 // Wavefront batches: searches advanced together (one round of launches and
 // one host check per level for the whole batch), from WF_BATCH, doubled
 // after every batch that fits the box budget up to WF_BATCH_MAX.  Workloads
@@ -1322,6 +1328,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         const int64_t nh = count(N_HEAVY);
         if (nh > 0) wavefront(nh);
     };
+    c.stat["ccd.expected"] = 0;
     c.stat["ccd.unmet"] = 0;
     c.stat["ccd.wavefront"] = 0;
     c.stat["ccd.spilled"] = 0;
@@ -1335,14 +1342,14 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         read_back(); // the root pass may have reported hits
         std::copy(run, run + nsc, step.begin());
     } else {
-        // With a low iteration limit the outcome of a search depends on how
-        // many boxes its bound hides: those keep to the running minimum.
         const bool expecting = A.bounded && (max_iter <= 0 || max_iter >= EXPECT_MIN_ITER);
         A.expect = expecting ? expect : nullptr;
         search();
         std::copy(run, run + nsc, step.begin());
         std::vector<uint8_t> again; // scenes whose expected minimum may not stand
         if (expecting) {
+            c.stat["ccd.expected"] =
+                std::count_if(expected, expected + nsc, [](double e) { return !std::isinf(e); });
             for (int k = 0; k < nsc; k++) {
                 if (run[k] < expected[k] || std::isinf(expected[k])) continue;
                 if (restarts[k]) {

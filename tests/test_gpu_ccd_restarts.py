@@ -1,4 +1,5 @@
-"""Expected minimums that do not stand.  Two edges in near contact, their
+"""Expected minimums: where they do not stand, and the iteration limits that
+search without one.  Two edges in near contact, their
 coordinates large against the gap: the first search ends at time 0 (the
 rounding filter fills the gap) and starts again from the minimum distance.
 CUT: the search outgrows a wave's lists on the way, so its earliest boxes
@@ -108,3 +109,22 @@ def test_only_its_scenes_are_searched_again(ctx, O, scenes, big):
     parts = [make(scenes, "sheets:8:3"), pair(scenes, CUT["tenth"]), make(scenes, "twisted:8:0"),
              pair(scenes, CUT["free"])] + [make(scenes, "sheets:40:1")] * big
     assert batched(ctx, O, scenes, parts) == 2
+
+
+@pytest.mark.parametrize("limit", [20_000, 999_999, 1_000_000, 9_999_999, 10_000_000, -1])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_step_at_iteration_limits(ctx, O, scenes, seed, limit):
+    """A minimum is expected from the default limit on.  A bound can only keep
+    searches from meeting the limit, so the step lies between the smallest
+    outcome of the searches alone and the step without a limit."""
+    s = scenes.two_sheets(10, seed=seed)
+    say("case limit", seed, limit)
+    upload(ctx, s)
+    t = ctx.stepsize(max_iterations=limit)
+    assert ctx.counter("ccd.expected") == int(limit < 0 or limit >= 10_000_000)
+    alone, free = (O.compute_collision_free_stepsize(s.V, s.V1, s.E, s.F,
+                                                     params=O.CCDParams(1e-6, n, 0.8))
+                   for n in (limit if limit > 0 else 10_000_000, 10_000_000))
+    assert alone <= t <= free
+    if limit < 0 or limit >= 10_000_000:
+        assert t == free
