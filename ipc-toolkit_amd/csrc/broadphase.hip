@@ -673,7 +673,9 @@ struct TraverseArgs {
     const int32_t* qmap;
     int2* out;
     Shards S;
-    int* deep; // TR_STACK - TR_LSTACK ints per lane of the launch
+    int* deep; // pool of `slots` spill stacks, TR_STACK - TR_LSTACK ints each
+    unsigned* claimed;
+    unsigned slots;
     int* status;
     ForestArgs fa;
     int qw; // queries a wave starts with (its first lanes; the others share)
@@ -696,8 +698,9 @@ __device__ __forceinline__ void wave_fence()
 
 // The walk of one workgroup's queries (block: its index in the query set's
 // launch range).  stack: postponed right children, the first TR_LSTACK
-// entries of each lane in LDS (small enough for full occupancy), deeper ones
-// in the lane's own HBM slots.
+// entries of each lane in LDS (small enough for full occupancy); a lane that
+// goes deeper claims a spill stack in HBM and keeps it.  (A spill stack per
+// lane is 12 KB per wave: with 8 queries a wave, 1.5 KB per query.)
 template <int MODE, int BLOCK>
 __device__ __forceinline__ void traverse(const TraverseArgs& A, unsigned block,
                                          TrShared<BLOCK>& sh_mem)
@@ -722,7 +725,7 @@ __device__ __forceinline__ void traverse(const TraverseArgs& A, unsigned block,
     const bool has_query = t % WAVE < A.qw && q0 < nq;
     const int qpos = has_query ? (int)q0 : 0;
     bool active = has_query;
-    int* const deep = A.deep + ((int64_t)block * BLOCK + t) * (TR_STACK - TR_LSTACK) - TR_LSTACK;
+    int* deep = nullptr; // its entry TR_LSTACK is the spill stack's first
     float q[6] = { 0, 0, 0, 0, 0, 0 };
     Query qr { 0, { -1, -1, -1 } };
     if (active) {
@@ -916,8 +919,18 @@ __device__ __forceinline__ void traverse(const TraverseArgs& A, unsigned block,
                 if (t0 && t1) {
                     if (sp < TR_LSTACK) stack[sp++][t] = nd.c1;
                     else if (sp < TR_STACK) {
-                        deep[sp] = nd.c1;
-                        sp++;
+                        if (!deep) {
+                            const unsigned k = atomicAdd(A.claimed, 1u);
+                            if (k < A.slots)
+                                deep = A.deep + (int64_t)k * (TR_STACK - TR_LSTACK) - TR_LSTACK;
+                        }
+                        if (deep) {
+                            deep[sp] = nd.c1;
+                            sp++;
+                        } else { // the host walks again with a larger pool
+                            atomicOr(status, 4);
+                            active = false;
+                        }
                     } else {
                         atomicOr(status, 1);
                         active = false;
@@ -963,11 +976,36 @@ unsigned traverse_blocks(int64_t nq, int qw, int block)
     return grid_for(nq, block / WAVE * qw);
 }
 
-// HBM stack ints of a walk of nq queries (its largest workgroup size)
-int64_t deep_ints(int64_t nq, int qw)
+// lanes of a walk of nq queries (its largest workgroup size)
+int64_t walk_lanes(int64_t nq, int qw) { return ((nq + qw - 1) / qw + 4) * WAVE; }
+
+// The pool of spill stacks: SLOTS_MIN of them (no sheet stack, sphere row or batch of
+// the benchmarks needs one), then as many as a walk has needed
+// (grown by 4 when one finds it empty, at most a stack per lane).
+constexpr int64_t SLOTS_MIN = 1024;
+constexpr size_t SLOT_BYTES = sizeof(int) * (TR_STACK - TR_LSTACK);
+
+unsigned reserve_slots(Ctx& c, int64_t lanes)
 {
-    return ((nq + qw - 1) / qw + 4) * WAVE * (TR_STACK - TR_LSTACK);
+    const int64_t n = std::min(std::max(c.tr_slots, SLOTS_MIN), lanes);
+    c.tr_deep.reserve(SLOT_BYTES * (size_t)n);
+    return (unsigned)n;
 }
+
+// after a walk: whether it has to run again with a larger pool
+bool slots_short(Ctx& c, int status, unsigned slots, int64_t lanes)
+{
+    if (!(status & 4)) return false;
+    if (slots >= lanes) throw Error(IPCG_ERR_NUMERIC, "LBVH spill stacks ran out");
+    c.tr_slots = std::min<int64_t>(4 * (int64_t)slots, lanes);
+    return true;
+}
+
+// the walks' status word, then the number of spill stacks claimed
+struct WalkStatus {
+    int status;
+    unsigned claimed;
+};
 
 // A walk of few queries leaves most of the chip idle and takes the time of
 // its longest wave: its waves start with part of their lanes busy, and the
@@ -998,7 +1036,8 @@ constexpr int TUNE_BLOCKS[3] = { 64, 128, 256 };
 // counters) and the fastest, by HIP events on the context stream, is kept.
 // Candidate sets do not depend on the size.
 template <class Launch>
-void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, Launch&& launch)
+void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, unsigned* claimed,
+                    Launch&& launch)
 {
     hipStream_t s = c.stream;
     auto it = c.launch_block.find(stage);
@@ -1010,6 +1049,7 @@ void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, L
         float best = INFINITY;
         for (int b : TUNE_BLOCKS) {
             IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES, s));
+            IPCG_HIP(hipMemsetAsync(claimed, 0, sizeof(unsigned), s));
             IPCG_HIP(hipEventRecord(e0, s));
             launch(b);
             IPCG_HIP(hipEventRecord(e1, s));
@@ -1026,6 +1066,7 @@ void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, L
         (void)hipEventDestroy(e1);
         c.launch_block[stage] = block;
         IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES, s));
+        IPCG_HIP(hipMemsetAsync(claimed, 0, sizeof(unsigned), s));
     }
     launch(block ? block : TR_BLOCK);
 }
@@ -1454,8 +1495,10 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
     c.counters.reserve(sizeof(unsigned long long) * 4);
     Filter flt { c.E.as<int32_t>(), c.F.as<int32_t>(), c.has_patch ? c.patch.as<int32_t>() : nullptr,
                  c.n_dynamic, c.n_codim_filter };
-    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(unsigned long long));
-    int* status = reinterpret_cast<int*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
+    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(WalkStatus));
+    WalkStatus* const ws = reinterpret_cast<WalkStatus*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
+    int* const status = &ws->status;
+    unsigned* const claimed = &ws->claimed;
     c.shard_off.reserve(sizeof(int64_t) * 4 * (SHARDS + 1));
     unsigned long long* cnt[4];
     for (int k = 0; k < 4; k++) cnt[k] = c.shard_cnt.as<unsigned long long>() + k * SHARDS * SHARD_PAD;
@@ -1467,19 +1510,18 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
     const int lists = codim ? 4 : 2;
     // one launch for both walks, unless the launch shapes are being tuned
     const bool both = !c.autotune && c.nE >= 2 && c.nF >= 1;
-    // deep traversal stack entries: per query of the largest query set, or
-    // of both sets when they walk at once
     const int qw = wave_queries((int64_t)c.nE + c.nV);
-    const int64_t deep_ee = deep_ints(c.nE, qw), deep_fv = deep_ints(c.nV, qw);
-    c.tr_deep.reserve(sizeof(int) * (size_t)(both ? deep_ee + deep_fv : std::max(deep_ee, deep_fv)));
-    int* deep = c.tr_deep.as<int>();
-    for (int attempt = 0; attempt < 3; attempt++) {
+    const int64_t lanes = walk_lanes(c.nE, qw) + walk_lanes(c.nV, qw)
+        + (codim ? 2 * walk_lanes(c.n_cv, qw) : 0);
+    for (int attempt = 0; attempt < 3;) {
+        const unsigned slots = reserve_slots(c, lanes);
+        int* const deep = c.tr_deep.as<int>();
         // per-shard regions; their sum bounds a list until a retry grows it
         for (int k = 0; k < lists; k++) {
             if (*scap[k] == 0) *scap[k] = std::max<int64_t>(1024, guess[k] / SHARDS);
             c.cand_stage[k].reserve(sizeof(int2) * (size_t)(SHARDS * *scap[k]));
         }
-        IPCG_HIP(hipMemsetAsync(c.shard_cnt.p, 0, 4 * SHARD_CNT_BYTES + sizeof(int), s));
+        IPCG_HIP(hipMemsetAsync(c.shard_cnt.p, 0, 4 * SHARD_CNT_BYTES + sizeof(WalkStatus), s));
         const Shards S0 { cnt[0], c.scap_ee }, S1 { cnt[1], c.scap_fv };
         if (sap) {
             c.stage_begin("bp_sweep");
@@ -1505,13 +1547,14 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
             const TraverseArgs ee { c.te.box.as<float>(), c.te.ids.as<uint32_t>(), c.nE,
                                     c.te.nodes.as<Node>(), c.te.root.as<int32_t>(),
                                     c.te.leaf.as<int4>(), c.te.box.as<float>(), c.nE, flt,
-                                    nullptr, c.cand_stage[0].as<int2>(), S0, deep, status,
+                                    nullptr, c.cand_stage[0].as<int2>(), S0, deep, claimed,
+                                    slots, status,
                                     forest_args(c, c.te), qw };
             const TraverseArgs fv { c.tv.box.as<float>(), c.tv.ids.as<uint32_t>(), c.nV,
                                     c.tf.nodes.as<Node>(), c.tf.root.as<int32_t>(),
                                     c.tf.leaf.as<int4>(), c.tf.box.as<float>(), c.nF, flt,
-                                    nullptr, c.cand_stage[1].as<int2>(), S1,
-                                    both ? deep + deep_ee : deep, status,
+                                    nullptr, c.cand_stage[1].as<int2>(), S1, deep, claimed,
+                                    slots, status,
                                     forest_args(c, c.tf), qw };
             if (both) {
                 const unsigned nb_ee = traverse_blocks(c.nE, qw, TR_BLOCK),
@@ -1527,7 +1570,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
             } else {
                 if (c.nE >= 2) {
                     c.stage_begin("bp_traverse_ee");
-                    tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], [&](int b) {
+                    tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], claimed, [&](int b) {
                         if (swept) launch_traverse<TR_EE, 1>(b, ee, s);
                         else launch_traverse<TR_EE, 0>(b, ee, s);
                     });
@@ -1535,7 +1578,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                 }
                 if (c.nF >= 1) {
                     c.stage_begin("bp_traverse_fv");
-                    tuned_traverse(c, "bp_traverse_fv" + tag, cnt[1], [&](int b) {
+                    tuned_traverse(c, "bp_traverse_fv" + tag, cnt[1], claimed, [&](int b) {
                         if (swept) launch_traverse<TR_FV, 1>(b, fv, s);
                         else launch_traverse<TR_FV, 0>(b, fv, s);
                     });
@@ -1551,7 +1594,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                                        c.tcv.nodes.as<Node>(), c.tcv.root.as<int32_t>(),
                                        c.tcv.leaf.as<int4>(), c.tcv.box.as<float>(), c.n_cv, flt,
                                        c.cv.as<int32_t>(), c.cand_stage[2].as<int2>(), S2, deep,
-                                       status, forest_args(c, c.tcv), qw };
+                                       claimed, slots, status, forest_args(c, c.tcv), qw };
                 if (swept) launch_traverse<TR_VV, 1>(TR_BLOCK, a, s);
                 else launch_traverse<TR_VV, 0>(TR_BLOCK, a, s);
             }
@@ -1560,7 +1603,7 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                                        c.tce.nodes.as<Node>(), c.tce.root.as<int32_t>(),
                                        c.tce.leaf.as<int4>(), c.tce.box.as<float>(), c.n_ce, flt,
                                        c.cv.as<int32_t>(), c.cand_stage[3].as<int2>(), S3, deep,
-                                       status, forest_args(c, c.tce), qw };
+                                       claimed, slots, status, forest_args(c, c.tce), qw };
                 if (swept) launch_traverse<TR_EV, 1>(TR_BLOCK, a, s);
                 else launch_traverse<TR_EV, 0>(TR_BLOCK, a, s);
             }
@@ -1569,12 +1612,16 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
         IPCG_CHECK_LAUNCH();
         // the lists' counts and the walk status in one read-back
         ShardCounts kc[4];
-        int st = 0;
+        WalkStatus walk {};
         c.shard_sum.reserve(256);
         shard_counts_n(cnt[0], lists, c.shard_sum.as<unsigned long long>(),
-                       c.shard_off.as<int64_t>(), c.pinned, s, kc, status, &st);
+                       c.shard_off.as<int64_t>(), c.pinned, s, kc, ws, &walk);
+        const int st = walk.status;
         if (st & 2) throw Error(IPCG_ERR_NUMERIC, "LBVH build produced an invalid tree");
         if (st & 1) throw Error(IPCG_ERR_NUMERIC, "LBVH traversal stack overflow (depth > 64)");
+        c.stat["bp.spill_stacks"] = walk.claimed;
+        if (slots_short(c, st, slots, lanes)) continue;
+        attempt++;
         bool again = false;
         for (int k = 0; k < lists; k++) {
             if (kc[k].max > *scap[k]) {
@@ -1628,33 +1675,41 @@ void bp_edge_face(Ctx& c, double inflation)
     Filter flt { c.E.as<int32_t>(), c.F.as<int32_t>(), c.has_patch ? c.patch.as<int32_t>() : nullptr,
                  c.n_dynamic, c.n_codim_filter };
     c.counters.reserve(sizeof(unsigned long long) * 4);
-    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(unsigned long long));
-    int* status = reinterpret_cast<int*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
+    c.shard_cnt.reserve(4 * SHARD_CNT_BYTES + sizeof(WalkStatus));
+    WalkStatus* const ws = reinterpret_cast<WalkStatus*>(c.shard_cnt.as<char>() + 4 * SHARD_CNT_BYTES);
+    int* const status = &ws->status;
+    unsigned* const claimed = &ws->claimed;
     c.shard_off.reserve(sizeof(int64_t) * 4 * (SHARDS + 1));
     unsigned long long* cnt = c.shard_cnt.as<unsigned long long>();
     const int qw = wave_queries(c.nE);
-    c.tr_deep.reserve(sizeof(int) * (size_t)deep_ints(c.nE, qw));
-    for (int attempt = 0; attempt < 3; attempt++) {
+    const int64_t lanes = walk_lanes(c.nE, qw);
+    for (int attempt = 0; attempt < 3;) {
+        const unsigned slots = reserve_slots(c, lanes);
         if (c.scap_ef == 0) c.scap_ef = std::max<int64_t>(1024, 8 * (int64_t)c.nE / SHARDS);
         c.cand_stage[0].reserve(sizeof(int2) * (size_t)(SHARDS * c.scap_ef));
         IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES, s));
-        IPCG_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
+        IPCG_HIP(hipMemsetAsync(ws, 0, sizeof(WalkStatus), s));
         const Shards S0 { cnt, c.scap_ef };
         c.stage_begin("bp_traverse_ef");
         const TraverseArgs a { c.te.box.as<float>(), c.te.ids.as<uint32_t>(), c.nE,
                                c.tf.nodes.as<Node>(), c.tf.root.as<int32_t>(), c.tf.leaf.as<int4>(),
                                c.tf.box.as<float>(), c.nF, flt, nullptr, c.cand_stage[0].as<int2>(),
-                               S0, c.tr_deep.as<int>(), status, forest_args(c, c.tf), qw };
+                               S0, c.tr_deep.as<int>(), claimed, slots, status,
+                               forest_args(c, c.tf), qw };
         launch_traverse<TR_EF, 0>(TR_BLOCK, a, s);
         IPCG_CHECK_LAUNCH();
         c.stage_end();
         ShardCounts kc;
-        int st = 0;
+        WalkStatus walk {};
         c.shard_sum.reserve(256);
         shard_counts_n(cnt, 1, c.shard_sum.as<unsigned long long>(), c.shard_off.as<int64_t>(),
-                       c.pinned, s, &kc, status, &st);
+                       c.pinned, s, &kc, ws, &walk);
+        const int st = walk.status;
         if (st & 2) throw Error(IPCG_ERR_NUMERIC, "LBVH build produced an invalid tree");
         if (st & 1) throw Error(IPCG_ERR_NUMERIC, "LBVH traversal stack overflow (depth > 64)");
+        c.stat["bp.spill_stacks"] = walk.claimed;
+        if (slots_short(c, st, slots, lanes)) continue;
+        attempt++;
         if (kc.max > c.scap_ef) {
             c.scap_ef = kc.max + kc.max / 4 + 1024;
             continue;

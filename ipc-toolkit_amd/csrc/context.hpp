@@ -111,7 +111,8 @@ struct Ctx {
     DevBuf isect;                      // intersection test: flag, deferred count, list
     int64_t scap_ee = 0, scap_fv = 0, scap_vv = 0, scap_ev = 0; // shard regions
     DevBuf cand_stage[4];              // sharded traversal output (ee, fv, vv, ev)
-    DevBuf tr_deep;                    // traversal stack entries beyond LDS
+    DevBuf tr_deep;                    // spill stacks of the walks, tr_slots of them (0: the least)
+    int64_t tr_slots = 0;
     DevBuf shard_sum;                  // per counter set: total, largest shard (u64)
     DevBuf shard_cnt, shard_off;       // shard counters / offsets of the append lists
 

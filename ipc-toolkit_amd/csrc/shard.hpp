@@ -51,13 +51,13 @@ struct ShardCounts {
 // (set k at cnt_dev + k * SHARDS * SHARD_PAD): one launch leaves the
 // exclusive offsets of each set's shards in off_dev (SHARDS + 1 int64 per
 // set) and reduces each set's total and largest shard into sum_dev (2 * nsets
-// u64, then *extra_dev), read back in one small copy with one synchronisation
-// of the stream.
+// u64, then the 8 bytes at extra_dev), read back in one small copy with one
+// synchronisation of the stream.
 ShardCounts shard_counts(const unsigned long long* cnt_dev, unsigned long long* sum_dev,
                          int64_t* off_dev, void* pinned, hipStream_t s);
 void shard_counts_n(const unsigned long long* cnt_dev, int nsets, unsigned long long* sum_dev,
                     int64_t* off_dev, void* pinned, hipStream_t s, ShardCounts* out,
-                    const int* extra_dev = nullptr, int* extra = nullptr);
+                    const void* extra_dev = nullptr, void* extra = nullptr);
 
 template <class T>
 __global__ __launch_bounds__(256) void k_shard_copy(const T* in, int64_t scap, const int64_t* off,

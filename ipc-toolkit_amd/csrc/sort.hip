@@ -29,6 +29,8 @@
 #include "shard.hpp"
 #include "sort.hpp"
 
+#include <cstring>
+
 namespace ipcg {
 
 namespace {
@@ -809,7 +811,8 @@ bool radix_sort_pairs(SortSpace& ws, uint32_t* keys, uint32_t* vals, uint32_t* k
 // one workgroup per counter set: the offsets of its shards, its total and its
 // largest shard count
 __global__ __launch_bounds__(SHARDS) void k_shard_summary(const unsigned long long* cnt,
-                                                          const int* extra, int64_t* off,
+                                                          const unsigned long long* extra,
+                                                          int64_t* off,
                                                           unsigned long long* out)
 {
     static_assert(SHARDS == SCAN_BLOCK, "block_exclusive_scan");
@@ -830,16 +833,16 @@ __global__ __launch_bounds__(SHARDS) void k_shard_summary(const unsigned long lo
         for (int w = 0; w < SHARDS / WAVE; w++) m = wmax[w] > m ? wmax[w] : m;
         out[2 * blockIdx.x] = total;
         out[2 * blockIdx.x + 1] = m;
-        if (blockIdx.x == 0) out[2 * gridDim.x] = extra ? (unsigned long long)(unsigned)*extra : 0ull;
+        if (blockIdx.x == 0) out[2 * gridDim.x] = extra ? *extra : 0ull;
     }
 }
 
 void shard_counts_n(const unsigned long long* cnt_dev, int nsets, unsigned long long* sum_dev,
                     int64_t* off_dev, void* pinned, hipStream_t s, ShardCounts* out,
-                    const int* extra_dev, int* extra)
+                    const void* extra_dev, void* extra)
 {
-    hipLaunchKernelGGL(k_shard_summary, dim3(nsets), dim3(SHARDS), 0, s, cnt_dev, extra_dev,
-                       off_dev, sum_dev);
+    hipLaunchKernelGGL(k_shard_summary, dim3(nsets), dim3(SHARDS), 0, s, cnt_dev,
+                       static_cast<const unsigned long long*>(extra_dev), off_dev, sum_dev);
     IPCG_CHECK_LAUNCH();
     unsigned long long* h = static_cast<unsigned long long*>(pinned);
     IPCG_HIP(hipMemcpyAsync(h, sum_dev, sizeof(unsigned long long) * (2 * nsets + 1),
@@ -849,7 +852,7 @@ void shard_counts_n(const unsigned long long* cnt_dev, int nsets, unsigned long 
         out[k].total = (int64_t)h[2 * k];
         out[k].max = (int64_t)h[2 * k + 1];
     }
-    if (extra) *extra = (int)h[2 * nsets];
+    if (extra) std::memcpy(extra, h + 2 * nsets, sizeof(*h));
 }
 
 ShardCounts shard_counts(const unsigned long long* cnt_dev, unsigned long long* sum_dev,

@@ -57,3 +57,28 @@ def test_walks_at_the_limits_of_the_starting_widths(ctx, O, scenes, n):
     finally:
         ctx.set_autotune(False)
     assert pair_set(ee) == pair_set(ee2) and pair_set(fv) == pair_set(fv2)
+
+
+def comb(spokes):
+    """Spokes from a corner hub, each spanning half the box, beside edges in
+    20 octaves towards the spokes' centres: a walk from a spoke postpones the
+    upper octave at each of 18 levels, more than a lane holds in LDS."""
+    rng = np.random.default_rng(spokes)
+    rim = 0.5 - 1e-6 * rng.uniform(0.1, 1, (spokes, 3))
+    c = (0.25 + 0.25 * 2.0 ** -np.arange(20)[:, None] * [1.0, 1.3]).ravel()
+    ends = c[:, None, None] + np.array([[-1e-9] * 3, [1e-9] * 3])
+    V = np.concatenate([[[0, 0, 0]], rim, ends.reshape(-1, 3), [[1, 1, 0.999], [1, 1, 1]]])
+    pairs = np.arange(spokes + 1, len(V)).reshape(-1, 2)
+    E = np.concatenate([np.stack([np.zeros(spokes), np.arange(1, spokes + 1)], 1), pairs])
+    return V, E.astype(np.int32), np.zeros((0, 3), np.int32)
+
+
+# spill stacks claimed from the first pool, and more of them than it has
+@pytest.mark.parametrize("spokes,least", [(40, 1), (12000, 1025)])
+def test_spill_stacks(ctx, O, spokes, least):
+    V, E, F = comb(spokes)
+    print("case", spokes, flush=True)
+    for _ in range(2):  # the second walk finds the pool at its size
+        ee, fv = check(ctx, O, V, E, F, 1e-12)
+        assert len(ee) >= 18 * 2 * spokes and len(fv) == 0
+        assert ctx.counter("bp.spill_stacks") >= least
