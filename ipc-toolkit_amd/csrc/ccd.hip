@@ -1076,7 +1076,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     unsigned long long* npend = reinterpret_cast<unsigned long long*>(st + 384); // [3]
     unsigned long long* cnt = reinterpret_cast<unsigned long long*>(st + 512);
     enum { N_SPILL_A, N_SPILL_A_DEEP, N_SPILL_B, N_SPILL_B_DEEP, N_SUB_A, N_SUB_B, N_OVER, N_WIDE, N_HEAVY,
-           WORK_SUB_A, WORK_SUB_B, WORK_A, WORK_B, WORK_WIDE, WORK_BLOCK, N_SLAB, N_TODO, N_CNT };
+           WORK_SUB_A, WORK_SUB_B, WORK_A, WORK_B, WORK_WIDE, WORK_BLOCK, N_SLAB, N_TODO,
+           N_LAST, WORK_LAST, N_CNT };
     static_assert(512 + 8 * N_CNT <= ST_BYTES, "status block");
     IPCG_HIP(hipMemsetAsync(st, 0, ST_BYTES, s));
     // batched contexts: running minimums, expected minimums, restart flags
@@ -1222,19 +1223,37 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         IPCG_CHECK_LAUNCH();
         c.stage_end();
     };
-    auto block_tier = [&]() {
+    // The lists past LDS are reserved (42 MB) when a search first asks for
+    // them: most contexts never get there.
+    constexpr size_t SLAB_BYTES = sizeof(unsigned long long) * 2 * SLAB_CAP * (size_t)SLABS;
+    auto block_tier = [&](const Searches& q, const Lists& to) {
         c.stage_begin("ccd_block");
-        c.ccd_slab.reserve(sizeof(unsigned long long) * 2 * SLAB_CAP * (size_t)SLABS);
         hipLaunchKernelGGL((k_ccd_group<BLOCK_NW, BLOCK_CAP>),
                            dim3((unsigned)std::min<int64_t>(n_todo, BLOCK_GROUPS)),
-                           dim3(BLOCK_NW * WAVE), 0, s, A,
-                           Searches { wide, cnt + N_WIDE, over, cnt + N_OVER, WIDE_MIN,
-                                     cnt + WORK_BLOCK, true },
-                           out(heavy, N_HEAVY),
-                           TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB, SLABS,
-                                     SLAB_CAP });
+                           dim3(BLOCK_NW * WAVE), 0, s, A, q, to,
+                           TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB,
+                                     c.ccd_slab.p ? SLABS : 0, SLAB_CAP });
         IPCG_CHECK_LAUNCH();
         c.stage_end();
+    };
+    // the workgroup tier, then a second time with slabs for the searches
+    // left over if one of them would have taken a slab; leaves the list for
+    // the wavefront in `last` (counts as read back)
+    uint32_t* last = heavy;
+    int n_last = N_HEAVY;
+    auto block_tiers = [&]() {
+        block_tier(Searches { wide, cnt + N_WIDE, over, cnt + N_OVER, WIDE_MIN, cnt + WORK_BLOCK,
+                              true },
+                   out(heavy, N_HEAVY));
+        read_back();
+        if (c.ccd_slab.p || count(N_SLAB) == 0 || count(N_HEAVY) == 0) return;
+        c.ccd_slab.reserve(SLAB_BYTES);
+        IPCG_HIP(hipMemsetAsync(cnt + N_SLAB, 0, sizeof(*cnt), s));
+        last = over; // (the workgroups have read it)
+        n_last = N_LAST;
+        block_tier(Searches { heavy, cnt + N_HEAVY, nullptr, nullptr, 0, cnt + WORK_LAST, true },
+                   Lists { last, cnt + N_LAST, last, cnt + N_LAST });
+        read_back();
     };
     // moves a tier's list to the wavefront's (counts as read back)
     auto to_heavy = [&](const uint32_t* list, int n_list) {
@@ -1243,7 +1262,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                                 hipMemcpyDeviceToDevice, s));
         h[512 / 8 + N_HEAVY] += (unsigned long long)m;
     };
-    auto wavefront = [&](int64_t nh) {
+    auto wavefront = [&](const uint32_t* list, int64_t nh) {
         c.stage_begin("ccd_wavefront");
         DevBuf& wst = c.ccd_bound; // per-candidate wavefront state
         wst.reserve(sizeof(WFState) * (size_t)std::min<int64_t>(nh, WF_BATCH_MAX));
@@ -1255,7 +1274,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         int64_t batch = std::min<int64_t>(WF_BATCH, nh);
         for (int64_t first = 0; first < nh;) {
             const int64_t nb = std::min<int64_t>(batch, nh - first);
-            const bool ok = wf_batch(c, A, heavy, first, nb, states, early_exit, any_hit, error,
+            const bool ok = wf_batch(c, A, list, first, nb, states, early_exit, any_hit, error,
                                      nroot, npend, h);
             if (!ok) {
                 if (nb == 1)
@@ -1277,6 +1296,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         hipLaunchKernelGGL(k_ccd_begin, dim3(1), dim3(WAVE), 0, s, cnt, (int)N_CNT, (int)N_TODO,
                            (unsigned long long)n_todo, restarted, nsc);
         IPCG_CHECK_LAUNCH();
+        last = heavy;
+        n_last = N_HEAVY;
         if (A.bounded) {
             // Face-vertex and codim candidates first: their roots are isolated
             // points, so they resolve fast and lower every scene's running and
@@ -1302,8 +1323,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
                 }
             }
             wide_tier();
-            block_tier();
-            read_back();
+            block_tiers();
         } else {
             lds_tier(0, n, spill_a, N_SPILL_A);
             sub_tier(spill_a, N_SPILL_A, WORK_SUB_A, N_SUB_A);
@@ -1318,18 +1338,23 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
             if (left > BLOCK_MAX) {
                 to_heavy(wide, N_WIDE);
             } else if (left > 0) {
-                block_tier();
-                read_back();
+                block_tiers();
             }
         }
         c.stat["ccd.spilled"] += count(N_SPILL_A) + count(N_SPILL_B);
         c.stat["ccd.spilled_deep"] += count(N_SPILL_A_DEEP) + count(N_SPILL_B_DEEP);
         c.stat["ccd.wavefront"] += count(N_OVER);
-        const int64_t nh = count(N_HEAVY);
-        if (nh > 0) wavefront(nh);
+        c.stat["ccd.past_sub"] += count(N_SUB_A) + count(N_SUB_B);
+        c.stat["ccd.past_wide"] += count(N_WIDE);
+        if (c.ccd_slab.p) c.stat["ccd.slabs"] += std::min<int64_t>(count(N_SLAB), SLABS);
+        const int64_t nh = count(n_last);
+        c.stat["ccd.by_level"] += nh;
+        if (nh > 0) wavefront(last, nh);
     };
     c.stat["ccd.expected"] = 0;
     c.stat["ccd.unmet"] = 0;
+    for (const char* k : { "past_sub", "past_wide", "slabs", "by_level" })
+        c.stat[std::string("ccd.") + k] = 0;
     c.stat["ccd.wavefront"] = 0;
     c.stat["ccd.spilled"] = 0;
     c.stat["ccd.spilled_deep"] = 0;
