@@ -27,9 +27,12 @@ namespace ipcg {
 
 namespace {
 
-// Device bytes a batched context holds per triangle and per vertex of its
-// scenes during a full step (collision build, energy, gradient, Hessian,
-// CCD), measured on sheet pairs and icosphere rows.
+// Estimate of the device bytes a batched context holds per triangle and per
+// vertex of its scenes through a full step (collision build, energy, gradient,
+// Hessian, CCD), for a mix of scenes in and out of contact.  Measured over the
+// estimate: 64 mixed scenes 0.91, 16 of them 0.45, rows of icospheres 0.25 to
+// 0.5, pairs of aligned sheets, in contact everywhere, 1.8 to 2.1 (and where
+// searches advance level by level, up to 0.1 GB whatever the size).
 constexpr int64_t BYTES_PER_TRI = 4096;
 constexpr int64_t BYTES_PER_VERTEX = 1024;
 

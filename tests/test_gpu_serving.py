@@ -123,3 +123,21 @@ def test_scene_beyond_the_budget_is_refused(capi, scenes):
         srv.run()
     assert e.value.code == capi.ERR_OOM
     srv.close()
+
+
+@pytest.mark.parametrize("rows", [[(2, 3)], [(8, 4)], [(16, 4)], [(2, 3), (8, 4), (3, 5)]])
+def test_scenes_hold_less_than_their_estimate(ctx, scenes, rows):
+    """rows of icospheres touch in few places: no fixed reserve of a context
+    may outweigh what the admission estimates for them"""
+    B = scenes.Batch([scenes.sphere_chain(c, sub, seed=3) for c, sub in rows])
+    ctx.upload_batch(B)
+    ctx.upload_positions(0, B.V)
+    ctx.upload_positions(1, B.V1)
+    ctx.build_collisions(DHAT)
+    ctx.energy_batched(DHAT, KAPPA)
+    ctx.gradient(DHAT, KAPPA, download=False)
+    ctx.hessian(DHAT, KAPPA, "clamp", download=False)
+    ctx.stepsize_batched()
+    nV, _, nF = B.sizes
+    say("rows", rows, ctx.device_bytes(), 4096 * nF + 1024 * nV)
+    assert ctx.device_bytes() <= 0.8 * (4096 * nF + 1024 * nV)
