@@ -241,8 +241,7 @@ def batched_form(args, capi, scenes):
     batched_step(ctx, dhat, kappa)  # warm-up: buffers reach their size, shapes are tuned
     progress("batched form: warm-up step done")
     shapes = {st: ctx.launch_shape(st)[0] for st in
-              ("bp_traverse_ee.static", "bp_traverse_fv.static", "bp_traverse_ee.swept",
-               "bp_traverse_fv.swept")}
+              ("bp_traverse_both.static", "bp_traverse_both.swept")}
     lat = []
     for _ in range(max(1, args.batch_steps)):
         t0 = time.perf_counter()

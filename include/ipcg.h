@@ -59,13 +59,15 @@ void* ipcg_ctx_stream(ipcg_ctx* ctx);
 /* bytes of device memory the context holds (its buffers only grow) */
 int ipcg_ctx_device_bytes(ipcg_ctx* ctx, int64_t* bytes);
 /* Launch-shape autotuning (no reference counterpart): with enable != 0,
- * the first broad phase of each kind ("bp_traverse_ee.static",
- * "bp_traverse_fv.static", "bp_traverse_ee.swept", "bp_traverse_fv.swept")
- * times the LBVH traversal at 64, 128 and 256 lanes per workgroup on the
- * real input and keeps the fastest for the context; results do not depend
- * on the choice.  Off (the default, and after turning it off): 128.
- * ipcg_launch_shape reports a stage's chosen size (0: not tuned) and its
- * measured time in milliseconds (ms may be NULL). */
+ * the first broad phase of each kind times the LBVH traversal at 64, 128 and
+ * 256 lanes per workgroup on the real input and keeps the fastest for the
+ * context; results do not depend on the choice.  Off (the default, and
+ * after turning it off): 128.  Edge-edge and face-vertex walks share a
+ * launch ("bp_traverse_both.static", "bp_traverse_both.swept"; a mesh without
+ * faces has "bp_traverse_ee.*" alone).  ipcg_launch_shape reports a stage's
+ * chosen size (0: not tuned) and its measured time in milliseconds (ms may be
+ * NULL); "bp_traverse_ee.*" and "bp_traverse_fv.*" answer for the launch that
+ * holds their walk. */
 int ipcg_ctx_set_autotune(ipcg_ctx* ctx, int enable);
 int ipcg_launch_shape(ipcg_ctx* ctx, const char* stage, int32_t* block, double* ms);
 
@@ -465,7 +467,13 @@ ipcg_ctx* ipcg_server_context(ipcg_server* srv);
 /* ---- timing of the last call's kernels (for benchmarks) ----------------- */
 /* Kernel time of named stages recorded with HIP events on the context
  * stream since the last reset; names are stage names, ms in milliseconds.
- * Returns the number of stages (up to max). */
+ * Returns the number of stages (up to max).  A stage is a launch or a few, so
+ * the names follow the launches: the walks of a broad phase are
+ * "bp_traverse_both" (".static" or ".swept" after every broad phase name),
+ * Hessian records of all kinds "hessian_records" with
+ * "hessian_records.mollified" for edge pairs under their mollifier, CCD
+ * searches "ccd_lds", "ccd_sub", "ccd_wave", "ccd_wide", "ccd_block" and
+ * "ccd_wavefront". */
 int ipcg_stage_times(ipcg_ctx* ctx, int max, const char** names, double* ms,
                      int64_t* calls);
 int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);

@@ -960,15 +960,15 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(TraverseArgs a)
 // from L2 (large ones).  With the wave's queue and the shared subtrees,
 // static walks of 4 sheets of 97^2 go from 0.395 + 0.292 to 0.138 ms, of
 // 8 sheets of 512^2 from 8.35 + 3.09 to 8.33 ms.
-template <int SWEPT>
-__global__ __launch_bounds__(TR_BLOCK) void k_traverse_both(TraverseArgs ee, TraverseArgs fv,
-                                                            unsigned nb_ee)
+template <int SWEPT, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_traverse_both(TraverseArgs ee, TraverseArgs fv,
+                                                         unsigned nb_ee)
 {
-    __shared__ TrShared<TR_BLOCK> m;
+    __shared__ TrShared<BLOCK> m;
     if (blockIdx.x < nb_ee)
-        traverse<TR_EE, TR_BLOCK>(ee, xcd_block(blockIdx.x, nb_ee), m);
+        traverse<TR_EE, BLOCK>(ee, xcd_block(blockIdx.x, nb_ee), m);
     else
-        traverse<TR_FV, TR_BLOCK>(fv, xcd_block(blockIdx.x - nb_ee, gridDim.x - nb_ee), m);
+        traverse<TR_FV, BLOCK>(fv, xcd_block(blockIdx.x - nb_ee, gridDim.x - nb_ee), m);
 }
 
 unsigned traverse_blocks(int64_t nq, int qw, int block)
@@ -1028,18 +1028,39 @@ template <int MODE, int SWEPT> void launch_traverse(int block, const TraverseArg
     else launch_traverse_b<MODE, SWEPT, TR_BLOCK>(a, s);
 }
 
+template <int SWEPT, int BLOCK>
+void launch_both_b(const TraverseArgs& ee, const TraverseArgs& fv, hipStream_t s)
+{
+    const unsigned nb_ee = traverse_blocks(ee.nq, ee.qw, BLOCK),
+                   nb_fv = traverse_blocks(fv.nq, fv.qw, BLOCK);
+    hipLaunchKernelGGL((k_traverse_both<SWEPT, BLOCK>), dim3(nb_ee + nb_fv), dim3(BLOCK), 0, s, ee,
+                       fv, nb_ee);
+}
+
+template <int SWEPT>
+void launch_both(int block, const TraverseArgs& ee, const TraverseArgs& fv, hipStream_t s)
+{
+    if (block == 64) launch_both_b<SWEPT, 64>(ee, fv, s);
+    else if (block == 256) launch_both_b<SWEPT, 256>(ee, fv, s);
+    else launch_both_b<SWEPT, TR_BLOCK>(ee, fv, s);
+}
+
 constexpr int TUNE_BLOCKS[3] = { 64, 128, 256 };
 
 // One traversal launch with the workgroup size tuned for this context: on
 // the first call of `stage` with autotuning on, every size runs once on the
-// real input (its output is discarded by resetting the list's shard
-// counters) and the fastest, by HIP events on the context stream, is kept.
-// Candidate sets do not depend on the size.
+// real input (its output is discarded by clearing the lists' shard counters,
+// `sets` of them from cnt) and the fastest, by HIP events on the context
+// stream, is kept.  Candidate sets do not depend on the size.
 template <class Launch>
-void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, unsigned* claimed,
-                    Launch&& launch)
+void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, int sets,
+                    unsigned* claimed, Launch&& launch)
 {
     hipStream_t s = c.stream;
+    auto clear = [&]() {
+        IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES * (size_t)sets, s));
+        IPCG_HIP(hipMemsetAsync(claimed, 0, sizeof(unsigned), s));
+    };
     auto it = c.launch_block.find(stage);
     int block = it != c.launch_block.end() ? it->second : 0;
     if (block == 0 && c.autotune) {
@@ -1048,8 +1069,7 @@ void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, u
         IPCG_HIP(hipEventCreate(&e1));
         float best = INFINITY;
         for (int b : TUNE_BLOCKS) {
-            IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES, s));
-            IPCG_HIP(hipMemsetAsync(claimed, 0, sizeof(unsigned), s));
+            clear();
             IPCG_HIP(hipEventRecord(e0, s));
             launch(b);
             IPCG_HIP(hipEventRecord(e1, s));
@@ -1065,8 +1085,7 @@ void tuned_traverse(Ctx& c, const std::string& stage, unsigned long long* cnt, u
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         c.launch_block[stage] = block;
-        IPCG_HIP(hipMemsetAsync(cnt, 0, SHARD_CNT_BYTES, s));
-        IPCG_HIP(hipMemsetAsync(claimed, 0, sizeof(unsigned), s));
+        clear();
     }
     launch(block ? block : TR_BLOCK);
 }
@@ -1508,8 +1527,6 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
     DevBuf* final_list[4] = { &c.cand_ee, &c.cand_fv, &c.cand_vv, &c.cand_ev };
     int64_t* final_n[4] = { &c.n_ee, &c.n_fv, &c.n_vv, &c.n_ev };
     const int lists = codim ? 4 : 2;
-    // one launch for both walks, unless the launch shapes are being tuned
-    const bool both = !c.autotune && c.nE >= 2 && c.nF >= 1;
     const int qw = wave_queries((int64_t)c.nE + c.nV);
     const int64_t lanes = walk_lanes(c.nE, qw) + walk_lanes(c.nV, qw)
         + (codim ? 2 * walk_lanes(c.n_cv, qw) : 0);
@@ -1556,34 +1573,20 @@ void bp_build(Ctx& c, bool swept, double inflation, int method)
                                     nullptr, c.cand_stage[1].as<int2>(), S1, deep, claimed,
                                     slots, status,
                                     forest_args(c, c.tf), qw };
-            if (both) {
-                const unsigned nb_ee = traverse_blocks(c.nE, qw, TR_BLOCK),
-                               nb_fv = traverse_blocks(c.nV, qw, TR_BLOCK);
+            if (c.nE >= 1 && c.nF >= 1) { // (a face brings its edges)
                 c.stage_begin("bp_traverse_both");
-                if (swept)
-                    hipLaunchKernelGGL(k_traverse_both<1>, dim3(nb_ee + nb_fv), dim3(TR_BLOCK), 0,
-                                       s, ee, fv, nb_ee);
-                else
-                    hipLaunchKernelGGL(k_traverse_both<0>, dim3(nb_ee + nb_fv), dim3(TR_BLOCK), 0,
-                                       s, ee, fv, nb_ee);
+                tuned_traverse(c, "bp_traverse_both" + tag, cnt[0], 2, claimed, [&](int b) {
+                    if (swept) launch_both<1>(b, ee, fv, s);
+                    else launch_both<0>(b, ee, fv, s);
+                });
                 c.stage_end();
-            } else {
-                if (c.nE >= 2) {
-                    c.stage_begin("bp_traverse_ee");
-                    tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], claimed, [&](int b) {
-                        if (swept) launch_traverse<TR_EE, 1>(b, ee, s);
-                        else launch_traverse<TR_EE, 0>(b, ee, s);
-                    });
-                    c.stage_end();
-                }
-                if (c.nF >= 1) {
-                    c.stage_begin("bp_traverse_fv");
-                    tuned_traverse(c, "bp_traverse_fv" + tag, cnt[1], claimed, [&](int b) {
-                        if (swept) launch_traverse<TR_FV, 1>(b, fv, s);
-                        else launch_traverse<TR_FV, 0>(b, fv, s);
-                    });
-                    c.stage_end();
-                }
+            } else if (c.nE >= 2) {
+                c.stage_begin("bp_traverse_ee");
+                tuned_traverse(c, "bp_traverse_ee" + tag, cnt[0], 1, claimed, [&](int b) {
+                    if (swept) launch_traverse<TR_EE, 1>(b, ee, s);
+                    else launch_traverse<TR_EE, 0>(b, ee, s);
+                });
+                c.stage_end();
             }
         }
         if (codim) {

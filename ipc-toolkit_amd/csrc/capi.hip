@@ -579,10 +579,16 @@ int ipcg_launch_shape(ipcg_ctx* ctx, const char* stage, int32_t* block, double* 
 {
     return guard(ctx, [&](Ctx& c) {
         if (!stage || !block) throw Error(IPCG_ERR_ARG, "null argument");
-        auto it = c.launch_block.find(stage);
+        std::string name = stage;
+        auto it = c.launch_block.find(name);
+        for (const char* walk : { "bp_traverse_ee.", "bp_traverse_fv." })
+            if (it == c.launch_block.end() && name.rfind(walk, 0) == 0) {
+                name = "bp_traverse_both." + name.substr(std::strlen(walk)); // the launch that holds it
+                it = c.launch_block.find(name);
+            }
         *block = it == c.launch_block.end() ? 0 : it->second;
         if (ms) {
-            auto t = c.tune_ms.find(std::string(stage) + "@" + std::to_string(*block));
+            auto t = c.tune_ms.find(name + "@" + std::to_string(*block));
             *ms = t == c.tune_ms.end() ? 0.0 : (double)t->second;
         }
     });

@@ -1,7 +1,7 @@
 """Tree walks: waves that start with 8, 16 or 64 queries, subtrees handed
 between lanes, the queue of overlapping leaves and edge-edge beside
 face-vertex walks in one launch, against the oracle's candidates and the
-separate launches of the autotuned path.  Candidate sets are exact."""
+launches of the autotuned path.  Candidate sets are exact."""
 import numpy as np
 import pytest
 
@@ -82,3 +82,29 @@ def test_spill_stacks(ctx, O, spokes, least):
         ee, fv = check(ctx, O, V, E, F, 1e-12)
         assert len(ee) >= 18 * 2 * spokes and len(fv) == 0
         assert ctx.counter("bp.spill_stacks") >= least
+
+
+def test_tuned_walks_share_a_launch(ctx, scenes):
+    """the tuner chooses the workgroup size of the launch that holds both
+    walks; the names of the walks answer for it"""
+    s = scenes.two_sheets(40, seed=3)
+    ctx.upload_mesh(s.V, s.E, s.F)
+    ctx.upload_positions(0, s.V)
+    ctx.set_autotune(True)
+    for _ in range(2):
+        ctx.timing(True)
+        ctx.broad_phase(False, 0.5 * s.dhat)
+        names = set(ctx.stage_times())
+        ctx.timing(False)
+        print("stages", sorted(names), flush=True)
+        assert "bp_traverse_both.static" in names and "bp_traverse_ee.static" not in names
+    b, ms = ctx.launch_shape("bp_traverse_both.static")
+    assert b in (64, 128, 256) and ms > 0
+    assert ctx.launch_shape("bp_traverse_ee.static") == (b, ms)
+    assert ctx.launch_shape("bp_traverse_fv.static") == (b, ms)
+    assert ctx.launch_shape("bp_traverse_both.swept")[0] == 0
+    # a mesh without faces: the edge-edge walk by itself
+    ctx.upload_mesh(s.V, s.E, s.F[:0])
+    ctx.upload_positions(0, s.V)
+    ctx.broad_phase(False, 0.5 * s.dhat)
+    assert ctx.launch_shape("bp_traverse_ee.static")[0] in (64, 128, 256)
