@@ -120,10 +120,10 @@ struct CCDArgs {
     double* bound;         // running minimum (double bits), one per scene
     double* expect;        // expected minimum, one per scene (null: none)
     int* restarted;        // one per scene: a search handed on by a group tier restarted
-    const uint8_t* redo;   // one per scene (null: all): search these only (LDS tier)
     const int32_t* vscene; // batched contexts: scene per vertex (null: one scene)
     double* toi_out;       // per-candidate toi (null: not recorded)
     int* any_hit;          // early exit flag (null: no early exit)
+    const uint8_t* redo;   // one per scene (null: all): search these only (LDS tier)
 };
 
 __device__ __forceinline__ void atomic_min_nonneg(double* p, double v)
