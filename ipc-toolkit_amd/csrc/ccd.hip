@@ -44,6 +44,7 @@
 #include "ti.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 
@@ -57,6 +58,12 @@ constexpr int LDS_CAP = 6;
 // 4.9 ms without, 4.7 at 32, 4.5 at 24, 4.5 at 16; two 193 x 193 sheets 2.9,
 // 2.9, 2.9 and 3.3)
 constexpr long LDS_BUDGET = 24;
+// Up to this many searches: past it (batches of hundreds of scenes) the tiers
+// above are as busy as this one, and 16 lanes spend more on a search of 25 to 100
+// boxes than one lane does.  LDS, sub-wave and wave tier with and without the
+// budget: 17 M searches of the 8 x 512 x 512 stack 5.5 and 5.9 ms, 56 M of 64
+// batch scenes 160 and 147, 194 M of 256 scenes 613 and 571.
+constexpr int64_t BUDGET_SEARCHES = 1 << 25;
 // Tiers above the LDS lists.  Their searches are chains of ~40 dependent
 // levels of a few boxes (median 5 a level on nearly parallel sheets, 18,000
 // at most below the expected minimum), so each tier gives a search the lanes
@@ -309,7 +316,7 @@ struct TIStrategy {
 // phase of the search; the others return at once)
 __global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo, int64_t n_todo,
                                                 uint32_t* spill, unsigned long long* n_spill,
-                                                int64_t ci_lo, int64_t ci_hi)
+                                                int64_t ci_lo, int64_t ci_hi, long budget)
 {
     __shared__ unsigned long long lists[3 * LDS_CAP * CB];
     const int64_t k = (int64_t)xcd_block() * CB + threadIdx.x;
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(CB) void k_ccd_lds(CCDArgs A, const uint32_t* todo,
     TIStrategy T(A, sc, eff, adj);
     int r;
     for (;;) {
-        r = ti_bfs_lds(q, T.delta, T.ms, T.max_iter, T.B, L, LDS_BUDGET, toi);
+        r = ti_bfs_lds(q, T.delta, T.ms, T.max_iter, T.B, L, budget, toi);
         if (!T.next(A, r, toi)) break;
         TIScale scale; // gathered again: too rare to keep
         (void)candidate_setup(A, ci, q, scale, eff, adj, sc);
@@ -1183,7 +1190,8 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
     auto lds_tier = [&](int64_t ci_lo, int64_t ci_hi, uint32_t* spill, int n_spill) {
         c.stage_begin("ccd_lds");
         hipLaunchKernelGGL(k_ccd_lds, dim3((unsigned)((n_todo + CB - 1) / CB)), dim3(CB), 0, s, A,
-                           c.ccd_todo.as<uint32_t>(), n_todo, spill, cnt + n_spill, ci_lo, ci_hi);
+                           c.ccd_todo.as<uint32_t>(), n_todo, spill, cnt + n_spill, ci_lo, ci_hi,
+                           n_todo <= BUDGET_SEARCHES ? LDS_BUDGET : LONG_MAX);
         IPCG_CHECK_LAUNCH();
         c.stage_end();
     };

@@ -87,3 +87,23 @@ def test_lists_past_lds_are_reserved_when_asked_for(ctx, O, scenes):
     upload(ctx, s)
     assert ctx.stepsize() == O.compute_collision_free_stepsize(s.V, s.V1, s.E, s.F)
     assert "slabs" in reached(ctx) and ctx.device_bytes() > small + (32 << 20)
+
+
+def test_more_searches_than_the_box_budget_is_for(ctx, capi, scenes):
+    """past 2^25 searches a lane's search is not cut at 24 boxes; the steps are
+    those of each scene alone"""
+    B = scenes.Batch(scenes.batch_scenes(48, seed=0))
+    say("batch", len(B.scenes), B.sizes)
+    ctx.upload_batch(B)
+    ctx.upload_positions(0, B.V)
+    ctx.upload_positions(1, B.V1)
+    steps = ctx.stepsize_batched()
+    assert ctx.counter("ccd.searched") > 1 << 25
+    alone = capi.Context(0)
+    try:
+        for k in np.argsort([len(s.F) for s in B.scenes])[::5]:
+            upload(alone, B.scenes[k])
+            assert alone.stepsize() == steps[k], k
+            assert alone.counter("ccd.searched") < 1 << 25
+    finally:
+        alone.close()
