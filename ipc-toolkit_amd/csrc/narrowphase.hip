@@ -445,38 +445,10 @@ template <int N, class W> __device__ __forceinline__ double network_sum(uint32_t
     return nan ? NAN : sum; // NaN contributions have no place in the order
 }
 
-// Repeated minimum scan, for runs that outgrow the other ways.
-template <class W> __device__ double scan_sum(uint32_t s, uint32_t e, W wt)
-{
-    double sum = 0.0, last = 0.0;
-    uint32_t done = 0;
-    bool first = true;
-    while (done < e - s) {
-        double v = INFINITY;
-        uint32_t c = 0;
-        for (uint32_t j = s; j < e; j++) {
-            const double x = wt(j);
-            if (!first && !(x > last)) continue;
-            if (c == 0 || x < v) {
-                v = x;
-                c = 1;
-            } else if (x == v) {
-                c++;
-            }
-        }
-        if (c == 0) return NAN; // NaN contributions have no place in the order
-        for (uint32_t t = 0; t < c; t++) sum += v;
-        done += c;
-        last = v;
-        first = false;
-    }
-    return sum;
-}
-
 // Sum of a run of n <= RUN_WAVE values by the wave: every value's rank by
 // comparison with the others in LDS (buf: 2 RUN_WAVE doubles), then the sum
 // of the ranked values.  All lanes call it, with the same run.
-constexpr uint32_t RUN_WAVE = 512;
+constexpr uint32_t RUN_WAVE = 128;
 
 template <class W>
 __device__ __forceinline__ double wave_sum(uint32_t s, uint32_t n, W wt, double* buf)
@@ -494,11 +466,13 @@ __device__ __forceinline__ double wave_sum(uint32_t s, uint32_t n, W wt, double*
     for (uint32_t j = l; j < n; j += WAVE) {
         const double x = buf[j];
         uint32_t rank = 0;
+#pragma unroll 8
         for (uint32_t k = 0; k < n; k++) rank += buf[k] < x || (buf[k] == x && k < j) ? 1u : 0u;
         by_rank[rank] = x;
     }
     wave_lds_fence();
     double sum = 0.0;
+#pragma unroll 8
     for (uint32_t k = 0; k < n; k++) sum += by_rank[k];
     wave_lds_fence();
     return sum;
@@ -507,37 +481,105 @@ __device__ __forceinline__ double wave_sum(uint32_t s, uint32_t n, W wt, double*
 // Sum of wt(j), j in [s, e) (none where s == e), taken in ascending order of
 // value (equal values in any order): the same double whatever order the
 // contributions arrived in.  All lanes of the wave call it.  Runs up to 16
-// go through a network in the lane's registers, longer ones are taken by the
-// wave one after the other; a minimum scan by each lane, e - s passes of dependent
-// loads, took 1.10 ms for the two launches of the area-weighted merge of 5 sheets of
-// 127^2, now 0.24.
-template <class W> __device__ __forceinline__ double sorted_sum(uint32_t s, uint32_t e, W wt, double* buf)
+// go through a network in the lane's registers, those up to RUN_WAVE are taken by
+// the wave one after the other, longer ones are left to k_long_runs (`left`).  A
+// minimum scan by each lane, e - s passes of dependent loads, took 1.10 ms for
+// the two launches of the area-weighted merge of 5 sheets of 127^2, now 0.24.
+template <class W>
+__device__ __forceinline__ double sorted_sum(uint32_t s, uint32_t e, W wt, double* buf, bool& left)
 {
     const uint32_t n = e - s;
     double sum = n <= 16 ? network_sum<16>(s, n, wt) : 0.0;
-    unsigned long long more = __ballot(n > 16);
+    left = n > RUN_WAVE;
+    unsigned long long more = __ballot(n > 16 && !left);
     while (more) {
         const int src = __ffsll(more) - 1;
         more &= more - 1;
         const uint32_t rs = __builtin_amdgcn_readlane(s, src), rn = __builtin_amdgcn_readlane(n, src);
-        double w;
-        if (rn <= RUN_WAVE) w = wave_sum(rs, rn, wt, buf);
-        else w = scan_sum(rs, rs + rn, wt);
+        const double w = wave_sum(rs, rn, wt, buf);
         if (lane_id() == src) sum = w;
     }
     return sum;
 }
 
+// Runs of more than RUN_WAVE contributions (vertices of high degree that touch),
+// listed by the kernels below: a workgroup each, ranks by comparison against
+// tiles in LDS, then the ranked values in order.  Collision merge of 400 pairs of
+// apexes of 24 (12) triangles: 110 (7.8) ms with a minimum scan by each lane,
+// 3.8 s (1.8 ms) with a wave's runs one after the other, 0.5 (0.24) ms now.
+struct LongRuns {
+    uint32_t* n;        // per kind: runs listed
+    uint32_t* list[3];
+    const uint32_t *start[3], *perm[3];
+    const double* cw[2];
+    const EERec* ee;
+    double* ranked[3];  // room for a kind's contributions
+    double* rw[3];
+    uint32_t* keep[3];
+};
+constexpr int LR_BLOCK = 1024;
+
+__device__ __forceinline__ void list_long_run(const LongRuns& L, int kind, bool left, int64_t i)
+{
+    if (left) L.list[kind][atomicAdd(L.n + kind, 1u)] = (uint32_t)i;
+}
+
+__global__ __launch_bounds__(LR_BLOCK) void k_long_runs(LongRuns L)
+{
+    __shared__ double tile[LR_BLOCK];
+    const int kind = blockIdx.y, t = threadIdx.x;
+    const uint32_t runs = L.n[kind];
+    const uint32_t* const perm = L.perm[kind];
+    auto wt = [&](uint32_t j) { return kind == 2 ? L.ee[perm[j]].w : L.cw[kind][perm[j]]; };
+    for (uint32_t q = blockIdx.x; q < runs; q += gridDim.x) {
+        const uint32_t i = L.list[kind][q], s = L.start[kind][i], n = L.start[kind][i + 1] - s;
+        double* const ranked = L.ranked[kind] + s;
+        bool nan = false;
+        for (uint32_t j0 = 0; j0 < n; j0 += LR_BLOCK) {
+            const uint32_t j = j0 + t;
+            const double x = j < n ? wt(s + j) : 0.0;
+            nan |= x != x;
+            uint32_t rank = 0;
+            for (uint32_t k0 = 0; k0 < n; k0 += LR_BLOCK) {
+                __syncthreads(); // the tile has been read
+                tile[t] = k0 + t < n ? wt(s + k0 + t) : 0.0;
+                __syncthreads();
+                const uint32_t m = n - k0 < (uint32_t)LR_BLOCK ? n - k0 : (uint32_t)LR_BLOCK;
+                for (uint32_t k = 0; k < m; k++)
+                    rank += tile[k] < x || (tile[k] == x && k0 + k < j) ? 1u : 0u;
+            }
+            if (j < n && x == x) ranked[rank] = x; // (< n: NaN counts for no rank)
+        }
+        const bool any_nan = __syncthreads_or(nan);
+        double sum = 0.0;
+        for (uint32_t k0 = 0; k0 < n; k0 += LR_BLOCK) {
+            tile[t] = !any_nan && k0 + t < n ? ranked[k0 + t] : 0.0;
+            __syncthreads();
+            const uint32_t m = n - k0 < (uint32_t)LR_BLOCK ? n - k0 : (uint32_t)LR_BLOCK;
+            if (t == 0)
+                for (uint32_t k = 0; k < m; k++) sum += tile[k];
+            __syncthreads();
+        }
+        if (t == 0) {
+            const double w = any_nan ? (double)NAN : sum; // (as wave_sum)
+            L.rw[kind][i] = w;
+            L.keep[kind][i] = w != 0.0;
+        }
+    }
+}
+
 // real-valued merge of a vertex-vertex / edge-vertex run
 __global__ __launch_bounds__(256) void k_run_sums(const uint32_t* start, int64_t nu,
                                                   const uint32_t* perm, const double* cw,
-                                                  double* rw, uint32_t* keep)
+                                                  double* rw, uint32_t* keep, LongRuns L, int kind)
 {
     __shared__ double buf[256 / WAVE][2 * RUN_WAVE];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const uint32_t s = i < nu ? start[i] : 0, e = i < nu ? start[i + 1] : 0;
+    bool left;
     const double w = sorted_sum(s, e, [&](uint32_t j) { return cw[perm[j]]; },
-                                buf[threadIdx.x / WAVE]);
+                                buf[threadIdx.x / WAVE], left);
+    list_long_run(L, kind, left, i);
     if (i < nu) {
         rw[i] = w;
         keep[i] = w != 0.0;
@@ -556,13 +598,15 @@ __global__ void k_run_scatter(const uint64_t* ukeys, int64_t nu, const double* r
 
 __global__ __launch_bounds__(256) void k_ee_runs(const uint32_t* start, int64_t nu,
                                                  const uint32_t* perm, const EERec* r, double* rw,
-                                                 uint32_t* rep, uint32_t* keep)
+                                                 uint32_t* rep, uint32_t* keep, LongRuns L)
 {
     __shared__ double buf[256 / WAVE][2 * RUN_WAVE];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const uint32_t s = i < nu ? start[i] : 0, e = i < nu ? start[i + 1] : 0;
+    bool left;
     const double w = sorted_sum(s, e, [&](uint32_t j) { return r[perm[j]].w; },
-                                buf[threadIdx.x / WAVE]);
+                                buf[threadIdx.x / WAVE], left);
+    list_long_run(L, 2, left, i);
     if (i < nu) {
         uint32_t best = perm[s];
         for (uint32_t j = s + 1; j < e; j++)
@@ -1067,27 +1111,51 @@ void np_build(Ctx& c, double dhat, double dmin)
         int64_t nu[3];
         read_three(nu_dev, nu);
         uint32_t* const kept_dev = nu_dev + 3;
+        // long runs: the sorts' other buffers are free for the list and the
+        // ranked values
+        LongRuns L {};
+        L.n = reinterpret_cast<uint32_t*>(c.counters.as<unsigned long long>() + 12);
+        L.ee = M.ee;
+        int64_t longest_list = 0; // contributions of the largest kind
         for (int k = 0; k < 3; k++) {
             if (m[k] == 0) nu[k] = 0;
+            longest_list = std::max(longest_list, m[k]);
+            L.list[k] = jobs[k].in_alt ? jobs[k].vals : jobs[k].vals_alt;
+            L.start[k] = start[k];
+            L.perm[k] = perm[k];
+            if (k < 2) L.cw[k] = M.cw + M.off[k];
+            L.ranked[k] = static_cast<double*>(jobs[k].in_alt ? jobs[k].keys : jobs[k].keys_alt);
+            L.rw[k] = c.np_rw.as<double>() + M.off[k];
+            L.keep[k] = c.np_flag.as<uint32_t>() + M.off[k];
+        }
+        const bool may_be_long = longest_list > (int64_t)RUN_WAVE;
+        if (may_be_long) IPCG_HIP(hipMemsetAsync(L.n, 0, 3 * sizeof(uint32_t), s));
+        for (int k = 0; k < 3; k++) {
+            if (!nu[k]) continue;
             const unsigned gu = grid_for(nu[k], 256, INT32_MAX);
-            double* const rw = c.np_rw.as<double>() + M.off[k];
-            uint32_t* const flag = c.np_flag.as<uint32_t>() + M.off[k];
-            uint32_t* const pos = c.np_pos.as<uint32_t>() + M.off[k];
-            uint32_t* const rep = c.np_rep.as<uint32_t>() + M.off[k];
-            if (nu[k] && k == 2)
+            if (k == 2)
                 hipLaunchKernelGGL(k_ee_runs, dim3(gu), dim3(256), 0, s, start[k], nu[k], perm[k],
-                                   M.ee, rw, rep, flag);
-            else if (nu[k])
+                                   M.ee, L.rw[k], c.np_rep.as<uint32_t>() + M.off[k], L.keep[k], L);
+            else
                 hipLaunchKernelGGL(k_run_sums, dim3(gu), dim3(256), 0, s, start[k], nu[k], perm[k],
-                                   M.cw + M.off[k], rw, flag);
-            exclusive_scan_u32(c.sort_space, flag, pos, nu[k], kept_dev + k, s);
+                                   L.cw[k], L.rw[k], L.keep[k], L, k);
+        }
+        if (may_be_long)
+            hipLaunchKernelGGL(k_long_runs, dim3(128, 3), dim3(LR_BLOCK), 0, s, L);
+        IPCG_CHECK_LAUNCH();
+        for (int k = 0; k < 3; k++) {
+            const unsigned gu = grid_for(nu[k], 256, INT32_MAX);
+            uint32_t* const pos = c.np_pos.as<uint32_t>() + M.off[k];
+            exclusive_scan_u32(c.sort_space, L.keep[k], pos, nu[k], kept_dev + k, s);
             if (nu[k] && k == 2)
-                hipLaunchKernelGGL(k_ee_scatter, dim3(gu), dim3(256), 0, s, M.ee, nu[k], rw, rep,
-                                   flag, pos, c.c_ids[2].as<int2>(), c.c_w[2].as<double>(),
+                hipLaunchKernelGGL(k_ee_scatter, dim3(gu), dim3(256), 0, s, M.ee, nu[k], L.rw[k],
+                                   c.np_rep.as<uint32_t>() + M.off[k], L.keep[k], pos,
+                                   c.c_ids[2].as<int2>(), c.c_w[2].as<double>(),
                                    c.c_eps.as<double>(), c.c_dtype.as<int32_t>());
             else if (nu[k])
-                hipLaunchKernelGGL(k_run_scatter, dim3(gu), dim3(256), 0, s, ukeys[k], nu[k], rw,
-                                   flag, pos, c.c_ids[k].as<int2>(), c.c_w[k].as<double>());
+                hipLaunchKernelGGL(k_run_scatter, dim3(gu), dim3(256), 0, s, ukeys[k], nu[k],
+                                   L.rw[k], L.keep[k], pos, c.c_ids[k].as<int2>(),
+                                   c.c_w[k].as<double>());
             IPCG_CHECK_LAUNCH();
         }
         if (m[3])

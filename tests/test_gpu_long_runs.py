@@ -28,7 +28,7 @@ def fans(deg):
     return V, E, F
 
 
-# runs of up to 16, of a wave (up to 512) and longer
+# runs of up to 16, of a wave (up to 128) and longer
 @pytest.mark.parametrize("deg", [3, 4, 5, 12, 22, 24, 40])
 @pytest.mark.parametrize("improved", [False, True])
 def test_runs_of_every_length(ctx, capi, O, deg, improved):
@@ -43,3 +43,27 @@ def test_runs_of_every_length(ctx, capi, O, deg, improved):
     print("case", deg, improved, [len(co.vv), len(co.ev), len(co.ee), len(co.fv)], flush=True)
     assert len(co.vv) == 1
     assert_same_set(ctx.collisions(), co)
+
+
+@pytest.mark.parametrize("deg", [11, 12, 24])
+def test_many_long_runs(ctx, capi, O, deg):
+    """300 apex pairs of a run each at both sides of a wave's buffer, all of
+    them in a few waves: equal weights, and not one long run after the other (24
+    triangles an apex took 2.8 s then)"""
+    V0, E0, F0 = fans(deg)
+    n = 300
+    V = np.concatenate([V0 + [4.0 * (k % 20), 4.0 * (k // 20), 0] for k in range(n)])
+    E = np.concatenate([E0 + len(V0) * k for k in range(n)]).astype(np.int32)
+    F = np.concatenate([F0 + len(V0) * k for k in range(n)]).astype(np.int32)
+    ctx.upload_mesh(V, E, F)
+    ctx.upload_positions(0, V)
+    ctx.set_area_weighting(True)
+    ctx.build_collisions(DHAT)
+    ctx.timing(True)
+    ctx.build_collisions(DHAT)
+    ms = ctx.stage_times()["np_merge"][0]
+    ctx.timing(False)
+    got = ctx.collisions()
+    print("case many", ms, [len(got[k]) for k in ("vv", "ev", "ee", "fv")], flush=True)
+    assert_same_set(got, oracle_set(ctx, O, V, E, F, DHAT, aw=True, improved=False))
+    assert len(got["vv"]) == n and ms < 100
