@@ -840,11 +840,20 @@ __device__ __forceinline__ void traverse(const TraverseArgs& A, unsigned block,
     // TR_SHARE steps the idle ones take the oldest postponed child, the
     // largest subtree left, of a busy lane each and walk it with that lane's
     // query (9.4 to 8.4 ms there, 0.29 to 0.21 ms on 4 sheets of 97^2).
-    int sb = 0, sp = 0, steps = 0, round = 0;
+    int sb = 0, sp = 0, steps = 0;
+    unsigned round = 0;
     int pos = qpos; // of the query walked
     unsigned char* const donor = sh_mem.donor[t / WAVE];
     const int max_steps = 2 * nleaves + 64; // each node is visited at most once per query
+    // A subtree that changes lanes starts a count of its own, so the wave's rounds
+    // are bounded too: in each of them a query that started here visits a node.
+    const int64_t visits = (int64_t)A.qw * max_steps;
+    const unsigned max_rounds = visits < (int64_t)UINT32_MAX ? (unsigned)visits : UINT32_MAX;
     while (__any(active)) {
+        if (round == max_rounds) {
+            atomicOr(status, 2);
+            break;
+        }
         if (++round % TR_SHARE == 0) {
             const bool gives = active && sp > sb && sb < TR_LSTACK;
             const bool takes = !active;
