@@ -1,11 +1,11 @@
 """Broad phase and merge at the sizes where their launches change: arrays at
 the edges of one workgroup's sort (8192 keys), of the sort's tiles, of the
 refit's leaf ranges (1024 leaves, 64 of them) and a forest of uneven scenes.
-Sets and orientations must equal the oracle's."""
+Sets and orientations must equal the oracle's, on every call."""
 import numpy as np
 import pytest
 
-from conftest import pair_set
+from conftest import pair_set, sparse_rel_err
 from test_gpu_parity import say
 
 pytestmark = pytest.mark.gpu
@@ -40,11 +40,43 @@ def test_sets(ctx, O, n):
     for k in ("vv", "ev", "ee", "fv"):
         assert np.array_equal(got[k], getattr(want, k)), k
         assert np.array_equal(got[k + "_w"], getattr(want, k + "_w")), k
-    for method in (0, 1):  # repeated calls and the sweep reuse the same scratch
-        ctx.broad_phase(False, 0.5 * dhat, method)
-        ee2, fv2 = ctx.candidates()
-        assert len(ee2) <= len(ee) and len(fv2) <= len(fv)
-        assert {tuple(sorted(p)) for p in ee2.tolist()} <= {tuple(sorted(p)) for p in ee.tolist()}
+    # a repeated call and the sweep reuse the same scratch
+    ctx.broad_phase(False, 0.5 * dhat, 0)
+    again = ctx.candidates()
+    for a, b in ((again[0], ee), (again[1], fv)):
+        assert len(a) == len(b) and pair_set(a) == pair_set(b)
+    ctx.broad_phase(False, 0.5 * dhat, 1)
+    swept = ctx.candidates()
+    for a, b in zip(swept, O.candidates(V, E, F, 0.5 * dhat, method="sap")):
+        assert len(a) == len(b) and pair_set(a) == pair_set(b)
+
+
+# one context through arrays of every sort path, up and down in size: 64-bit
+# keys (trees, merges), 32-bit keys (incidences), scans and run lengths share
+# look-back words, ticket and histograms with the calls before
+@pytest.mark.parametrize("order", [[8193, 2, 21846, 1, 43691, 683, 8193],
+                                   [43691, 43691, 5, 2731, 341, 21845, 1024],
+                                   [1, 8193, 8193, 1, 8193, 2, 43691]])
+def test_scratch_across_calls(ctx, O, order):
+    for n in order:
+        V, E, F = soup(n)
+        say("case", order, n)
+        ctx.upload_mesh(V, E, F)
+        ctx.upload_positions(0, V)
+        dhat = 1.5e-3
+        eo, fo = O.candidates(V, E, F, 0.5 * dhat)
+        want = O.build_collisions(V, E, F, eo, fo, dhat)
+        Ho = O.barrier_hessian(want, V, E, F, dhat, 1e3, "clamp")
+        for _ in range(2):
+            ctx.build_collisions(dhat)
+            ee, fv = ctx.candidates()
+            assert len(ee) == len(eo) and pair_set(ee) == pair_set(eo)
+            assert len(fv) == len(fo) and pair_set(fv) == pair_set(fo)
+            got = ctx.collisions()
+            for k in ("vv", "ev", "ee", "fv"):
+                assert np.array_equal(got[k], getattr(want, k)), k
+                assert np.array_equal(got[k + "_w"], getattr(want, k + "_w")), k
+            assert sparse_rel_err(ctx.hessian(dhat, 1e3, "clamp"), Ho) <= 1e-10
 
 
 @pytest.mark.parametrize("sizes", [(1, 1, 1), (1, 400, 2), (342, 1, 5000, 1, 341), (22000, 3, 700)])
