@@ -1,5 +1,5 @@
 // Broad phase on the GPU: conservative boxes, 63-bit Morton codes, LBVH
-// (Apetrei 2014 single bottom-up pass) and candidate traversal.
+// (Karras 2012 hierarchy, boxes refit in three steps) and candidate traversal.
 //
 // Boxes follow aabb.cpp:35-126 (nextafter(p -/+ r) outward in FP64, unions
 // for edges and faces) and lbvh.cpp:29-41 (FP32 with one more outward ulp).
@@ -120,10 +120,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_mesh_aabb_final(const double* part
     }
 }
 
-// Batched contexts: the mesh box of each scene's vertex boxes, one
-// workgroup per scene (min / max are exact, so the box equals the one a
-// context holding the scene alone computes).
-// Scene boxes in two steps: workgroup (scene, chunk) reduces every
+// Batched contexts: scene boxes in two steps: workgroup (scene, chunk) reduces every
 // SCENE_CHUNKS-th stretch of the scene's vertices into a partial box, then a
 // lane per scene combines its partials (min / max are exact, so the box is
 // the one the scene alone gets).
@@ -574,14 +571,6 @@ __device__ __forceinline__ bool can_ee(const Filter& f, int ea, int eb)
     const int b0 = f.E[2 * (int64_t)eb], b1 = f.E[2 * (int64_t)eb + 1];
     if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return false;
     return can_vv(f, a0, b0) || can_vv(f, a0, b1) || can_vv(f, a1, b0) || can_vv(f, a1, b1);
-}
-
-// lbvh.cpp:800-807 can_edge_vertex_collide
-__device__ __forceinline__ bool can_ev(const Filter& f, int ei, int vi)
-{
-    const int e0 = f.E[2 * (int64_t)ei], e1 = f.E[2 * (int64_t)ei + 1];
-    if (vi == e0 || vi == e1) return false;
-    return can_vv(f, vi, e0) || can_vv(f, vi, e1);
 }
 
 // lbvh.cpp:851-858 can_face_vertex_collide

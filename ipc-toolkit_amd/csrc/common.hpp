@@ -91,14 +91,6 @@ __device__ __forceinline__ unsigned xcd_block() { return xcd_block(blockIdx.x, g
 // ---- wave64 helpers -------------------------------------------------------
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
-// exclusive prefix count of `pred` among lower lanes, and the wave total
-__device__ __forceinline__ unsigned wave_prefix(bool pred, unsigned& total)
-{
-    const unsigned long long m = __ballot(pred);
-    total = (unsigned)__popcll(m);
-    return (unsigned)__popcll(m & ((1ull << lane_id()) - 1ull));
-}
-
 // wave-aggregated append of `cnt` items; returns this lane's first slot
 __device__ __forceinline__ unsigned long long wave_append(unsigned long long* counter,
                                                           unsigned cnt)

@@ -402,8 +402,6 @@ struct ContactFrame {
     double y1, y2;
 };
 
-IPCG_HD d3 unit(const d3& v) { return scale(v, 1.0 / sqrt(sqn(v))); }
-
 // two axes completing the unit vector a (Duff et al., "Building an
 // Orthonormal Basis, Revisited", JCGT 2017)
 IPCG_HD void complement(const d3& a, d3& b, d3& c)

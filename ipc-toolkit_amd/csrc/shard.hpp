@@ -28,15 +28,10 @@ __device__ __forceinline__ int wave_shard()
     return (int)((blockIdx.x * wpb + threadIdx.x / WAVE) & (SHARDS - 1));
 }
 
-// Reserves `cnt` slots for this lane in shard `sh`; returns the first slot's
-// position inside the shard region (may be >= scap: the region overflowed,
-// the caller must not write and the host retries with a larger region).
-__device__ __forceinline__ unsigned long long shard_append(const Shards& S, int sh, unsigned cnt)
-{
-    return wave_append(S.cnt + (int64_t)sh * SHARD_PAD, cnt);
-}
-
-// Ballot form for lanes appending at most two items (a, then b).
+// Reserves a slot in shard `sh` for each lane with a set and one for each with b
+// set (a's item, then b's; `pre`: the lane's offset).  Returns the wave's first
+// position inside the shard region (positions >= scap: the region overflowed, the
+// caller must not write there and the host retries with a larger region).
 __device__ __forceinline__ unsigned long long shard_append_bits(const Shards& S, int sh, bool a,
                                                                 bool b, unsigned& pre)
 {

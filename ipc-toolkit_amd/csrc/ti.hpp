@@ -81,8 +81,10 @@ IPCG_HD double ti_corner(const TIQuery& q, int k, double t, double u, double v)
 // monotone in each operand, so the extremes over the corners of one t are
 // the same chain of operations over the extremes of the products: the same
 // doubles as the eight corners give, in about 55 operations an axis instead
-// of 75.  Where overflow, infinities or NaN occur (the range is not finite)
-// the corners are compared one by one.
+// of 75.  Where the range is not finite (overflow, infinities, NaN) the corners
+// are compared one by one; edges whose differences overflow to NaN at one t alone
+// show the other t's range, where their filter, which grows with the cube of the
+// coordinates, is infinite and takes the box either way.
 template <bool VF>
 IPCG_HD void ti_range(const TIQuery& q, int k, double t0, double t1, double u0, double u1,
                       double v0, double v1, double& mn, double& mx)
