@@ -48,11 +48,13 @@ PSD_FLOPS = {n: SWEEPS[n] * (n * (n - 1) // 2 * (12 * n + 7) + n * (n + 1))
 # Unmollified collision: the frame of the closest points (about 200 flops),
 # the 5 x 5 matrix and its projection, and the record from it (about 150).
 FRAME_FLOPS = 350 + PSD_FLOPS[5]
-# Tight-Inclusion: one box = the 8 corners of F along 3 axes (about 70 flops
-# per axis); a candidate that survives the root pass visits 5.0 boxes on
-# average on the sheet-stack workload (counted in-kernel).
-TI_BOX_FLOPS = 210
-TI_BOXES_PER_SEARCH = 5.0
+# Tight-Inclusion: one box = the extremes of the 8 corners of F along 3 axes,
+# from the extremes of the u and v products (about 55 flops per axis); the
+# one-lane search of a candidate that survives the root pass visits 5.1 boxes
+# on average on the sheet-stack workload (88.1 M for 17.35 M searches, counted
+# in-kernel).
+TI_BOX_FLOPS = 165
+TI_BOXES_PER_SEARCH = 5.1
 
 
 def parse():

@@ -957,7 +957,8 @@ __global__ __launch_bounds__(BLOCK) void k_traverse(TraverseArgs a)
 // (small scenes: two launches in a row take two of them) and by node reads
 // from L2 (large ones).  With the wave's queue and the shared subtrees,
 // static walks of 4 sheets of 97^2 go from 0.395 + 0.292 to 0.138 ms, of
-// 8 sheets of 512^2 from 8.35 + 3.09 to 8.33 ms.
+// 8 sheets of 512^2 from 8.35 + 3.09 to 8.33 ms (vertices off the grid; 9.5 ms
+// with the sheets exactly above each other).
 template <int SWEPT, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_traverse_both(TraverseArgs ee, TraverseArgs fv,
                                                          unsigned nb_ee)

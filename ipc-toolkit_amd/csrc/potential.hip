@@ -839,7 +839,8 @@ __device__ __forceinline__ void row_add(double* acc, uint32_t* msk, const double
 
 // full matrices among a wave's 64 incidences from which each lane expands
 // its own: one after the other they take about 1.5 us a pair (two aligned
-// sheets have dozens a row: the rows of 64 such scenes 11.9 -> 9.3 ms)
+// sheets have dozens a row: the rows of 64 such scenes 11.9 -> 9.3 ms, with
+// 4 the same, with 16 as without; 8 sheets of 512^2: 9.0 to 9.1 ms with any)
 constexpr int ROW_FULL = 8;
 
 // A full matrix by one lane, one block row r at a time, so few values are
@@ -898,6 +899,9 @@ __device__ __forceinline__ void row_add_full(const double* rec, const double* ex
 // LDS adds of a wave off one address.  The few full matrices are expanded by
 // the whole wave, a lane per entry of the four blocks: as a branch of each
 // lane they doubled the kernel's time (spills, and most waves hold one).
+// 20 M collisions of 8 sheets of 512^2: 8.95 ms with the 9 x 9 records, 8.3 now
+// where the vertices are off the grid; 8.6 and 8.9 where the sheets lie exactly
+// above each other (every Hessian call gains: 26.1 -> 17.8 ms there).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_hessian_rows(
     const double* rec, const double* ext, int64_t ee0, const uint32_t* vptr, const uint32_t* inc,
     const int4* inc_vtx, const uint32_t* bptr, const int32_t* bcol, int nV, double* bval,

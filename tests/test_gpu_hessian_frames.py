@@ -2,7 +2,8 @@
 expand them, against the CPU oracle: every stencil kind and edge-edge type,
 with and without a mollifier, one collision and rows of several column
 windows.  The bound is the contract's 1e-10 of the Frobenius norm (triangles
-are kept fat: a frame loses |u| |v| / |u x v| roundings)."""
+are kept fat: both sides lose |u| |v| / |u x v| roundings, the oracle's
+point-space derivatives as much as the frame)."""
 import numpy as np
 import pytest
 
