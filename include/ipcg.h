@@ -483,7 +483,7 @@ int ipcg_stage_times_reset(ipcg_ctx* ctx, int enable);
  * lists), "ccd.wavefront" (searches that outgrew a wave's lists too: a workgroup
  * or the level-by-level wavefront takes them), "ccd.past_sub" (searches that
  * outgrew a sub-wave's lists), "ccd.past_wide" (those of a wave with long
- * lists), "ccd.slabs" (searches whose lists left a workgroup's LDS),
+ * lists), "ccd.slabs" (searches that took lists past a workgroup's LDS),
  * "ccd.by_level" (searches that the level-by-level wavefront took),
  * "ccd.expected" (scenes, at most 1 in a plain context, for which a search cut
  * to its earliest boxes gave an expected minimum; iteration limits below the

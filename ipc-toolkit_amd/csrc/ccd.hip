@@ -83,6 +83,13 @@ constexpr int WIDE_GROUPS = 2304;
 constexpr int BLOCK_GROUPS = 256;
 constexpr int SLAB_CAP = 1 << 16;
 constexpr int SLABS = 32; // 1 MB each
+// slabs a context starts with: a single scene's step bound takes none or 1,
+// seldom 2 (23 where sheets are exactly aligned), 16 scenes in a batch up to 10.
+// The first bound of two 8 x 8 sheets takes 1.83 ms if none is there and the
+// tier runs twice, 1.43 ms with one; of 16 scenes (2.5 M searches) 10.6 ms with
+// 5, 9.8 ms with all.  A context of that many searches holds gigabytes.
+constexpr int SLABS_MIN = 1;
+constexpr int64_t SLABS_ALL = 1ll << 21; // searches
 // Where a tier's searches all fit the chip at once in the next tier, the
 // tier only adds its own longest search to the chain of launches:
 constexpr int64_t DIRECT_MAX = 4096; // searches: no LDS tier (1,021: 0.87 -> 0.14 ms)
@@ -1231,31 +1238,34 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         IPCG_CHECK_LAUNCH();
         c.stage_end();
     };
-    // The lists past LDS are reserved (42 MB) when a search first asks for
-    // them: most contexts never get there.
-    constexpr size_t SLAB_BYTES = sizeof(unsigned long long) * 2 * SLAB_CAP * (size_t)SLABS;
+    // The lists past LDS: SLABS_MIN (1.3 MB), and SLABS (42 MB) with SLABS_ALL
+    // searches or once searches have asked for more.
+    constexpr size_t SLAB_BYTES = sizeof(unsigned long long) * 2 * SLAB_CAP;
+    auto slabs = [&]() { return (int)std::min<size_t>(c.ccd_slab.bytes / SLAB_BYTES, SLABS); };
     auto block_tier = [&](const Searches& q, const Lists& to) {
         c.stage_begin("ccd_block");
         hipLaunchKernelGGL((k_ccd_group<BLOCK_NW, BLOCK_CAP>),
                            dim3((unsigned)std::min<int64_t>(n_todo, BLOCK_GROUPS)),
                            dim3(BLOCK_NW * WAVE), 0, s, A, q, to,
-                           TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB,
-                                     c.ccd_slab.p ? SLABS : 0, SLAB_CAP });
+                           TISlabs { c.ccd_slab.as<unsigned long long>(), cnt + N_SLAB, slabs(),
+                                     SLAB_CAP });
         IPCG_CHECK_LAUNCH();
         c.stage_end();
     };
-    // the workgroup tier, then a second time with slabs for the searches
-    // left over if one of them would have taken a slab; leaves the list for
-    // the wavefront in `last` (counts as read back)
+    // the workgroup tier, then a second time with all slabs for the searches
+    // left over if one of them found none; leaves the list for the wavefront
+    // in `last` (counts as read back)
     uint32_t* last = heavy;
     int n_last = N_HEAVY;
     auto block_tiers = [&]() {
+        c.ccd_slab.reserve(SLAB_BYTES * (n_todo < SLABS_ALL ? SLABS_MIN : SLABS));
         block_tier(Searches { wide, cnt + N_WIDE, over, cnt + N_OVER, WIDE_MIN, cnt + WORK_BLOCK,
                               true },
                    out(heavy, N_HEAVY));
         read_back();
-        if (c.ccd_slab.p || count(N_SLAB) == 0 || count(N_HEAVY) == 0) return;
-        c.ccd_slab.reserve(SLAB_BYTES);
+        if (slabs() == SLABS || count(N_SLAB) <= slabs() || count(N_HEAVY) == 0) return;
+        c.stat["ccd.slabs"] += slabs();
+        c.ccd_slab.reserve(SLAB_BYTES * SLABS);
         IPCG_HIP(hipMemsetAsync(cnt + N_SLAB, 0, sizeof(*cnt), s));
         last = over; // (the workgroups have read it)
         n_last = N_LAST;
@@ -1354,7 +1364,7 @@ double ccd_stepsize(Ctx& c, double min_distance, double tol, int64_t max_iter, d
         c.stat["ccd.wavefront"] += count(N_OVER);
         c.stat["ccd.past_sub"] += count(N_SUB_A) + count(N_SUB_B);
         c.stat["ccd.past_wide"] += count(N_WIDE);
-        if (c.ccd_slab.p) c.stat["ccd.slabs"] += std::min<int64_t>(count(N_SLAB), SLABS);
+        c.stat["ccd.slabs"] += std::min<int64_t>(count(N_SLAB), slabs());
         const int64_t nh = count(n_last);
         c.stat["ccd.by_level"] += nh;
         if (nh > 0) wavefront(last, nh);
